@@ -249,10 +249,13 @@ __device__ __forceinline__ uint32_t tile_window_bytes(int64_t d_sq, int NP, int 
   return left <= 0 ? 0u : (left > 0xFFFFFFFFll ? 0xFFFFFFFFu : (uint32_t)left);
 }
 
-// Fast path 1: pure integer epilogue with alpha, beta scalars and beta == 0 on a full tile with
-// 16-byte aligned columns: D = alpha * acc straight from the accumulator registers.  Lanes 0..31 of
-// a store hold 32 consecutive int32 of one D column (one 128-byte line), so no LDS staging is
-// needed; two instructions per output element.
+// Offset bit that puts a lane of a buffer store outside every window (the store is dropped): lanes past the end of P.
+constexpr int kStoreNowhere = (int)0x80000000;
+
+// Fast path 1: pure integer epilogue with alpha, beta scalars and beta == 0: D = alpha * acc straight from the accumulator
+// registers.  Lanes 0..31 of a store hold 32 consecutive int32 of one D column (one 128-byte line), so no LDS staging is
+// needed; two instructions per output element.  Tiles that hang over the end of P mask their lanes, columns past the end
+// fall outside the window.
 template <int WP, int WQ, int WTP, int WTQ>
 __device__ __forceinline__ void mfma_store_tile_i32(const MfmaParams &prm, v16i (&acc)[WTQ / 32][WTP / 32],
                                                     int p0, int q0, int NP, int NQ, int bt, int ialpha) {
@@ -269,7 +272,9 @@ __device__ __forceinline__ void mfma_store_tile_i32(const MfmaParams &prm, v16i 
   const int64_t corner = (int64_t)(q0 + wq * WTQ) * d_sq + (p0 + wp * WTP);
   int32_t *Dw = (int32_t *)g.D + g.d_sb * bt + corner;
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dw, 0, tile_window_bytes(d_sq, NP, NQ, corner, 4), 0x00020000);
-  const int voff = (4 * gsel * d_sq + lr) * 4;
+  int voff[TP];
+#pragma unroll
+  for (int b = 0; b < TP; b++) voff[b] = p0 + wp * WTP + b * 32 + lr < NP ? (4 * gsel * d_sq + lr) * 4 : kStoreNowhere;
   // alpha == 1 (the usual case) stores the accumulator registers as they are
   if (ialpha == 1) {
 #pragma unroll
@@ -278,7 +283,7 @@ __device__ __forceinline__ void mfma_store_tile_i32(const MfmaParams &prm, v16i 
       for (int v = 0; v < 16; v++) {
         const int soff = (a * 32 + 8 * (v >> 2) + (v & 3)) * d_sq * 4;  // uniform
 #pragma unroll
-        for (int b = 0; b < TP; b++) __builtin_amdgcn_raw_buffer_store_b32(acc[a][b][v], rs, voff, soff + b * 128, 0);
+        for (int b = 0; b < TP; b++) __builtin_amdgcn_raw_buffer_store_b32(acc[a][b][v], rs, voff[b], soff + b * 128, 0);
       }
   } else {
 #pragma unroll
@@ -288,7 +293,7 @@ __device__ __forceinline__ void mfma_store_tile_i32(const MfmaParams &prm, v16i 
         const int soff = (a * 32 + 8 * (v >> 2) + (v & 3)) * d_sq * 4;
 #pragma unroll
         for (int b = 0; b < TP; b++)
-          __builtin_amdgcn_raw_buffer_store_b32(acc[a][b][v] * ialpha, rs, voff, soff + b * 128, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(acc[a][b][v] * ialpha, rs, voff[b], soff + b * 128, 0);
       }
   }
 }
@@ -314,107 +319,21 @@ __device__ __forceinline__ void mfma_store_tile_raw(int32_t *ws_tile, int ws_pit
     }
 }
 
-// Fast path 2: float epilogue without a C read (beta == 0) on a full tile, D of type bf16, f16 or
-// f32 with aligned columns.  The accumulators are staged through LDS so that a lane owns four
-// consecutive elements of a D column (8- or 16-byte stores, 256/512 contiguous bytes per column and
-// instruction).  Everything that does not change inside the inner loop is hoisted; the loop body is
-// one ds_read_b128, the arithmetic and one store.
-template <int KIND, int WP, int WQ, int WTP, int WTQ, int ACT, int DT, class AccV>
-__device__ __forceinline__ void mfma_store_tile_f(const MfmaParams &prm, AccV (&acc)[WTQ / 32][WTP / 32],
-                                                  int *lds_words, int p0, int q0, int NP, int NQ, int bt) {
-  constexpr int TP = WTP / 32, TQ = WTQ / 32;
-  constexpr int SROW = WTP + 8, LPR = WTP / 4, RPI = 64 / LPR, ITER = 16 / RPI;
-  static_assert(16 % RPI == 0, "whole passes");
-  constexpr int ESZ = DT == 2 ? 4 : 2;
-  const GemmArgs &g = prm.g;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wp = wave % WP, wq = wave / WP;
-  const int lr = lane & 31, gsel = lane >> 5;
-  int *stage = lds_words + wave * (16 * SROW);
-  Epilogue ep(g, bt);
-  const bool swp = prm.swapped != 0;
-  const int pl = (lane % LPR) * 4, qsub = lane / LPR;
-  const int pi0 = p0 + wp * WTP + pl;
-  float p_scale[4], p_bias[4];
-#pragma unroll
-  for (int e = 0; e < 4; e++) {
-    p_scale[e] = swp ? ep.col_scale(pi0 + e) : ep.row_scale(pi0 + e);
-    p_bias[e] = swp ? 0.0f : ep.bias_at(pi0 + e);
-  }
-  // vectors that run along Q (per-column scale, or per-row quantities of a row-major D)
-  const bool q_vec = swp ? (ep.alpha_v || ep.sa_v || g.bias) : (ep.sb_v != nullptr);
-  const float q_scale_u = swp ? ep.row_scale(0) : ep.col_scale(0);  // used when !q_vec
-  const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < 2^22 (checked by the dispatcher)
-  // buffer stores: uniform descriptor at the wave tile, per-lane byte offset (row qsub, column pl)
-  const int64_t corner = (int64_t)(q0 + wq * WTQ) * d_sq + (p0 + wp * WTP);
-  char *Dw = (char *)g.D + (g.d_sb * bt + corner) * ESZ;
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dw, 0, tile_window_bytes(d_sq, NP, NQ, corner, ESZ), 0x00020000);
-  const int voff = (qsub * d_sq + pl) * ESZ;
-  const int read_off = qsub * SROW + pl;
-
-  auto do_pass = [&](auto pass_c) {
-    constexpr int pass = decltype(pass_c)::value;
-    constexpr int a = pass >> 1, h = pass & 1;
-#pragma unroll
-    for (int b = 0; b < TP; b++)
-#pragma unroll
-      for (int vv = 0; vv < 8; vv++) {
-        const int ql = 8 * (vv >> 2) + 4 * gsel + (vv & 3);
-        stage[ql * SROW + b * 32 + lr] = to_bits(acc[a][b][h * 8 + vv]);
-      }
-    // no workgroup barrier: the staging rows belong to this wave alone, and LDS executes the
-    // writes and reads of one wave in program order
-#pragma unroll 2
-    for (int it = 0; it < ITER; it++) {
-      if (64 % LPR != 0 && qsub >= RPI) continue;  // 96-wide wave tiles: lanes beyond the last whole staged row
-      const v4i raw = *(const v4i *)&stage[it * RPI * SROW + read_off];
-      float qs = q_scale_u, qb = 0.0f;
-      if (q_vec) {
-        const int qi = min(q0 + wq * WTQ + a * 32 + h * 16 + it * RPI + qsub, NQ - 1);  // columns past the end: dropped stores
-        qs = swp ? ep.row_scale(qi) : ep.col_scale(qi);
-        qb = swp ? ep.bias_at(qi) : 0.0f;
-      }
-      float x[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int rawe = raw[e];
-        const float accf = KIND == KIND_I8 ? (float)rawe : bits2f((uint32_t)rawe);
-        float y = (swp ? qs * p_scale[e] : p_scale[e] * qs) * accf + (swp ? qb : p_bias[e]);
-        if (ACT == ACT_RELU) y = y > 0.0f ? y : 0.0f;
-        else if (ACT == ACT_GELU) y = gelu_tanh(y);
-        x[e] = y * ep.sd;
-      }
-      const int soff = (a * 32 + h * 16 + it * RPI) * d_sq * ESZ;  // uniform
-      if constexpr (DT == 2) {
-        const v4i pk = {(int)f2bits(x[0]), (int)f2bits(x[1]), (int)f2bits(x[2]), (int)f2bits(x[3])};
-        buffer_store_b128_guarded(pk, rs, voff, soff);
-      } else {
-        v2i pk;
-        if constexpr (DT == 0) {
-          pk[0] = (int)pack_bf16x2(x[0], x[1]);
-          pk[1] = (int)pack_bf16x2(x[2], x[3]);
-        } else {
-          pk[0] = (int)pack_f16x2(x[0], x[1]);
-          pk[1] = (int)pack_f16x2(x[2], x[3]);
-        }
-        buffer_store_b64_guarded(pk, rs, voff, soff);
-      }
-    }
-  };
-  static_for<TQ * 2>(do_pass);
-}
-
-// Fast path 3: the same float epilogue when nothing varies along Q (no per-column scale vector for a
-// column-major D, no per-row vectors for a row-major one), D bf16 or f16: straight from the
-// accumulator registers, no LDS.  Lane (lr, gsel) holds element (column lr, row 8*(v/4)+4*gsel+v%4)
-// of each 32x32 tile; rows 2k and 2k+1 are paired: after one DPP swap with the neighbouring lane the
-// even lane owns columns (lr, lr+1) of row 2k and the odd lane columns (lr-1, lr) of row 2k+1, so
-// every lane stores one dword of two 16-bit results and a store instruction writes four 64-byte row
-// segments.
-template <int KIND, int WP, int WQ, int WTP, int WTQ, int ACT, int DT, class AccV>
-__device__ __forceinline__ void mfma_store_tile_f16_direct(const MfmaParams &prm, AccV (&acc)[WTQ / 32][WTP / 32],
-                                                           int p0, int q0, int NP, int NQ, int bt) {
-  static_assert(DT == 0 || DT == 1, "16-bit outputs");
+// Fast path 2: float epilogue without a C read (beta == 0), D of type bf16, f16 or f32 at any element's address and any
+// pitch, straight from the accumulator registers.  One 32 x 32 tile (16 accumulators per lane) at a time: the activation and
+// the type of D are uniform branches around whole tiles, so one body serves every combination.
+// f32: lanes 0..31 of a store hold 32 consecutive elements of one D column.  16-bit types: lane (lr, gsel) holds element
+// (column lr, row 8*(v/4)+4*gsel+v%4); rows 2k and 2k+1 are paired: after one DPP swap with the neighbouring lane the even
+// lane owns columns (lr, lr+1) of row 2k and the odd lane columns (lr-1, lr) of row 2k+1, so every lane stores one dword of
+// two results and a store instruction writes four 64-byte row segments.  (The memory system takes those dwords at 2-byte
+// alignment as well: an odd pitch of D costs nothing here.)
+// A tile that hangs over the end of P masks its lanes; the pair that straddles an odd end is stored as one 16-bit element.
+// Measured (MI355X, us, before: the element-wise path through LDS on every tile that was not whole or not 16-byte aligned):
+// bf16 1000 x 1000 x 128, 64 batches, with the product that follows it 286 -> 146; int8 -> int32 5004 x 3000 x 4096 110 -> 61;
+// bf16 5001 x 4099 x 4096 + bias + GELU 258 -> 186; whole tiles as before (fp8 and bf16 within the noise).
+template <int KIND, int WP, int WQ, int WTP, int WTQ, class AccV>
+__device__ __forceinline__ void mfma_store_tile_float(const MfmaParams &prm, AccV (&acc)[WTQ / 32][WTP / 32],
+                                                      int p0, int q0, int NP, int NQ, int bt) {
   constexpr int TP = WTP / 32, TQ = WTQ / 32;
   const GemmArgs &g = prm.g;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -422,103 +341,130 @@ __device__ __forceinline__ void mfma_store_tile_f16_direct(const MfmaParams &prm
   const int lr = lane & 31, gsel = lane >> 5, odd = lane & 1;
   Epilogue ep(g, bt);
   const bool swp = prm.swapped != 0;
-  const float q_scale = swp ? ep.row_scale(0) : ep.col_scale(0);
+  const bool to_f32 = g.d_type == CUDA_R_32F, to_bf16 = g.d_type == CUDA_R_16BF;
+  const int esz = to_f32 ? 4 : 2;
+  const int pc = p0 + wp * WTP, qc = q0 + wq * WTQ;
+  // vectors that run along Q (per-column scale, or per-row quantities of a row-major D)
+  const bool q_vec = swp ? (ep.alpha_v || ep.sa_v || g.bias) : (ep.sb_v != nullptr);
+  const float q_scale = swp ? ep.row_scale(0) : ep.col_scale(0);  // used when !q_vec
   float p_scale[TP], p_bias[TP];
 #pragma unroll
   for (int b = 0; b < TP; b++) {
-    const int pi = p0 + wp * WTP + b * 32 + lr;
+    const int pi = min(pc + b * 32 + lr, NP - 1);
     p_scale[b] = swp ? ep.col_scale(pi) : ep.row_scale(pi);
     p_bias[b] = swp ? 0.0f : ep.bias_at(pi);
+    if (!q_vec) p_scale[b] *= q_scale;
+  }
+  // the vectors along Q, lane l holding entry l % 32 of each 32 columns (one burst of loads up front: a load per column
+  // where it is used costs a memory round trip per 32 columns -- 4096 x 777 x 14336 int8 with per-token scales 92 us against 88)
+  float q_lane[TQ], qb_lane[TQ];
+#pragma unroll
+  for (int a = 0; a < TQ; a++) {
+    const int qi = min(qc + a * 32 + lr, NQ - 1);  // columns past the end: dropped stores
+    q_lane[a] = q_vec ? (swp ? ep.row_scale(qi) : ep.col_scale(qi)) : 1.0f;
+    qb_lane[a] = q_vec && swp ? ep.bias_at(qi) : 0.0f;
   }
   const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < 2^22 (checked by the dispatcher)
-  const int64_t corner = (int64_t)(q0 + wq * WTQ) * d_sq + (p0 + wp * WTP);
-  char *Dw = (char *)g.D + (g.d_sb * bt + corner) * 2;
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dw, 0, tile_window_bytes(d_sq, NP, NQ, corner, 2), 0x00020000);
-  const int voff = ((4 * gsel + odd) * d_sq + (lr & ~1)) * 2;
-  auto value = [&](float accf, int b) {
-    float y = (swp ? q_scale * p_scale[b] : p_scale[b] * q_scale) * accf + p_bias[b];
-    if (ACT == ACT_RELU) y = y > 0.0f ? y : 0.0f;
-    else if (ACT == ACT_GELU) y = gelu_tanh(y);
-    return y * ep.sd;
-  };
+  const int64_t corner = (int64_t)qc * d_sq + pc;
+  char *Dw = (char *)g.D + (g.d_sb * bt + corner) * esz;
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dw, 0, tile_window_bytes(d_sq, NP, NQ, corner, esz), 0x00020000);
+  const int col = to_f32 ? lr : lr & ~1, last = to_f32 ? lr : lr | 1;  // first / last P index of the lane's store inside a tile
+  const int voff_in = to_f32 ? (4 * gsel * d_sq + lr) * 4 : ((4 * gsel + odd) * d_sq + col) * 2;
+  const bool odd_end = !to_f32 && (NP & 1) && NP < pc + WTP;  // (uniform) some pair of the wave tile straddles the end
+
 #pragma unroll
-  for (int a = 0; a < TQ; a++)
+  for (int a = 0; a < TQ; a++) {
+    float qs[16], qb[16];
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const int soff = (a * 32 + 8 * (k >> 1) + 2 * (k & 1)) * d_sq * 2;  // uniform: row 2k of tile a
+    for (int v = 0; v < 16; v++) { qs[v] = 1.0f; qb[v] = 0.0f; }
+    if (q_vec) {
 #pragma unroll
-      for (int b = 0; b < TP; b++) {
-        const float fa = KIND == KIND_I8 ? (float)to_bits(acc[a][b][2 * k]) : bits2f((uint32_t)to_bits(acc[a][b][2 * k]));
-        const float fb = KIND == KIND_I8 ? (float)to_bits(acc[a][b][2 * k + 1]) : bits2f((uint32_t)to_bits(acc[a][b][2 * k + 1]));
-        const float ya = value(fa, b), yb = value(fb, b);
-        // even lanes keep row 2k and need the neighbour's row-2k value; odd lanes the other way round
-        const float mine = odd ? yb : ya, give = odd ? ya : yb;
-        const float got = bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(give), 0xB1 /* quad_perm [1,0,3,2] */, 0xF, 0xF, true));
-        const float lo = odd ? got : mine, hi = odd ? mine : got;
-        const uint32_t pk = DT == 0 ? pack_bf16x2(lo, hi) : pack_f16x2(lo, hi);
-        __builtin_amdgcn_raw_buffer_store_b32((int)pk, rs, voff, soff + b * 64, 0);
+      for (int v = 0; v < 16; v++) {
+        const int from = (8 * (v >> 2) + 4 * gsel + (v & 3)) * 4;  // the lane that holds the column, in bytes
+        qs[v] = bits2f((uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)f2bits(q_lane[a])));
+        if (swp) qb[v] = bits2f((uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)f2bits(qb_lane[a])));
       }
     }
+#pragma unroll
+    for (int b = 0; b < TP; b++) {
+      float x[16];
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const float accf = KIND == KIND_I8 ? (float)to_bits(acc[a][b][v]) : bits2f((uint32_t)to_bits(acc[a][b][v]));
+        x[v] = accf;
+      }
+      if (q_vec) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) x[v] = (p_scale[b] * qs[v]) * x[v] + (p_bias[b] + qb[v]);
+      } else {
+#pragma unroll
+        for (int v = 0; v < 16; v++) x[v] = p_scale[b] * x[v] + p_bias[b];
+      }
+      if (g.act == ACT_GELU) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) x[v] = gelu_tanh(x[v]);
+      } else if (g.act == ACT_RELU) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) x[v] = x[v] > 0.0f ? x[v] : 0.0f;
+      }
+#pragma unroll
+      for (int v = 0; v < 16; v++) x[v] *= ep.sd;
+      const int tile_p = pc + b * 32;
+      const int voff = tile_p + last < NP ? voff_in : kStoreNowhere;
+      if (to_f32) {
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+          __builtin_amdgcn_raw_buffer_store_b32((int)f2bits(x[v]), rs, voff, (a * 32 + 8 * (v >> 2) + (v & 3)) * d_sq * 4 + b * 128, 0);
+      } else {
+        uint32_t pk[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          // even lanes keep row 2k and need the neighbour's row-2k value; odd lanes the other way round
+          const float mine = odd ? x[2 * k + 1] : x[2 * k], give = odd ? x[2 * k] : x[2 * k + 1];
+          const float got = bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(give), 0xB1 /* quad_perm [1,0,3,2] */, 0xF, 0xF, true));
+          x[2 * k] = odd ? got : mine;
+          x[2 * k + 1] = odd ? mine : got;
+        }
+        if (to_bf16) {
+#pragma unroll
+          for (int k = 0; k < 8; k++) pk[k] = pack_bf16x2(x[2 * k], x[2 * k + 1]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 8; k++) pk[k] = pack_f16x2(x[2 * k], x[2 * k + 1]);
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+          __builtin_amdgcn_raw_buffer_store_b32((int)pk[k], rs, voff, (a * 32 + 8 * (k >> 1) + 2 * (k & 1)) * d_sq * 2 + b * 64, 0);
+        if (odd_end) {
+          const int vedge = tile_p + col == NP - 1 ? voff_in : kStoreNowhere;
+#pragma unroll
+          for (int k = 0; k < 8; k++)
+            __builtin_amdgcn_raw_buffer_store_b16((short)pk[k], rs, vedge, (a * 32 + 8 * (k >> 1) + 2 * (k & 1)) * d_sq * 2 + b * 64, 0);
+        }
+      }
+    }
+  }
 }
 
-// Epilogue dispatch: the fast paths for the common configurations on tiles that are complete along
-// P (columns past the end of D are dropped by the store window, so a ragged token count keeps the
-// fast path), the general path for the rest.  All conditions are workgroup-uniform.
+// Epilogue dispatch: the fast paths for the common configurations, the general path for the rest (C reads, 8-bit outputs,
+// integer outputs of a float epilogue, vectors of alpha in the integer one).  All conditions are workgroup-uniform.
 template <int KIND, int WP, int WQ, int WTP, int WTQ, class AccV>
 __device__ __forceinline__ void mfma_store_tile(const MfmaParams &prm, AccV (&acc)[WTQ / 32][WTP / 32],
                                                 int *lds_words, size_t lds_bytes, int p0, int q0, int NP,
                                                 int NQ, int bt) {
   const GemmArgs &g = prm.g;
-  const bool swp = prm.swapped != 0;
-  const int64_t d_sq = swp ? g.d_si : g.d_sj;
-  const bool full = p0 + WP * WTP <= NP;  // along Q the store window cuts the tile
-  const int dbytes = (g.d_type == CUDA_R_32F || g.d_type == CUDA_R_32I) ? 4 : (g.d_type == CUDA_R_8I ? 1 : 2);
-  // columns of the tile start 16-byte aligned and the lane offsets fit 32 bits
-  const bool aligned = (((uintptr_t)g.D) & 15) == 0 && ((d_sq * dbytes) & 15) == 0 &&
-                       ((g.d_sb * dbytes) & 15) == 0 && d_sq < (1 << 22);
+  const int64_t d_sq = prm.swapped ? g.d_si : g.d_sj;
+  const bool narrow = d_sq < (1 << 22);  // the lane offsets fit 32 bits
   if constexpr (KIND == KIND_I8) {
-    if (g.int_scale && full && aligned && g.alpha_mode != VECTOR_DEV && g.beta_mode == SCALAR_VALUE &&
-        g.beta_val.i == 0) {
+    if (g.int_scale && narrow && g.alpha_mode != VECTOR_DEV && g.beta_mode == SCALAR_VALUE && g.beta_val.i == 0) {
       const int ialpha = g.alpha_mode == SCALAR_VALUE ? g.alpha_val.i : *(const int32_t *)g.alpha_ptr;
       mfma_store_tile_i32<WP, WQ, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, ialpha);
       return;
     }
   }
-  if (!g.int_scale && full && aligned && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
+  if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
       (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F)) {
-    const int dt = g.d_type == CUDA_R_16BF ? 0 : (g.d_type == CUDA_R_16F ? 1 : 2);
-    // vectors that run along Q need the LDS-staged form
-    const bool q_vec = swp ? (g.alpha_mode == VECTOR_DEV || g.a_scale_mode == SCALE_OUTER_VEC || g.bias != nullptr)
-                           : (g.b_scale_mode == SCALE_OUTER_VEC);
-    if (!q_vec && dt != 2) {
-#define ZLUDA_EPI_D(ACT_, DT_) mfma_store_tile_f16_direct<KIND, WP, WQ, WTP, WTQ, ACT_, DT_>(prm, acc, p0, q0, NP, NQ, bt)
-      if (dt == 0) {
-        if (g.act == ACT_GELU) ZLUDA_EPI_D(ACT_GELU, 0);
-        else if (g.act == ACT_RELU) ZLUDA_EPI_D(ACT_RELU, 0);
-        else ZLUDA_EPI_D(ACT_NONE, 0);
-      } else {
-        if (g.act == ACT_GELU) ZLUDA_EPI_D(ACT_GELU, 1);
-        else if (g.act == ACT_RELU) ZLUDA_EPI_D(ACT_RELU, 1);
-        else ZLUDA_EPI_D(ACT_NONE, 1);
-      }
-#undef ZLUDA_EPI_D
-      return;
-    }
-#define ZLUDA_EPI(ACT_, DT_) mfma_store_tile_f<KIND, WP, WQ, WTP, WTQ, ACT_, DT_>(prm, acc, lds_words, p0, q0, NP, NQ, bt)
-    if (dt == 0) {
-      if (g.act == ACT_GELU) ZLUDA_EPI(ACT_GELU, 0);
-      else if (g.act == ACT_RELU) ZLUDA_EPI(ACT_RELU, 0);
-      else ZLUDA_EPI(ACT_NONE, 0);
-    } else if (dt == 1) {
-      if (g.act == ACT_GELU) ZLUDA_EPI(ACT_GELU, 1);
-      else if (g.act == ACT_RELU) ZLUDA_EPI(ACT_RELU, 1);
-      else ZLUDA_EPI(ACT_NONE, 1);
-    } else {
-      if (g.act == ACT_GELU) ZLUDA_EPI(ACT_GELU, 2);
-      else if (g.act == ACT_RELU) ZLUDA_EPI(ACT_RELU, 2);
-      else ZLUDA_EPI(ACT_NONE, 2);
-    }
-#undef ZLUDA_EPI
+    mfma_store_tile_float<KIND, WP, WQ, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt);
     return;
   }
   mfma_store_tile_general<KIND, WP, WQ, WTP, WTQ>(prm, acc, lds_words, lds_bytes, p0, q0, NP, NQ, bt);

@@ -36,12 +36,18 @@ namespace zluda_amd {
 // acc[a][b] is the 16 x 16 tile at (P tile a, Q tile b) of the wave tile; lane l holds elements
 // P = 16a + 4*(l/16) + v (v = 0..3), Q = 16b + l%16.
 
+// A lane's store of four consecutive elements along P: where the four end past P's last index it is dropped, and those of
+// them that exist are stored one by one.  `left`: P indices from the lane's first one to the end.
+__device__ __forceinline__ int store4_offset(int left, int voff) { return left >= 4 ? voff : kStoreNowhere; }
+__device__ __forceinline__ int store1_offset(int left, int e, int voff, int esz) { return left < 4 && e < left ? voff + e * esz : kStoreNowhere; }
+
 // raw accumulators (int32 or fp32 bits) of a whole wave tile into a matrix of `pitch` dwords per Q column
-// through the window `rs` that starts at the wave tile's corner
+// through the window `rs` that starts at the wave tile's corner; `p_left`: P indices from that corner to the end of P
 template <int TP, int TQ, class AccV>
-__device__ __forceinline__ void mfma16_store_raw(__amdgpu_buffer_rsrc_t rs, int pitch, AccV (&acc)[TP][TQ], int mul) {
+__device__ __forceinline__ void mfma16_store_raw(__amdgpu_buffer_rsrc_t rs, int pitch, AccV (&acc)[TP][TQ], int mul, int p_left = TP * 16) {
   const int lane = threadIdx.x & 63;
   const int voff = ((lane & 15) * pitch + 4 * (lane >> 4)) * 4;
+  const bool ragged = p_left < TP * 16 && (p_left & 3);  // (uniform) some lane's four straddle the end
 #pragma unroll
   for (int b = 0; b < TQ; b++)
 #pragma unroll
@@ -50,19 +56,21 @@ __device__ __forceinline__ void mfma16_store_raw(__amdgpu_buffer_rsrc_t rs, int 
 #pragma unroll
       for (int e = 0; e < 4; e++) v[e] = to_bits(acc[a][b][e]);
       if (mul != 1) v *= mul;
-      buffer_store_b128_guarded(v, rs, voff, (b * 16 * pitch + a * 16) * 4);
+      const int left = p_left - (a * 16 + 4 * (lane >> 4));
+      buffer_store_b128_guarded(v, rs, store4_offset(left, voff), (b * 16 * pitch + a * 16) * 4);
+      if (ragged) {
+#pragma unroll
+        for (int e = 0; e < 3; e++) __builtin_amdgcn_raw_buffer_store_b32(v[e], rs, store1_offset(left, e, voff, 4), (b * 16 * pitch + a * 16) * 4, 0);
+      }
     }
 }
 
-// float epilogue without a C read on tiles complete along P: D bf16 / f16 (8-byte stores) or f32 (WIDE:
-// 16-byte stores).  The activation and the 16-bit format are workgroup-uniform branches per 16 x 16 tile
-// (one instantiation serves them all: the 64 tiles of a wave are unrolled, so every further template
-// argument multiplies a large body).
-// FENCE: the scheduler may not move instructions from one row of 16 x 16 tiles to the next (a wave that holds more
-// than the accumulators across the epilogue has no registers for what the scheduler would otherwise hoist).
-// ACT_T / BF16_T >= 0 fix the activation / the 16-bit format at compile time (no branch per tile: a wave that has its
-// SIMD to itself cannot hide them behind another wave's work).
-template <int KIND, int WP, int WQ, int TP, int TQ, bool WIDE, bool FENCE = false, int ACT_T = -1, int BF16_T = -1, class AccV>
+// float epilogue without a C read: D bf16 / f16 (8-byte stores) or f32 (WIDE: 16-byte stores), at any element's address
+// and any pitch (the memory system takes such stores unaligned).  The activation and the 16-bit format are
+// workgroup-uniform branches per 16 x 16 tile (one instantiation serves them all: the 64 tiles of a wave are unrolled, so
+// every further template argument multiplies a large body).  A tile that hangs over the end of P drops the lanes past it
+// and stores the elements of a group of four that straddles the end one by one.
+template <int KIND, int WP, int WQ, int TP, int TQ, bool WIDE, class AccV>
 __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt) {
   constexpr int WTP = TP * 16, WTQ = TQ * 16;
   constexpr int ESZ = WIDE ? 4 : 2;
@@ -71,8 +79,9 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
   const int wp = wave % WP, wq = wave / WP;
   Epilogue ep(g, bt);
   const bool swp = prm.swapped != 0;
-  const int act = ACT_T >= 0 ? ACT_T : g.act;
-  const bool to_bf16 = BF16_T >= 0 ? BF16_T != 0 : g.d_type == CUDA_R_16BF;
+  const int act = g.act;
+  const bool to_bf16 = g.d_type == CUDA_R_16BF;
+  const bool ragged = NP < p0 + wp * WTP + WTP && (NP & 3);  // (uniform) some lane's four straddle the end of P
   const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < 2^22 (checked by the dispatcher)
   const int pc = p0 + wp * WTP, qc = q0 + wq * WTQ;
   const int64_t corner = (int64_t)qc * d_sq + pc;
@@ -92,11 +101,12 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
   const int bsz = g.bias_type == CUDA_R_32F ? 4 : 2;
   const bool pbias = !swp && g.bias != nullptr;
   const char *bias_b = (const char *)g.bias + g.bias_sb * bt * bsz;
-  const bool wide_bias = pbias && (((uintptr_t)bias_b) & (4 * bsz - 1)) == 0;  // rows start at multiples of 4
+  // (rows start at multiples of 4)
+  const bool wide_bias = pbias && (((uintptr_t)bias_b) & (4 * bsz - 1)) == 0 && p0 + WP * WTP <= NP;
   v4i braw[TP];
 #pragma unroll
   for (int a = 0; a < TP; a++) {
-    const int pi = pc + a * 16 + 4 * (lane >> 4);  // + 3 < NP: the tile is complete along P
+    const int pi = pc + a * 16 + 4 * (lane >> 4);
     braw[a] = v4i{0, 0, 0, 0};
     if (wide_bias) {
       if (bsz == 4) braw[a] = *(const v4i *)(bias_b + (int64_t)pi * 4);
@@ -106,7 +116,7 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
       }
     } else if (pbias) {
 #pragma unroll
-      for (int e = 0; e < 4; e++) braw[a][e] = (int)ep.bias_raw(pi + e);
+      for (int e = 0; e < 4; e++) braw[a][e] = (int)ep.bias_raw(min(pi + e, NP - 1));
     }
   }
 #pragma unroll
@@ -114,7 +124,7 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
     float ps[4], pb[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const int pi = pc + a * 16 + 4 * (lane >> 4) + e;
+      const int pi = min(pc + a * 16 + 4 * (lane >> 4) + e, NP - 1);
       ps[e] = swp ? ep.col_scale(pi) : ep.row_scale(pi);
       pb[e] = pbias ? ep.bias_from_raw((uint32_t)braw[a][e]) : 0.0f;
     }
@@ -136,17 +146,26 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
 #pragma unroll
       for (int e = 0; e < 4; e++) x[e] *= ep.sd;
       const int soff = (b * 16 * d_sq + a * 16) * ESZ;  // uniform
+      const int left = NP - (pc + a * 16 + 4 * (lane >> 4));
       if constexpr (WIDE) {
         const v4i pk = {(int)f2bits(x[0]), (int)f2bits(x[1]), (int)f2bits(x[2]), (int)f2bits(x[3])};
-        buffer_store_b128_guarded(pk, rs, voff, soff);
+        buffer_store_b128_guarded(pk, rs, store4_offset(left, voff), soff);
+        if (ragged) {
+#pragma unroll
+          for (int e = 0; e < 3; e++) __builtin_amdgcn_raw_buffer_store_b32(pk[e], rs, store1_offset(left, e, voff, 4), soff, 0);
+        }
       } else {
         v2i pk;
         if (to_bf16) { pk[0] = (int)pack_bf16x2(x[0], x[1]); pk[1] = (int)pack_bf16x2(x[2], x[3]); }
         else { pk[0] = (int)pack_f16x2(x[0], x[1]); pk[1] = (int)pack_f16x2(x[2], x[3]); }
-        buffer_store_b64_guarded(pk, rs, voff, soff);
+        buffer_store_b64_guarded(pk, rs, store4_offset(left, voff), soff);
+        if (ragged) {
+          __builtin_amdgcn_raw_buffer_store_b16((short)pk[0], rs, store1_offset(left, 0, voff, 2), soff, 0);
+          __builtin_amdgcn_raw_buffer_store_b16((short)(pk[0] >> 16), rs, store1_offset(left, 1, voff, 2), soff, 0);
+          __builtin_amdgcn_raw_buffer_store_b16((short)pk[1], rs, store1_offset(left, 2, voff, 2), soff, 0);
+        }
       }
     }
-    if constexpr (FENCE) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -157,7 +176,7 @@ constexpr int staging_columns(int fit, int tq) {
   return c;
 }
 
-// everything else (partial tiles along P, C reads, 8-bit outputs, unaligned D, integer alpha vectors):
+// everything else (C reads, 8-bit outputs, integer outputs of a float epilogue, integer alpha vectors):
 // element by element through the scalar epilogue.  Correct for whatever the planner admits; not fast.
 // The accumulators are staged in the wave's share of the (now free) LDS, as many tile columns per pass as
 // fit, so that the scalar epilogue is a rolled loop (a function call would do as well, but a call anywhere
@@ -209,23 +228,20 @@ __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&
   const GemmArgs &g = prm.g;
   const bool swp = prm.swapped != 0;
   const int64_t d_sq = swp ? g.d_si : g.d_sj;
-  const bool full = p0 + WP * WTP <= NP;  // along Q the store window cuts the tile
-  const int dbytes = (g.d_type == CUDA_R_32F || g.d_type == CUDA_R_32I) ? 4 : (g.d_type == CUDA_R_8I ? 1 : 2);
-  const bool aligned = (((uintptr_t)g.D) & 15) == 0 && ((d_sq * dbytes) & 15) == 0 && ((g.d_sb * dbytes) & 15) == 0 &&
-                       d_sq < (1 << 22);
+  const bool narrow = d_sq < (1 << 22);  // the lane offsets fit 32 bits
   if constexpr (KIND == KIND_I8) {
-    if (g.int_scale && full && aligned && g.alpha_mode != VECTOR_DEV && g.beta_mode == SCALAR_VALUE && g.beta_val.i == 0) {
+    if (g.int_scale && narrow && g.alpha_mode != VECTOR_DEV && g.beta_mode == SCALAR_VALUE && g.beta_val.i == 0) {
       const int ialpha = g.alpha_mode == SCALAR_VALUE ? g.alpha_val.i : *(const int32_t *)g.alpha_ptr;
       const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
       const int pc = p0 + (wave % WP) * WTP, qc = q0 + (wave / WP) * WTQ;
       const int64_t corner = (int64_t)qc * d_sq + pc;
       int32_t *Dw = (int32_t *)g.D + g.d_sb * bt + corner;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dw, 0, tile_window_bytes(d_sq, NP, NQ, corner, 4), 0x00020000);
-      mfma16_store_raw<TP, TQ>(rs, (int)d_sq, acc, ialpha);
+      mfma16_store_raw<TP, TQ>(rs, (int)d_sq, acc, ialpha, NP - pc);
       return;
     }
   }
-  if (!g.int_scale && full && aligned && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
+  if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
       (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F)) {
     if (g.d_type == CUDA_R_32F) mfma16_store_f<KIND, WP, WQ, TP, TQ, true>(prm, acc, p0, q0, NP, NQ, bt);
     else mfma16_store_f<KIND, WP, WQ, TP, TQ, false>(prm, acc, p0, q0, NP, NQ, bt);

@@ -47,8 +47,7 @@ __device__ __forceinline__ bool w4_stream_d_i32(const GemmArgs &g) {
   return d_bytes >= (256ll << 20) && ab_bytes >= (128ll << 20);
 }
 
-// the fast epilogue an instantiation carries; everything else a problem may ask for (and every tile that is not
-// complete along P) takes the element-wise path through LDS
+// the epilogue an instantiation carries; the planner sends it the problems that one serves (w4_epilogue_class)
 enum { W4_EPI_I32 = 0, W4_EPI_BF16 = 1, W4_EPI_BF16_GELU = 2 };
 
 // one accumulator element, AGPR -> VGPR
@@ -96,6 +95,14 @@ __device__ __forceinline__ void w4_scalar_here(float &v) {
   v = bits2f((uint32_t)b);
 }
 
+// The same for a vector register: masks computed from it are computed at each use instead of all at once in front.
+__device__ __forceinline__ int w4_vector_here(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(v));
+#endif
+  return v;
+}
+
 // What a wave has staged in LDS for the epilogue of its current tile: up to three vectors along P, WTP = 128 entries each
 // (slot 0: the per-P scale vector alpha[] or, for a row-major D, B's; slot 1: A's; slot 2: the bias in its storage type),
 // and up to two scale vectors along Q, WTQ = 128 entries each (slot 3: B's outer scales or, for a row-major D, alpha[];
@@ -110,13 +117,13 @@ struct W4Staged {
 };
 
 // Float epilogue of the four-wave kernel: D bf16 / f16 = act((scale_p * scale_q) * acc + bias) * scale_d straight from the
-// accumulators (layout of gemm_mfma_pipe16.hpp: lane l holds P = 16a + 4 (l / 16) + e, Q = 16b + l % 16) on tiles complete
-// along P, for problems in which nothing varies along Q (no per-column scale vector; for a row-major D no per-row vector
+// accumulators (layout of gemm_mfma_pipe16.hpp: lane l holds P = 16a + 4 (l / 16) + e, Q = 16b + l % 16), for problems in which nothing varies along Q (no per-column scale vector; for a row-major D no per-row vector
 // or bias).  A wave that has its SIMD to itself cannot hide branches or dependent chains behind another wave, so everything
 // that depends on the problem's modes is decided once, up front, into per-lane factors, and the 64 tiles are straight-line
 // code: one FMA per element, then the activation (ACT fixed at compile time) with D's scale folded into it.
 // QV: the problem has a scale vector along Q (one more multiplication per element, which problems without one are spared).
-template <int KIND, int ACT, bool BF16, bool QV, int WTP, int WTQ, int TP, int TQ, class AccV>
+// EDGE: the tile hangs over the end of P (its masks cost the whole tiles of fp8 8192^3 2 us: a body of its own).
+template <int KIND, int ACT, bool EDGE, bool QV, int WTP, int WTQ, int TP, int TQ, class AccV>
 __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt,
                                              int wp, int wq, const EpilogueScalars &scalars, const W4Staged &st) {
   const GemmArgs &g = prm.g;
@@ -222,7 +229,11 @@ __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[
   // lane, and a store instruction writes 64 contiguous bytes of each of 16 columns instead of 32.
   static_assert(TP % 2 == 0, "tiles along P are stored in pairs");
   const int grp = lane >> 4;
-  const int voff16 = ((lane & 15) * d_sq + ((grp & 1) ? 4 * grp + 12 : 4 * grp)) * 2;
+  // Tiles that hang over the end of P: a lane whose elements do not all exist stores nowhere, and those of a group that
+  // straddles the end go out one by one (only in the pair of tiles that holds the end).
+  const int first = (grp & 1) ? 4 * grp + 12 : 4 * grp;  // the lane's first P index inside a pair of tiles
+  const int voff16 = ((lane & 15) * d_sq + first) * 2;
+  const int p_left = NP - pc;  // P indices from the wave tile's corner to the end
 #pragma unroll
   for (int b = 0; b < TQ; b++) {
     // The column's accumulators first, by explicit reads (left to itself the register allocator parks most accumulators
@@ -305,7 +316,18 @@ __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[
 #else
         pk = v4i{(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
 #endif
-        buffer_store_b128_guarded(pk, rs, voff16, (b * 16 * d_sq + a * 16) * 2);
+        const int soff = (b * 16 * d_sq + a * 16) * 2;
+        if constexpr (!EDGE) {
+          buffer_store_b128_guarded(pk, rs, voff16, soff);
+        } else {
+          const int left = w4_vector_here(p_left - a * 16 - first);
+          buffer_store_b128_guarded(pk, rs, left >= 8 ? voff16 : kStoreNowhere, soff);
+          if (p_left > a * 16 && p_left < a * 16 + 32 && (p_left & 7)) {  // (uniform)
+#pragma unroll
+            for (int e = 0; e < 7; e++)
+              __builtin_amdgcn_raw_buffer_store_b16((short)(pk[e >> 1] >> (16 * (e & 1))), rs, left < 8 && e < left ? voff16 + e * 2 : kStoreNowhere, soff, 0);
+          }
+        }
       }
     };
     if (to_f32) {
@@ -313,7 +335,17 @@ __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[
 #pragma unroll
       for (int a = 0; a < TP; a++) {
         const v4i pk = {(int)f2bits(x[a][0]), (int)f2bits(x[a][1]), (int)f2bits(x[a][2]), (int)f2bits(x[a][3])};
-        buffer_store_b128_guarded(pk, rs, voff32, (b * 16 * d_sq + a * 16) * 4);
+        const int soff = (b * 16 * d_sq + a * 16) * 4;
+        if constexpr (!EDGE) {
+          buffer_store_b128_guarded(pk, rs, voff32, soff);
+        } else {
+          const int left = w4_vector_here(p_left - a * 16 - 4 * grp);
+          buffer_store_b128_guarded(pk, rs, store4_offset(left, voff32), soff);
+          if (p_left > a * 16 && p_left < a * 16 + 16 && (p_left & 3)) {
+#pragma unroll
+            for (int e = 0; e < 3; e++) __builtin_amdgcn_raw_buffer_store_b32(pk[e], rs, store1_offset(left, e, voff32, 4), soff, 0);
+          }
+        }
       }
     } else if (to_bf16) {
       pack_store(std::integral_constant<int, 1>{});
@@ -324,8 +356,8 @@ __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[
   }
 }
 
-// Integer epilogue of the four-wave kernel: D int32 = alpha * acc (beta == 0, scalar alpha) on tiles complete along P
-// with 16-byte aligned columns: 16 bytes per lane straight from the accumulators.
+// Integer epilogue of the four-wave kernel: D int32 = alpha * acc (beta == 0, scalar alpha) with 16-byte aligned columns:
+// 16 bytes per lane straight from the accumulators; the end of P as in the float epilogue.
 template <int WTP, int WTQ, int AUX, int TP, int TQ, class AccV>
 __device__ __forceinline__ void w4_store_i32(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt,
                                              int wp, int wq, int ialpha) {
@@ -340,6 +372,8 @@ __device__ __forceinline__ void w4_store_i32(const MfmaParams &prm, AccV (&acc)[
   const int voff = ((lane & 15) * pitch + 4 * (lane >> 4)) * 4;
 #pragma unroll
   for (int a = 0; a < TP; a++) {
+    const int left = w4_vector_here(NP - (pc + a * 16 + 4 * (lane >> 4)));
+    const bool ragged = NP > pc + a * 16 && NP < pc + a * 16 + 16 && (NP & 3);  // (uniform)
     v4i v[TQ];
 #pragma unroll
     for (int b = 0; b < TQ; b++)
@@ -348,69 +382,13 @@ __device__ __forceinline__ void w4_store_i32(const MfmaParams &prm, AccV (&acc)[
 #pragma unroll
     for (int b = 0; b < TQ; b++) {
       if (ialpha != 1) v[b] *= ialpha;
-      buffer_store_b128_guarded<AUX>(v[b], rs, voff, (b * 16 * pitch + a * 16) * 4);
+      buffer_store_b128_guarded<AUX>(v[b], rs, store4_offset(left, voff), (b * 16 * pitch + a * 16) * 4);
+      if (ragged) {
+#pragma unroll
+        for (int e = 0; e < 3; e++) __builtin_amdgcn_raw_buffer_store_b32(v[b][e], rs, store1_offset(left, e, voff, 4), (b * 16 * pitch + a * 16) * 4, AUX);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
-// Everything else (tiles that are partial along P, C reads, other output types, vectors along Q, unaligned D): element by
-// element through the scalar epilogue, one row of 16 x 16 tiles at a time staged in the wave's share of LDS.  Correct for
-// whatever the planner admits; not fast.  The caller guarantees that no wave still needs the LDS tiles.
-template <int KIND, int WTP, int WTQ, int TP, int TQ, class AccV>
-__device__ __forceinline__ void w4_store_general(const MfmaParams &prm, AccV (&acc)[TP][TQ], int *lds_words, int p0, int q0, int NP,
-                                                 int NQ, int bt, int wp, int wq) {
-  const GemmArgs &g = prm.g;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int *stage = lds_words + wave * (WTQ * 16);  // [Q index of the wave tile][16 P indices of the row]
-  Epilogue ep(g, bt);
-  const bool swp = prm.swapped != 0;
-#pragma unroll
-  for (int a = 0; a < TP; a++) {
-#pragma unroll
-    for (int b = 0; b < TQ; b++) {
-      v4i v;
-#pragma unroll
-      for (int e = 0; e < 4; e++) v[e] = w4_acc_read(acc[a][b][e]);
-      *(v4i *)&stage[(b * 16 + (lane & 15)) * 16 + 4 * (lane >> 4)] = v;
-    }
-    // (LDS executes the writes and reads of one wave in program order: no barrier for wave-private rows)
-#pragma unroll 1
-    for (int e = lane; e < WTQ * 16; e += 64) {
-      const int ql = e / 16, pl = e % 16;
-      const int pi = p0 + wp * WTP + a * 16 + pl, qi = q0 + wq * WTQ + ql;
-      if (pi >= NP || qi >= NQ) continue;
-      const int raw = stage[ql * 16 + pl];
-      const int i = swp ? qi : pi, j = swp ? pi : qi;
-      if (g.int_scale) ep.store_int(i, j, raw);
-      else ep.store_f(i, j, KIND == KIND_I8 ? (float)raw : bits2f((uint32_t)raw));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
-// whether the instantiation's fast epilogue serves the problem (on tiles complete along P)
-template <int KIND, int EPI>
-__device__ __forceinline__ bool w4_fast_epilogue_ok(const MfmaParams &prm) {
-  const GemmArgs &g = prm.g;
-  const int64_t d_sq = prm.swapped ? g.d_si : g.d_sj;
-  const int dbytes = (EPI == W4_EPI_I32 || g.d_type == CUDA_R_32F) ? 4 : 2;
-  const bool aligned = (((uintptr_t)g.D) & 15) == 0 && ((d_sq * dbytes) & 15) == 0 && ((g.d_sb * dbytes) & 15) == 0 &&
-                       d_sq < (1 << 22);
-  if (!aligned) return false;
-  if constexpr (EPI == W4_EPI_I32) {
-    return KIND == KIND_I8 && g.int_scale && g.d_type == CUDA_R_32I && g.alpha_mode != VECTOR_DEV && g.beta_mode == SCALAR_VALUE &&
-           g.beta_val.i == 0;
-  } else {
-    // a bias that runs along Q (a row-major D's) is not served; scale vectors along Q are
-    const bool q_vec = prm.swapped && g.bias != nullptr;
-    // (MXFP4 has no room in LDS for staged vectors: no alpha[], no bias)
-    const bool p_vec = g.alpha_mode == VECTOR_DEV || g.bias != nullptr;
-    // bf16, f16 and f32 outputs; the GELU instantiation for GELU, the plain one without an activation and for ReLU
-    const bool act_ok = EPI == W4_EPI_BF16_GELU ? g.act == ACT_GELU : (g.act == ACT_NONE || g.act == ACT_RELU);
-    return !g.int_scale && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
-           (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F) &&
-           !q_vec && !(KIND == KIND_MXF4 && p_vec) && act_ok;
   }
 }
 
@@ -782,16 +760,12 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
     static_for<NRD>([&](auto r_c) { read_piece(0, fragP, pf[0], P0{}, r_c); });
     static_for<NRD>([&](auto r_c) { read_piece(0, fragQ, qf[0], P0{}, r_c); });
   };
-  // (re)starts the stream at tile n: its first two stages requested and landed, its first fragments in registers
-  auto prime = [&](int n) __attribute__((always_inline)) {
-    d_live = -1;
-    dma_tile(n);
+  // starts the stream: the first tile's first two stages requested and landed, its first fragments in registers
+  auto prime = [&]() __attribute__((always_inline)) {
+    dma_tile(0);
     if constexpr (MX) {
-      // (only the stream's very first tile: later ones had their chunk 0 requested in the tile before)
-      if (n == 0) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) issue_scale_part(0, j);
-      }
+      for (int j = 0; j < 4; j++) issue_scale_part(0, j);
     }
     issue_part(0, 0, std::integral_constant<int, 0>{}, std::integral_constant<int, NLOAD>{}, std::integral_constant<int, 0>{}, wave * RPW * CPR);
     issue_part(1, STAGE_V4, std::integral_constant<int, 0>{}, std::integral_constant<int, NLOAD>{}, std::integral_constant<int, 0>{}, wave * RPW * CPR);
@@ -799,7 +773,6 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
     first_frags();
   };
 
-  const bool fast = w4_fast_epilogue_ok<KIND, EPI>(prm);
   // The scalars behind device pointers, once for all tiles and wave-uniform (SGPRs): fetched in a tile's epilogue each
   // would first wait for the next tile's stages, which are in flight and older.
   EpilogueScalars scalars(g);
@@ -813,29 +786,28 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
     ialpha = (int)f2bits(w4_uniform_now(bits2f((uint32_t)raw)));
   }
   W4Staged staged{(const int *)&lds[2 * STAGE_V4] + (STG_V4 == 0 ? 0 : wave * STG_WAVE), {false, false, false, false, false}, 0};
-  // epilogue of the tile at (p0, q0, bt); returns false when it needed the LDS (the stream must be primed again)
-  auto epilogue = [&](int p0, int q0, int bt) __attribute__((always_inline)) -> bool {
+  // epilogue of the tile at (p0, q0, bt)
+  auto epilogue = [&](int p0, int q0, int bt) __attribute__((always_inline)) {
     // MFMA write -> read of the accumulators: the wait states the compiler would insert if it could see the MFMAs.
     // Nothing that reads an accumulator may be scheduled in front of them (every MFMA is followed by a scheduling
     // barrier, and so are they).
     asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    if (fast && p0 + BP <= NP) {
-      if constexpr (EPI == W4_EPI_I32) {
-        if (stream_d) w4_store_i32<WTP, WTQ, 2>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, ialpha);
-        else w4_store_i32<WTP, WTQ, 0>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, ialpha);
+    if constexpr (EPI == W4_EPI_I32) {
+      if (stream_d) w4_store_i32<WTP, WTQ, 2>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, ialpha);
+      else w4_store_i32<WTP, WTQ, 0>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, ialpha);
+    } else {
+      constexpr int ACT = EPI == W4_EPI_BF16_GELU ? ACT_GELU : ACT_NONE;
+      const bool qv = staged.has[3] || staged.has[4];
+      if (p0 + BP <= NP) {
+        if (qv) w4_store_f16<KIND, ACT, false, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+        else w4_store_f16<KIND, ACT, false, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+      } else if (qv) {
+        w4_store_f16<KIND, ACT, true, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+      } else {
+        w4_store_f16<KIND, ACT, true, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
       }
-      else if (staged.has[3] || staged.has[4])
-        w4_store_f16<KIND, EPI == W4_EPI_BF16_GELU ? ACT_GELU : ACT_NONE, true, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
-      else
-        w4_store_f16<KIND, EPI == W4_EPI_BF16_GELU ? ACT_GELU : ACT_NONE, true, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
-      return true;
     }
-    // the element-wise epilogue stages the accumulators in LDS: let the stages in flight land first
-    wait_vmcnt_barrier<0>();
-    w4_store_general<KIND, WTP, WTQ>(prm, acc, (int *)&lds[0], p0, q0, NP, NQ, bt, wp, wq);
-    __syncthreads();
-    return false;
   };
 
   // The vectors along P that the epilogue of the tile at (p0, bt) needs, this wave's WTP entries of each, into the wave's
@@ -845,9 +817,11 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
     if constexpr (EPI != W4_EPI_I32 && !MX) {
       staged.has[0] = staged.has[1] = staged.has[2] = staged.has[3] = staged.has[4] = false;
       staged.bias_skip = 0;
-      if (fast && p0 + BP <= NP) {
+      {
         const int ln4 = w4_lane_here() * 4;
-        const int pc = p0 + wp * WTP;
+        // (a ragged last tile: what the vectors have of this wave's entries; the rest reads as zero and belongs to rows
+        // nobody stores)
+        const int pc = p0 + wp * WTP, pn = min(WTP, NP - pc);
         int *const area = (int *)&lds[2 * STAGE_V4] + wave * STG_WAVE;
         // 128 dwords of a slot (and the one behind them); what lies past `bytes` is out of range and lands as zero
         auto copy = [&](const void *src, int bytes, int slot) __attribute__((always_inline)) {
@@ -859,15 +833,15 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
         const float *v1 = swp ? (g.b_scale_mode == SCALE_OUTER_VEC ? (const float *)g.b_scale : nullptr)
                               : (g.alpha_mode == VECTOR_DEV ? (const float *)g.alpha_ptr + g.alpha_sb * bt : nullptr);
         const float *v2 = !swp && g.a_scale_mode == SCALE_OUTER_VEC ? (const float *)g.a_scale : nullptr;
-        if (v1 != nullptr) { copy(v1 + pc, WTP * 4, 0); staged.has[0] = true; }
-        if (v2 != nullptr) { copy(v2 + pc, WTP * 4, 1); staged.has[1] = true; }
-        if (!swp && g.bias != nullptr) {
+        if (v1 != nullptr && pn > 0) { copy(v1 + pc, pn * 4, 0); staged.has[0] = true; }
+        if (v2 != nullptr && pn > 0) { copy(v2 + pc, pn * 4, 1); staged.has[1] = true; }
+        if (!swp && g.bias != nullptr && pn > 0) {
           const int es = g.bias_type == CUDA_R_32F ? 4 : 2;
           const char *src = (const char *)g.bias + (g.bias_sb * bt + pc) * es;
           const int skip = (int)(((uintptr_t)src) & 3) >> 1;  // (dword loads)
-          // (whole dwords are range-checked: the last one of a skipped start ends two bytes past the vector, inside
-          // the aligned dword that holds the vector's last element)
-          copy(src - 2 * skip, WTP * es + 4 * skip, 2);
+          // (whole dwords are range-checked: the last one may end two bytes past the vector, inside the aligned dword that
+          // holds the vector's last element)
+          copy(src - 2 * skip, (pn * es + 2 * skip + 3) & ~3, 2);
           staged.has[2] = true;
           staged.bias_skip = skip;
         }
@@ -885,7 +859,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
 
   // ---- the stream -------------------------------------------------------------------------------------------------
   static_assert(!MX || NM >= NRD + TP + TQ, "room for the scale reads in a sub-step");
-  prime(0);
+  prime();
   if constexpr (MX) {
     scale_addr(0);
     static_for<TP + TQ>([&](auto r_c) { read_scale(std::integral_constant<int, 0>{}, r_c); });
@@ -908,13 +882,10 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
     if (n + 1 < my_tiles) dma_tile(n + 1);
     else d_live = 0;
     do_pair(0, std::integral_constant<int, 2>{});
-    const bool kept = epilogue(p0, q0, bt);
+    epilogue(p0, q0, bt);
     // The first fragments of the next tile are fetched again behind the epilogue (its first stage landed before the
     // last barrier): holding them across it would take 64 of the registers the epilogue needs.
-    if (n + 1 < my_tiles) {
-      if (kept) first_frags();
-      else prime(n + 1);
-    }
+    if (n + 1 < my_tiles) first_frags();
   }
   __builtin_amdgcn_s_waitcnt(0);  // the loads past the end of the list have landed before the wave ends
 }
