@@ -65,6 +65,13 @@ __device__ __forceinline__ void transpose2x2(int x0, int x1, int &lo, int &hi) {
   hi = __builtin_amdgcn_perm(x1, x0, 0x07060302);  // x0.h1 x1.h1
 }
 
+// Everything in flight has landed, said about these registers: what reads them is not moved in front of the wait.
+template <int N>
+__device__ __forceinline__ void wait_regs(int (&r)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; i++) asm volatile("s_waitcnt vmcnt(0)" : "+v"(r[i]));
+}
+
 // Global -> register -> LDS path of ROWS rows of a tile operand, served by 256 threads; KC: unit
 // stride along K; ESZ: bytes per element.
 template <int ROWS, bool KC, int ESZ = 1>
@@ -79,42 +86,60 @@ struct TrOperand {
   static_assert(ESZ == 1 || ESZ == 2 || ESZ == 4, "8-, 16- or 32-bit elements");
   static_assert(ROWS == 64 || ROWS == 128 || ROWS == 256, "64, 128 or 256 rows per group of 256 threads");
 
+  static constexpr int NX = ESZ == 2 ? (KC ? NCH : KR) : 1;  // 16-bit elements loaded on their own in the last stage
+
   __amdgpu_buffer_rsrc_t rs;
   int voff[KC ? NCH : 1];
   int kstep;     // byte offset of one stage
   int kbytes;    // bytes of K per row
   int ld;        // MC: stride of one K row
   int tc;        // KC: byte offset of this lane's chunk in a stage
+  int left;      // MC: row indices the matrix has from the lane's first one on (0: the lane lies behind the last row)
+  int x[NX];
 
   // base: first byte of the operand (this batch); row0: first tile row; nrows: rows of the whole
   // operand; ld_row / ld_k: byte strides (one of them is ESZ); K: elements along K
   // t: index of the thread among the 256 that load this operand
+  //
+  // Alignment-bound problems ran on the scalar kernel before this path existed (MI355X, us): bf16 1024 x 512 x 32003 with
+  // 32003-element pitches 7637 -> 62, 1024 x 32003 x 512 1086 -> 110; f32 1000 x 777 x 1003 219 -> 21; f16 701 x 333 x 517 99 -> 11.
+  //
+  // Neither the base nor the pitches need more alignment than an element (8-bit elements: a dword); the memory system
+  // takes dwords at any element's address.  The window is the operand's extent, and a dword counts as inside it when all
+  // of its bytes are (checked per dword, against the unaligned address), so no load reaches past the operand.
   __device__ __forceinline__ void init(int t, const uint8_t *base, int row0, int nrows, int ld_row, int ld_k, int K) {
     kbytes = K * ESZ;
     tc = (t & 3) * 16;
+    left = 0;
+#pragma unroll
+    for (int n = 0; n < NX; n++) x[n] = 0;
+    // (8-bit elements: up to the end of the last dword; base and pitches are multiples of 4 then)
+    constexpr int UP = ESZ == 1 ? 3 : 0;
     if constexpr (KC) {
-      rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 0x80000000, 0x00020000);
+      rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, ((nrows - 1) * ld_row + kbytes + UP) & ~UP, 0x00020000);
 #pragma unroll
       for (int n = 0; n < NCH; n++) voff[n] = min(row0 + (t >> 2) + 64 * n, nrows - 1) * ld_row + (t & 3) * 16;
       kstep = 64;
       ld = 0;
     } else {
-      // the operand's extent, up to the end of its last dword (the range check is per dword; base
-      // and ld_k are multiples of 4, so that dword lies in the same allocation granule): K rows past
-      // the end read as zero
-      rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, K > 0 ? (((K - 1) * ld_k + nrows * ESZ + 3) & ~3) : 0, 0x00020000);
-      voff[0] = ((t >> 4) * KR) * ld_k + (row0 + (t & 15) * IW) * ESZ;
+      // K rows past the end lie outside the window and read as zero
+      rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, K > 0 ? ((K - 1) * ld_k + nrows * ESZ + UP) & ~UP : 0, 0x00020000);
+      // (a lane behind the last row index reads the first ones instead: nobody stores what it multiplies, and an
+      // instruction of a stage in front of the last one is then never wholly out of range)
+      const int row = row0 + (t & 15) * IW;
+      left = max(nrows - row, 0);
+      voff[0] = ((t >> 4) * KR) * ld_k + (left > 0 ? row : 0) * ESZ;
       kstep = (64 / ESZ) * ld_k;
       ld = ld_k;
     }
   }
 
+  // stage kt, not the last one: every K index of it exists
   __device__ __forceinline__ void load(int kt, int (&regs)[NREG]) const {
     if constexpr (KC) {
 #pragma unroll
       for (int n = 0; n < NCH; n++) {
-        const int oob = kt * 64 + tc < kbytes ? 0 : (int)0x80000000;
-        const v4i v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, voff[n] | oob, kt * kstep, 0));
+        const v4i v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, voff[n], kt * kstep, 0));
         regs[n * 4 + 0] = v[0]; regs[n * 4 + 1] = v[1]; regs[n * 4 + 2] = v[2]; regs[n * 4 + 3] = v[3];
       }
     } else {
@@ -133,6 +158,51 @@ struct TrOperand {
           }
         }
       }
+    }
+  }
+
+  // The last stage (kt = the last stage that holds data), which may end inside a lane's piece.  A KC piece past the end of
+  // K is not fetched, one that holds the end brings what follows it in memory (finish_last() clears that).  Of 16-bit elements
+  // the operand's very last one may sit in a dword that lies only half inside the window and reads as zero: the last element
+  // along K (KC) or along the row index (MC) is therefore fetched on its own as well.
+  __device__ __forceinline__ void load_last(int kt, int (&regs)[NREG]) {
+    if constexpr (KC) {
+      const int have = kbytes - kt * 64 - tc;  // bytes of the lane's piece that exist
+#pragma unroll
+      for (int n = 0; n < NCH; n++) {
+        const v4i v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, have > 0 ? voff[n] : (int)0x80000000, kt * kstep, 0));
+        regs[n * 4 + 0] = v[0]; regs[n * 4 + 1] = v[1]; regs[n * 4 + 2] = v[2]; regs[n * 4 + 3] = v[3];
+        if constexpr (ESZ == 2)
+          x[n] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, have > 0 && have <= 16 ? voff[n] + have - 2 : (int)0x80000000, kt * kstep, 0);
+      }
+    } else {
+      load(kt, regs);
+      if constexpr (ESZ == 2) {
+#pragma unroll
+        for (int j = 0; j < KR; j++)
+          x[j] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, left > 0 && left <= IW ? voff[0] + j * ld + (left - 1) * 2 : (int)0x80000000, kt * kstep, 0);
+      }
+    }
+  }
+  // what load_last() brought, made whole; the caller has waited for everything in flight
+  __device__ __forceinline__ void finish_last(int kt, int (&regs)[NREG]) {
+    if constexpr (KC) {
+      const int have = kbytes - kt * 64 - tc;
+#pragma unroll
+      for (int n = 0; n < NCH; n++)
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+          const int b = have - 4 * d;  // bytes of this dword that exist
+          int r = regs[n * 4 + d];
+          if constexpr (ESZ == 2) r = b == 2 ? x[n] : r;
+          else if constexpr (ESZ == 1) r = b < 4 ? r & ((1 << (8 * max(b, 0))) - 1) : r;
+          regs[n * 4 + d] = b > 0 ? r : 0;
+        }
+    } else if constexpr (ESZ == 2) {
+#pragma unroll
+      for (int j = 0; j < KR; j++)
+#pragma unroll
+        for (int c = 0; c < NW; c++) regs[j * NW + c] = left == 2 * c + 1 ? x[j] : regs[j * NW + c];
     }
   }
 
@@ -230,14 +300,16 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
   }
   const int KT = (Kl * ESZ + 63) / 64;
   const int KL = max(KT - 1, 0);  // last stage that holds data
-  // K % 64 != 0: in the last stage a load instruction of an operand without unit K stride covers K rows
-  // 16 * wave + j + 4 * {0..3}; when even the first of them is past the end every lane of the instruction
-  // is out of range.  Such an instruction completes without a memory round trip and may be counted as done
-  // ahead of older loads, so a wait that leaves "the younger stage" in flight (what the compiler emits in
-  // front of the LDS stores, which consume the older stage's registers) could pass too early.  From the
-  // first trip whose younger stage is that last stage (stage kt + 2 >= KL) the stores are therefore preceded
-  // by a wait for everything.  With K % 64 == 0 no such instruction exists and nothing is added.
-  const int tail_from = tr_tail_from(Kl * ESZ);  // (mfma_wait_counts.hpp, where a host program checks it)
+  // The last stage goes its own way (load_last / finish_last), and so do the trips around it: whole trips (TAIL = 0) run
+  // while the stage they request, kt + 3, lies in front of it.
+  // In the last stage an instruction can have all of its lanes out of range (K rows past the end, the extra element of a
+  // lane that has none).  Such an instruction completes without a memory round trip and may be counted as done ahead of
+  // older loads, so a wait that leaves "the younger stage" in flight (what the compiler emits in front of the LDS stores,
+  // which consume the older stage's registers) could pass too early.  From the first trip whose younger stage is that
+  // last stage (stage kt + 2 >= KL) the stores are therefore preceded by a wait for everything.  With K % 64 == 0 no such
+  // instruction exists for 8- and 32-bit elements and nothing is added.
+  int tail_from = tr_tail_from(Kl * ESZ);  // (mfma_wait_counts.hpp, where a host program checks it)
+  if (ESZ == 2) tail_from = min(tail_from, KL - 2);
 
   // LDS rows (in v4i units) of this lane's fragment rows
   int prow[TP], qrow[TQ];
@@ -372,11 +444,25 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
   //   second half: loads of stage kt+3 into the sets just emptied, fragment reads of stage kt+1's
   //                sub-step 0, and the MFMAs of sub-step 1 that cover both.
   // (fp8 stages have a single sub-step: its MFMAs all run in the first half.)
-  auto stage_trip = [&](int kt, const v4i *cur, v4i *nxt, int (&sp)[P.NREG], int (&sq)[Q.NREG], Frags &f0) {
-    Frags f1;
-    // K tail: see tail_from above.  (The branch sits right behind the sched_barrier that ends the previous
-    // trip, so it does not cut a scheduling region.)
+  // stage kt whichever it is; nothing past the last one (nobody multiplies that)
+  auto load_any = [&](int kt, int (&sp)[P.NREG], int (&sq)[Q.NREG]) {
+    if (kt < KL) { P.load(kt, sp); Q.load(kt, sq); }
+    else if (kt == KL) { P.load_last(kt, sp); Q.load_last(kt, sq); }
+  };
+  // tail_c: the trips around the last stage (see tail_from above).  (The branches sit right behind the sched_barrier that
+  // ends the previous trip, so they do not cut a scheduling region.)
+  auto enter_tail = [&](int kt, int (&sp)[P.NREG], int (&sq)[Q.NREG]) {
     if (kt >= tail_from) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (kt + 1 == KL) {
+      wait_regs(sp); wait_regs(P.x); wait_regs(sq); wait_regs(Q.x);
+      P.finish_last(KL, sp); Q.finish_last(KL, sq);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto stage_trip = [&](int kt, const v4i *cur, v4i *nxt, int (&sp)[P.NREG], int (&sq)[Q.NREG], Frags &f0, auto tail_c) {
+    constexpr bool TAIL = decltype(tail_c)::value != 0;
+    Frags f1;
+    if constexpr (TAIL) enter_tail(kt, sp, sq);
     if constexpr (KS == 2) read_frags(cur, 1, f1);
     P.store(tl, nxt + lds_p, sp);
     Q.store(tl, nxt + lds_q, sq);
@@ -406,16 +492,17 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
-    // Past the end the last stage is fetched once more (nothing multiplies it).  Not an out-of-range
-    // stage: instructions whose lanes are all out of range complete without a memory round trip and
-    // can retire ahead of older loads, while the compiler's vmcnt waits count on in-order return.
-    P.load(min(kt + 3, KL), sp);
-    Q.load(min(kt + 3, KL), sq);
+    if constexpr (TAIL) {
+      load_any(kt + 3, sp, sq);
+    } else {
+      P.load(kt + 3, sp);
+      Q.load(kt + 3, sq);
+    }
     read_frags(nxt, 0, f0);
     if constexpr (KS == 2) {
       mfma_all(f1);
       constexpr int NM = TP * TQ * MPS, NDR = TP + TQ;
-      constexpr int NVM = P.NLOADS + Q.NLOADS;
+      constexpr int NVM = TAIL ? 0 : P.NLOADS + Q.NLOADS;
       static_for<NM>([&](auto i_c) {
         constexpr int i = decltype(i_c)::value;
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -433,13 +520,14 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
   //   first half : MFMAs of P half 0; P half 1 is read and stage kt+1 transposed into `nxt` between them;
   //   barrier;
   //   second half: MFMAs of P half 1 cover the loads of stage kt+3 and the reads of stage kt+1's P half 0 and Q.
-  auto stage_trip16 = [&](int kt, const v4i *cur, v4i *nxt, int (&sp)[P.NREG], int (&sq)[Q.NREG], auto par_c) {
+  auto stage_trip16 = [&](int kt, const v4i *cur, v4i *nxt, int (&sp)[P.NREG], int (&sq)[Q.NREG], auto par_c, auto tail_c) {
+    constexpr bool TAIL = decltype(tail_c)::value != 0;
     constexpr int PAR = decltype(par_c)::value;
     using H0 = std::integral_constant<int, 0>;
     using H1 = std::integral_constant<int, 1>;
     using SC = std::integral_constant<int, PAR>;
     using SN = std::integral_constant<int, 1 - PAR>;
-    if (kt >= tail_from) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (TAIL) enter_tail(kt, sp, sq);
     read_p16(cur, H1{});
     P.store(tl, nxt + lds_p, sp);
     Q.store(tl, nxt + lds_q, sq);
@@ -466,14 +554,18 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
-    P.load(min(kt + 3, KL), sp);
-    Q.load(min(kt + 3, KL), sq);
+    if constexpr (TAIL) {
+      load_any(kt + 3, sp, sq);
+    } else {
+      P.load(kt + 3, sp);
+      Q.load(kt + 3, sq);
+    }
     read_p16(nxt, H0{});
     read_q16(nxt, SN{});
     mfma16(H1{}, SC{});
     {
       constexpr int NM = HP16 * TQ16, NDR = HP16 + TQ16;
-      constexpr int NVM = P.NLOADS + Q.NLOADS;
+      constexpr int NVM = TAIL ? 0 : P.NLOADS + Q.NLOADS;
       static_for<NM>([&](auto i_c) {
         constexpr int i = decltype(i_c)::value;
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -490,25 +582,42 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
   int rp0[P.NREG], rp1[P.NREG], rq0[Q.NREG], rq1[Q.NREG];
   v4i *buf0 = &lds[0], *buf1 = &lds[STAGE_V4];
   Frags f0;
-  P.load(0, rp0); Q.load(0, rq0);
-  P.load(min(1, KL), rp1); Q.load(min(1, KL), rq1);
+  load_any(0, rp0, rq0);
+  load_any(1, rp1, rq1);
   if (tail_from < 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // stage 1 is already the K tail
+  if (KL == 0) {
+    wait_regs(rp0); wait_regs(P.x); wait_regs(rq0); wait_regs(Q.x);
+    P.finish_last(0, rp0); Q.finish_last(0, rq0);
+  }
   P.store(tl, buf0 + lds_p, rp0);
   Q.store(tl, buf0 + lds_q, rq0);
   __syncthreads();
-  P.load(min(2, KL), rp0); Q.load(min(2, KL), rq0);
+  load_any(2, rp0, rq0);
+  using W = std::integral_constant<int, 0>;
+  using T = std::integral_constant<int, 1>;
+  int kt = 0;
   if constexpr (M16) {
-    read_p16(buf0, std::integral_constant<int, 0>{});
-    read_q16(buf0, std::integral_constant<int, 0>{});
-    for (int kt = 0; kt < KT; kt += 2) {
-      stage_trip16(kt, buf0, buf1, rp1, rq1, std::integral_constant<int, 0>{});
-      if (kt + 1 < KT) stage_trip16(kt + 1, buf1, buf0, rp0, rq0, std::integral_constant<int, 1>{});
+    using E = std::integral_constant<int, 0>;
+    using O = std::integral_constant<int, 1>;
+    read_p16(buf0, E{});
+    read_q16(buf0, E{});
+    for (; kt + 4 < KL; kt += 2) {
+      stage_trip16(kt, buf0, buf1, rp1, rq1, E{}, W{});
+      stage_trip16(kt + 1, buf1, buf0, rp0, rq0, O{}, W{});
+    }
+    for (; kt < KT; kt += 2) {
+      stage_trip16(kt, buf0, buf1, rp1, rq1, E{}, T{});
+      if (kt + 1 < KT) stage_trip16(kt + 1, buf1, buf0, rp0, rq0, O{}, T{});
     }
   } else {
     read_frags(buf0, 0, f0);
-    for (int kt = 0; kt < KT; kt += 2) {
-      stage_trip(kt, buf0, buf1, rp1, rq1, f0);
-      if (kt + 1 < KT) stage_trip(kt + 1, buf1, buf0, rp0, rq0, f0);
+    for (; kt + 4 < KL; kt += 2) {
+      stage_trip(kt, buf0, buf1, rp1, rq1, f0, W{});
+      stage_trip(kt + 1, buf1, buf0, rp0, rq0, f0, W{});
+    }
+    for (; kt < KT; kt += 2) {
+      stage_trip(kt, buf0, buf1, rp1, rq1, f0, T{});
+      if (kt + 1 < KT) stage_trip(kt + 1, buf1, buf0, rp0, rq0, f0, T{});
     }
   }
 

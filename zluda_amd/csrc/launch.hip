@@ -285,6 +285,11 @@ uint32_t launch_planned(const zluda_gemm_problem *p, const zluda_gemm_plan *plan
   }
   switch (plan->kernel) {
   case ZLUDA_KERNEL_GENERIC: {
+    zluda_gemm_plan tr;
+    if (plan_transposing_under_generic(l, zluda_gemm_device_cu_count(), plan->workspace, &tr)) {
+      st = launch_tr(l, tr, ws, ws_size, s);
+      break;
+    }
     dim3 grid(plan->grid_x, plan->grid_y, plan->grid_z);
     const bool int_acc = l.g.a_type == CUDA_R_8I;
     st = int_acc ? launch_kernel(gemm_generic_kernel<true>, grid, dim3(256), s, l.g)

@@ -279,11 +279,42 @@ static bool any_decode_variant_ok(const Lowered &l) {
   return false;
 }
 
+static bool d_type_fast(const GemmArgs &g) {
+  return g.d_type == CUDA_R_32I || g.d_type == CUDA_R_32F || g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_8I;
+}
+
+// The family of the transposing kernel that runs the operands (TR8: 8-bit, TR16: 16-bit, TR32: f32), each with unit stride
+// along K or along its row index, or 0.  The families themselves take dword-aligned operands whose K-contiguous rows are
+// whole 16-byte pieces; the kernel takes more (`any_pitch`): 16-bit and f32 operands at any element's address and any
+// pitch, and K-contiguous rows that end anywhere.
+static uint32_t transposing_family(const Lowered &l, bool any_pitch) {
+  const GemmArgs &g = l.g;
+  const bool h16 = g.a_type == CUDA_R_16F || g.a_type == CUDA_R_16BF, f32 = g.a_type == CUDA_R_32F;
+  const bool i8 = g.a_type == CUDA_R_8I && g.b_type == CUDA_R_8I;
+  const bool f8 = is_f8(g.a_type) && is_f8(g.b_type) && !(g.a_type == CUDA_R_8F_E5M2 && g.b_type == CUDA_R_8F_E5M2);
+  if (!d_type_fast(g) || g.a_scale_mode == SCALE_BLOCK32_UE8M0 || g.b_scale_mode == SCALE_BLOCK32_UE8M0) return 0;
+  if (!(i8 || f8 || ((h16 || f32) && g.b_type == g.a_type))) return 0;
+  const int64_t esz = f32 ? 4 : h16 ? 2 : 1;
+  const int64_t align = (any_pitch && h16 ? 2 : 4) - 1;
+  // (strides in bytes from here on)
+  auto operand_ok = [&](const void *ptr, int64_t s_row, int64_t s_k, int64_t s_b, int rows) {
+    s_row *= esz; s_k *= esz; s_b *= esz;
+    if ((((uintptr_t)ptr) & align) || (g.batch > 1 && (s_b & align))) return false;
+    const int64_t span = (int64_t)(rows - 1) * s_row + (int64_t)(g.K - 1) * s_k + esz;
+    if (span >= 0x7fffffffll) return false;
+    if (s_k == esz) return (s_row & align) == 0 && (any_pitch || ((g.K * esz) & 15) == 0);
+    // (offsets of K rows up to three stages past the end must stay below 2^32, where they are out
+    // of range instead of wrapping into it)
+    return s_row == esz && (s_k & align) == 0 && (int64_t)(g.K + 256) * s_k < 0xffffffffll;
+  };
+  if (!operand_ok(g.A, g.a_si, g.a_sk, g.a_sb, g.M) || !operand_ok(g.B, g.b_sj, g.b_sk, g.b_sb, g.N)) return 0;
+  return f32 ? ZLUDA_KERNEL_MFMA_TR32 : h16 ? ZLUDA_KERNEL_MFMA_TR16 : ZLUDA_KERNEL_MFMA_TR8;
+}
+
 bool family_supports(uint32_t kernel, const Lowered &l) {
   const GemmArgs &g = l.g;
   const bool fast_layout = l.a_kcontig && l.b_kcontig && l.aligned16;
-  const bool d_fast = g.d_type == CUDA_R_32I || g.d_type == CUDA_R_32F || g.d_type == CUDA_R_16BF ||
-                      g.d_type == CUDA_R_16F || g.d_type == CUDA_R_8I;
+  const bool d_fast = d_type_fast(g);
   switch (kernel) {
   case ZLUDA_KERNEL_GENERIC: return true;
   case ZLUDA_KERNEL_MFMA_I8:
@@ -302,29 +333,8 @@ bool family_supports(uint32_t kernel, const Lowered &l) {
            g.a_scale_mode != SCALE_BLOCK32_UE8M0 && g.b_scale_mode != SCALE_BLOCK32_UE8M0 && d_fast;
   case ZLUDA_KERNEL_MFMA_F32:
     return fast_layout && l.span_ok && g.a_type == CUDA_R_32F && g.b_type == CUDA_R_32F && d_fast;
-  case ZLUDA_KERNEL_MFMA_TR8: case ZLUDA_KERNEL_MFMA_TR16: case ZLUDA_KERNEL_MFMA_TR32: {
-    // 8-bit (TR8), 16-bit (TR16) or f32 (TR32) operands, each with unit stride along K or along its row index; dword-aligned loads
-    const bool h16 = g.a_type == CUDA_R_16F || g.a_type == CUDA_R_16BF, f32 = g.a_type == CUDA_R_32F;
-    const bool types = kernel == ZLUDA_KERNEL_MFMA_TR32 ? (f32 && g.b_type == CUDA_R_32F)
-                       : kernel == ZLUDA_KERNEL_MFMA_TR16
-                           ? (h16 && g.b_type == g.a_type)
-                           : ((g.a_type == CUDA_R_8I && g.b_type == CUDA_R_8I) ||
-                              (is_f8(g.a_type) && is_f8(g.b_type) && !(g.a_type == CUDA_R_8F_E5M2 && g.b_type == CUDA_R_8F_E5M2)));
-    const int64_t esz = f32 ? 4 : h16 ? 2 : 1;
-    // (strides in bytes from here on)
-    auto operand_ok = [&](const void *ptr, int64_t s_row, int64_t s_k, int64_t s_b, int rows) {
-      s_row *= esz; s_k *= esz; s_b *= esz;
-      if ((((uintptr_t)ptr) & 3) || (g.batch > 1 && (s_b & 3))) return false;
-      const int64_t span = (int64_t)(rows - 1) * s_row + (int64_t)(g.K - 1) * s_k + esz;
-      if (span >= 0x7fffffffll) return false;
-      if (s_k == esz) return (s_row & 3) == 0 && ((g.K * esz) & 15) == 0;  // 16-byte pieces along K
-      // (offsets of K rows up to three stages past the end must stay below 2^32, where they are out
-      // of range instead of wrapping into it)
-      return s_row == esz && (s_k & 3) == 0 && (int64_t)(g.K + 256) * s_k < 0xffffffffll;
-    };
-    return types && d_fast && g.a_scale_mode != SCALE_BLOCK32_UE8M0 && g.b_scale_mode != SCALE_BLOCK32_UE8M0 &&
-           operand_ok(g.A, g.a_si, g.a_sk, g.a_sb, g.M) && operand_ok(g.B, g.b_sj, g.b_sk, g.b_sb, g.N);
-  }
+  case ZLUDA_KERNEL_MFMA_TR8: case ZLUDA_KERNEL_MFMA_TR16: case ZLUDA_KERNEL_MFMA_TR32:
+    return transposing_family(l, false) == kernel;
   case ZLUDA_KERNEL_DECODE_W8A8:
     // int8, or e4m3 x e4m3 without block scales (the LDS-streaming variants only), or f16 / bf16 (the slab form only)
     return fast_layout && ((g.a_type == CUDA_R_8I && g.b_type == CUDA_R_8I) ||
@@ -539,6 +549,17 @@ static int pick_tr_variant(const Lowered &l, uint32_t cus) {
   return best;
 }
 
+uint32_t plan_transposing_under_generic(const Lowered &l, uint32_t cus, uint64_t workspace_size, zluda_gemm_plan *plan) {
+  const uint32_t family = transposing_family(l, true);
+  if (!family || transposing_family(l, false)) return 0;
+  for (uint32_t k : {ZLUDA_KERNEL_MFMA_I8, ZLUDA_KERNEL_MFMA_F8, ZLUDA_KERNEL_MFMA_H16, ZLUDA_KERNEL_MFMA_F32})
+    if (family_supports(k, l)) return 0;
+  memset(plan, 0, sizeof(*plan));
+  plan->kernel = family;
+  fill_tr_plan(l, pick_tr_variant(l, cus), cus, workspace_size, plan);
+  return family;
+}
+
 static void fill_decode_plan(const Lowered &l, int variant, uint32_t cus, zluda_gemm_plan *plan) {
   const GemmArgs &g = l.g;
   const DecodeVariant &v = kDecodeVariants[variant];
@@ -664,6 +685,12 @@ extern "C" uint32_t zluda_gemm_plan_problem(const zluda_gemm_problem *p, uint32_
     plan->block = 256;
     plan->waves = (float)plan->grid_x * plan->grid_y * plan->grid_z / (float)(cu_count * 8);
     if (plan->grid_y > 65535) return CUBLAS_STATUS_NOT_SUPPORTED;
+    {
+      // what only alignment or a ragged K keeps from the transposing kernel runs on it all the same (launch_planned); its
+      // split along K wants scratch like any other
+      zluda_gemm_plan tr;
+      if (plan_transposing_under_generic(l, cu_count, p->workspace_size, &tr)) { plan->workspace = tr.workspace; plan->waves = tr.waves; }
+    }
     break;
   case ZLUDA_KERNEL_MFMA_I8: case ZLUDA_KERNEL_MFMA_F8: case ZLUDA_KERNEL_MFMA_MXF4: case ZLUDA_KERNEL_MFMA_H16:
   case ZLUDA_KERNEL_MFMA_F32: {
