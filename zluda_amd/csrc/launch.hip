@@ -75,7 +75,7 @@ uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws,
   if (plan.grid_z > 1) {
     // split-K: partial tiles go through the caller's workspace
     const uint64_t need = (uint64_t)plan.grid_z * l.g.batch * prm.tiles_p * v.bp * prm.tiles_q * v.bq * 4;
-    if (!ws || (((uintptr_t)ws) & 15) || ws_size < need || plan.workspace != need) return CUBLAS_STATUS_INVALID_VALUE;
+    if (!ws || (((uintptr_t)ws) & 15) || ws_size < need || plan.workspace < need) return CUBLAS_STATUS_INVALID_VALUE;
     const bool mx = plan.kernel == ZLUDA_KERNEL_MFMA_MXF4;
     const int kbytes = mx ? l.g.K / 2 : (plan.kernel == ZLUDA_KERNEL_MFMA_H16 ? l.g.K * 2 : plan.kernel == ZLUDA_KERNEL_MFMA_F32 ? l.g.K * 4 : l.g.K);
     const int stages = (kbytes + v.bkb - 1) / v.bkb;
@@ -128,7 +128,7 @@ uint32_t launch_tr(const Lowered &l, const zluda_gemm_plan &plan, void *ws, uint
   if (plan.grid_z > 1) {
     // split-K: partial tiles go through the caller's workspace (64 K bytes per stage)
     const uint64_t need = (uint64_t)plan.grid_z * l.g.batch * prm.tiles_p * v.bp * prm.tiles_q * v.bq * 4;
-    if (!ws || (((uintptr_t)ws) & 15) || ws_size < need || plan.workspace != need) return CUBLAS_STATUS_INVALID_VALUE;
+    if (!ws || (((uintptr_t)ws) & 15) || ws_size < need || plan.workspace < need) return CUBLAS_STATUS_INVALID_VALUE;
     const int stages = (l.g.K * (plan.kernel == ZLUDA_KERNEL_MFMA_TR16 ? 2 : plan.kernel == ZLUDA_KERNEL_MFMA_TR32 ? 4 : 1) + 63) / 64;
     prm.splits = (int32_t)plan.grid_z;
     prm.split_stages = (stages + prm.splits - 1) / prm.splits;
@@ -248,12 +248,36 @@ extern "C" uint32_t zluda_gemm_device_cu_count(void) {
 
 namespace zluda_amd {
 
+namespace {
+
+uint32_t finish_sums(const void *part, int shares, int rows, int batch, bool ints, void *out, uint32_t out_type, int64_t out_sb, hipStream_t s) {
+  BgradFinishParams f{part, shares, rows, ints ? 1 : 0, out, out_type, out_sb};
+  return launch_kernel(bgrad_finish_kernel, dim3((rows + 63) / 64, 1, batch), dim3(256), s, f);
+}
+
+// LANES of the row-sum kernels: 16-byte pieces side by side.  Four (whole 64-byte pieces of memory) give the most
+// workgroups, which is what a share-less reduction wants; with K shared out eight read whole cache lines.
+template <uint32_t TYPE>
+uint32_t launch_bgrad_typed(BgradParams &b, void *ws, uint64_t ws_size, hipStream_t s) {
+  constexpr int V = elems16(TYPE), ESZ = 16 / V;
+  b.wide = !(((uintptr_t)b.src | (uintptr_t)(b.s_b * ESZ) | (uintptr_t)((b.s_k <= b.s_row ? b.s_row : b.s_k) * ESZ)) & 15);
+  if (b.s_k <= b.s_row) return launch_kernel(bgrad_rows_kernel<TYPE>, dim3(b.rows, 1, b.batch), dim3(256), s, b);
+  const uint32_t shares = row_sum_shares(b.rows, b.K, b.batch, ws ? ws_size : 0);
+  b.per_block = (int32_t)((b.K + shares - 1) / shares);
+  b.part = ws;
+  uint32_t st;
+  if (shares > 1) st = launch_kernel(bgrad_cols_kernel<TYPE, 8>, dim3((b.rows + 8 * V - 1) / (8 * V), shares, b.batch), dim3(512), s, b);
+  else st = launch_kernel(bgrad_cols_kernel<TYPE, 4>, dim3((b.rows + 4 * V - 1) / (4 * V), 1, b.batch), dim3(512), s, b);
+  if (st || shares == 1) return st;
+  return finish_sums(ws, (int)shares, b.rows, b.batch, TYPE == CUDA_R_8I, b.out, b.out_type, b.out_sb, s);
+}
+
 // BGRADA / BGRADB: the K sums of one operand into the bias buffer, behind the matmul on its stream
-static uint32_t launch_bgrad(const GemmArgs &g, hipStream_t s) {
+uint32_t launch_bgrad(const GemmArgs &g, void *ws, uint64_t ws_size, hipStream_t s) {
   BgradParams b;
+  memset(&b, 0, sizeof(b));
   const bool of_a = g.bgrad_src == 1;
   b.src = of_a ? g.A : g.B;
-  b.type = of_a ? g.a_type : g.b_type;
   b.rows = of_a ? g.M : g.N;
   b.K = g.K;
   b.batch = g.batch;
@@ -263,9 +287,56 @@ static uint32_t launch_bgrad(const GemmArgs &g, hipStream_t s) {
   b.out = g.bgrad;
   b.out_type = g.bias_type;
   b.out_sb = g.bias_sb;
-  if (b.s_k <= b.s_row) return launch_kernel(bgrad_rows_kernel, dim3(b.rows, b.batch), dim3(256), s, b);
-  return launch_kernel(bgrad_cols_kernel, dim3((b.rows + 255) / 256, b.batch), dim3(256), s, b);
+  switch (of_a ? g.a_type : g.b_type) {
+  case CUDA_R_32F: return launch_bgrad_typed<CUDA_R_32F>(b, ws, ws_size, s);
+  case CUDA_R_16F: return launch_bgrad_typed<CUDA_R_16F>(b, ws, ws_size, s);
+  case CUDA_R_16BF: return launch_bgrad_typed<CUDA_R_16BF>(b, ws, ws_size, s);
+  case CUDA_R_8I: return launch_bgrad_typed<CUDA_R_8I>(b, ws, ws_size, s);
+  case CUDA_R_8F_E4M3: return launch_bgrad_typed<CUDA_R_8F_E4M3>(b, ws, ws_size, s);
+  case CUDA_R_8F_E5M2: return launch_bgrad_typed<CUDA_R_8F_E5M2>(b, ws, ws_size, s);
+  default: return CUBLAS_STATUS_NOT_SUPPORTED;
+  }
 }
+
+template <uint32_t TYPE>
+uint32_t launch_aux_typed(const GemmArgs &g, void *ws, uint64_t ws_size, hipStream_t s) {
+  constexpr int V = elems16(TYPE), ESZ = 16 / V;
+  const bool col = g.d_si == 1;
+  AuxParams a;
+  memset(&a, 0, sizeof(a));
+  a.D = g.D; a.aux = g.aux;
+  a.NP = col ? g.M : g.N; a.NQ = col ? g.N : g.M; a.batch = g.batch;
+  a.d_sq = col ? g.d_sj : g.d_si; a.d_sb = g.d_sb;
+  a.aux_sq = col ? g.aux_sj : g.aux_si; a.aux_sb = g.aux_sb;
+  a.d_scale = g.d_scale;
+  a.wide = !(((uintptr_t)a.D | (uintptr_t)a.aux | (uintptr_t)(a.d_sq * ESZ) | (uintptr_t)(a.aux_sq * ESZ) |
+              (g.batch > 1 ? (uintptr_t)(a.d_sb * ESZ) | (uintptr_t)(a.aux_sb * ESZ) : 0)) & 15);
+  const uint64_t pieces = (uint64_t)((a.NP + V - 1) / V) * a.NQ;
+  if (g.aux_mode == 1) return launch_kernel(aux_gelu_kernel<TYPE>, dim3((uint32_t)((pieces + 255) / 256), 1, g.batch), dim3(256), s, a);
+  a.sums = g.aux_bgrad;
+  a.out = g.bgrad; a.out_type = g.bias_type; a.out_sb = g.bias_sb;
+  if (!col && a.sums) return launch_kernel(aux_dgelu_rows_kernel<TYPE>, dim3(a.NQ, 1, g.batch), dim3(256), s, a);
+  // (without sums nothing is carried from one share of Q to another)
+  const uint32_t shares = row_sum_shares(a.NP, a.NQ, g.batch, !a.sums ? ~0ull : ws ? ws_size : 0);
+  a.per_block = (int32_t)((a.NQ + shares - 1) / shares);
+  a.part = ws;
+  uint32_t st;
+  if (shares > 1) st = launch_kernel(aux_dgelu_kernel<TYPE, 32>, dim3((a.NP + 32 * V - 1) / (32 * V), shares, g.batch), dim3(512), s, a);
+  else st = launch_kernel(aux_dgelu_kernel<TYPE, 4>, dim3((a.NP + 4 * V - 1) / (4 * V), 1, g.batch), dim3(512), s, a);
+  if (st || shares == 1 || !a.sums) return st;
+  return finish_sums(ws, (int)shares, a.NP, g.batch, false, g.bgrad, g.bias_type, g.bias_sb, s);
+}
+
+uint32_t launch_aux(const GemmArgs &g, void *ws, uint64_t ws_size, hipStream_t s) {
+  switch (g.d_type) {
+  case CUDA_R_32F: return launch_aux_typed<CUDA_R_32F>(g, ws, ws_size, s);
+  case CUDA_R_16F: return launch_aux_typed<CUDA_R_16F>(g, ws, ws_size, s);
+  case CUDA_R_16BF: return launch_aux_typed<CUDA_R_16BF>(g, ws, ws_size, s);
+  default: return CUBLAS_STATUS_NOT_SUPPORTED;
+  }
+}
+
+} // namespace
 
 uint32_t launch_planned(const zluda_gemm_problem *p, const zluda_gemm_plan *plan, void *ws, uint64_t ws_size, void *stream) {
   hipStream_t s = (hipStream_t)stream;
@@ -304,11 +375,10 @@ uint32_t launch_planned(const zluda_gemm_problem *p, const zluda_gemm_plan *plan
   case ZLUDA_KERNEL_MFMA_TR8: case ZLUDA_KERNEL_MFMA_TR16: case ZLUDA_KERNEL_MFMA_TR32: st = launch_tr(l, *plan, ws, ws_size, s); break;
   default: return CUBLAS_STATUS_NOT_SUPPORTED;
   }
-  if (st == CUBLAS_STATUS_SUCCESS && l.g.bgrad_src) st = launch_bgrad(l.g, s);
-  if (st == CUBLAS_STATUS_SUCCESS && whole.aux_mode == 1)
-    st = launch_kernel(aux_gelu_kernel, dim3((uint32_t)(((int64_t)whole.M * whole.N + 255) / 256), whole.batch), dim3(256), s, whole);
-  if (st == CUBLAS_STATUS_SUCCESS && whole.aux_mode == 2)
-    st = launch_kernel(aux_dgelu_kernel, dim3((whole.M + (whole.d_si == 1 ? 63 : 3)) / (whole.d_si == 1 ? 64 : 4), whole.batch), dim3(256), s, whole);
+  // (the kernels behind the matmul on its stream take over its scratch)
+  void *const sums = (((uintptr_t)ws) & 15) ? nullptr : ws;
+  if (st == CUBLAS_STATUS_SUCCESS && l.g.bgrad_src) st = launch_bgrad(l.g, sums, ws_size, s);
+  if (st == CUBLAS_STATUS_SUCCESS && whole.aux_mode) st = launch_aux(whole, sums, ws_size, s);
   return st;
 }
 

@@ -116,6 +116,10 @@ uint32_t plan_transposing_under_generic(const Lowered &l, uint32_t cus, uint64_t
 // which kernel families can run the lowered problem
 bool family_supports(uint32_t kernel, const Lowered &l);
 
+// Row sums along the longer stride (bias gradients): how many workgroups share the `len` terms of each of `rows` sums, given
+// scratch for shares * rows * batch partial sums of 4 bytes; 1: no scratch is used
+uint32_t row_sum_shares(int64_t rows, int64_t len, int64_t batch, uint64_t workspace_size);
+
 // Lowers `p` with its real pointers and enqueues the kernel `plan` names on `stream` (a hipStream_t).
 // `ws` / `ws_size`: device scratch for split-K partial tiles, at least plan->workspace bytes.
 uint32_t launch_planned(const zluda_gemm_problem *p, const zluda_gemm_plan *plan, void *ws, uint64_t ws_size, void *stream);
