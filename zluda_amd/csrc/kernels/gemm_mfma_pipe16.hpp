@@ -26,6 +26,18 @@
 //     there ("|"), and behind it the slot is refilled with stage kt+2 while the last two sub-steps fetch
 //     the first fragments of stage kt+1 from the other slot into the registers that have just become free.
 //     The fragment registers (both P halves, both Q halves) are as many as in gemm_mfma_pipe.hpp.
+//
+// 16-bit operands with unit stride along their row index ("MC": PMC / QMC; D^T and the gradients of a training step) go
+// through the same loop: the DMA copies 64 K rows of 128 or 256 elements as they lie in memory, and ds_read_b64_tr_b16
+// (16 lanes read 4 K rows x 16 elements; lane i gets the four K elements of row i) transposes on the way into the
+// fragments, so there is no work in registers and no store to LDS.  The kernel of gemm_mfma_tr.hpp, which transposes in
+// registers, spends its stages on that: bf16 8192^3 A:N B:N 1019 us there, 808 here; 4096^3 A:N B:N 107; 128 x 128 tiles,
+// 2048 x 4096 x 8192 A:N B:N 183 and 133 inside a training step.
+// LDS layout of such an operand: blocks of 1 KiB, one DMA instruction of a wave each, at a pitch of 1056 bytes.  A block
+// holds the K rows {k, k + 4} (256 elements a row) or {k, k + 4, k + 32, k + 36} (128), and the blocks run over k = 0..3,
+// 8..11, 16..19, ...: a ds_read_b64_tr_b16 takes the rows k..k+3 of four blocks for each of its groups of 16 lanes, 32
+// bytes of each; the pitch puts eight blocks in a row on different banks, and every fragment of a stage is one register
+// plus an immediate away.
 #pragma once
 #include "gemm_mfma_pipe.hpp"
 #include "mfma_wait_counts.hpp"
@@ -252,8 +264,36 @@ __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&
 }
 
 // ---- the kernel ----------------------------------------------------------------------------------------
-template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ>
+// An MC operand's block of LDS (head of this file): the K row of its first lane, and where K row `k` & 36 lies in its block
+__host__ __device__ constexpr int mc_block_k(int blk) { return (blk & 3) + 8 * ((blk >> 2) & 3) + 32 * (blk >> 4); }
+constexpr int kMcPitch = 1056;
+typedef short v4s_tr __attribute__((ext_vector_type(4)));
+
+// four K elements of one row of an MC operand: 16 lanes, each with the address of 8 bytes (lane 4r + c: K row r, elements
+// 4c .. 4c+3), get the K rows 0..3 of element `lane`
+__device__ __forceinline__ v2i lds_read_tr16(const char *src) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_tr *)src));
+#else
+  return v2i{0, 0};
+#endif
+}
+
+// lds_dma16() where ds_read_b64_tr_b16 reads what it brings: the compiler would put s_waitcnt vmcnt(0) in front of every
+// such read that follows the builtin (it does not follow which slot is read), i.e. wait for the stage just requested.  The
+// waits for it are the kernel's own.  The wait states: after M0, and for a resource or offset that came out of a VALU
+// instruction (v_readlane of a spilled SGPR).
+__device__ __forceinline__ void lds_dma16_uncounted(v4i rs, const void *lds_dst, int voff, int soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char *)lds_dst;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(voff), "s"(rs), "s"(soff) : "m0");
+#endif
+}
+
+template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, bool PMC = false, bool QMC = false>
 __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParams prm) {
+  static_assert(!(PMC || QMC) || kind_is_h16(KIND), "the transposing LDS reads are those of 16-bit elements");
+  static_assert((!PMC || BP == 256 || BP == 128) && (!QMC || BQ == 256 || BQ == 128), "rows of 1 KiB / 2 or / 4");
   static_assert(KIND == KIND_I8 || KIND == KIND_F8 || kind_is_h16(KIND), "int8, fp8, f16 and bf16 operands");
   constexpr int ESZ = kind_esz(KIND);          // f16 / bf16: the byte geometry of int8 (v_mfma_f32_16x16x32_*: 16 bytes of K per lane)
   constexpr int NT = WP * WQ * 64, NWV = NT / 64;
@@ -267,7 +307,9 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   constexpr int HP = TP / 2, HQ = TQ / 2;      // fragments per half of the wave tile
   constexpr int KS = KIND == KIND_F8 ? 1 : 2;  // MFMAs per fragment pair (K halves of the 128-byte stage)
   constexpr int NSTAGE = 2;
-  constexpr int STAGE_V4 = (BP + BQ) * CPR;    // one slot in 16-byte words: P rows, then Q rows
+  // one slot in 16-byte words: P rows, then Q rows
+  constexpr int P_V4 = PMC ? BP / 8 * (kMcPitch / 16) : BP * CPR, Q_V4 = QMC ? BQ / 8 * (kMcPitch / 16) : BQ * CPR;
+  constexpr int STAGE_V4 = P_V4 + Q_V4;
   static_assert(BP % RPP == 0 && BQ % RPP == 0, "tile / copy-pass mismatch");
   static_assert(WTP % 32 == 0 && WTQ % 32 == 0, "wave tiles start on multiples of 32 rows (fragment swizzle)");
   static_assert(NSTAGE * STAGE_V4 * 16 <= 160 * 1024, "LDS capacity");
@@ -298,11 +340,11 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   const uint8_t *Pg, *Qg;
   int ldp, ldq;
   if (!prm.swapped) {
-    Pg = (const uint8_t *)g.A + g.a_sb * bt * ESZ; ldp = (int)g.a_si * ESZ;
-    Qg = (const uint8_t *)g.B + g.b_sb * bt * ESZ; ldq = (int)g.b_sj * ESZ;
+    Pg = (const uint8_t *)g.A + g.a_sb * bt * ESZ; ldp = (int)(PMC ? g.a_sk : g.a_si) * ESZ;
+    Qg = (const uint8_t *)g.B + g.b_sb * bt * ESZ; ldq = (int)(QMC ? g.b_sk : g.b_sj) * ESZ;
   } else {
-    Pg = (const uint8_t *)g.B + g.b_sb * bt * ESZ; ldp = (int)g.b_sj * ESZ;
-    Qg = (const uint8_t *)g.A + g.a_sb * bt * ESZ; ldq = (int)g.a_si * ESZ;
+    Pg = (const uint8_t *)g.B + g.b_sb * bt * ESZ; ldp = (int)(PMC ? g.b_sk : g.b_sj) * ESZ;
+    Qg = (const uint8_t *)g.A + g.a_sb * bt * ESZ; ldq = (int)(QMC ? g.a_sk : g.a_si) * ESZ;
   }
   // split-K: this workgroup's share of the stages starts k0 bytes into every row
   int Kbytes_local = Kbytes, k0 = 0;
@@ -323,29 +365,53 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   const int drow = wave * RPW + dr;  // passes advance by RPP, a multiple of 32: same swizzle
   const int dcg = dslot ^ swz(drow);
   int voffP[LP], voffQ[LQ];
+  // MC: an instruction fills a block; lane l -> K row and 16-byte piece of it.  A piece past the last one of the row index
+  // loads that one (rows past the end of D are dropped), which holds at least one element of the operand: with the
+  // 16-byte aligned pitch the planner asks for it lies in the operand's own 16-byte granules.
+  const int mkP = mc_block_k(wave) + (BP == 256 ? 4 * (lane >> 5) : 4 * ((lane >> 4) & 1) + 32 * (lane >> 5));
+  const int mkQ = mc_block_k(wave) + (BQ == 256 ? 4 * (lane >> 5) : 4 * ((lane >> 4) & 1) + 32 * (lane >> 5));
 #pragma unroll
-  for (int i = 0; i < LP; i++) voffP[i] = min(p0 + drow + RPP * i, NP - 1) * ldp + dcg * 16;
+  for (int i = 0; i < LP; i++)
+    if constexpr (PMC) voffP[i] = i ? 0 : mkP * ldp + min(p0 + 8 * (lane & (BP / 8 - 1)), (NP - 1) & ~7) * ESZ;
+    else voffP[i] = min(p0 + drow + RPP * i, NP - 1) * ldp + dcg * 16;
 #pragma unroll
-  for (int i = 0; i < LQ; i++) voffQ[i] = min(q0 + drow + RPP * i, NQ - 1) * ldq + dcg * 16;
+  for (int i = 0; i < LQ; i++)
+    if constexpr (QMC) voffQ[i] = i ? 0 : mkQ * ldq + min(q0 + 8 * (lane & (BQ / 8 - 1)), (NQ - 1) & ~7) * ESZ;
+    else voffQ[i] = min(q0 + drow + RPP * i, NQ - 1) * ldq + dcg * 16;
   const int tail_bytes = Kbytes_local - (KT - 1) * BKB;
   const int oob_last = dcg * 16 < tail_bytes ? 0 : (int)0x80000000;
 
-  // stage kt -> LDS slot at 16-byte offset `so`.  Stages kt >= KT are never multiplied; they are issued
-  // only so that every stage has the same vector memory operations in flight, as real loads of one cache
+  const v4i rawP = {(int)(uintptr_t)Pg, (int)((uintptr_t)Pg >> 32) & 0xffff, (int)0x80000000, 0x00020000};
+  const v4i rawQ = {(int)(uintptr_t)Qg, (int)((uintptr_t)Qg >> 32) & 0xffff, (int)0x80000000, 0x00020000};
+  constexpr bool MC = PMC || QMC;
+
+  // stage kt -> LDS slot at 16-byte offset `so`, DMA instruction `n` of LP + LQ.  Stages kt >= KT are never multiplied; they
+  // are issued only so that every stage has the same vector memory operations in flight, as real loads of one cache
   // line (an instruction whose lanes are all out of range completes without a memory round trip and can
   // retire ahead of older loads).
-  auto issue_stage = [&](int kt, int so) {
+  auto issue_one = [&](int kt, int so, auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    constexpr bool is_p = n < LP, mc = is_p ? PMC : QMC;
+    constexpr int i = is_p ? n : n - LP;
     const int live = kt < KT ? -1 : 0;  // uniform
-    const int oob = kt == KT - 1 ? oob_last : 0;
-    const int soff = (k0 + kt * BKB) & live;
-    v4i *base = &lds[so];
-#pragma unroll
-    for (int i = 0; i < LP; i++)
-      lds_dma16(rsP, base + (wave * RPW + RPP * i) * CPR, (voffP[i] | oob) & live, soff);
-#pragma unroll
-    for (int i = 0; i < LQ; i++)
-      lds_dma16(rsQ, base + (BP + wave * RPW + RPP * i) * CPR, (voffQ[i] | oob) & live, soff);
+    const int *voff = is_p ? voffP : voffQ;
+    v4i *base = &lds[so] + (is_p ? 0 : P_V4);
+    if constexpr (mc) {
+      // K rows from `klim` on are past the end (an offset of bit 31 alone, which no stage's offset carries beyond 2^32);
+      // the blocks of a wave lie whole K rows apart: in the scalar offset
+      const int klim = kt == KT - 1 ? tail_bytes / ESZ : BKB / ESZ;
+      const int vo = ((is_p ? mkP : mkQ) < klim - mc_block_k(i * NWV) ? voff[0] : (int)0x80000000) & live;
+      const int soff = (((k0 + kt * BKB) / ESZ + mc_block_k(i * NWV)) & live) * (is_p ? ldp : ldq);
+      lds_dma16_uncounted(is_p ? rawP : rawQ, base + (wave + NWV * i) * (kMcPitch / 16), vo, soff);
+    } else {
+      const int oob = kt == KT - 1 ? oob_last : 0;
+      const int soff = (k0 + kt * BKB) & live;
+      v4i *dst = base + (wave * RPW + RPP * i) * CPR;
+      if constexpr (MC) lds_dma16_uncounted(is_p ? rawP : rawQ, dst, (voff[i] | oob) & live, soff);
+      else lds_dma16(is_p ? rsP : rsQ, dst, (voff[i] | oob) & live, soff);
+    }
   };
+  auto issue_stage = [&](int kt, int so) { static_for<NLOAD>([&](auto n_c) { issue_one(kt, so, n_c); }); };
 
   // ---- fragment addressing --------------------------------------------------------------------------------
   // Tiles start on multiples of 16 rows; the swizzle depends on the row mod 32, so even and odd tiles
@@ -358,8 +424,11 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
       const int row = par * 16 + r16;
       const int ch = (KIND == KIND_F8 ? 2 * g4 + kk : 4 * kk + g4) ^ swz(row);
       fragP[par][kk] = (wp * WTP + row) * CPR + ch;
-      fragQ[par][kk] = (BP + wq * WTQ + row) * CPR + ch;
+      fragQ[par][kk] = (P_V4 + (wq * WTQ + row) * CPR) + ch;
     }
+  // MC: K row 8 * (l / 16) + (l % 16) / 4, elements 4 * (l % 4) .. +3 of the wave tile, in bytes inside a slot
+  const int mfrag = ((r16 >> 2) + 4 * g4) * kMcPitch + 8 * (r16 & 3);
+  const int mfragP = mfrag + wp * WTP * 2, mfragQ = P_V4 * 16 + mfrag + wq * WTQ * 2;
   // 16-row tile `tile` of the wave tile, from the stage in the slot at `so`
   auto load_frag = [&](int so, const int (&fr)[2][2], auto tile_c, Frag &f) {
     constexpr int tile = decltype(tile_c)::value;
@@ -370,6 +439,17 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     } else {
       f.k[0] = lo;
       f.k[1] = hi;
+    }
+  };
+
+  auto load_frag_mc = [&](int so, int fr, auto rows_c, auto tile_c, Frag &f) {
+    constexpr int B = decltype(rows_c)::value, tile = decltype(tile_c)::value;
+    constexpr int UP4 = B == 256 ? 512 : 256, UP32 = B == 256 ? 16 * kMcPitch : 512;  // bytes to the K row 4 / 32 further on
+    const char *base = (const char *)&lds[so] + fr + tile * 32;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      const v2i lo = lds_read_tr16(base + ks * UP32), hi = lds_read_tr16(base + ks * UP32 + UP4);
+      f.k[ks] = frag_v{lo[0], lo[1], hi[0], hi[1]};
     }
   };
 
@@ -387,7 +467,8 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     constexpr int h = decltype(h_c)::value, I0 = decltype(i0_c)::value, I1 = decltype(i1_c)::value;
     static_for<I1 - I0>([&](auto i_c) {
       constexpr int i = I0 + decltype(i_c)::value;
-      load_frag(so, fragP, std::integral_constant<int, h * HP + i>{}, pf[h][i]);
+      if constexpr (PMC) load_frag_mc(so, mfragP, std::integral_constant<int, BP>{}, std::integral_constant<int, h * HP + i>{}, pf[h][i]);
+      else load_frag(so, fragP, std::integral_constant<int, h * HP + i>{}, pf[h][i]);
     });
   };
   auto load_p_half = [&](int so, auto h_c) {
@@ -397,18 +478,17 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     constexpr int h = decltype(h_c)::value;
     static_for<HQ>([&](auto i_c) {
       constexpr int i = decltype(i_c)::value;
-      load_frag(so, fragQ, std::integral_constant<int, h * HQ + i>{}, qf[h][i]);
+      if constexpr (QMC) load_frag_mc(so, mfragQ, std::integral_constant<int, BQ>{}, std::integral_constant<int, h * HQ + i>{}, qf[h][i]);
+      else load_frag(so, fragQ, std::integral_constant<int, h * HQ + i>{}, qf[h][i]);
     });
   };
   // the MFMAs of P half ph against Q half qh; K half by K half, so that the two instructions of a tile
   // (int8) are a whole sub-step's worth of independent instructions apart
-  auto mfma_halves = [&](auto ph_c, auto qh_c) {
+  auto mfma_part = [&](auto ph_c, auto qh_c, auto n0_c, auto n1_c) {  // number n0 .. n1 - 1 of them
     constexpr int ph = decltype(ph_c)::value, qh = decltype(qh_c)::value;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++)
-#pragma unroll
-      for (int x = 0; x < HP * HQ; x++) {
-          const int i = x / HQ, j = x % HQ;
+    for (int n = decltype(n0_c)::value; n < decltype(n1_c)::value; n++) {
+          const int ks = n / (HP * HQ), x = n % (HP * HQ), i = x / HQ, j = x % HQ;
           acc_v &c = acc[ph * HP + i][qh * HQ + j];
           if constexpr (KIND == KIND_I8) c = __builtin_amdgcn_mfma_i32_16x16x64_i8(pf[ph][i].k[ks], qf[qh][j].k[ks], c, 0, 0, 0);
           else if constexpr (KIND == KIND_F16)
@@ -416,7 +496,10 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
           else if constexpr (KIND == KIND_BF16)
             c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8b, pf[ph][i].k[ks]), __builtin_bit_cast(v8b, qf[qh][j].k[ks]), c, 0, 0, 0);
           else c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(pf[ph][i].k[ks], qf[qh][j].k[ks], c, FP, FQ, 0, 0, 0, 0);
-        }
+    }
+  };
+  auto mfma_halves = [&](auto ph_c, auto qh_c) {
+    mfma_part(ph_c, qh_c, std::integral_constant<int, 0>{}, std::integral_constant<int, HP * HQ * KS>{});
   };
   // issue order of a sub-step: its NM MFMAs back to back, with the NDS fragment reads slotted PER_DS at a
   // time behind the first ones (what they fetch is needed one sub-step later, or by the barrier) and the
@@ -444,6 +527,9 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   // ---- prologue: stages 0 and 1 in flight, stage 0 landed, its first fragments in registers -----------------
   issue_stage(0, 0);
   issue_stage(1, STAGE_V4);
+  // (MC: an instruction of the last stage's K tail may hold no K row that exists and retires early, so nothing is counted
+  // where one is in flight)
+  if (MC && KT <= 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   wait_vmcnt_barrier<PC.wait_prologue>();
   load_p_half(0, std::integral_constant<int, 0>{});
   load_q_half(0, std::integral_constant<int, 0>{});
@@ -457,7 +543,8 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     using P1 = std::integral_constant<int, 1>;
     using QAc = std::integral_constant<int, QA>;
     using QBc = std::integral_constant<int, QB_>;
-    constexpr int DSP = 2 * HP, DSQ = 2 * HQ;  // ds_read_b128 per half
+    constexpr int PD = PMC ? 4 : 2, QD = QMC ? 4 : 2;  // LDS reads per fragment
+    constexpr int DSP = PD * HP, DSQ = QD * HQ;        // and per half
     // The fragment reads are spread over the four sub-steps (the LDS is the busiest unit of the loop: 24 KiB
     // per wave and stage): EARLY fragments of P half 1 come with QB, LATE fragments of the next stage's P
     // half 0 with its first Q half.
@@ -470,24 +557,35 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     load_q_half(so, QBc{});
     load_p_part(so, P1{}, I0{}, IE{});
     mfma_halves(P0{}, QAc{});
-    pattern(std::integral_constant<int, DSQ + 2 * EARLY>{}, std::integral_constant<int, 0>{});
+    pattern(std::integral_constant<int, DSQ + PD * EARLY>{}, std::integral_constant<int, 0>{});
     // (P0, QB) while P1 arrives
     load_p_part(so, P1{}, IE{}, IH{});
     mfma_halves(P0{}, QBc{});
-    pattern(std::integral_constant<int, DSP - 2 * EARLY>{}, std::integral_constant<int, 0>{});
+    pattern(std::integral_constant<int, DSP - PD * EARLY>{}, std::integral_constant<int, 0>{});
     // every fragment of the stage has been requested: wait for them and for this wave's share of stage
     // kt+1, meet the other waves; then the slot is free and the other one readable
     wait_vmcnt_barrier<PC.wait_stage>();
     // (P1, QB): refill this slot with stage kt+2, P half 0 of stage kt+1 arrives
     load_p_part(so_next, P0{}, I0{}, IL{});
-    issue_stage(kt + NSTAGE, so);
-    mfma_halves(P1{}, QBc{});
-    pattern(std::integral_constant<int, DSP - 2 * LATE>{}, std::integral_constant<int, NLOAD>{});
+    if constexpr (MC) {
+      // (the scheduler does not know the asm for a memory instruction: its place among the MFMAs is written out)
+      constexpr int NM = HP * HQ * KS;
+      static_for<NLOAD>([&](auto n_c) {
+        constexpr int n = decltype(n_c)::value;
+        mfma_part(P1{}, QBc{}, std::integral_constant<int, NM * n / NLOAD>{}, std::integral_constant<int, NM * (n + 1) / NLOAD>{});
+        issue_one(kt + NSTAGE, so, n_c);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    } else {
+      issue_stage(kt + NSTAGE, so);
+      mfma_halves(P1{}, QBc{});
+      pattern(std::integral_constant<int, DSP - PD * LATE>{}, std::integral_constant<int, NLOAD>{});
+    }
     // (P1, QA): Q half QB of stage kt+1 arrives (that stage starts with it)
     load_p_part(so_next, P0{}, IL{}, IH{});
     load_q_half(so_next, QBc{});
     mfma_halves(P1{}, QAc{});
-    pattern(std::integral_constant<int, DSQ + 2 * LATE>{}, std::integral_constant<int, 0>{});
+    pattern(std::integral_constant<int, DSQ + PD * LATE>{}, std::integral_constant<int, 0>{});
   };
 
   int kt = 0;

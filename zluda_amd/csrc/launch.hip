@@ -125,11 +125,13 @@ uint32_t launch_tr(const Lowered &l, const zluda_gemm_plan &plan, void *ws, uint
   prm.group_p = 8;
   prm.splits = 1; prm.split_stages = 0; prm.ws = nullptr;
   if ((uint32_t)(prm.tiles_p * prm.tiles_q) != plan.grid_x) return CUBLAS_STATUS_INVALID_VALUE;
+  // aligned 16-bit operands: the same tiles, transposed by the LDS reads, 128 K bytes per stage
+  const bool lds_reads = (plan.variant == 1 || plan.variant == 3) && lds_transposable(l);
   if (plan.grid_z > 1) {
     // split-K: partial tiles go through the caller's workspace (64 K bytes per stage)
     const uint64_t need = (uint64_t)plan.grid_z * l.g.batch * prm.tiles_p * v.bp * prm.tiles_q * v.bq * 4;
     if (!ws || (((uintptr_t)ws) & 15) || ws_size < need || plan.workspace < need) return CUBLAS_STATUS_INVALID_VALUE;
-    const int stages = (l.g.K * (plan.kernel == ZLUDA_KERNEL_MFMA_TR16 ? 2 : plan.kernel == ZLUDA_KERNEL_MFMA_TR32 ? 4 : 1) + 63) / 64;
+    const int stages = (l.g.K * (plan.kernel == ZLUDA_KERNEL_MFMA_TR16 ? 2 : plan.kernel == ZLUDA_KERNEL_MFMA_TR32 ? 4 : 1) + (lds_reads ? 127 : 63)) / (lds_reads ? 128 : 64);
     prm.splits = (int32_t)plan.grid_z;
     prm.split_stages = (stages + prm.splits - 1) / prm.splits;
     prm.ws = ws;
@@ -137,7 +139,9 @@ uint32_t launch_tr(const Lowered &l, const zluda_gemm_plan &plan, void *ws, uint
   // P is op(A) for a column-major D, op(B)^T otherwise
   const bool pkc = plan.swapped ? l.b_kcontig : l.a_kcontig, qkc = plan.swapped ? l.a_kcontig : l.b_kcontig;
   uint32_t st;
-  if (l.g.a_type == CUDA_R_8I) {
+  if (lds_reads) {
+    st = l.g.a_type == CUDA_R_16BF ? launch_trl_bf16(prm, plan, pkc, qkc, s) : launch_trl_f16(prm, plan, pkc, qkc, s);
+  } else if (l.g.a_type == CUDA_R_8I) {
     st = launch_tr_i8(prm, plan, pkc, qkc, s);
   } else if (l.g.a_type == CUDA_R_16F) {
     st = launch_tr_f16(prm, plan, pkc, qkc, s);

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "kernels/gemm_mfma_pipe16.hpp"
 #include "kernels/gemm_mfma_tr.hpp"
 #include "launch_util.hpp"
 #include "planner.hpp"
@@ -46,6 +47,9 @@ inline uint32_t launch_tr_variant(const MfmaParams &prm, const zluda_gemm_plan &
   return CUBLAS_STATUS_INVALID_VALUE;
 }
 
+// the variants 1 and 3 on 16-byte aligned 16-bit operands: their grids, with the transposition in the LDS reads
+uint32_t launch_trl_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
+uint32_t launch_trl_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_i8(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_f8(const MfmaParams &prm, const zluda_gemm_plan &plan, int fq, int fp, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_f8_e5m2q(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
@@ -53,5 +57,28 @@ uint32_t launch_tr_f8_e5m2p(const MfmaParams &prm, const zluda_gemm_plan &plan, 
 uint32_t launch_tr_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_f32(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
+
+template <int KIND>
+inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s) {
+  const dim3 grid(plan.grid_x, plan.grid_y, plan.grid_z > 1 ? plan.grid_z : 1);
+#define ZLUDA_TRL_MODE(BP, BQ, WP, WQ, PK, QK)                                                                       \
+  if (pkc == PK && qkc == QK)                                                                                        \
+    return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, BP, BQ, WP, WQ, !PK, !QK>, grid, dim3(WP * WQ * 64), s, prm);
+#define ZLUDA_TRL_CASE(V, BP, BQ, WP, WQ)                                                                            \
+  case V:                                                                                                            \
+    static_assert(kTrVariants[V].bp == BP && kTrVariants[V].bq == BQ && kTrVariants[V].wp == WP &&                   \
+                  kTrVariants[V].wq == WQ, "variant table mismatch");                                                \
+    ZLUDA_TRL_MODE(BP, BQ, WP, WQ, false, false) ZLUDA_TRL_MODE(BP, BQ, WP, WQ, false, true)                         \
+    ZLUDA_TRL_MODE(BP, BQ, WP, WQ, true, false)                                                                      \
+    break;
+  switch (plan.variant) {
+    ZLUDA_TRL_CASE(1, 128, 128, 2, 2)
+    ZLUDA_TRL_CASE(3, 256, 256, 2, 4)
+  default: break;
+  }
+#undef ZLUDA_TRL_CASE
+#undef ZLUDA_TRL_MODE
+  return CUBLAS_STATUS_INVALID_VALUE;
+}
 
 } // namespace zluda_amd

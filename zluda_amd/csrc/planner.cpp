@@ -311,6 +311,18 @@ static uint32_t transposing_family(const Lowered &l, bool any_pitch) {
   return f32 ? ZLUDA_KERNEL_MFMA_TR32 : h16 ? ZLUDA_KERNEL_MFMA_TR16 : ZLUDA_KERNEL_MFMA_TR8;
 }
 
+bool lds_transposable(const Lowered &l) {
+  const GemmArgs &g = l.g;
+  if ((g.a_type != CUDA_R_16F && g.a_type != CUDA_R_16BF) || g.b_type != g.a_type || (l.a_kcontig && l.b_kcontig)) return false;
+  auto ok = [&](const void *ptr, int64_t s_row, int64_t s_k, int64_t s_b) {
+    if ((((uintptr_t)ptr) & 15) || (g.batch > 1 && ((s_b * 2) & 15))) return false;
+    if (s_k == 1) return ((s_row * 2) & 15) == 0 && (g.K & 7) == 0;
+    // (the K rows of the last stage past the end stay below 2 GiB too: the scalar offset of its loads counts them)
+    return s_row == 1 && ((s_k * 2) & 15) == 0 && ((int64_t)g.K + 64) * s_k * 2 < 0x7fffffffll;
+  };
+  return ok(g.A, g.a_si, g.a_sk, g.a_sb) && ok(g.B, g.b_sj, g.b_sk, g.b_sb);
+}
+
 bool family_supports(uint32_t kernel, const Lowered &l) {
   const GemmArgs &g = l.g;
   const bool fast_layout = l.a_kcontig && l.b_kcontig && l.aligned16;
@@ -527,8 +539,38 @@ static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t w
 struct TrCost { uint32_t per_cu; float base, slope; };
 static const TrCost kTrCost[kNumTrVariants] = {{1, 0.0f, 71.0f}, {2, 26.0f, 11.0f}, {4, 16.0f, 6.0f}, {1, 0.0f, 67.0f}};
 
-static int pick_tr_variant(const Lowered &l, uint32_t cus) {
+// f16 and bf16: the split along K that the variant would get counts as well, and with operands that the LDS reads
+// transpose (lds_transposable()) the variants 1 and 3 are that kernel, with times of its own.  us for 4096 bytes of K:
+// 128x128 25 + 3.3 n, 256x256 53 on a full chip (8192 x 4096 x 2048 121 us against 174 on 128x128; 2048 x 4096 x 8192, 128
+// tiles, 164 against 130); the others as above.  Around the loop 4 us, and for a split the second kernel and the partial
+// tiles' way through memory at 3 TB/s (1024 x 512 x 1024 on 128x128 would take 20 us split, 64x64 take 10).
+static const TrCost kTrCostLds[kNumTrVariants] = {{1, 0.0f, 71.0f}, {2, 25.0f, 3.3f}, {4, 16.0f, 6.0f}, {1, 0.0f, 53.0f}};
+
+static int pick_tr_variant_h16(const Lowered &l, uint32_t cus, uint64_t workspace_size) {
+  const bool lds = lds_transposable(l);
+  const double units = (double)l.g.K * 2 / 4096;
+  int best = 0;
+  double best_cost = 0;
+  for (int v = 0; v < kNumTrVariants; v++) {
+    const TrCost &c = (lds ? kTrCostLds : kTrCost)[v];
+    zluda_gemm_plan p;
+    memset(&p, 0, sizeof(p));
+    fill_tr_plan(l, v, cus, workspace_size, &p);
+    const uint64_t groups = (uint64_t)p.grid_x * p.grid_y * p.grid_z, slots = (uint64_t)cus * c.per_cu;
+    if (kTrVariants[v].m16 && !lds && groups * 4 < (uint64_t)cus * 3) continue;
+    const uint64_t full = groups / slots, rem = groups % slots;
+    double cost = (double)full * (c.base + c.slope * c.per_cu);
+    if (rem) cost += c.base + c.slope * (double)((rem + cus - 1) / cus);
+    cost = 4.0 + cost * units / p.grid_z;
+    if (p.grid_z > 1) cost += 4.0 + (double)p.workspace * 2 / 3e6;
+    if (v == 0 || cost < best_cost) { best = v; best_cost = cost; }
+  }
+  return best;
+}
+
+static int pick_tr_variant(const Lowered &l, uint32_t cus, uint64_t workspace_size) {
   const GemmArgs &g = l.g;
+  if (g.a_type == CUDA_R_16F || g.a_type == CUDA_R_16BF) return pick_tr_variant_h16(l, cus, workspace_size);
   const bool swapped = g.d_si != 1;
   const uint32_t np = swapped ? g.N : g.M, nq = swapped ? g.M : g.N;
   int best = 0;
@@ -577,7 +619,7 @@ uint32_t plan_transposing_under_generic(const Lowered &l, uint32_t cus, uint64_t
     if (family_supports(k, l)) return 0;
   memset(plan, 0, sizeof(*plan));
   plan->kernel = family;
-  fill_tr_plan(l, pick_tr_variant(l, cus), cus, workspace_size, plan);
+  fill_tr_plan(l, pick_tr_variant(l, cus, workspace_size), cus, workspace_size, plan);
   return family;
 }
 
@@ -736,7 +778,7 @@ extern "C" uint32_t zluda_gemm_plan_problem(const zluda_gemm_problem *p, uint32_
     break;
   }
   case ZLUDA_KERNEL_MFMA_TR8: case ZLUDA_KERNEL_MFMA_TR16: case ZLUDA_KERNEL_MFMA_TR32: {
-    int v = forced_variant >= 0 ? forced_variant : pick_tr_variant(l, cu_count);
+    int v = forced_variant >= 0 ? forced_variant : pick_tr_variant(l, cu_count, p->workspace_size);
     if (v >= kNumTrVariants || (kTrVariants[v].m16 && l.g.a_type != CUDA_R_8I && l.g.a_type != CUDA_R_16F && l.g.a_type != CUDA_R_16BF))
       return CUBLAS_STATUS_INVALID_VALUE;
     fill_tr_plan(l, v, cu_count, p->workspace_size, plan);

@@ -116,6 +116,10 @@ uint32_t plan_transposing_under_generic(const Lowered &l, uint32_t cus, uint64_t
 // which kernel families can run the lowered problem
 bool family_supports(uint32_t kernel, const Lowered &l);
 
+// whether a 16-bit problem of the transposing family can read its operands through ds_read_b64_tr_b16: one of them not
+// K-contiguous, both 16-byte aligned with 16-byte aligned pitches, K-contiguous rows of whole 16-byte pieces
+bool lds_transposable(const Lowered &l);
+
 // Row sums along the longer stride (bias gradients): how many workgroups share the `len` terms of each of `rows` sums, given
 // scratch for shares * rows * batch partial sums of 4 bytes; 1: no scratch is used
 uint32_t row_sum_shares(int64_t rows, int64_t len, int64_t batch, uint64_t workspace_size);
