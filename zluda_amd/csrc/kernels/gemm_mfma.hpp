@@ -21,6 +21,7 @@
 // groups).
 #pragma once
 #include "numeric.hpp"
+#include "store_window.hpp"
 
 namespace zluda_amd {
 
@@ -240,18 +241,6 @@ __device__ __forceinline__ void mfma_store_tile_general(const MfmaParams &prm, A
   static_for<TQ * 2>(do_pass);
 }
 
-// Size of the buffer window of a wave tile whose corner is `base_elems` elements into this batch's D:
-// what is left of the matrix (NQ columns of pitch d_sq, the last one NP long).  Stores of a tile that
-// hangs over the last column fall outside the window and are dropped by the hardware, which is what
-// lets the fast paths below take tiles that are complete along P only.
-__device__ __forceinline__ uint32_t tile_window_bytes(int64_t d_sq, int NP, int NQ, int64_t base_elems, int esz) {
-  const int64_t left = ((int64_t)(NQ - 1) * d_sq + NP - base_elems) * esz;
-  return left <= 0 ? 0u : (left > 0xFFFFFFFFll ? 0xFFFFFFFFu : (uint32_t)left);
-}
-
-// Offset bit that puts a lane of a buffer store outside every window (the store is dropped): lanes past the end of P.
-constexpr int kStoreNowhere = (int)0x80000000;
-
 // Fast path 1: pure integer epilogue with alpha, beta scalars and beta == 0: D = alpha * acc straight from the accumulator
 // registers.  Lanes 0..31 of a store hold 32 consecutive int32 of one D column (one 128-byte line), so no LDS staging is
 // needed; two instructions per output element.  Tiles that hang over the end of P mask their lanes, columns past the end
@@ -266,7 +255,7 @@ __device__ __forceinline__ void mfma_store_tile_i32(const MfmaParams &prm, v16i 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wp = wave % WP, wq = wave / WP;
   const int lr = lane & 31, gsel = lane >> 5;
-  const int d_sq = (int)(prm.swapped ? g.d_si : g.d_sj);  // < 2^22 (checked by the dispatcher)
+  const int d_sq = (int)(prm.swapped ? g.d_si : g.d_sj);  // < kNarrowPitch (checked by the dispatcher)
   // Buffer stores: wave-uniform descriptor at the wave tile, per-lane byte offset of (row 4*gsel,
   // column lr) in a VGPR, everything else in the scalar offset.
   const int64_t corner = (int64_t)(q0 + wq * WTQ) * d_sq + (p0 + wp * WTP);
@@ -364,7 +353,7 @@ __device__ __forceinline__ void mfma_store_tile_float(const MfmaParams &prm, Acc
     q_lane[a] = q_vec ? (swp ? ep.row_scale(qi) : ep.col_scale(qi)) : 1.0f;
     qb_lane[a] = q_vec && swp ? ep.bias_at(qi) : 0.0f;
   }
-  const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < 2^22 (checked by the dispatcher)
+  const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < kNarrowPitch (checked by the dispatcher)
   const int64_t corner = (int64_t)qc * d_sq + pc;
   char *Dw = (char *)g.D + (g.d_sb * bt + corner) * esz;
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dw, 0, tile_window_bytes(d_sq, NP, NQ, corner, esz), 0x00020000);
@@ -454,7 +443,7 @@ __device__ __forceinline__ void mfma_store_tile(const MfmaParams &prm, AccV (&ac
                                                 int NQ, int bt) {
   const GemmArgs &g = prm.g;
   const int64_t d_sq = prm.swapped ? g.d_si : g.d_sj;
-  const bool narrow = d_sq < (1 << 22);  // the lane offsets fit 32 bits
+  const bool narrow = d_sq < kNarrowPitch;  // the lane offsets fit 32 bits
   if constexpr (KIND == KIND_I8) {
     if (g.int_scale && narrow && g.alpha_mode != VECTOR_DEV && g.beta_mode == SCALAR_VALUE && g.beta_val.i == 0) {
       const int ialpha = g.alpha_mode == SCALAR_VALUE ? g.alpha_val.i : *(const int32_t *)g.alpha_ptr;

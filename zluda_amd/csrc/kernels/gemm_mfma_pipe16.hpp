@@ -94,7 +94,7 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
   const int act = g.act;
   const bool to_bf16 = g.d_type == CUDA_R_16BF;
   const bool ragged = NP < p0 + wp * WTP + WTP && (NP & 3);  // (uniform) some lane's four straddle the end of P
-  const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < 2^22 (checked by the dispatcher)
+  const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < kNarrowPitch (checked by the dispatcher)
   const int pc = p0 + wp * WTP, qc = q0 + wq * WTQ;
   const int64_t corner = (int64_t)qc * d_sq + pc;
   char *Dw = (char *)g.D + (g.d_sb * bt + corner) * ESZ;
@@ -240,7 +240,7 @@ __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&
   const GemmArgs &g = prm.g;
   const bool swp = prm.swapped != 0;
   const int64_t d_sq = swp ? g.d_si : g.d_sj;
-  const bool narrow = d_sq < (1 << 22);  // the lane offsets fit 32 bits
+  const bool narrow = d_sq < kNarrowPitch;  // the lane offsets fit 32 bits
   if constexpr (KIND == KIND_I8) {
     if (g.int_scale && narrow && g.alpha_mode != VECTOR_DEV && g.beta_mode == SCALAR_VALUE && g.beta_val.i == 0) {
       const int ialpha = g.alpha_mode == SCALAR_VALUE ? g.alpha_val.i : *(const int32_t *)g.alpha_ptr;

@@ -131,7 +131,7 @@ __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[
   EpilogueScalars here = scalars;
   w4_scalar_here(here.alpha_s); w4_scalar_here(here.sa_s); w4_scalar_here(here.sb_s); w4_scalar_here(here.sd);
   const bool swp = prm.swapped != 0;
-  const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < 2^22 (checked before this path is taken)
+  const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < kNarrowPitch (checked before this path is taken)
   const int pc = p0 + wp * WTP, qc = q0 + wq * WTQ;
   const int64_t corner = (int64_t)qc * d_sq + pc;
   const bool to_f32 = g.d_type == CUDA_R_32F;  // (four bytes per element: a lane's four rows are its 16 bytes, no trade)

@@ -5,6 +5,8 @@
 // path needs: scale pointers/modes, pointer modes, FP4/UE8M0 types.
 #include "planner.hpp"
 
+#include "kernels/store_window.hpp"
+
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -368,7 +370,7 @@ int w4_epilogue_class(const Lowered &l, bool dry) {
   const bool swapped = g.d_si != 1;
   const int64_t d_sq = swapped ? g.d_si : g.d_sj;
   const int dbytes = (g.d_type == CUDA_R_32I || g.d_type == CUDA_R_32F) ? 4 : 2;
-  if (((d_sq * dbytes) & 15) || (g.batch > 1 && ((g.d_sb * dbytes) & 15)) || d_sq >= (1 << 22) || (((uintptr_t)g.D) & 15))
+  if (((d_sq * dbytes) & 15) || (g.batch > 1 && ((g.d_sb * dbytes) & 15)) || d_sq >= kNarrowPitch || (((uintptr_t)g.D) & 15))
     return W4_CLASS_NONE;
   const bool i8 = g.a_type == CUDA_R_8I && g.b_type == CUDA_R_8I;
   if (i8 && g.int_scale) {
