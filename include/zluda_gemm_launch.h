@@ -108,21 +108,22 @@ uint32_t zluda_gemm_plan_problem(const zluda_gemm_problem *p, uint32_t forced_ke
                                  zluda_gemm_plan *plan);
 
 /* Enqueue the matmul on `stream` (a hipStream_t).  Asynchronous; no allocation; the workspace in
- * `p` must be at least plan->workspace bytes. */
+ * `p` must be at least plan->workspace bytes, of which no more than plan->workspace are written. */
 uint32_t zluda_gemm_launch(const zluda_gemm_problem *p, const zluda_gemm_plan *plan,
                            void *stream);
 
 /* zluda_gemm_launch for callers that cannot hand over device scratch and cannot allocate any (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the
- * reference.  Same arguments and results as zluda_gemm_launch, but split-K partial tiles go to an array of
- * ZLUDA_GEMM_STATIC_SCRATCH_BYTES of device memory that is part of the library image (every device the
- * library runs on holds its own copy until the process ends); `p->workspace` is ignored.  Plan with
- * p->workspace_size = ZLUDA_GEMM_STATIC_SCRATCH_BYTES so that zluda_gemm_plan_problem sizes the split for it;
- * a plan that needs more returns CUBLAS_STATUS_ALLOC_FAILED (3) and launches nothing.  The call allocates and
+ * reference.  Same arguments and results as zluda_gemm_launch, but what the plan counts as workspace (split-K
+ * partial tiles, partial sums of a bias gradient) goes to an array of ZLUDA_GEMM_STATIC_SCRATCH_BYTES of device
+ * memory that is part of the library image (every device the library runs on holds its own copy until the process
+ * ends); `p->workspace` is ignored.  Plan with p->workspace_size = ZLUDA_GEMM_STATIC_SCRATCH_BYTES so that
+ * zluda_gemm_plan_problem sizes splits and sums for it; a plan that needs more returns CUBLAS_STATUS_ALLOC_FAILED (3)
+ * and launches nothing, one that needs none leaves the array alone.  The call allocates and
  * frees nothing.  The first call on a device looks up the array's address, which it will not do while `stream` is
  * being captured (CUBLAS_STATUS_NOT_SUPPORTED): make one call on the device outside the capture first; from then on
- * calls may be captured.  All calls on one device -- replays of a captured graph included -- share that
- * device's array: calls that may overlap on one device (two streams, two threads) race on it and must be
+ * calls may be captured.  All calls on one device whose plans need scratch -- replays of a captured graph included --
+ * share that device's array: calls that may overlap on one device (two streams, two threads) race on it and must be
  * serialised by the caller; nothing in it needs clearing between calls. */
 #define ZLUDA_GEMM_STATIC_SCRATCH_BYTES (32u << 20)
 uint32_t zluda_gemm_launch_noalloc(const zluda_gemm_problem *p, const zluda_gemm_plan *plan,

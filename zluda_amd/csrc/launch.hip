@@ -3,6 +3,7 @@
 #include <atomic>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 
 #include "decode_launch.hpp"
@@ -266,7 +267,7 @@ uint32_t launch_bgrad_typed(BgradParams &b, void *ws, uint64_t ws_size, hipStrea
   constexpr int V = elems16(TYPE), ESZ = 16 / V;
   b.wide = !(((uintptr_t)b.src | (uintptr_t)(b.s_b * ESZ) | (uintptr_t)((b.s_k <= b.s_row ? b.s_row : b.s_k) * ESZ)) & 15);
   if (b.s_k <= b.s_row) return launch_kernel(bgrad_rows_kernel<TYPE>, dim3(b.rows, 1, b.batch), dim3(256), s, b);
-  const uint32_t shares = row_sum_shares(b.rows, b.K, b.batch, ws ? ws_size : 0);
+  const uint32_t shares = row_sum_shares(b.rows, b.K, b.batch, ws_size);
   b.per_block = (int32_t)((b.K + shares - 1) / shares);
   b.part = ws;
   uint32_t st;
@@ -321,7 +322,7 @@ uint32_t launch_aux_typed(const GemmArgs &g, void *ws, uint64_t ws_size, hipStre
   a.out = g.bgrad; a.out_type = g.bias_type; a.out_sb = g.bias_sb;
   if (!col && a.sums) return launch_kernel(aux_dgelu_rows_kernel<TYPE>, dim3(a.NQ, 1, g.batch), dim3(256), s, a);
   // (without sums nothing is carried from one share of Q to another)
-  const uint32_t shares = row_sum_shares(a.NP, a.NQ, g.batch, !a.sums ? ~0ull : ws ? ws_size : 0);
+  const uint32_t shares = row_sum_shares(a.NP, a.NQ, g.batch, a.sums ? ws_size : ~0ull);
   a.per_block = (int32_t)((a.NQ + shares - 1) / shares);
   a.part = ws;
   uint32_t st;
@@ -379,10 +380,11 @@ uint32_t launch_planned(const zluda_gemm_problem *p, const zluda_gemm_plan *plan
   case ZLUDA_KERNEL_MFMA_TR8: case ZLUDA_KERNEL_MFMA_TR16: case ZLUDA_KERNEL_MFMA_TR32: st = launch_tr(l, *plan, ws, ws_size, s); break;
   default: return CUBLAS_STATUS_NOT_SUPPORTED;
   }
-  // (the kernels behind the matmul on its stream take over its scratch)
-  void *const sums = (((uintptr_t)ws) & 15) ? nullptr : ws;
-  if (st == CUBLAS_STATUS_SUCCESS && l.g.bgrad_src) st = launch_bgrad(l.g, sums, ws_size, s);
-  if (st == CUBLAS_STATUS_SUCCESS && whole.aux_mode) st = launch_aux(whole, sums, ws_size, s);
+  // The kernels behind the matmul on its stream take over its scratch: what the plan counted, however much there is, so that
+  // a plan that asks for none writes none and the shares of a sum (its last bits) follow from the plan alone.
+  const uint64_t sums = ws && !(((uintptr_t)ws) & 15) ? std::min<uint64_t>(ws_size, plan->workspace) : 0;
+  if (st == CUBLAS_STATUS_SUCCESS && l.g.bgrad_src) st = launch_bgrad(l.g, ws, sums, s);
+  if (st == CUBLAS_STATUS_SUCCESS && whole.aux_mode) st = launch_aux(whole, ws, sums, s);
   return st;
 }
 

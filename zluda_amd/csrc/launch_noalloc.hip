@@ -1,4 +1,4 @@
-// The launch entry point that allocates nothing: split-K partial tiles go to an array in device memory
+// The launch entry point that allocates nothing: a plan's scratch is an array in device memory
 // that is part of the library image instead of a caller workspace.
 #include <atomic>
 #include <hip/hip_runtime.h>
@@ -8,8 +8,8 @@
 
 using namespace zluda_amd;
 
-// Split-K partial tiles go to this array instead of a caller workspace.  Every device the library runs
-// on holds its own copy (at its own address) until the process ends.  In host code the array's name is
+// Split-K partial tiles and the partial sums of bias gradients go to this array instead of a caller workspace, as far as
+// the plan counts them.  Every device the library runs on holds its own copy (at its own address) until the process ends.  In host code the array's name is
 // only a handle for hipGetSymbolAddress: the device address it returns is what kernels and copies get.
 static __device__ __align__(256) unsigned char scratch[ZLUDA_GEMM_STATIC_SCRATCH_BYTES];
 
@@ -34,7 +34,7 @@ extern "C" uint32_t zluda_gemm_launch_noalloc(const zluda_gemm_problem *p, const
     scratch_of[dev].store(ptr, std::memory_order_release);
     ws = ptr;
   }
-  // nothing in the array has to start at zero: every split writes its whole partial tile before the
+  // nothing in the array has to start at zero: every split and every share of a sum writes its whole part before the
   // reduction kernel of the same call reads it
   return launch_planned(p, plan, ws, ZLUDA_GEMM_STATIC_SCRATCH_BYTES, stream);
 }

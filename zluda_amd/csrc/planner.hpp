@@ -125,7 +125,8 @@ bool lds_transposable(const Lowered &l);
 uint32_t row_sum_shares(int64_t rows, int64_t len, int64_t batch, uint64_t workspace_size);
 
 // Lowers `p` with its real pointers and enqueues the kernel `plan` names on `stream` (a hipStream_t).
-// `ws` / `ws_size`: device scratch for split-K partial tiles, at least plan->workspace bytes.
+// `ws` / `ws_size`: device scratch, at least plan->workspace bytes, of which plan->workspace are used (split-K partial tiles,
+// then the partial sums of bias gradients).
 uint32_t launch_planned(const zluda_gemm_problem *p, const zluda_gemm_plan *plan, void *ws, uint64_t ws_size, void *stream);
 
 } // namespace zluda_amd
