@@ -1,0 +1,51 @@
+"""The 256 x 256 tiles on the 16x16 MFMA shapes use every register of their waves in the K loop: whatever an epilogue keeps live
+across the loop, and every address the compiler hoists in front of it, is spilled, and a reload inside the loop waits for the
+stages in flight (bf16 8192 x 4096 x 1024 took 8 % longer).  Read off the assembly of two instantiations (hipcc, device pass
+only, no GPU needed)."""
+import os
+import re
+import subprocess
+import tempfile
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "zluda_amd", "csrc")
+HIPCC = "/opt/rocm/bin/hipcc"
+pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
+
+
+def kernels(instances):
+    """the instruction lines of the kernels instantiated in `instances`, in their order"""
+    with tempfile.TemporaryDirectory() as tmp:
+        src, out = os.path.join(tmp, "k.hip"), os.path.join(tmp, "k.s")
+        with open(src, "w") as f:
+            f.write('#include "mfma_launch.hpp"\nnamespace zluda_amd {\n%s\n}\n' % "\n".join("template __global__ void %s(MfmaParams);" % i for i in instances))
+        cmd = [HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Xclang", "-target-feature", "-Xclang",
+               "-packed-fp32-ops", "--cuda-device-only", "-S", "-I" + CSRC, src, "-o", out]
+        res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        assert res.returncode == 0, res.stdout[-2000:]
+        text = open(out).read()
+    found = [[l.strip() for l in m.group(1).split("\n")]
+             for m in re.finditer(r"^_ZN9zluda_amd\S*gemm_mfma_pipe16\S*:\s*;.*?\n(.*?)^\.Lfunc_end", text, re.S | re.M)]
+    assert len(found) == len(instances)
+    return found
+
+
+def k_loop(lines):
+    """the loop with the most MFMAs"""
+    labels = {m.group(1): i for i, l in enumerate(lines) for m in [re.match(r"(\.LBB\d+_\d+):", l)] if m}
+    loops = []
+    for i, l in enumerate(lines):
+        m = re.match(r"s_c?branch\S*\s+(\.LBB\d+_\d+)", l)
+        if m and labels.get(m.group(1), i) < i:
+            loops.append(lines[labels[m.group(1)]:i])
+    return max(loops, key=lambda b: sum(x.startswith("v_mfma") for x in b))
+
+
+def test_no_reload_in_the_loop_of_a_256x256_tile():
+    kinds = ["KIND_I8", "KIND_BF16"]
+    for kind, lines in zip(kinds, kernels(["gemm_mfma_pipe16_kernel<%s, 0, 0, 256, 256, 2, 4>" % k for k in kinds])):
+        body = k_loop(lines)
+        assert sum(x.startswith("v_mfma") for x in body) == 128, kind
+        assert not [x for x in body if x.startswith("scratch_")], kind

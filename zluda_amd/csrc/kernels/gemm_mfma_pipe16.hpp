@@ -44,6 +44,17 @@
 
 namespace zluda_amd {
 
+// The lane number, computed where it is used.  Nothing an epilogue needs per lane may stay live across the K loop of a
+// 256 x 256 tile: the loop has no register to spare, what is kept is spilled to scratch memory, and a reload from there (like
+// every load from memory) first waits for the stages in flight, which are older.
+__device__ __forceinline__ int lane_here() {
+  int l = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+#endif
+  return l;
+}
+
 // ---- epilogues for the 16x16 accumulator layout ------------------------------------------------------
 // acc[a][b] is the 16 x 16 tile at (P tile a, Q tile b) of the wave tile; lane l holds elements
 // P = 16a + 4*(l/16) + v (v = 0..3), Q = 16b + l%16.
@@ -54,12 +65,13 @@ __device__ __forceinline__ int store4_offset(int left, int voff) { return left >
 __device__ __forceinline__ int store1_offset(int left, int e, int voff, int esz) { return left < 4 && e < left ? voff + e * esz : kStoreNowhere; }
 
 // raw accumulators (int32 or fp32 bits) of a whole wave tile into a matrix of `pitch` dwords per Q column
-// through the window `rs` that starts at the wave tile's corner; `p_left`: P indices from that corner to the end of P
-template <int TP, int TQ, class AccV>
-__device__ __forceinline__ void mfma16_store_raw(__amdgpu_buffer_rsrc_t rs, int pitch, AccV (&acc)[TP][TQ], int mul, int p_left = TP * 16) {
-  const int lane = threadIdx.x & 63;
+// through the window `rs` that starts at the wave tile's corner; EDGE: the tile may hang over the end of P, `p_left` indices
+// from the corner
+template <bool EDGE, int TP, int TQ, class AccV>
+__device__ __forceinline__ void mfma16_store_raw(__amdgpu_buffer_rsrc_t rs, int pitch, AccV (&acc)[TP][TQ], int mul, int p_left) {
+  const int lane = lane_here();
   const int voff = ((lane & 15) * pitch + 4 * (lane >> 4)) * 4;
-  const bool ragged = p_left < TP * 16 && (p_left & 3);  // (uniform) some lane's four straddle the end
+  const bool ragged = EDGE && p_left < TP * 16 && (p_left & 3);  // (uniform) some lane's four straddle the end
 #pragma unroll
   for (int b = 0; b < TQ; b++)
 #pragma unroll
@@ -69,7 +81,7 @@ __device__ __forceinline__ void mfma16_store_raw(__amdgpu_buffer_rsrc_t rs, int 
       for (int e = 0; e < 4; e++) v[e] = to_bits(acc[a][b][e]);
       if (mul != 1) v *= mul;
       const int left = p_left - (a * 16 + 4 * (lane >> 4));
-      buffer_store_b128_guarded(v, rs, store4_offset(left, voff), (b * 16 * pitch + a * 16) * 4);
+      buffer_store_b128_guarded(v, rs, EDGE ? store4_offset(left, voff) : voff, (b * 16 * pitch + a * 16) * 4);
       if (ragged) {
 #pragma unroll
         for (int e = 0; e < 3; e++) __builtin_amdgcn_raw_buffer_store_b32(v[e], rs, store1_offset(left, e, voff, 4), (b * 16 * pitch + a * 16) * 4, 0);
@@ -77,23 +89,25 @@ __device__ __forceinline__ void mfma16_store_raw(__amdgpu_buffer_rsrc_t rs, int 
     }
 }
 
-// float epilogue without a C read: D bf16 / f16 (8-byte stores) or f32 (WIDE: 16-byte stores), at any element's address
-// and any pitch (the memory system takes such stores unaligned).  The activation and the 16-bit format are
-// workgroup-uniform branches per 16 x 16 tile (one instantiation serves them all: the 64 tiles of a wave are unrolled, so
-// every further template argument multiplies a large body).  A tile that hangs over the end of P drops the lanes past it
+// float epilogue without a C read: D bf16 / f16 (8-byte stores) or f32 (16-byte stores), at any element's address and any
+// pitch (the memory system takes such stores unaligned).  A tile that hangs over the end of P (EDGE) drops the lanes past it
 // and stores the elements of a group of four that straddles the end one by one.
-template <int KIND, int WP, int WQ, int TP, int TQ, bool WIDE, class AccV>
-__device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt) {
+// DT: 0 bf16, 1 f16, 2 f32, -1 one of the 16-bit types; ACT: the activation, -1 any.  Whole tiles have both fixed at compile
+// time (int8 4096 x 4096 x 1024 -> bf16 + GELU: 31.3 us with run-time branches per 16 x 16 tile, 28.7).  Edge tiles branch: the
+// 64 tiles of a wave are unrolled, and a grid has few of them.
+template <int KIND, int WP, int WQ, int TP, int TQ, int DT, int ACT, bool EDGE, class AccV>
+__device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt, int wave) {
   constexpr int WTP = TP * 16, WTQ = TQ * 16;
+  constexpr bool WIDE = DT == 2;
   constexpr int ESZ = WIDE ? 4 : 2;
   const GemmArgs &g = prm.g;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = lane_here();
   const int wp = wave % WP, wq = wave / WP;
   Epilogue ep(g, bt);
   const bool swp = prm.swapped != 0;
-  const int act = g.act;
-  const bool to_bf16 = g.d_type == CUDA_R_16BF;
-  const bool ragged = NP < p0 + wp * WTP + WTP && (NP & 3);  // (uniform) some lane's four straddle the end of P
+  const int act = ACT >= 0 ? ACT : (int)g.act;
+  const bool to_bf16 = DT >= 0 ? DT == 0 : g.d_type == CUDA_R_16BF;
+  const bool ragged = EDGE && NP < p0 + wp * WTP + WTP && (NP & 3);  // (uniform) some lane's four straddle the end of P
   const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < kNarrowPitch (checked by the dispatcher)
   const int pc = p0 + wp * WTP, qc = q0 + wq * WTQ;
   const int64_t corner = (int64_t)qc * d_sq + pc;
@@ -114,7 +128,7 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
   const bool pbias = !swp && g.bias != nullptr;
   const char *bias_b = (const char *)g.bias + g.bias_sb * bt * bsz;
   // (rows start at multiples of 4)
-  const bool wide_bias = pbias && (((uintptr_t)bias_b) & (4 * bsz - 1)) == 0 && p0 + WP * WTP <= NP;
+  const bool wide_bias = pbias && (((uintptr_t)bias_b) & (4 * bsz - 1)) == 0 && !EDGE;
   v4i braw[TP];
 #pragma unroll
   for (int a = 0; a < TP; a++) {
@@ -128,7 +142,7 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
       }
     } else if (pbias) {
 #pragma unroll
-      for (int e = 0; e < 4; e++) braw[a][e] = (int)ep.bias_raw(min(pi + e, NP - 1));
+      for (int e = 0; e < 4; e++) braw[a][e] = (int)ep.bias_raw(EDGE ? min(pi + e, NP - 1) : pi + e);
     }
   }
 #pragma unroll
@@ -136,7 +150,7 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
     float ps[4], pb[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const int pi = min(pc + a * 16 + 4 * (lane >> 4) + e, NP - 1);
+      const int pi = EDGE ? min(pc + a * 16 + 4 * (lane >> 4) + e, NP - 1) : pc + a * 16 + 4 * (lane >> 4) + e;
       ps[e] = swp ? ep.col_scale(pi) : ep.row_scale(pi);
       pb[e] = pbias ? ep.bias_from_raw((uint32_t)braw[a][e]) : 0.0f;
     }
@@ -161,7 +175,7 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
       const int left = NP - (pc + a * 16 + 4 * (lane >> 4));
       if constexpr (WIDE) {
         const v4i pk = {(int)f2bits(x[0]), (int)f2bits(x[1]), (int)f2bits(x[2]), (int)f2bits(x[3])};
-        buffer_store_b128_guarded(pk, rs, store4_offset(left, voff), soff);
+        buffer_store_b128_guarded(pk, rs, EDGE ? store4_offset(left, voff) : voff, soff);
         if (ragged) {
 #pragma unroll
           for (int e = 0; e < 3; e++) __builtin_amdgcn_raw_buffer_store_b32(pk[e], rs, store1_offset(left, e, voff, 4), soff, 0);
@@ -170,7 +184,7 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
         v2i pk;
         if (to_bf16) { pk[0] = (int)pack_bf16x2(x[0], x[1]); pk[1] = (int)pack_bf16x2(x[2], x[3]); }
         else { pk[0] = (int)pack_f16x2(x[0], x[1]); pk[1] = (int)pack_f16x2(x[2], x[3]); }
-        buffer_store_b64_guarded(pk, rs, store4_offset(left, voff), soff);
+        buffer_store_b64_guarded(pk, rs, EDGE ? store4_offset(left, voff) : voff, soff);
         if (ragged) {
           __builtin_amdgcn_raw_buffer_store_b16((short)pk[0], rs, store1_offset(left, 0, voff, 2), soff, 0);
           __builtin_amdgcn_raw_buffer_store_b16((short)(pk[0] >> 16), rs, store1_offset(left, 1, voff, 2), soff, 0);
@@ -197,13 +211,13 @@ constexpr int staging_columns(int fit, int tq) {
 // K loop); `lds_words` / `lds_bytes`: the workgroup's LDS.
 template <int KIND, int WP, int WQ, int TP, int TQ, int LDS_BYTES, class AccV>
 __device__ __forceinline__ void mfma16_store_general(const MfmaParams &prm, AccV (&acc)[TP][TQ], int *lds_words, int p0, int q0,
-                                                     int NP, int NQ, int bt) {
+                                                     int NP, int NQ, int bt, int wave) {
   constexpr int WTP = TP * 16, WTQ = TQ * 16;
   constexpr int PER_WAVE = LDS_BYTES / (WP * WQ);            // bytes of staging per wave
   constexpr int COLS = staging_columns(PER_WAVE / (16 * WTP * 4), TQ);  // tile columns per pass
   static_assert(COLS >= 1 && TQ % COLS == 0, "staging passes");
   const GemmArgs &g = prm.g;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = lane_here();
   const int wp = wave % WP, wq = wave / WP;
   int *stage = lds_words + wave * (PER_WAVE / 4);
   Epilogue ep(g, bt);
@@ -235,32 +249,48 @@ __device__ __forceinline__ void mfma16_store_general(const MfmaParams &prm, AccV
 
 template <int KIND, int WP, int WQ, int TP, int TQ, int LDS_BYTES, class AccV>
 __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&acc)[TP][TQ], int *lds_words, int p0, int q0, int NP,
-                                                  int NQ, int bt) {
+                                                  int NQ, int bt, int wave) {
   constexpr int WTP = TP * 16, WTQ = TQ * 16;
   const GemmArgs &g = prm.g;
   const bool swp = prm.swapped != 0;
   const int64_t d_sq = swp ? g.d_si : g.d_sj;
   const bool narrow = d_sq < kNarrowPitch;  // the lane offsets fit 32 bits
+  const bool whole = p0 + WP * WTP <= NP;
   if constexpr (KIND == KIND_I8) {
     if (g.int_scale && narrow && g.alpha_mode != VECTOR_DEV && g.beta_mode == SCALAR_VALUE && g.beta_val.i == 0) {
       const int ialpha = g.alpha_mode == SCALAR_VALUE ? g.alpha_val.i : *(const int32_t *)g.alpha_ptr;
-      const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
       const int pc = p0 + (wave % WP) * WTP, qc = q0 + (wave / WP) * WTQ;
       const int64_t corner = (int64_t)qc * d_sq + pc;
       int32_t *Dw = (int32_t *)g.D + g.d_sb * bt + corner;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dw, 0, tile_window_bytes(d_sq, NP, NQ, corner, 4), 0x00020000);
-      mfma16_store_raw<TP, TQ>(rs, (int)d_sq, acc, ialpha, NP - pc);
+      if (whole) mfma16_store_raw<false>(rs, (int)d_sq, acc, ialpha, 0);
+      else mfma16_store_raw<true>(rs, (int)d_sq, acc, ialpha, NP - pc);
       return;
     }
   }
   if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
       (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F)) {
-    if (g.d_type == CUDA_R_32F) mfma16_store_f<KIND, WP, WQ, TP, TQ, true>(prm, acc, p0, q0, NP, NQ, bt);
-    else mfma16_store_f<KIND, WP, WQ, TP, TQ, false>(prm, acc, p0, q0, NP, NQ, bt);
+#define ZLUDA_EPI16(DT_, ACT_, EDGE_) mfma16_store_f<KIND, WP, WQ, TP, TQ, DT_, ACT_, EDGE_>(prm, acc, p0, q0, NP, NQ, bt, wave)
+#define ZLUDA_EPI16_ACT(DT_)                                 \
+  if (g.act == ACT_GELU) ZLUDA_EPI16(DT_, ACT_GELU, false);  \
+  else if (g.act == ACT_RELU) ZLUDA_EPI16(DT_, ACT_RELU, false); \
+  else ZLUDA_EPI16(DT_, ACT_NONE, false);
+    if (!whole) {
+      if (g.d_type == CUDA_R_32F) ZLUDA_EPI16(2, -1, true);
+      else ZLUDA_EPI16(-1, -1, true);
+    } else if (g.d_type == CUDA_R_16BF) {
+      ZLUDA_EPI16_ACT(0)
+    } else if (g.d_type == CUDA_R_16F) {
+      ZLUDA_EPI16_ACT(1)
+    } else {
+      ZLUDA_EPI16_ACT(2)
+    }
+#undef ZLUDA_EPI16_ACT
+#undef ZLUDA_EPI16
     return;
   }
   __syncthreads();  // (workgroup-uniform branch) the LDS tiles become staging
-  mfma16_store_general<KIND, WP, WQ, TP, TQ, LDS_BYTES>(prm, acc, lds_words, p0, q0, NP, NQ, bt);
+  mfma16_store_general<KIND, WP, WQ, TP, TQ, LDS_BYTES>(prm, acc, lds_words, p0, q0, NP, NQ, bt, wave);
 }
 
 // ---- the kernel ----------------------------------------------------------------------------------------
@@ -424,7 +454,9 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
       const int row = par * 16 + r16;
       const int ch = (KIND == KIND_F8 ? 2 * g4 + kk : 4 * kk + g4) ^ swz(row);
       fragP[par][kk] = (wp * WTP + row) * CPR + ch;
-      fragQ[par][kk] = (P_V4 + (wq * WTQ + row) * CPR) + ch;
+      // (summed in this order: the other one has the compiler hoist two more addresses than the loop has registers for, and
+      // their reloads cost 7 % of int8 and bf16 8192 x 4096 x 1024)
+      fragQ[par][kk] = PMC ? P_V4 + (wq * WTQ + row) * CPR + ch : (BP + wq * WTQ + row) * CPR + ch;
     }
   // MC: K row 8 * (l / 16) + (l % 16) / 4, elements 4 * (l % 4) .. +3 of the wave tile, in bytes inside a slot
   const int mfrag = ((r16 >> 2) + 4 * g4) * kMcPitch + 8 * (r16 & 3);
@@ -600,10 +632,10 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
     int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)blockIdx.z * g.batch + bt) * ws_np * ws_nq + (int64_t)(q0 + wq * WTQ) * ws_np + p0 + wp * WTP;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)ws_tile, 0, 0xFFFFFFFF, 0x00020000);
-    mfma16_store_raw<TP, TQ>(rs, ws_np, acc, 1);
+    mfma16_store_raw<false>(rs, ws_np, acc, 1, 0);
     return;
   }
-  mfma16_store_tile<KIND, WP, WQ, TP, TQ, (int)sizeof(lds)>(prm, acc, (int *)&lds[0], p0, q0, NP, NQ, bt);
+  mfma16_store_tile<KIND, WP, WQ, TP, TQ, (int)sizeof(lds)>(prm, acc, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
 }
 
 } // namespace zluda_amd

@@ -628,10 +628,10 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
       const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
       int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)blockIdx.z * g.batch + bt) * ws_np * ws_nq + (int64_t)(q0 + wq * WTQ) * ws_np + p0 + wp * WTP;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)ws_tile, 0, 0xFFFFFFFF, 0x00020000);
-      mfma16_store_raw<TP16, TQ16>(rs, ws_np, acc16, 1);
+      mfma16_store_raw<false>(rs, ws_np, acc16, 1, 0);
       return;
     }
-    mfma16_store_tile<KIND, WP, WQ, TP16, TQ16, (int)sizeof(lds)>(prm, acc16, (int *)&lds[0], p0, q0, NP, NQ, bt);
+    mfma16_store_tile<KIND, WP, WQ, TP16, TQ16, (int)sizeof(lds)>(prm, acc16, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
   } else {
   if (prm.splits > 1) {
     const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;

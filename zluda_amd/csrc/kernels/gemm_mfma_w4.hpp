@@ -62,17 +62,6 @@ __device__ __forceinline__ int w4_acc_read(const T &elem) {
   return raw;
 }
 
-// The lane number, computed where it is used.  Nothing an epilogue needs per lane may stay live across the K loop: the
-// loop has no register to spare, what is kept is spilled to scratch memory, and a reload from there (like every load from
-// memory in an epilogue) first waits for the next tile's stages, which are in flight and older.
-__device__ __forceinline__ int w4_lane_here() {
-  int l = 0;
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-#endif
-  return l;
-}
-
 // A value every lane holds alike, moved to a scalar register now (not where the compiler would next need it).  The
 // compiler does not look inside the assembly, so the wait states it would add around the instruction are written out:
 // one between a VALU write of the source and the read, two between the write of the SGPR and a VALU read of it.
@@ -127,7 +116,7 @@ template <int KIND, int ACT, bool EDGE, bool QV, int WTP, int WTQ, int TP, int T
 __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt,
                                              int wp, int wq, const EpilogueScalars &scalars, const W4Staged &st) {
   const GemmArgs &g = prm.g;
-  const int lane = w4_lane_here();
+  const int lane = lane_here();
   EpilogueScalars here = scalars;
   w4_scalar_here(here.alpha_s); w4_scalar_here(here.sa_s); w4_scalar_here(here.sb_s); w4_scalar_here(here.sd);
   const bool swp = prm.swapped != 0;
@@ -362,7 +351,7 @@ template <int WTP, int WTQ, int AUX, int TP, int TQ, class AccV>
 __device__ __forceinline__ void w4_store_i32(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt,
                                              int wp, int wq, int ialpha) {
   const GemmArgs &g = prm.g;
-  const int lane = w4_lane_here();
+  const int lane = lane_here();
   const int64_t d_sq = prm.swapped ? g.d_si : g.d_sj;
   const int pc = p0 + wp * WTP, qc = q0 + wq * WTQ;
   const int64_t corner = (int64_t)qc * d_sq + pc;
@@ -818,7 +807,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
       staged.has[0] = staged.has[1] = staged.has[2] = staged.has[3] = staged.has[4] = false;
       staged.bias_skip = 0;
       {
-        const int ln4 = w4_lane_here() * 4;
+        const int ln4 = lane_here() * 4;
         // (a ragged last tile: what the vectors have of this wave's entries; the rest reads as zero and belongs to rows
         // nobody stores)
         const int pc = p0 + wp * WTP, pn = min(WTP, NP - pc);
