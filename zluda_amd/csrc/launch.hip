@@ -126,8 +126,9 @@ uint32_t launch_tr(const Lowered &l, const zluda_gemm_plan &plan, void *ws, uint
   prm.group_p = 8;
   prm.splits = 1; prm.split_stages = 0; prm.ws = nullptr;
   if ((uint32_t)(prm.tiles_p * prm.tiles_q) != plan.grid_x) return CUBLAS_STATUS_INVALID_VALUE;
-  // aligned 16-bit operands: the same tiles, transposed by the LDS reads, 128 K bytes per stage
-  const bool lds_reads = (plan.variant == 1 || plan.variant == 3) && lds_transposable(l);
+  // the same tiles, transposed by the LDS reads: 128 K bytes per stage
+  const bool lds_reads = tr_lds_reads(l, (int)plan.variant, (uint64_t)plan.grid_x * plan.grid_y * std::max(plan.grid_z, 1u), plan.grid_z,
+                                      zluda_gemm_device_cu_count());
   if (plan.grid_z > 1) {
     // split-K: partial tiles go through the caller's workspace (64 K bytes per stage)
     const uint64_t need = (uint64_t)plan.grid_z * l.g.batch * prm.tiles_p * v.bp * prm.tiles_q * v.bq * 4;

@@ -501,6 +501,23 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus) {
   return best;
 }
 
+// The 128 x 128 tile exists in both forms for 16-bit operands.  us of `groups` workgroups, n = groups / CUs of them side by
+// side or in turn, u = bytes of K in a share / 4096 (bf16, MI355X, 128 to 768 tiles, K = 256 .. 1280; the choice is within 3 %
+// of the better one there):
+//   transposed in registers  4.6 + 1.2 n + (7.5 + 15.3 n) u
+//   by the LDS reads         6.2 + 1.45 n + 2.4 per round behind the first + 27.8 u per round of two on a CU, 17.4 u for one
+// -- level at K = 700 for n = 1, 430 for two, 1200 for three.  (2048 x 2048 x 128: 7.5 us in registers, 9.7 by the LDS reads;
+// 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 tile is faster by the LDS reads at every K.
+bool tr_lds_reads(const Lowered &l, int variant, uint64_t groups, uint32_t splits, uint32_t cus) {
+  if ((variant != 1 && variant != 3) || !lds_transposable(l)) return false;
+  if (variant == 3) return true;
+  const uint64_t n = (groups + cus - 1) / std::max(cus, 1u), rounds = (n + 1) / 2;
+  const double u = (double)l.g.K * 2 / 4096 / std::max(splits, 1u);
+  const double regs = 4.6 + 1.2 * (double)n + (7.5 + 15.3 * (double)n) * u;
+  const double lds = 6.2 + 1.45 * (double)n + 2.4 * (double)(rounds - 1) + (27.8 * (double)(n / 2) + 17.4 * (double)(n % 2)) * u;
+  return lds < regs;
+}
+
 static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t workspace_size, zluda_gemm_plan *plan) {
   const GemmArgs &g = l.g;
   const TrVariant &v = kTrVariants[variant];
@@ -510,8 +527,10 @@ static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t w
   plan->swapped = swapped;
   plan->grid_x = ceil_div(np, v.bp) * ceil_div(nq, v.bq); plan->grid_y = g.batch; plan->grid_z = 1;
   plan->block = v.wp * v.wq * 64;
-  const uint32_t per_cu = 160u * 1024u / (2u * (v.bp + v.bq) * 80u);  // LDS: two stages of 80-byte rows
-  plan->waves = (float)plan->grid_x * plan->grid_y / (float)(cus * std::min(per_cu, 4u));
+  // workgroups that share a CU: two stages of 80-byte rows each, or two of 128 K bytes at a pitch of 1056 bytes per KiB
+  const bool lds_reads = tr_lds_reads(l, variant, (uint64_t)plan->grid_x * plan->grid_y, 1, cus);
+  const uint32_t per_cu = std::min(160u * 1024u / (lds_reads ? 2u * (v.bp + v.bq) * 132u : 2u * (v.bp + v.bq) * 80u), 4u);
+  plan->waves = (float)plan->grid_x * plan->grid_y / (float)(cus * per_cu);
   plan->workspace = 0;
   // Split-K as for the K-contiguous kernels: grid_z workgroups share a tile's K range through the
   // caller's workspace when K has at least 16 stages and the tiles leave half of the chip idle --
@@ -519,7 +538,7 @@ static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t w
   // only ~16 KiB in flight), half of the workgroup slots.  N-contiguous weights, 16 tokens, us:
   // 4096x14336 89 -> 25, 4096x4096 31 -> 14, 14336x4096 31 -> 24; 14336x128x4096 would lose (37 -> 42).
   const uint64_t tiles = (uint64_t)plan->grid_x * plan->grid_y;
-  const uint64_t slots = (uint64_t)cus * std::min(per_cu, 4u);
+  const uint64_t slots = (uint64_t)cus * per_cu;
   const bool skinny = std::min(g.M, g.N) <= 64;
   const uint64_t kbytes = (uint64_t)g.K * type_bits(g.a_type) / 8;
   if (tiles * 2 <= (skinny ? slots : (uint64_t)cus) && kbytes >= 1024 && (uint64_t)ceil_div(np, v.bp) * v.bp <= (1u << 20)) {
@@ -541,24 +560,25 @@ static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t w
 struct TrCost { uint32_t per_cu; float base, slope; };
 static const TrCost kTrCost[kNumTrVariants] = {{1, 0.0f, 71.0f}, {2, 26.0f, 11.0f}, {4, 16.0f, 6.0f}, {1, 0.0f, 67.0f}};
 
-// f16 and bf16: the split along K that the variant would get counts as well, and with operands that the LDS reads
-// transpose (lds_transposable()) the variants 1 and 3 are that kernel, with times of its own.  us for 4096 bytes of K:
+// f16 and bf16: the split along K that the variant would get counts as well, and where the LDS reads transpose
+// (tr_lds_reads()) the variants 1 and 3 have times of their own.  us for 4096 bytes of K:
 // 128x128 25 + 3.3 n, 256x256 53 on a full chip (8192 x 4096 x 2048 121 us against 174 on 128x128; 2048 x 4096 x 8192, 128
 // tiles, 164 against 130); the others as above.  Around the loop 4 us, and for a split the second kernel and the partial
 // tiles' way through memory at 3 TB/s (1024 x 512 x 1024 on 128x128 would take 20 us split, 64x64 take 10).
 static const TrCost kTrCostLds[kNumTrVariants] = {{1, 0.0f, 71.0f}, {2, 25.0f, 3.3f}, {4, 16.0f, 6.0f}, {1, 0.0f, 53.0f}};
 
 static int pick_tr_variant_h16(const Lowered &l, uint32_t cus, uint64_t workspace_size) {
-  const bool lds = lds_transposable(l);
   const double units = (double)l.g.K * 2 / 4096;
   int best = 0;
   double best_cost = 0;
   for (int v = 0; v < kNumTrVariants; v++) {
-    const TrCost &c = (lds ? kTrCostLds : kTrCost)[v];
     zluda_gemm_plan p;
     memset(&p, 0, sizeof(p));
     fill_tr_plan(l, v, cus, workspace_size, &p);
-    const uint64_t groups = (uint64_t)p.grid_x * p.grid_y * p.grid_z, slots = (uint64_t)cus * c.per_cu;
+    const uint64_t groups = (uint64_t)p.grid_x * p.grid_y * p.grid_z;
+    const bool lds = tr_lds_reads(l, v, groups, p.grid_z, cus);
+    const TrCost &c = (lds ? kTrCostLds : kTrCost)[v];
+    const uint64_t slots = (uint64_t)cus * c.per_cu;
     if (kTrVariants[v].m16 && !lds && groups * 4 < (uint64_t)cus * 3) continue;
     const uint64_t full = groups / slots, rem = groups % slots;
     double cost = (double)full * (c.base + c.slope * c.per_cu);

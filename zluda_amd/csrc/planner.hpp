@@ -120,6 +120,10 @@ bool family_supports(uint32_t kernel, const Lowered &l);
 // K-contiguous, both 16-byte aligned with 16-byte aligned pitches, K-contiguous rows of whole 16-byte pieces
 bool lds_transposable(const Lowered &l);
 
+// whether `groups` workgroups (all shares and batches) of a variant of the transposing family do so, each share holding
+// K / splits: the tiles 1 and 3 of operands that allow it, the former from the K on where that is the faster form
+bool tr_lds_reads(const Lowered &l, int variant, uint64_t groups, uint32_t splits, uint32_t cus);
+
 // Row sums along the longer stride (bias gradients): how many workgroups share the `len` terms of each of `rows` sums, given
 // scratch for shares * rows * batch partial sums of 4 bytes; 1: no scratch is used
 uint32_t row_sum_shares(int64_t rows, int64_t len, int64_t batch, uint64_t workspace_size);
