@@ -241,6 +241,31 @@ __device__ __forceinline__ void mfma_store_tile_general(const MfmaParams &prm, A
   static_for<TQ * 2>(do_pass);
 }
 
+// The kernel's arguments lie in host memory: a cache line of them that a scalar load asks for first costs most of a
+// microsecond.  Asked for where they are used, in batches, the lines come one after the other; here all of them are asked for
+// together at the kernel's entry (one dword of each), and what is read later comes out of the scalar cache.
+__device__ __forceinline__ void fetch_args(const MfmaParams &prm) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int LINES = (sizeof(MfmaParams) + 63) / 64;
+  static_assert(LINES == 6, "one operand per line below");
+  const uint32_t *w = (const uint32_t *)&prm;
+  asm volatile("" ::"s"(w[0]), "s"(w[16]), "s"(w[32]), "s"(w[48]), "s"(w[64]), "s"(w[80]));
+#endif
+}
+
+// The arguments once more, for what runs behind the K loop.  Read through `prm` the compiler keeps everything an epilogue may
+// ask for from the kernel's entry on, has no scalar registers for it and spills.
+__device__ __forceinline__ const MfmaParams &args_again(const MfmaParams &prm) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef const __attribute__((address_space(4))) MfmaParams *arg_ptr;
+  uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();  // (the kernels' one argument lies at its start)
+  asm volatile("" : "+s"(at));
+  return *(const MfmaParams *)(arg_ptr)at;
+#else
+  return prm;
+#endif
+}
+
 // Fast path 1: pure integer epilogue with alpha, beta scalars and beta == 0: D = alpha * acc straight from the accumulator
 // registers.  Lanes 0..31 of a store hold 32 consecutive int32 of one D column (one 128-byte line), so no LDS staging is
 // needed; two instructions per output element.  Tiles that hang over the end of P (EDGE) mask their lanes, columns past the
@@ -515,28 +540,31 @@ __device__ __forceinline__ void mfma_store_tile(const MfmaParams &prm, AccV (&ac
   }
   if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
       (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F)) {
+    if (!whole) {
+      mfma_store_tile_float<KIND, WP, WQ, WTP, WTQ, true>(prm, acc, p0, q0, NP, NQ, bt);
+      return;
+    }
     // what varies along Q: a scale vector of B's, or a row-major D's per-row quantities
     const bool q_vec = prm.swapped ? g.alpha_mode == VECTOR_DEV || g.a_scale_mode == SCALE_OUTER_VEC || g.bias != nullptr
                                    : g.b_scale_mode == SCALE_OUTER_VEC;
-    if (whole && !q_vec) {
+    if (q_vec) {
+      mfma_store_tile_float<KIND, WP, WQ, WTP, WTQ, false>(prm, acc, p0, q0, NP, NQ, bt);
+      return;
+    }
 #define ZLUDA_EPI_PLAIN(ACT_, DT_) mfma_store_tile_plain<KIND, WP, WQ, WTP, WTQ, ACT_, DT_>(prm, acc, p0, q0, NP, NQ, bt)
 #define ZLUDA_EPI_ACT(DT_)                                  \
   if (g.act == ACT_GELU) ZLUDA_EPI_PLAIN(ACT_GELU, DT_);    \
   else if (g.act == ACT_RELU) ZLUDA_EPI_PLAIN(ACT_RELU, DT_); \
   else ZLUDA_EPI_PLAIN(ACT_NONE, DT_);
-      if (g.d_type == CUDA_R_16BF) {
-        ZLUDA_EPI_ACT(0)
-      } else if (g.d_type == CUDA_R_16F) {
-        ZLUDA_EPI_ACT(1)
-      } else {
-        ZLUDA_EPI_ACT(2)
-      }
+    if (g.d_type == CUDA_R_16BF) {
+      ZLUDA_EPI_ACT(0)
+    } else if (g.d_type == CUDA_R_16F) {
+      ZLUDA_EPI_ACT(1)
+    } else {
+      ZLUDA_EPI_ACT(2)
+    }
 #undef ZLUDA_EPI_ACT
 #undef ZLUDA_EPI_PLAIN
-      return;
-    }
-    if (whole) mfma_store_tile_float<KIND, WP, WQ, WTP, WTQ, false>(prm, acc, p0, q0, NP, NQ, bt);
-    else mfma_store_tile_float<KIND, WP, WQ, WTP, WTQ, true>(prm, acc, p0, q0, NP, NQ, bt);
     return;
   }
   mfma_store_tile_general<KIND, WP, WQ, WTP, WTQ>(prm, acc, lds_words, lds_bytes, p0, q0, NP, NQ, bt);

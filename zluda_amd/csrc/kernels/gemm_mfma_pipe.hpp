@@ -73,6 +73,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
 
   __shared__ v4i lds[NSTAGE * STAGE_V4 + 2 * CHUNK_V4];
 
+  fetch_args(prm);
   const GemmArgs &g = prm.g;
   // the wave index is uniform by construction; readfirstlane tells the compiler (LDS DMA bases and
   // buffer descriptors derived from it then live in SGPRs)
@@ -381,7 +382,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
     mfma_store_tile_raw<WP, WQ, WTP, WTQ>(ws_tile, ws_np, acc);
     return;
   }
-  mfma_store_tile<KIND, WP, WQ, WTP, WTQ>(prm, acc, (int *)&lds[0], sizeof(lds), p0, q0, NP, NQ, bt);
+  mfma_store_tile<KIND, WP, WQ, WTP, WTQ>(args_again(prm), acc, (int *)&lds[0], sizeof(lds), p0, q0, NP, NQ, bt);
 }
 
 } // namespace zluda_amd

@@ -349,6 +349,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
 
   __shared__ v4i lds[NSTAGE * STAGE_V4];
 
+  fetch_args(prm);
   const GemmArgs &g = prm.g;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wp = wave % WP, wq = wave / WP;
@@ -635,7 +636,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     mfma16_store_raw<false>(rs, ws_np, acc, 1, 0);
     return;
   }
-  mfma16_store_tile<KIND, WP, WQ, TP, TQ, (int)sizeof(lds)>(prm, acc, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
+  mfma16_store_tile<KIND, WP, WQ, TP, TQ, (int)sizeof(lds)>(args_again(prm), acc, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
 }
 
 } // namespace zluda_amd
