@@ -73,7 +73,8 @@ typedef struct zluda_gemm_problem {
 /* Kernel families the planner can choose. */
 enum {
   ZLUDA_KERNEL_AUTO = 0,
-  ZLUDA_KERNEL_GENERIC = 1,   /* any layout / type: LDS-tiled scalar kernel (correctness net) */
+  ZLUDA_KERNEL_GENERIC = 1,   /* any layout / type: LDS-tiled scalar kernel (correctness net), or the transposing kernel
+                                 where only alignment or a ragged K kept a problem from its family */
   ZLUDA_KERNEL_MFMA_I8 = 2,   /* v_mfma_i32_32x32x32_i8, K-contiguous A and B */
   ZLUDA_KERNEL_MFMA_F8 = 3,   /* v_mfma_f32_32x32x64_f8f6f4 (e4m3/e5m2) */
   ZLUDA_KERNEL_MFMA_MXF4 = 4, /* v_mfma_scale_f32_32x32x64_f8f6f4, E2M1 + UE8M0/32 */
@@ -92,7 +93,8 @@ enum {
 #define ZLUDA_ALGO_MAGIC 0x5a4c4441u /* "ZLDA" */
 typedef struct zluda_gemm_plan {
   uint32_t kernel;        /* ZLUDA_KERNEL_* */
-  uint32_t variant;       /* tile configuration index inside the family */
+  uint32_t variant;       /* tile configuration index inside the family; ZLUDA_KERNEL_GENERIC: 0 the scalar kernel, 1 + v
+                             variant v of the transposing kernel for the operands' type (unaligned operands, ragged K) */
   uint64_t workspace;     /* bytes of workspace the plan needs */
   uint32_t swapped;       /* 1 if the planner computes D^T = op(B)^T op(A)^T */
   uint32_t grid_x, grid_y, grid_z, block;

@@ -303,7 +303,8 @@ cublasStatus_t build_problem(cublasLtMatmulDesc_t op, cublasLtMatrixLayout_t A, 
 void pack_algo(const zluda_gemm_plan &plan, cublasLtMatmulAlgo_t *algo) {
   memset(algo, 0, sizeof(*algo));
   algo->data[0] = ((uint64_t)ZLUDA_ALGO_MAGIC << 32) | plan.kernel;
-  algo->data[1] = plan.variant;
+  // (the generic family chooses by itself for each call, from the pointers it is given)
+  algo->data[1] = plan.kernel == ZLUDA_KERNEL_GENERIC ? 0 : plan.variant;
   algo->data[2] = plan.workspace;
 }
 bool unpack_algo(const cublasLtMatmulAlgo_t *algo, uint32_t *kernel, int32_t *variant) {

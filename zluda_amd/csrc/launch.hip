@@ -362,12 +362,16 @@ uint32_t launch_planned(const zluda_gemm_problem *p, const zluda_gemm_plan *plan
   }
   switch (plan->kernel) {
   case ZLUDA_KERNEL_GENERIC: {
-    zluda_gemm_plan tr;
-    if (plan_transposing_under_generic(l, zluda_gemm_device_cu_count(), plan->workspace, &tr)) {
+    const uint32_t family = plan->variant ? transposing_under_generic(l) : 0;
+    if (family) {
+      zluda_gemm_plan tr = *plan;
+      tr.kernel = family;
+      tr.variant--;
       st = launch_tr(l, tr, ws, ws_size, s);
       break;
     }
-    dim3 grid(plan->grid_x, plan->grid_y, plan->grid_z);
+    // (also where a plan for that kernel meets pointers it does not take)
+    dim3 grid((l.g.M + 63) / 64, (l.g.N + 63) / 64, l.g.batch);
     const bool int_acc = l.g.a_type == CUDA_R_8I;
     st = int_acc ? launch_kernel(gemm_generic_kernel<true>, grid, dim3(256), s, l.g)
                  : launch_kernel(gemm_generic_kernel<false>, grid, dim3(256), s, l.g);

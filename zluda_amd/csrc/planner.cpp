@@ -634,14 +634,11 @@ static uint64_t row_sum_workspace(const GemmArgs &g, uint64_t workspace_size) {
   return s > 1 ? (uint64_t)s * rows * g.batch * 4 : 0;
 }
 
-uint32_t plan_transposing_under_generic(const Lowered &l, uint32_t cus, uint64_t workspace_size, zluda_gemm_plan *plan) {
+uint32_t transposing_under_generic(const Lowered &l) {
   const uint32_t family = transposing_family(l, true);
   if (!family || transposing_family(l, false)) return 0;
   for (uint32_t k : {ZLUDA_KERNEL_MFMA_I8, ZLUDA_KERNEL_MFMA_F8, ZLUDA_KERNEL_MFMA_H16, ZLUDA_KERNEL_MFMA_F32})
     if (family_supports(k, l)) return 0;
-  memset(plan, 0, sizeof(*plan));
-  plan->kernel = family;
-  fill_tr_plan(l, pick_tr_variant(l, cus, workspace_size), cus, workspace_size, plan);
   return family;
 }
 
@@ -770,11 +767,10 @@ extern "C" uint32_t zluda_gemm_plan_problem(const zluda_gemm_problem *p, uint32_
     plan->block = 256;
     plan->waves = (float)plan->grid_x * plan->grid_y * plan->grid_z / (float)(cu_count * 8);
     if (plan->grid_y > 65535) return CUBLAS_STATUS_NOT_SUPPORTED;
-    {
-      // what only alignment or a ragged K keeps from the transposing kernel runs on it all the same (launch_planned); its
-      // split along K wants scratch like any other
-      zluda_gemm_plan tr;
-      if (plan_transposing_under_generic(l, cu_count, p->workspace_size, &tr)) { plan->workspace = tr.workspace; plan->waves = tr.waves; }
+    // what only alignment or a ragged K keeps from the transposing kernel runs on it all the same: variant 1 + v
+    if (transposing_under_generic(l)) {
+      fill_tr_plan(l, pick_tr_variant(l, cu_count, p->workspace_size), cu_count, p->workspace_size, plan);
+      plan->variant++;
     }
     break;
   case ZLUDA_KERNEL_MFMA_I8: case ZLUDA_KERNEL_MFMA_F8: case ZLUDA_KERNEL_MFMA_MXF4: case ZLUDA_KERNEL_MFMA_H16:

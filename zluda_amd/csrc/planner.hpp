@@ -109,9 +109,9 @@ uint32_t lower_problem(const zluda_gemm_problem *p, bool dry, Lowered *out);
 int w4_epilogue_class(const Lowered &l, bool dry);
 
 // The generic family's fast road: problems that only alignment or a K-contiguous row that ends inside a 16-byte piece keeps
-// from every MFMA family run on the transposing kernel.  Fills `plan` for it (kernel = the family whose launcher takes it)
-// and returns that family, or 0: the scalar kernel.
-uint32_t plan_transposing_under_generic(const Lowered &l, uint32_t cus, uint64_t workspace_size, zluda_gemm_plan *plan);
+// from every MFMA family run on the transposing kernel (plan.variant = 1 + its variant, with its grid).  The family whose
+// launcher takes them, or 0: the scalar kernel (plan.variant = 0).
+uint32_t transposing_under_generic(const Lowered &l);
 
 // which kernel families can run the lowered problem
 bool family_supports(uint32_t kernel, const Lowered &l);
