@@ -268,7 +268,7 @@ uint32_t launch_bgrad_typed(BgradParams &b, void *ws, uint64_t ws_size, hipStrea
   constexpr int V = elems16(TYPE), ESZ = 16 / V;
   b.wide = !(((uintptr_t)b.src | (uintptr_t)(b.s_b * ESZ) | (uintptr_t)((b.s_k <= b.s_row ? b.s_row : b.s_k) * ESZ)) & 15);
   if (b.s_k <= b.s_row) return launch_kernel(bgrad_rows_kernel<TYPE>, dim3(b.rows, 1, b.batch), dim3(256), s, b);
-  const uint32_t shares = row_sum_shares(b.rows, b.K, b.batch, ws_size);
+  const uint32_t shares = row_sum_shares(b.rows, b.K, b.batch, ws_size, zluda_gemm_device_cu_count());
   b.per_block = (int32_t)((b.K + shares - 1) / shares);
   b.part = ws;
   uint32_t st;
@@ -323,7 +323,7 @@ uint32_t launch_aux_typed(const GemmArgs &g, void *ws, uint64_t ws_size, hipStre
   a.out = g.bgrad; a.out_type = g.bias_type; a.out_sb = g.bias_sb;
   if (!col && a.sums) return launch_kernel(aux_dgelu_rows_kernel<TYPE>, dim3(a.NQ, 1, g.batch), dim3(256), s, a);
   // (without sums nothing is carried from one share of Q to another)
-  const uint32_t shares = row_sum_shares(a.NP, a.NQ, g.batch, a.sums ? ws_size : ~0ull);
+  const uint32_t shares = row_sum_shares(a.NP, a.NQ, g.batch, a.sums ? ws_size : ~0ull, zluda_gemm_device_cu_count());
   a.per_block = (int32_t)((a.NQ + shares - 1) / shares);
   a.part = ws;
   uint32_t st;

@@ -613,24 +613,25 @@ static int pick_tr_variant(const Lowered &l, uint32_t cus, uint64_t workspace_si
   return best;
 }
 
-// A workgroup of the row-sum kernels takes 64 to 256 rows.  Enough shares for about four workgroups per CU, 64 terms at the
-// least in each: 2048 sums of 4096 terms take 1024 workgroups in 32 shares.
-uint32_t row_sum_shares(int64_t rows, int64_t len, int64_t batch, uint64_t workspace_size) {
+// Enough shares for about four workgroups per CU at 64 rows a workgroup, 64 terms at the least in each: 2048 sums of 4096 terms
+// take 1024 workgroups in 32 shares on 256 CUs.  (A workgroup takes 16 bytes' worth of rows per lane: with K shared out 32 to 128
+// of an operand, 128 or 256 of a GELU gradient; unshared half of the former and 16 or 32.)
+uint32_t row_sum_shares(int64_t rows, int64_t len, int64_t batch, uint64_t workspace_size, uint32_t cus) {
   const int64_t groups = (rows + 63) / 64 * batch;
-  int64_t s = std::min<int64_t>({(1024 + groups - 1) / groups, len / 64, 65535});
+  int64_t s = std::min<int64_t>({(4 * (int64_t)cus + groups - 1) / groups, len / 64, 65535});
   const uint64_t per_share = (uint64_t)rows * batch * 4;
   if (s > 1 && (uint64_t)s * per_share > workspace_size) s = (int64_t)(workspace_size / per_share);
   return s > 1 ? (uint32_t)s : 1u;
 }
 
 // scratch the bias-gradient sums of the problem would use, within `workspace_size`
-static uint64_t row_sum_workspace(const GemmArgs &g, uint64_t workspace_size) {
+static uint64_t row_sum_workspace(const GemmArgs &g, uint64_t workspace_size, uint32_t cus) {
   int64_t rows = 0, len = 0;
   if (g.bgrad_src == 1 && g.a_sk > g.a_si) { rows = g.M; len = g.K; }
   else if (g.bgrad_src == 2 && g.b_sk > g.b_sj) { rows = g.N; len = g.K; }
   else if (g.aux_bgrad && g.d_si == 1) { rows = g.M; len = g.N; }
   if (rows == 0) return 0;
-  const uint32_t s = row_sum_shares(rows, len, g.batch, workspace_size);
+  const uint32_t s = row_sum_shares(rows, len, g.batch, workspace_size, cus);
   return s > 1 ? (uint64_t)s * rows * g.batch * 4 : 0;
 }
 
@@ -812,6 +813,6 @@ extern "C" uint32_t zluda_gemm_plan_problem(const zluda_gemm_problem *p, uint32_
   default: return CUBLAS_STATUS_NOT_SUPPORTED;
   }
   // (the sums run behind the matmul and its reduction, in the same scratch)
-  plan->workspace = std::max(plan->workspace, row_sum_workspace(l.g, p->workspace_size));
+  plan->workspace = std::max(plan->workspace, row_sum_workspace(l.g, p->workspace_size, cu_count));
   return CUBLAS_STATUS_SUCCESS;
 }

@@ -126,7 +126,7 @@ bool tr_lds_reads(const Lowered &l, int variant, uint64_t groups, uint32_t split
 
 // Row sums along the longer stride (bias gradients): how many workgroups share the `len` terms of each of `rows` sums, given
 // scratch for shares * rows * batch partial sums of 4 bytes; 1: no scratch is used
-uint32_t row_sum_shares(int64_t rows, int64_t len, int64_t batch, uint64_t workspace_size);
+uint32_t row_sum_shares(int64_t rows, int64_t len, int64_t batch, uint64_t workspace_size, uint32_t cus);
 
 // Lowers `p` with its real pointers and enqueues the kernel `plan` names on `stream` (a hipStream_t).
 // `ws` / `ws_size`: device scratch, at least plan->workspace bytes, of which plan->workspace are used (split-K partial tiles,
