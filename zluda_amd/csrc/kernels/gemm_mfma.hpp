@@ -521,7 +521,8 @@ __device__ __forceinline__ void mfma_store_tile_plain(const MfmaParams &prm, Acc
 }
 
 // Epilogue dispatch: the fast paths for the common configurations, the general path for the rest (C reads, 8-bit outputs,
-// integer outputs of a float epilogue, vectors of alpha in the integer one).  All conditions are workgroup-uniform.
+// integer outputs of a float epilogue, vectors of alpha in the integer one).  All conditions are workgroup-uniform.  What they
+// and the integer path read is few enough to be kept from the kernel's entry on; the float paths read the arguments again.
 template <int KIND, int WP, int WQ, int WTP, int WTQ, class AccV>
 __device__ __forceinline__ void mfma_store_tile(const MfmaParams &prm, AccV (&acc)[WTQ / 32][WTP / 32],
                                                 int *lds_words, size_t lds_bytes, int p0, int q0, int NP,
@@ -538,20 +539,21 @@ __device__ __forceinline__ void mfma_store_tile(const MfmaParams &prm, AccV (&ac
       return;
     }
   }
+  const MfmaParams &late = args_again(prm);
   if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
       (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F)) {
     if (!whole) {
-      mfma_store_tile_float<KIND, WP, WQ, WTP, WTQ, true>(prm, acc, p0, q0, NP, NQ, bt);
+      mfma_store_tile_float<KIND, WP, WQ, WTP, WTQ, true>(late, acc, p0, q0, NP, NQ, bt);
       return;
     }
     // what varies along Q: a scale vector of B's, or a row-major D's per-row quantities
-    const bool q_vec = prm.swapped ? g.alpha_mode == VECTOR_DEV || g.a_scale_mode == SCALE_OUTER_VEC || g.bias != nullptr
-                                   : g.b_scale_mode == SCALE_OUTER_VEC;
+    const bool q_vec = prm.swapped ? g.alpha_mode == VECTOR_DEV || late.g.a_scale_mode == SCALE_OUTER_VEC || late.g.bias != nullptr
+                                   : late.g.b_scale_mode == SCALE_OUTER_VEC;
     if (q_vec) {
-      mfma_store_tile_float<KIND, WP, WQ, WTP, WTQ, false>(prm, acc, p0, q0, NP, NQ, bt);
+      mfma_store_tile_float<KIND, WP, WQ, WTP, WTQ, false>(late, acc, p0, q0, NP, NQ, bt);
       return;
     }
-#define ZLUDA_EPI_PLAIN(ACT_, DT_) mfma_store_tile_plain<KIND, WP, WQ, WTP, WTQ, ACT_, DT_>(prm, acc, p0, q0, NP, NQ, bt)
+#define ZLUDA_EPI_PLAIN(ACT_, DT_) mfma_store_tile_plain<KIND, WP, WQ, WTP, WTQ, ACT_, DT_>(late, acc, p0, q0, NP, NQ, bt)
 #define ZLUDA_EPI_ACT(DT_)                                  \
   if (g.act == ACT_GELU) ZLUDA_EPI_PLAIN(ACT_GELU, DT_);    \
   else if (g.act == ACT_RELU) ZLUDA_EPI_PLAIN(ACT_RELU, DT_); \
@@ -567,7 +569,7 @@ __device__ __forceinline__ void mfma_store_tile(const MfmaParams &prm, AccV (&ac
 #undef ZLUDA_EPI_PLAIN
     return;
   }
-  mfma_store_tile_general<KIND, WP, WQ, WTP, WTQ>(prm, acc, lds_words, lds_bytes, p0, q0, NP, NQ, bt);
+  mfma_store_tile_general<KIND, WP, WQ, WTP, WTQ>(late, acc, lds_words, lds_bytes, p0, q0, NP, NQ, bt);
 }
 
 } // namespace zluda_amd

@@ -382,7 +382,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
     mfma_store_tile_raw<WP, WQ, WTP, WTQ>(ws_tile, ws_np, acc);
     return;
   }
-  mfma_store_tile<KIND, WP, WQ, WTP, WTQ>(args_again(prm), acc, (int *)&lds[0], sizeof(lds), p0, q0, NP, NQ, bt);
+  mfma_store_tile<KIND, WP, WQ, WTP, WTQ>(prm, acc, (int *)&lds[0], sizeof(lds), p0, q0, NP, NQ, bt);
 }
 
 } // namespace zluda_amd

@@ -268,9 +268,10 @@ __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&
       return;
     }
   }
+  const MfmaParams &late = args_again(prm);
   if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
       (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F)) {
-#define ZLUDA_EPI16(DT_, ACT_, EDGE_) mfma16_store_f<KIND, WP, WQ, TP, TQ, DT_, ACT_, EDGE_>(prm, acc, p0, q0, NP, NQ, bt, wave)
+#define ZLUDA_EPI16(DT_, ACT_, EDGE_) mfma16_store_f<KIND, WP, WQ, TP, TQ, DT_, ACT_, EDGE_>(late, acc, p0, q0, NP, NQ, bt, wave)
 #define ZLUDA_EPI16_ACT(DT_)                                 \
   if (g.act == ACT_GELU) ZLUDA_EPI16(DT_, ACT_GELU, false);  \
   else if (g.act == ACT_RELU) ZLUDA_EPI16(DT_, ACT_RELU, false); \
@@ -290,7 +291,7 @@ __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&
     return;
   }
   __syncthreads();  // (workgroup-uniform branch) the LDS tiles become staging
-  mfma16_store_general<KIND, WP, WQ, TP, TQ, LDS_BYTES>(prm, acc, lds_words, p0, q0, NP, NQ, bt, wave);
+  mfma16_store_general<KIND, WP, WQ, TP, TQ, LDS_BYTES>(late, acc, lds_words, p0, q0, NP, NQ, bt, wave);
 }
 
 // ---- the kernel ----------------------------------------------------------------------------------------
@@ -636,7 +637,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     mfma16_store_raw<false>(rs, ws_np, acc, 1, 0);
     return;
   }
-  mfma16_store_tile<KIND, WP, WQ, TP, TQ, (int)sizeof(lds)>(args_again(prm), acc, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
+  mfma16_store_tile<KIND, WP, WQ, TP, TQ, (int)sizeof(lds)>(prm, acc, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
 }
 
 } // namespace zluda_amd

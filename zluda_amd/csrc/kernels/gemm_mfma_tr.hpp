@@ -632,7 +632,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
       mfma16_store_raw<false>(rs, ws_np, acc16, 1, 0);
       return;
     }
-    mfma16_store_tile<KIND, WP, WQ, TP16, TQ16, (int)sizeof(lds)>(args_again(prm), acc16, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
+    mfma16_store_tile<KIND, WP, WQ, TP16, TQ16, (int)sizeof(lds)>(prm, acc16, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
   } else {
   if (prm.splits > 1) {
     const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
@@ -640,7 +640,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
     mfma_store_tile_raw<WP, WQ, WTP, WTQ>(ws_tile, ws_np, acc);
     return;
   }
-  mfma_store_tile<KIND, WP, WQ, WTP, WTQ>(args_again(prm), acc, (int *)&lds[0], sizeof(lds), p0, q0, NP, NQ, bt);
+  mfma_store_tile<KIND, WP, WQ, WTP, WTQ>(prm, acc, (int *)&lds[0], sizeof(lds), p0, q0, NP, NQ, bt);
   }
 }
 
