@@ -120,26 +120,50 @@ static void check_pipe16(int variant) {
   }
 }
 
-// gemm_mfma_tr_kernel: trip kt stores stage kt + 1's registers while stage min(kt + 2, kl)'s loads are in flight
-static void check_tr() {
-  for (int kbytes = 1; kbytes <= 64 * 9; kbytes++) {
-    const int KT = (kbytes + 63) / 64, KL = KT > 0 ? KT - 1 : 0;
-    const int tail_from = tr_tail_from(kbytes);
-    auto may_hold_lanes_past_k = [&](int stage) { return stage >= KL && (kbytes & 63) != 0; };
-    // the prologue stores stage 0 with the loads of stage min(1, KL) in flight
-    if (may_hold_lanes_past_k(1 < KL ? 1 : KL) && !(tail_from < 0)) {
-      printf("transposing kernel, K = %d bytes: the prologue counts past a stage that can retire early\n", kbytes);
-      exit(1);
-    }
-    for (int kt = 0; kt + 1 <= KL; kt++) {  // trips that still store a stage
-      const int younger = kt + 2 < KL ? kt + 2 : KL;
-      if (may_hold_lanes_past_k(younger) && !(kt >= tail_from)) {
-        printf("transposing kernel, K = %d bytes, trip %d: counts past a stage that can retire early\n", kbytes, kt);
-        exit(1);
-      }
+// The form of gemm_mfma_pipe16_kernel for operands along their row index, on tiles of bp x bq: what the prologue counts on --
+// stage 0 landed with stage 1's instructions outstanding -- holds only while neither stage can retire ahead of its turn, i.e.
+// neither is the last one, whose K tail an instruction may miss altogether.  (The waits of the loop count nothing.)
+static void check_pipe16_mc(int bp, int bq, int wp, int wq) {
+  const Pipe16Counts c = pipe16_counts(bp, bq, wp, wq);
+  if (c.wait_stage != 0) fail("a wait of the loop that counts", -1, 0, 0, 0, 0);
+  for (int KT = 1; KT <= 9; KT++) {
+    const int last = KT - 1;
+    if (last <= 1 && !pipe16_drains_prologue(true, KT)) fail("the prologue counts past a stage that can retire early", -1, 0, 0, 0, KT);
+    if (last > 1 && pipe16_drains_prologue(true, KT)) fail("needless wait in the prologue", -1, 0, 0, 0, KT);
+    if (pipe16_drains_prologue(false, KT)) fail("needless wait in the prologue", -1, 0, 0, 0, KT);
+    checked++;
+  }
+}
+
+// gemm_mfma_tr_kernel: the stages are requested in order, nothing past the last one, kl.  The prologue stores stage 0's registers
+// with stage 1 in flight, trip kt those of stage kt + 1 with stage kt + 2 in flight.
+static void check_tr(int esz) {
+  for (int kbytes = esz; kbytes <= 64 * 9; kbytes += esz) {
+    const int KT = (kbytes + 63) / 64, KL = KT - 1;
+    const int tail_from = tr_tail_from(kbytes, esz);
+    const bool last_retires_early = (kbytes & 63) != 0 || esz == 2;  // lanes past the end of K; the extra loads of 2-byte elements
+    std::vector<int> in_flight;  // stages, oldest first
+    auto request = [&](int stage) { if (stage <= KL) in_flight.push_back(stage); };
+    auto store = [&](int stage, bool waits_for_all, const char *where, int kt) {
+      // counted: everything but the stages younger than `stage` has landed -- unless one of those can be done before its turn
+      for (int s : in_flight)
+        if (s > stage && s == KL && last_retires_early && !waits_for_all) {
+          printf("transposing kernel, K = %d bytes of %d-byte elements, %s %d: counts past a stage that can retire early\n", kbytes, esz, where, kt);
+          exit(1);
+        }
+      if (waits_for_all) in_flight.clear();
+      while (!in_flight.empty() && in_flight[0] <= stage) in_flight.erase(in_flight.begin());
       checked++;
+    };
+    request(0); request(1);
+    store(0, tail_from < 0, "prologue", 0);
+    request(2);
+    for (int kt = 0; kt + 1 <= KL; kt++) {  // trips that still store a stage
+      store(kt + 1, kt >= tail_from, "trip", kt);
+      request(kt + 3);
     }
-    if ((kbytes & 63) == 0 && tail_from != 0x7fffffff) { printf("transposing kernel, K = %d bytes: needless waits\n", kbytes); exit(1); }
+    if (!last_retires_early && tail_from != 0x7fffffff) { printf("transposing kernel, K = %d bytes: needless waits\n", kbytes); exit(1); }
+    if (last_retires_early && KL >= 3 && KL - 3 >= tail_from) { printf("transposing kernel, K = %d bytes: waits a trip early\n", kbytes); exit(1); }
   }
 }
 
@@ -152,7 +176,8 @@ int main() {
     for (int ks : {v.bkb / 32, v.bkb / 64}) check_pipe(variant, false, ks);
     if (variant < kNumMfmaVariants32) check_pipe(variant, true, v.bkb / 32);
   }
-  check_tr();
+  for (int v : {1, 3}) check_pipe16_mc(kTrVariants[v].bp, kTrVariants[v].bq, kTrVariants[v].wp, kTrVariants[v].wq);
+  for (int esz : {1, 2, 4}) check_tr(esz);
   printf("%ld waits checked\n", checked);
   return 0;
 }

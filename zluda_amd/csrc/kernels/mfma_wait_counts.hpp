@@ -67,14 +67,19 @@ constexpr Pipe16Counts pipe16_counts(int bp, int bq, int wp, int wq) {
   return c;
 }
 
+// The form of gemm_mfma_pipe16.hpp whose operands lie along their row index ("MC"): an instruction of the last stage may hold
+// no K row that exists.  The prologue, the one place that counts, waits for everything where stage 0 or 1 is that stage.
+constexpr bool pipe16_drains_prologue(bool mc, int kt) { return mc && kt <= 2; }
+
 // gemm_mfma_tr.hpp leaves its waits to the compiler, which counts: before the LDS stores of trip kt (stage kt + 1's
-// registers) it waits until only stage kt + 2's loads are outstanding.  Stages hold 64 K bytes; only the last one that
-// holds data, stage kl = ceil(kbytes / 64) - 1, can have lanes past the end of K (later trips load it again), and only
-// when kbytes is no multiple of 64.  From the first trip whose younger stage is that one, the kernel waits for
+// registers) it waits until only stage kt + 2's loads are outstanding.  Stages hold 64 K bytes; nothing past the last one that
+// holds data, stage kl = ceil(kbytes / 64) - 1, is fetched.  Instructions of that stage can have all of their lanes out of
+// range when kbytes is no multiple of 64, and with 2-byte elements always (the last element of a row, fetched on its own by
+// the lanes that have one).  From the first trip whose younger stage is that one, the kernel waits for
 // everything instead: the value below, compared with kt (0x7fffffff: never; negative: the prologue waits as well).
-constexpr int tr_tail_from(int kbytes) {
+constexpr int tr_tail_from(int kbytes, int esz) {
   const int kt = (kbytes + 63) / 64, kl = kt > 0 ? kt - 1 : 0;
-  return (kbytes & 63) ? kl - 2 : 0x7fffffff;
+  return (kbytes & 63) || esz == 2 ? kl - 2 : 0x7fffffff;
 }
 
 } // namespace zluda_amd
