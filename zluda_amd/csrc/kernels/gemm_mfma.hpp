@@ -260,7 +260,12 @@ __device__ __forceinline__ const MfmaParams &args_again(const MfmaParams &prm) {
   typedef const __attribute__((address_space(4))) MfmaParams *arg_ptr;
   uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();  // (the kernels' one argument lies at its start)
   asm volatile("" : "+s"(at));
-  return *(const MfmaParams *)(arg_ptr)at;
+  const MfmaParams &again = *(const MfmaParams *)(arg_ptr)at;
+  // (what every float epilogue asks for, in one go: left to its first uses it is a chain of loads and branches)
+  const GemmArgs &g = again.g;
+  asm volatile("" ::"s"(g.alpha_mode), "s"(g.alpha_val.i), "s"(g.alpha_ptr), "s"(g.a_scale_mode), "s"(g.b_scale_mode), "s"(g.a_scale),
+               "s"(g.b_scale), "s"(g.d_scale), "s"(g.bias), "s"(g.bias_type), "s"(g.D), "s"(g.d_sb));
+  return again;
 #else
   return prm;
 #endif
