@@ -31,7 +31,7 @@
 // through the same loop: the DMA copies 64 K rows of 128 or 256 elements as they lie in memory, and ds_read_b64_tr_b16
 // (16 lanes read 4 K rows x 16 elements; lane i gets the four K elements of row i) transposes on the way into the
 // fragments, so there is no work in registers and no store to LDS.  The kernel of gemm_mfma_tr.hpp, which transposes in
-// registers, spends its stages on that: bf16 8192^3 A:N B:N 1019 us there, 808 here; 4096^3 A:N B:N 107; 128 x 128 tiles,
+// registers, spends its stages on that: bf16 8192^3 A:N B:N 1019 us there, 808 here; 4096^3 A:N B:N 110; 128 x 128 tiles,
 // 2048 x 4096 x 8192 A:N B:N 183 and 133 inside a training step.
 // LDS layout of such an operand: blocks of 1 KiB, one DMA instruction of a wave each, at a pitch of 1056 bytes.  A block
 // holds the K rows {k, k + 4} (256 elements a row) or {k, k + 4, k + 32, k + 36} (128), and the blocks run over k = 0..3,

@@ -47,7 +47,7 @@ inline uint32_t launch_tr_variant(const MfmaParams &prm, const zluda_gemm_plan &
   return CUBLAS_STATUS_INVALID_VALUE;
 }
 
-// the variants 1 and 3 on 16-byte aligned 16-bit operands: their grids, with the transposition in the LDS reads
+// the variants 1 and 3 where tr_lds_reads() says so: their grids, with the transposition in the LDS reads
 uint32_t launch_trl_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_trl_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_i8(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
