@@ -80,17 +80,10 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wp = wave % WP, wq = wave / WP;
   const int lr = lane & 31, gsel = lane >> 5;
-  const int bt = blockIdx.y;
 
-  // ---- workgroup -> tile (see gemm_mfma.hpp) ---------------------------------------------------
-  const int total = prm.tiles_p * prm.tiles_q;
-  int w = blockIdx.x;
-  if ((total & 7) == 0) w = (w & 7) * (total >> 3) + (w >> 3);
-  const int group = prm.group_p * prm.tiles_q;
-  const int gid = w / group, first_p = gid * prm.group_p;
-  const int gsz = min(prm.tiles_p - first_p, prm.group_p);
-  const int tile_p = first_p + (w % group) % gsz, tile_q = (w % group) / gsz;
-  const int p0 = tile_p * BP, q0 = tile_q * BQ;
+  const WorkItem item = work_item(prm);
+  const int bt = item.bt;
+  const int p0 = item.p * BP, q0 = item.q * BQ;
 
   const int NP = prm.swapped ? g.N : g.M, NQ = prm.swapped ? g.M : g.N;
   constexpr int ebits = KIND == KIND_MXF4 ? 4 : 8 * kind_esz(KIND);
@@ -111,7 +104,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
   int sk0 = 0;  // MX: first scale byte of this workgroup's K range in a row of scales (the host keeps
                 // split_stages a multiple of the CH stages of a scale chunk)
   if (prm.splits > 1) {
-    k0 = (int)blockIdx.z * prm.split_stages * BKB_;
+    k0 = item.z * prm.split_stages * BKB_;
     Kbytes_local = max(0, min(Kbytes - k0, prm.split_stages * BKB_));
     sk0 = k0 / 16;
   }
@@ -378,7 +371,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
   __syncthreads();
   if (prm.splits > 1) {
     const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
-    int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)blockIdx.z * g.batch + bt) * ws_np * ws_nq + (int64_t)q0 * ws_np + p0;
+    int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)item.z * g.batch + bt) * ws_np * ws_nq + (int64_t)q0 * ws_np + p0;
     mfma_store_tile_raw<WP, WQ, WTP, WTQ>(ws_tile, ws_np, acc);
     return;
   }

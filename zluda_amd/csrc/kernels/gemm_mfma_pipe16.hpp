@@ -355,17 +355,10 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wp = wave % WP, wq = wave / WP;
   const int r16 = lane & 15, g4 = lane >> 4;
-  const int bt = blockIdx.y;
 
-  // ---- workgroup -> tile (as in gemm_mfma_pipe_kernel) ----------------------------------------------------
-  const int total = prm.tiles_p * prm.tiles_q;
-  int w = blockIdx.x;
-  if ((total & 7) == 0) w = (w & 7) * (total >> 3) + (w >> 3);
-  const int group = prm.group_p * prm.tiles_q;
-  const int gid = w / group, first_p = gid * prm.group_p;
-  const int gsz = min(prm.tiles_p - first_p, prm.group_p);
-  const int tile_p = first_p + (w % group) % gsz, tile_q = (w % group) / gsz;
-  const int p0 = tile_p * BP, q0 = tile_q * BQ;
+  const WorkItem item = work_item(prm);
+  const int bt = item.bt;
+  const int p0 = item.p * BP, q0 = item.q * BQ;
 
   const int NP = prm.swapped ? g.N : g.M, NQ = prm.swapped ? g.M : g.N;
   const int Kbytes = g.K * ESZ;
@@ -381,7 +374,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   // split-K: this workgroup's share of the stages starts k0 bytes into every row
   int Kbytes_local = Kbytes, k0 = 0;
   if (prm.splits > 1) {
-    k0 = (int)blockIdx.z * prm.split_stages * BKB;
+    k0 = item.z * prm.split_stages * BKB;
     Kbytes_local = max(0, min(Kbytes - k0, prm.split_stages * BKB));
   }
   const int KT = (Kbytes_local + BKB - 1) / BKB;  // real stages
@@ -632,7 +625,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   __builtin_amdgcn_s_waitcnt(0);  // every DMA of the padding stages has landed before the LDS is reused or the wave ends
   if (prm.splits > 1) {
     const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
-    int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)blockIdx.z * g.batch + bt) * ws_np * ws_nq + (int64_t)(q0 + wq * WTQ) * ws_np + p0 + wp * WTP;
+    int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)item.z * g.batch + bt) * ws_np * ws_nq + (int64_t)(q0 + wq * WTQ) * ws_np + p0 + wp * WTP;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)ws_tile, 0, 0xFFFFFFFF, 0x00020000);
     mfma16_store_raw<false>(rs, ws_np, acc, 1, 0);
     return;

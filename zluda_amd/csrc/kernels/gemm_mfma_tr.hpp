@@ -263,17 +263,10 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wp = wave % WP, wq = wave / WP;
   const int lr = lane & 31, gsel = lane >> 5;
-  const int bt = blockIdx.y;
 
-  // workgroup -> tile: as in gemm_mfma_pipe_kernel
-  const int total = prm.tiles_p * prm.tiles_q;
-  int w = blockIdx.x;
-  if ((total & 7) == 0) w = (w & 7) * (total >> 3) + (w >> 3);
-  const int group = prm.group_p * prm.tiles_q;
-  const int gid = w / group, first_p = gid * prm.group_p;
-  const int gsz = min(prm.tiles_p - first_p, prm.group_p);
-  const int tile_p = first_p + (w % group) % gsz, tile_q = (w % group) / gsz;
-  const int p0 = tile_p * BP, q0 = tile_q * BQ;
+  const WorkItem item = work_item(prm);
+  const int bt = item.bt;
+  const int p0 = item.p * BP, q0 = item.q * BQ;
   const int NP = prm.swapped ? g.N : g.M, NQ = prm.swapped ? g.M : g.N;
 
   TrOperand<LP, PKC, ESZ> P;
@@ -285,7 +278,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
   // (k0, Kl in elements; a stage is 64 bytes of K)
   int k0 = 0, Kl = g.K;
   if (prm.splits > 1) {
-    k0 = (int)blockIdx.z * prm.split_stages * (64 / ESZ);
+    k0 = item.z * prm.split_stages * (64 / ESZ);
     Kl = max(0, min(g.K - k0, prm.split_stages * (64 / ESZ)));
   }
   {
@@ -626,7 +619,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
   if constexpr (M16) {
     if (prm.splits > 1) {
       const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
-      int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)blockIdx.z * g.batch + bt) * ws_np * ws_nq + (int64_t)(q0 + wq * WTQ) * ws_np + p0 + wp * WTP;
+      int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)item.z * g.batch + bt) * ws_np * ws_nq + (int64_t)(q0 + wq * WTQ) * ws_np + p0 + wp * WTP;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)ws_tile, 0, 0xFFFFFFFF, 0x00020000);
       mfma16_store_raw<false>(rs, ws_np, acc16, 1, 0);
       return;
@@ -635,7 +628,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
   } else {
   if (prm.splits > 1) {
     const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
-    int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)blockIdx.z * g.batch + bt) * ws_np * ws_nq + (int64_t)q0 * ws_np + p0;
+    int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)item.z * g.batch + bt) * ws_np * ws_nq + (int64_t)q0 * ws_np + p0;
     mfma_store_tile_raw<WP, WQ, WTP, WTQ>(ws_tile, ws_np, acc);
     return;
   }

@@ -431,19 +431,12 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
   const int ldp = ((int)(prm.swapped ? g.b_sj : g.a_si) << (H16 ? 1 : 0)) >> (MX ? 1 : 0);  // bytes
   const int ldq = ((int)(prm.swapped ? g.a_si : g.b_sj) << (H16 ? 1 : 0)) >> (MX ? 1 : 0);
 
-  // n-th tile of this workgroup -> tile corner and batch (the order of gemm_mfma_pipe_kernel: the 8 XCDs take
-  // turns at workgroup ids, so ids are spread over 8 contiguous ranges of the tile order, which walks groups
-  // of group_p tiles along P; G is a multiple of 8 whenever total is)
+  // n-th tile of this workgroup -> tile corner and batch (G is a multiple of 8 whenever a workgroup has more than one tile)
   auto tile_coords = [&](int n, int &p0, int &q0, int &bt) __attribute__((always_inline)) {
-    const int idx = (int)blockIdx.x + n * G;
-    bt = idx / total;
-    int w = idx - bt * total;
-    if ((total & 7) == 0) w = (w & 7) * (total >> 3) + (w >> 3);
-    const int group = prm.group_p * prm.tiles_q;
-    const int gid = w / group, first_p = gid * prm.group_p;
-    const int gsz = min(prm.tiles_p - first_p, prm.group_p);
-    p0 = (first_p + (w % group) % gsz) * BP;
-    q0 = ((w % group) / gsz) * BQ;
+    const WorkItem it = work_item(prm, blockIdx.x + (uint32_t)(n * G));
+    p0 = it.p * BP;
+    q0 = it.q * BQ;
+    bt = it.bt;
   };
 
   // ---- MXFP4 block scales ---------------------------------------------------------------------------------------
