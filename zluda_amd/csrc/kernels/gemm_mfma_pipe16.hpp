@@ -13,8 +13,8 @@
 // What differs from gemm_mfma_pipe.hpp:
 //   * P is the MFMA operand "A": the 16x16 result layout then gives every lane FOUR CONSECUTIVE elements
 //     along D's unit-stride dimension (rows 4*(lane/16) .. +3 of a 16-row tile, column lane%16), so the
-//     epilogue stores 16 bytes (int32 / f32) or 8 bytes (bf16 / f16) per lane straight from the
-//     accumulators: no LDS staging, no lane exchange.
+//     epilogue stores 16 bytes per lane straight from the accumulators (bf16 / f16: the 8 bytes of two tiles, traded
+//     between neighbouring lane groups): no LDS staging.
 //   * A fragment is 16 rows x 128 K bytes: lane l holds row l%16 and the K bytes of lane group l/16 --
 //     fp8: chunks 2*(l/16) and 2*(l/16)+1 of the 128-byte row (one instruction per stage and tile pair);
 //     int8: chunks l/16 and 4 + l/16 (two instructions, K halves).  Both operands use the same assignment,
@@ -55,6 +55,8 @@ __device__ __forceinline__ int lane_here() {
   return l;
 }
 
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+
 // ---- epilogues for the 16x16 accumulator layout ------------------------------------------------------
 // acc[a][b] is the 16 x 16 tile at (P tile a, Q tile b) of the wave tile; lane l holds elements
 // P = 16a + 4*(l/16) + v (v = 0..3), Q = 16b + l%16.
@@ -89,12 +91,14 @@ __device__ __forceinline__ void mfma16_store_raw(__amdgpu_buffer_rsrc_t rs, int 
     }
 }
 
-// float epilogue without a C read: D bf16 / f16 (8-byte stores) or f32 (16-byte stores), at any element's address and any
+// float epilogue without a C read: D bf16, f16 or f32 in 16-byte stores, at any element's address and any
 // pitch (the memory system takes such stores unaligned).  A tile that hangs over the end of P (EDGE) drops the lanes past it
-// and stores the elements of a group of four that straddles the end one by one.
+// and stores the elements of a lane's 16 bytes that straddle the end one by one.
 // DT: 0 bf16, 1 f16, 2 f32, -1 one of the 16-bit types; ACT: the activation, -1 any.  Whole tiles have both fixed at compile
 // time (int8 4096 x 4096 x 1024 -> bf16 + GELU: 31.3 us with run-time branches per 16 x 16 tile, 28.7).  Edge tiles branch: the
 // 64 tiles of a wave are unrolled, and a grid has few of them.
+// (us, 8-byte stores and a branch per factor and element before: bf16 4096 x 4096 x 512 27.0 -> 22.4, with a D pitch of 4100 34.6 -> 23.6;
+// 32000 x 512 x 1024 with pitches of 32004 49.7 -> 40.8 and 32003 53.2 -> 46.2: stores at 2-byte alignment cost more.)
 template <int KIND, int WP, int WQ, int TP, int TQ, int DT, int ACT, bool EDGE, class AccV>
 __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt, int wave) {
   constexpr int WTP = TP * 16, WTQ = TQ * 16;
@@ -110,85 +114,174 @@ __device__ __forceinline__ void mfma16_store_f(const MfmaParams &prm, AccV (&acc
   const bool ragged = EDGE && NP < p0 + wp * WTP + WTP && (NP & 3);  // (uniform) some lane's four straddle the end of P
   const int d_sq = (int)(swp ? g.d_si : g.d_sj);  // < kNarrowPitch (checked by the dispatcher)
   const int pc = p0 + wp * WTP, qc = q0 + wq * WTQ;
+  const int p_left = NP - pc;  // P indices from the wave tile's corner to the end
   const int64_t corner = (int64_t)qc * d_sq + pc;
   char *Dw = (char *)g.D + (g.d_sb * bt + corner) * ESZ;
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dw, 0, tile_window_bytes(d_sq, NP, NQ, corner, ESZ), 0x00020000);
   const int voff = ((lane & 15) * d_sq + 4 * (lane >> 4)) * ESZ;
-  // per-Q factors (one Q index per lane and tile column); columns past the end are dropped by the window
-  float qs[TQ], qb[TQ];
+  // The factors along Q (one index per lane and tile column; columns past the end are dropped by the window) and along P (a
+  // lane's four consecutive indices of each tile).  Whether a factor is a vector is decided once for all of them: decided
+  // where each is used, the kernel is a chain of hundreds of branches around single loads.
+  float qs[TQ], qb[TQ], ps[TP][4];
+  const float *q_v = swp ? ep.alpha_v : ep.sb_v, *p_v = swp ? ep.sb_v : ep.alpha_v;
+  const float q_s = swp ? ep.alpha_s : ep.sb_s, p_s = swp ? ep.sb_s : ep.alpha_s;
+  const int q_lane = qc + (lane & 15), p_lane = pc + 4 * (lane >> 4);
 #pragma unroll
-  for (int b = 0; b < TQ; b++) {
-    const int qi = min(qc + b * 16 + (lane & 15), NQ - 1);
-    qs[b] = swp ? ep.row_scale(qi) : ep.col_scale(qi);
-    qb[b] = swp ? ep.bias_at(qi) : 0.0f;
+  for (int b = 0; b < TQ; b++) { qs[b] = q_s; qb[b] = 0.0f; }
+#pragma unroll
+  for (int a = 0; a < TP; a++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) ps[a][e] = p_s;
+  if (q_v) {
+#pragma unroll
+    for (int b = 0; b < TQ; b++) qs[b] = q_v[min(q_lane + b * 16, NQ - 1)];
   }
-  // per-P bias: the four consecutive rows of a lane are fetched with one load where the vector's type and
-  // alignment allow (raw bits now, all tiles of the wave in one burst; values when they are used)
-  const int bsz = g.bias_type == CUDA_R_32F ? 4 : 2;
-  const bool pbias = !swp && g.bias != nullptr;
-  const char *bias_b = (const char *)g.bias + g.bias_sb * bt * bsz;
-  // (rows start at multiples of 4)
-  const bool wide_bias = pbias && (((uintptr_t)bias_b) & (4 * bsz - 1)) == 0 && !EDGE;
-  v4i braw[TP];
+  if (p_v) {
 #pragma unroll
-  for (int a = 0; a < TP; a++) {
-    const int pi = pc + a * 16 + 4 * (lane >> 4);
-    braw[a] = v4i{0, 0, 0, 0};
-    if (wide_bias) {
-      if (bsz == 4) braw[a] = *(const v4i *)(bias_b + (int64_t)pi * 4);
-      else {
-        const v2i h = *(const v2i *)(bias_b + (int64_t)pi * 2);
-        braw[a] = v4i{h[0] & 0xffff, (int)((uint32_t)h[0] >> 16), h[1] & 0xffff, (int)((uint32_t)h[1] >> 16)};
-      }
-    } else if (pbias) {
+    for (int a = 0; a < TP; a++)
 #pragma unroll
-      for (int e = 0; e < 4; e++) braw[a][e] = (int)ep.bias_raw(EDGE ? min(pi + e, NP - 1) : pi + e);
-    }
+      for (int e = 0; e < 4; e++) ps[a][e] = p_v[EDGE ? min(p_lane + a * 16 + e, NP - 1) : p_lane + a * 16 + e];
   }
+  if (ep.sa_v) {
+    if (swp) {
 #pragma unroll
-  for (int a = 0; a < TP; a++) {
-    float ps[4], pb[4];
+      for (int b = 0; b < TQ; b++) qs[b] *= ep.sa_v[min(q_lane + b * 16, NQ - 1)];
+    } else {
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int pi = EDGE ? min(pc + a * 16 + 4 * (lane >> 4) + e, NP - 1) : pc + a * 16 + 4 * (lane >> 4) + e;
-      ps[e] = swp ? ep.col_scale(pi) : ep.row_scale(pi);
-      pb[e] = pbias ? ep.bias_from_raw((uint32_t)braw[a][e]) : 0.0f;
+      for (int a = 0; a < TP; a++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) ps[a][e] *= ep.sa_v[EDGE ? min(p_lane + a * 16 + e, NP - 1) : p_lane + a * 16 + e];
     }
+  } else if (swp) {
 #pragma unroll
-    for (int b = 0; b < TQ; b++) {
-      float x[4];
+    for (int b = 0; b < TQ; b++) qs[b] *= ep.sa_s;
+  } else {
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const float accf = KIND == KIND_I8 ? (float)to_bits(acc[a][b][e]) : bits2f((uint32_t)to_bits(acc[a][b][e]));
-        x[e] = (swp ? qs[b] * ps[e] : ps[e] * qs[b]) * accf + (swp ? qb[b] : pb[e]);
-      }
-      if (act == ACT_GELU) {
+    for (int a = 0; a < TP; a++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) x[e] = gelu_tanh(x[e]);
-      } else if (act == ACT_RELU) {
+      for (int e = 0; e < 4; e++) ps[a][e] *= ep.sa_s;
+  }
+  if (swp && g.bias) {
+    uint32_t raw[TQ];
 #pragma unroll
-        for (int e = 0; e < 4; e++) x[e] = x[e] > 0.0f ? x[e] : 0.0f;
-      }
+    for (int b = 0; b < TQ; b++) raw[b] = ep.bias_raw(min(q_lane + b * 16, NQ - 1));
 #pragma unroll
-      for (int e = 0; e < 4; e++) x[e] *= ep.sd;
-      const int soff = (b * 16 * d_sq + a * 16) * ESZ;  // uniform
-      const int left = NP - (pc + a * 16 + 4 * (lane >> 4));
-      if constexpr (WIDE) {
-        const v4i pk = {(int)f2bits(x[0]), (int)f2bits(x[1]), (int)f2bits(x[2]), (int)f2bits(x[3])};
-        buffer_store_b128_guarded(pk, rs, EDGE ? store4_offset(left, voff) : voff, soff);
-        if (ragged) {
+    for (int b = 0; b < TQ; b++) qb[b] = ep.bias_from_raw(raw[b]);
+  }
+  // the bias, along P (a row-major D: along Q): raw bits of all tiles in one burst, then their values
+  float pb[TP][4];
 #pragma unroll
-          for (int e = 0; e < 3; e++) __builtin_amdgcn_raw_buffer_store_b32(pk[e], rs, store1_offset(left, e, voff, 4), soff, 0);
+  for (int a = 0; a < TP; a++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) pb[a][e] = 0.0f;
+  if (g.bias && !swp) {
+    uint32_t raw[TP][4];
+    if (g.bias_type == CUDA_R_32F) {
+      const uint32_t *v = (const uint32_t *)g.bias + g.bias_sb * bt;
+#pragma unroll
+      for (int a = 0; a < TP; a++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) pb[a][e] = bits2f(v[EDGE ? min(p_lane + a * 16 + e, NP - 1) : p_lane + a * 16 + e]);
+    } else {
+      const uint16_t *v = (const uint16_t *)g.bias + g.bias_sb * bt;
+      if (!EDGE && (((uintptr_t)v) & 7) == 0) {  // (rows start at multiples of 4)
+        v2i t[TP];
+#pragma unroll
+        for (int a = 0; a < TP; a++) t[a] = *(const v2i *)(v + p_lane + a * 16);
+#pragma unroll
+        for (int a = 0; a < TP; a++) {
+          raw[a][0] = (uint32_t)t[a][0] & 0xffffu; raw[a][1] = (uint32_t)t[a][0] >> 16;
+          raw[a][2] = (uint32_t)t[a][1] & 0xffffu; raw[a][3] = (uint32_t)t[a][1] >> 16;
         }
       } else {
-        v2i pk;
-        if (to_bf16) { pk[0] = (int)pack_bf16x2(x[0], x[1]); pk[1] = (int)pack_bf16x2(x[2], x[3]); }
-        else { pk[0] = (int)pack_f16x2(x[0], x[1]); pk[1] = (int)pack_f16x2(x[2], x[3]); }
-        buffer_store_b64_guarded(pk, rs, EDGE ? store4_offset(left, voff) : voff, soff);
-        if (ragged) {
-          __builtin_amdgcn_raw_buffer_store_b16((short)pk[0], rs, store1_offset(left, 0, voff, 2), soff, 0);
-          __builtin_amdgcn_raw_buffer_store_b16((short)(pk[0] >> 16), rs, store1_offset(left, 1, voff, 2), soff, 0);
-          __builtin_amdgcn_raw_buffer_store_b16((short)pk[1], rs, store1_offset(left, 2, voff, 2), soff, 0);
+#pragma unroll
+        for (int a = 0; a < TP; a++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) raw[a][e] = v[EDGE ? min(p_lane + a * 16 + e, NP - 1) : p_lane + a * 16 + e];
+      }
+      if (g.bias_type == CUDA_R_16BF) {
+#pragma unroll
+        for (int a = 0; a < TP; a++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) pb[a][e] = dec_bf16((uint16_t)raw[a][e]);
+      } else {
+#pragma unroll
+        for (int a = 0; a < TP; a++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) pb[a][e] = dec_f16((uint16_t)raw[a][e]);
+      }
+    }
+  }
+  // Two tiles along P at a time: the 16-bit results of a lane's four rows are 8 bytes of either, and the lane groups g and g ^ 1
+  // trade halves (v_permlane16_swap), after which a lane of an even group holds rows 4g .. 4g + 7 of the first tile and a lane
+  // of an odd one rows 4(g-1) .. 4(g-1) + 7 of the second: 16 bytes a lane, 64 contiguous bytes of each of 16 columns.
+  static_assert(TP % 2 == 0, "tiles along P are stored in pairs");
+  const int grp = lane >> 4, first = (grp & 1) ? 4 * grp + 12 : 4 * grp;  // the lane's first P index inside a pair
+  const int voff_pair = ((lane & 15) * d_sq + first) * 2;
+#pragma unroll
+  for (int a = 0; a < TP; a += 2) {
+#pragma unroll
+    for (int b = 0; b < TQ; b++) {
+      float x[2][4];
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float accf = KIND == KIND_I8 ? (float)to_bits(acc[a + h][b][e]) : bits2f((uint32_t)to_bits(acc[a + h][b][e]));
+          x[h][e] = ps[a + h][e] * qs[b] * accf + (swp ? qb[b] : pb[a + h][e]);
+        }
+      if (act == ACT_GELU) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) x[h][e] = gelu_tanh(x[h][e]);
+      } else if (act == ACT_RELU) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) x[h][e] = x[h][e] > 0.0f ? x[h][e] : 0.0f;
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[h][e] *= ep.sd;
+      const int soff = (b * 16 * d_sq + a * 16) * ESZ;  // uniform
+      if constexpr (WIDE) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const int left = NP - (pc + (a + h) * 16 + 4 * (lane >> 4));
+          const v4i pk = {(int)f2bits(x[h][0]), (int)f2bits(x[h][1]), (int)f2bits(x[h][2]), (int)f2bits(x[h][3])};
+          buffer_store_b128_guarded(pk, rs, EDGE ? store4_offset(left, voff) : voff, soff + h * 16 * ESZ);
+          if (ragged) {
+#pragma unroll
+            for (int e = 0; e < 3; e++) __builtin_amdgcn_raw_buffer_store_b32(pk[e], rs, store1_offset(left, e, voff, 4), soff + h * 16 * ESZ, 0);
+          }
+        }
+      } else {
+        uint32_t lo[2], hi[2];  // the first and the second tile
+        if (to_bf16) {
+          lo[0] = pack_bf16x2(x[0][0], x[0][1]); lo[1] = pack_bf16x2(x[0][2], x[0][3]);
+          hi[0] = pack_bf16x2(x[1][0], x[1][1]); hi[1] = pack_bf16x2(x[1][2], x[1][3]);
+        } else {
+          lo[0] = pack_f16x2(x[0][0], x[0][1]); lo[1] = pack_f16x2(x[0][2], x[0][3]);
+          hi[0] = pack_f16x2(x[1][0], x[1][1]); hi[1] = pack_f16x2(x[1][2], x[1][3]);
+        }
+        v4i pk = {(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
+#if defined(__HIP_DEVICE_COMPILE__)
+        const v2u s0 = __builtin_amdgcn_permlane16_swap(lo[0], hi[0], false, false);
+        const v2u s1 = __builtin_amdgcn_permlane16_swap(lo[1], hi[1], false, false);
+        pk = v4i{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
+#endif
+        if constexpr (!EDGE) {
+          buffer_store_b128_guarded(pk, rs, voff_pair, soff);
+        } else {
+          const int left = NP - (pc + a * 16 + first);
+          buffer_store_b128_guarded(pk, rs, left >= 8 ? voff_pair : kStoreNowhere, soff);
+          if (p_left > a * 16 && p_left < a * 16 + 32 && (p_left & 7)) {  // (uniform) some lane's eight straddle the end
+#pragma unroll
+            for (int e = 0; e < 7; e++)
+              __builtin_amdgcn_raw_buffer_store_b16((short)(pk[e >> 1] >> (16 * (e & 1))), rs, left < 8 && e < left ? voff_pair + e * 2 : kStoreNowhere, soff, 0);
+          }
         }
       }
     }
@@ -247,9 +340,9 @@ __device__ __forceinline__ void mfma16_store_general(const MfmaParams &prm, AccV
   }
 }
 
-template <int KIND, int WP, int WQ, int TP, int TQ, int LDS_BYTES, class AccV>
-__device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&acc)[TP][TQ], int *lds_words, int p0, int q0, int NP,
-                                                  int NQ, int bt, int wave) {
+// The epilogues that store straight from the accumulators; false: this problem needs the general one
+template <int KIND, int WP, int WQ, int TP, int TQ, class AccV>
+__device__ __forceinline__ bool mfma16_store_direct(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt, int wave) {
   constexpr int WTP = TP * 16, WTQ = TQ * 16;
   const GemmArgs &g = prm.g;
   const bool swp = prm.swapped != 0;
@@ -265,7 +358,7 @@ __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dw, 0, tile_window_bytes(d_sq, NP, NQ, corner, 4), 0x00020000);
       if (whole) mfma16_store_raw<false>(rs, (int)d_sq, acc, ialpha, 0);
       else mfma16_store_raw<true>(rs, (int)d_sq, acc, ialpha, NP - pc);
-      return;
+      return true;
     }
   }
   const MfmaParams &late = args_again(prm);
@@ -288,10 +381,17 @@ __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&
     }
 #undef ZLUDA_EPI16_ACT
 #undef ZLUDA_EPI16
-    return;
+    return true;
   }
+  return false;
+}
+
+template <int KIND, int WP, int WQ, int TP, int TQ, int LDS_BYTES, class AccV>
+__device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&acc)[TP][TQ], int *lds_words, int p0, int q0, int NP,
+                                                  int NQ, int bt, int wave) {
+  if (mfma16_store_direct<KIND, WP, WQ, TP, TQ>(prm, acc, p0, q0, NP, NQ, bt, wave)) return;
   __syncthreads();  // (workgroup-uniform branch) the LDS tiles become staging
-  mfma16_store_general<KIND, WP, WQ, TP, TQ, LDS_BYTES>(late, acc, lds_words, p0, q0, NP, NQ, bt, wave);
+  mfma16_store_general<KIND, WP, WQ, TP, TQ, LDS_BYTES>(args_again(prm), acc, lds_words, p0, q0, NP, NQ, bt, wave);
 }
 
 // ---- the kernel ----------------------------------------------------------------------------------------

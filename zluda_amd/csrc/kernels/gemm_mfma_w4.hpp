@@ -51,8 +51,6 @@ __device__ __forceinline__ bool w4_stream_d_i32(const GemmArgs &g) {
 enum { W4_EPI_I32 = 0, W4_EPI_BF16 = 1, W4_EPI_BF16_GELU = 2 };
 
 // one accumulator element, AGPR -> VGPR
-typedef unsigned v2u __attribute__((ext_vector_type(2)));
-
 template <class T>
 __device__ __forceinline__ int w4_acc_read(const T &elem) {
   int raw = 0;
