@@ -32,6 +32,20 @@ namespace {
 
 inline int f8_fmt(uint32_t t) { return t == CUDA_R_8F_E5M2 ? 1 : 0; }
 
+uint32_t launch_splitk_reduce(const SplitKReduceParams &rp, int np, int nq, hipStream_t s) {
+  const dim3 grid((np + 1023) / 1024, nq, rp.g.batch), block(256);
+  switch (rp.splits) {  // (the planner's shares are 2 .. 8)
+  case 2: return launch_kernel(splitk_reduce_kernel<2>, grid, block, s, rp);
+  case 3: return launch_kernel(splitk_reduce_kernel<3>, grid, block, s, rp);
+  case 4: return launch_kernel(splitk_reduce_kernel<4>, grid, block, s, rp);
+  case 5: return launch_kernel(splitk_reduce_kernel<5>, grid, block, s, rp);
+  case 6: return launch_kernel(splitk_reduce_kernel<6>, grid, block, s, rp);
+  case 7: return launch_kernel(splitk_reduce_kernel<7>, grid, block, s, rp);
+  case 8: return launch_kernel(splitk_reduce_kernel<8>, grid, block, s, rp);
+  default: return launch_kernel(splitk_reduce_kernel<0>, grid, block, s, rp);
+  }
+}
+
 // `ws` / `ws_size`: the scratch that holds split-K partial tiles (the caller's workspace, or the library's own)
 uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws, uint64_t ws_size, hipStream_t s) {
   MfmaParams prm;
@@ -111,7 +125,7 @@ uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws,
   rp.ws_np = prm.tiles_p * v.bp;
   rp.ws_nq = prm.tiles_q * v.bq;
   rp.ws = (const int32_t *)ws;
-  return launch_kernel(splitk_reduce_kernel, dim3((np + 1023) / 1024, nq, l.g.batch), dim3(256), s, rp);
+  return launch_splitk_reduce(rp, np, nq, s);
 }
 
 uint32_t launch_tr(const Lowered &l, const zluda_gemm_plan &plan, void *ws, uint64_t ws_size, hipStream_t s) {
@@ -164,7 +178,7 @@ uint32_t launch_tr(const Lowered &l, const zluda_gemm_plan &plan, void *ws, uint
   rp.ws_np = prm.tiles_p * v.bp;
   rp.ws_nq = prm.tiles_q * v.bq;
   rp.ws = (const int32_t *)ws;
-  return launch_kernel(splitk_reduce_kernel, dim3((np + 1023) / 1024, nq, l.g.batch), dim3(256), s, rp);
+  return launch_splitk_reduce(rp, np, nq, s);
 }
 
 template <int NW, int STEPS>
