@@ -1,0 +1,40 @@
+"""Many tiles of a short K (at most 128 elements of f16 / bf16): workgroups that walk the tiles with both operands of a tile in LDS
+at once.  Ends of K inside and between its two chunks; ends of both extents inside a tile, in runs of one to a few tiles per
+workgroup that turn over within a run; every output type; a row-major D; and what runs on other kernels all the same: a beta that
+is not zero, columns of D at odd 16-bit addresses."""
+import pytest
+
+from oracle.cases import Case
+from zluda_amd import abi as K
+
+pytestmark = pytest.mark.gpu
+
+
+def run(gpu_api, m, n, k, batch, t=K.CUDA_R_16BF, d=None, **more):
+    s = dict(a_type=t, b_type=t, d_type=d if d is not None else t, c_type=d if d is not None else t, compute_type=K.CUBLAS_COMPUTE_32F,
+             scale_type=K.CUDA_R_32F, m=m, n=n, k=k, transa=1, batch=batch)
+    s.update(more)
+    print("case", s, flush=True)
+    case = Case(s, 7700 + m + k)
+    st, got, kernel, variant = case.run_gpu(gpu_api)
+    assert st == 0 and kernel == K.ZLUDA_KERNEL_MFMA_H16
+    case.compare(got, case.run_oracle(), tol=1e-2)   # one rounding to 16 bits of sums in another order
+
+
+@pytest.mark.parametrize("m,n,k,batch", [(130, 130, 8, 130), (128, 256, 64, 260), (300, 70, 72, 175), (66, 65, 128, 520), (256, 384, 120, 90), (1026, 200, 104, 40)])
+def test_edges(gpu_api, m, n, k, batch):
+    run(gpu_api, m, n, k, batch)
+
+
+@pytest.mark.parametrize("t,d", [(K.CUDA_R_16F, K.CUDA_R_16F), (K.CUDA_R_16BF, K.CUDA_R_32F), (K.CUDA_R_16F, K.CUDA_R_32F), (K.CUDA_R_16BF, K.CUDA_R_16F)])
+def test_output_types(gpu_api, t, d):
+    run(gpu_api, 202, 130, 96, 133, t, d, alpha=0.125)
+    run(gpu_api, 131, 129, 64, 133, t, K.CUDA_R_32F, ldd=133)
+
+
+def test_row_major_scales_and_other_roads(gpu_api):
+    run(gpu_api, 130, 202, 96, 133, order_c=1, order_d=1, ldc=208, ldd=208)
+    run(gpu_api, 130, 130, 80, 133, with_scalar_scales=True, scale_range=(0.5, 1.5))
+    run(gpu_api, 130, 130, 80, 133, with_c=True, beta=0.5)       # a tile per workgroup
+    run(gpu_api, 131, 130, 80, 133, ldd=131)
+    run(gpu_api, 130, 130, 80, 133, epilogue=K.CUBLASLT_EPILOGUE_GELU_BIAS)

@@ -55,6 +55,8 @@ uint32_t launch_mfma_f8(const MfmaParams &prm, const zluda_gemm_plan &plan, int 
 uint32_t launch_mfma_mxf4(const MfmaParams &prm, const zluda_gemm_plan &plan, hipStream_t s);
 uint32_t launch_mfma_h16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool bf16, hipStream_t s);
 uint32_t launch_mfma_f32(const MfmaParams &prm, const zluda_gemm_plan &plan, hipStream_t s);
+// variant 3 in the form of kernels/gemm_mfma_short.hpp; `grid` workgroups, prm.split_stages the same number
+uint32_t launch_mfma_short(const MfmaParams &prm, bool bf16, uint32_t grid, hipStream_t s);
 // the four-wave persistent kernel (variant 11; kernels/gemm_mfma_w4.hpp), `epi` = W4_CLASS_* of planner.hpp, `grid` workgroups
 uint32_t launch_mfma_w4_i8(const MfmaParams &prm, int epi, uint32_t grid, hipStream_t s);
 uint32_t launch_mfma_w4_i8f(const MfmaParams &prm, int epi, uint32_t grid, hipStream_t s);

@@ -401,6 +401,21 @@ int w4_epilogue_class(const Lowered &l, bool dry) {
   return W4_CLASS_NONE;
 }
 
+// All of K in LDS at once and more tiles than the two workgroups of every CU take in one go: those walk the tiles.  (Columns of
+// D at odd 16-bit addresses are left to the tile kernels, whose narrower stores mind them less: bf16 2459 x 351 x 80, 21
+// batches 23.3 us here, 19.4 there; with a pitch of 2462 or 2464 16 here and 18.5 there.)
+bool mfma_short_k(const Lowered &l, bool dry, uint32_t cus) {
+  const GemmArgs &g = l.g;
+  if ((g.a_type != CUDA_R_16F && g.a_type != CUDA_R_16BF) || g.K > 128 || std::min(g.M, g.N) <= 64) return false;
+  if (g.beta_mode != SCALAR_VALUE || (!dry && g.beta_val.f != 0.0f) || (g.d_si != 1 ? g.d_si : g.d_sj) >= kNarrowPitch) return false;
+  if (g.d_type != CUDA_R_16F && g.d_type != CUDA_R_16BF && g.d_type != CUDA_R_32F) return false;
+  const int64_t d_sq = g.d_si != 1 ? g.d_si : g.d_sj;
+  if (g.d_type != CUDA_R_32F && ((d_sq & 1) || (g.batch > 1 && (g.d_sb & 1)) || (!dry && (((uintptr_t)g.D) & 3)))) return false;
+  // (its epilogue has one factor for all of D)
+  if (g.act != ACT_NONE || l.has_bias || g.alpha_mode == VECTOR_DEV || g.a_scale_mode == SCALE_OUTER_VEC || g.b_scale_mode == SCALE_OUTER_VEC) return false;
+  return (uint64_t)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch > 2 * (uint64_t)cus;
+}
+
 static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t workspace_size,
                            zluda_gemm_plan *plan) {
   const GemmArgs &g = l.g;
@@ -420,6 +435,13 @@ static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t
     plan->grid_x = (uint32_t)std::min<uint64_t>(all, slots);
     plan->grid_y = 1;
     plan->waves = (float)all / (float)cus;
+    plan->workspace = 0;
+    return;
+  }
+  if (variant == 3 && mfma_short_k(l, true, cus)) {
+    plan->waves = (float)((double)plan->grid_x * plan->grid_y / (2.0 * cus));
+    plan->grid_x = std::max(2 * cus / 8 * 8, 8u);
+    plan->grid_y = 1;
     plan->workspace = 0;
     return;
   }
@@ -467,6 +489,7 @@ static const float kMfmaVariantEfficiency[kNumMfmaVariants] = {1.00f, 0.95f, 0.8
 
 static int pick_mfma_variant(const Lowered &l, uint32_t cus) {
   const GemmArgs &g = l.g;
+  if (mfma_short_k(l, true, cus)) return 3;
   const bool swapped = g.d_si != 1;
   const uint32_t np = swapped ? g.N : g.M, nq = swapped ? g.M : g.N;
   // cost = rounds of workgroups over the CUs x time of one tile; the tile shapes trade efficiency

@@ -14,7 +14,7 @@ constexpr MfmaVariant kMfmaVariants[] = {
     {256, 256, 2, 4, 128, 2, 0, 0},  // 0: 8 waves, 128x64 per wave
     {256, 256, 2, 2, 128, 2, 0, 0},  // 1: 4 waves, 128x128 per wave
     {256, 128, 2, 2, 128, 2, 0, 0},  // 2: 4 waves, 128x64 per wave
-    {128, 128, 2, 2, 128, 2, 0, 0},  // 3: 4 waves, 64x64 per wave, two workgroups per CU
+    {128, 128, 2, 2, 128, 2, 0, 0},  // 3: 4 waves, 64x64 per wave, two workgroups per CU; many tiles of a short K: mfma_short_k()
     {128, 128, 2, 2, 64, 4, 0, 0},   // 4: same tile, half-line stages, deeper ring (short K)
     {128, 64, 2, 2, 128, 3, 0, 0},   // 5: 4 waves, 64x32 per wave: skinny problems
     {64, 64, 2, 2, 128, 3, 0, 0},    // 6: 4 waves, 32x32 per wave: problems of a few hundred tiles at most
@@ -107,6 +107,9 @@ uint32_t lower_problem(const zluda_gemm_problem *p, bool dry, Lowered *out);
 // the fast epilogue of the four-wave kernel that serves the problem, or W4_CLASS_NONE; `dry`: planning (beta and the
 // pointers are not known yet and are taken to be zero / aligned)
 int w4_epilogue_class(const Lowered &l, bool dry);
+
+// whether a 16-bit problem runs on the short-K form of variant 3 (kernels/gemm_mfma_short.hpp); `dry` as above
+bool mfma_short_k(const Lowered &l, bool dry, uint32_t cus);
 
 // The generic family's fast road: problems that only alignment or a K-contiguous row that ends inside a 16-byte piece keeps
 // from every MFMA family run on the transposing kernel (plan.variant = 1 + its variant, with its grid).  The family whose
