@@ -58,6 +58,13 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
   constexpr int TP = WTP / 32, TQ = WTQ / 32;
   constexpr int KS = BKB_ / (KIND == KIND_F8 ? 64 : 32);  // MFMA sub-steps per stage
   constexpr int SPT = (KS & 1) ? 2 : 1;        // stages per loop trip (fragment roles must realign)
+  // Wave tiles of up to 64 x 64 fetch the fragments of a whole stage ahead (twice 64 registers): a sub-step of theirs is 1 to 4
+  // MFMAs, shorter than an LDS read takes.  Larger ones have no registers for it and fetch one sub-step ahead.  Time of a stage
+  // on a chip that is not full (int8, one workgroup per CU, us), one sub-step ahead and a whole stage: 64x64 tile
+  // 0.28 -> 0.19, 128x64 0.34 -> 0.27, 128x128 0.43 -> 0.35, 256x128 on eight waves 0.67 -> 0.53 (128 KiB of LDS traffic
+  // and 48 KiB of DMA, which bound it now).  On rings of two stages it gains nothing: they wait for memory.
+  // (Nor on the 64x64 tile of MXFP4, which runs the skinny problems that wait for memory too: 10240 x 64 x 8192 16.0 -> 17.3.)
+  constexpr bool AHEAD = WTP * WTQ <= 64 * 64 && NSTAGE > 2 && !(MX && WTP * WTQ <= 32 * 32);
   constexpr int STAGE_V4 = (BP + BQ) * CPR;    // one stage in 16-byte units: P rows, then Q rows
   static_assert(BKB_ == 64 || BKB_ == 128, "row segments are half or whole cache lines");
   static_assert(BP % RPP == 0 && BQ % RPP == 0 && RPP % 32 == 0, "tile / copy-pass mismatch");
@@ -294,8 +301,51 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
   }
   wait_vmcnt_barrier<PC.wait_prologue>();
 
-  Frags fa, fb;
   Scales sc_cur, sc_nxt;
+  int so = 0, kt = 0;
+  if constexpr (AHEAD) {
+  // All fragments of a stage are fetched while the one before it is multiplied: on entry those of stage kt are in fr[CUR] or on
+  // their way there.  Wait for them and for stage kt+1, barrier; the slot of stage kt is free then (refilled with stage
+  // kt+NSTAGE), the fragments of stage kt+1 arrive behind the first MFMAs of stage kt.
+  Frags fr[2][KS];
+  static_for<KS>([&](auto s_c) { load_frags(0, s_c, fr[0][decltype(s_c)::value]); });
+  load_scales(0, sc_nxt);
+  auto do_stage = [&](auto cur_c) {
+    constexpr int CUR = decltype(cur_c)::value;
+    const int so_next = so == (NSTAGE - 1) * STAGE_V4 ? 0 : so + STAGE_V4;
+    wait_vmcnt_barrier<PC.wait_stage>();
+    if constexpr (MX) sc_cur = sc_nxt;
+    // (reads in front of the DMA, as below)
+    static_for<KS>([&](auto s_c) { load_frags(so_next, s_c, fr[1 - CUR][decltype(s_c)::value]); });
+    load_scales(kt + 1, sc_nxt);  // (their chunk landed at least one barrier ago, see below)
+    issue_scales_for(kt, so);
+    issue_stage(kt + NSTAGE, so);
+    static_for<KS>([&](auto s_c) { mfma_all(fr[CUR][decltype(s_c)::value], sc_cur, s_c); });
+    // the reads behind the first five eighths of the MFMAs, the DMA behind the rest
+    constexpr int NM = TP * TQ * MPS * KS, NDS = (TP + TQ) * KS * (KIND == KIND_F8 ? 2 : 1) + (MX ? TP + TQ : 0);
+    constexpr int H1 = NM * 5 / 8 > 0 ? NM * 5 / 8 : 1, H2 = NM - H1 > 0 ? NM - H1 : 1;
+    static_for<NM>([&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+      if constexpr (i < H1) {
+        constexpr int n = NDS * (i + 1) / H1 - NDS * i / H1;
+        if constexpr (n > 0) __builtin_amdgcn_sched_group_barrier(0x100, n, 0);  // DS reads
+      } else {
+        constexpr int j = i - H1, n = NLOAD * (j + 1) / H2 - NLOAD * j / H2;
+        if constexpr (n > 0) __builtin_amdgcn_sched_group_barrier(0x010, n, 0);  // VMEM (LDS DMA)
+      }
+    });
+    __builtin_amdgcn_sched_barrier(0);
+    so = so_next;
+    kt++;
+  };
+  while (kt + 2 <= KT) {
+    do_stage(std::integral_constant<int, 0>{});
+    do_stage(std::integral_constant<int, 1>{});
+  }
+  if (kt < KT) do_stage(std::integral_constant<int, 0>{});
+  } else {
+  Frags fa, fb;
   load_frags(0, std::integral_constant<int, 0>{}, fa);
   load_scales(0, sc_nxt);
 
@@ -352,8 +402,6 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
 
   // K loop: SPT stages per trip, no other control flow; with two stages per trip (the fragment
   // roles realign every other stage) an odd last stage follows on its own
-  int so = 0;
-  int kt = 0;
   for (; kt + SPT <= KT; kt += SPT) {
     do_stage(kt, so, fa, fb);
     so = so == (NSTAGE - 1) * STAGE_V4 ? 0 : so + STAGE_V4;
@@ -364,6 +412,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
   }
   if constexpr (SPT == 2) {
     if (kt < KT) do_stage(kt, so, fa, fb);
+  }
   }
 
   // every wave is done with the LDS tiles (and every DMA has landed) before they become staging

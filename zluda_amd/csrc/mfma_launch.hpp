@@ -21,11 +21,16 @@ inline uint32_t launch_mfma_variant(const MfmaParams &prm, const zluda_gemm_plan
     return launch_kernel(gemm_mfma_pipe_kernel<KIND, FQ, FP, BP, BQ, WP, WQ, BKB, NS>, grid,               \
                          dim3(WP * WQ * 64), s, prm);
   switch (plan.variant) {
+  case 2:  // (two forms of one tile, see mfma_eight_waves())
+    static_assert(kMfmaVariants[2].bp == 256 && kMfmaVariants[2].bq == 128 && kMfmaVariants[2].wp == 2 && kMfmaVariants[2].wq == 2 &&
+                  kMfmaVariants[2].bkb == 128 && kMfmaVariants[2].stages == 2 && !kMfmaVariants[2].m16, "variant table mismatch");
+    if (plan.block != 512) return launch_kernel(gemm_mfma_pipe_kernel<KIND, FQ, FP, 256, 128, 2, 2, 128, 2>, grid, dim3(256), s, prm);
+    if constexpr (KIND == KIND_MXF4) return CUBLAS_STATUS_INVALID_VALUE;
+    else return launch_kernel(gemm_mfma_pipe_kernel<KIND, FQ, FP, 256, 128, 4, 2, 128, 3>, grid, dim3(512), s, prm);
     ZLUDA_MFMA_CASE(0, 256, 256, 2, 4, 128, 2)
     ZLUDA_MFMA_CASE(1, 256, 256, 2, 2, 128, 2)
-    ZLUDA_MFMA_CASE(2, 256, 128, 2, 2, 128, 2)
     ZLUDA_MFMA_CASE(3, 128, 128, 2, 2, 128, 2)
-    ZLUDA_MFMA_CASE(4, 128, 128, 2, 2, 64, 4)
+    ZLUDA_MFMA_CASE(4, 128, 128, 2, 2, 128, 3)
     ZLUDA_MFMA_CASE(5, 128, 64, 2, 2, 128, 3)
     ZLUDA_MFMA_CASE(6, 64, 64, 2, 2, 128, 3)
     ZLUDA_MFMA_CASE(7, 192, 256, 2, 4, 128, 2)

@@ -416,6 +416,17 @@ bool mfma_short_k(const Lowered &l, bool dry, uint32_t cus) {
   return (uint64_t)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch > 2 * (uint64_t)cus;
 }
 
+// The 256 x 128 tile has a second form on eight waves with three stages, faster on grids of less than two rounds (int8, us:
+// 6144 x 777 x 4096 39.6 -> 30.6, 4096 x 2048 x 4096 42 -> 38, 28672 x 777 x 4096, three rounds, 163 -> 131, where the larger
+// tiles take 105).  Results of 4 bytes on a grid that fills the chip need a longer K for it: int8 -> int32 5372 x 1428 x 1536 20.9 us on
+// four waves, 24.3 on eight, x 4096 43 and 37; 2048 x 2048 x 1024 13.7 and 12.3.  MXFP4 has no room in LDS for the third stage beside
+// its scale chunks.
+static bool mfma_eight_waves(const Lowered &l, uint64_t tiles, uint32_t cus) {
+  if (l.g.a_type == CUDA_R_4F_E2M1 || tiles >= 2 * (uint64_t)cus) return false;
+  const bool wide_d = l.g.d_type == CUDA_R_32I || l.g.d_type == CUDA_R_32F;
+  return !wide_d || tiles * 4 <= 3 * (uint64_t)cus || (int64_t)l.g.K * type_bits(l.g.a_type) / 8 > 2048;
+}
+
 static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t workspace_size,
                            zluda_gemm_plan *plan) {
   const GemmArgs &g = l.g;
@@ -445,8 +456,10 @@ static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t
     plan->workspace = 0;
     return;
   }
+  const bool eight = variant == 2 && mfma_eight_waves(l, (uint64_t)tp * tq * g.batch, cus);
+  if (eight) plan->block = 512;
   // data stages, plus two chunks of 32 scale bytes per tile row for MXFP4
-  const uint32_t lds = (uint32_t)v.stages * (v.bp + v.bq) * v.bkb + (l.g.a_type == CUDA_R_4F_E2M1 ? 64u * (v.bp + v.bq) : 0u);
+  const uint32_t lds = (uint32_t)(eight ? 3 : v.stages) * (v.bp + v.bq) * v.bkb + (l.g.a_type == CUDA_R_4F_E2M1 ? 64u * (v.bp + v.bq) : 0u);
   const uint32_t per_cu = std::max(1u, std::min(160u * 1024u / lds, 2048u / plan->block));
   plan->waves = (float)plan->grid_x * plan->grid_y / (float)(cus * per_cu);
   plan->workspace = 0;
@@ -476,16 +489,22 @@ static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t
   }
 }
 
-// Relative throughput of one CU running tiles of each variant (measured on MI355X, int8 and fp8, K >= 1024;
-// variant 0 = 1).  Smaller tiles read more LDS and L2 bytes per MFMA.
-// The variants on the 16x16 MFMA shapes (8, 9) need less energy per multiply-add, which is what bounds a GEMM
-// that keeps the whole chip busy (the board sits at its power cap): at 4096^3 and 8192^3 they take 8-10 % less
-// time than their 32x32 counterparts for int8 and 1-3 % less for fp8.  On a chip that is partly idle the clock
-// is the bound instead and they lose (their epilogue is ~3 us per tile slower: 2048^3 int8 30.5 us against
-// 27.5), so they are only chosen for grids that fill the chip; the same tiles at 256x128 and 128x128 measured
-// no better than the 32x32 ones anywhere and are not instantiated.
-static const float kMfmaVariantEfficiency[kNumMfmaVariants] = {1.00f, 0.95f, 0.80f, 0.70f, 0.72f, 0.55f, 0.40f, 0.85f,
-                                                               1.05f, 0.89f, 0.40f, 1.10f};
+// Relative throughput of one CU inside the K loop on tiles of each variant (variant 0 = 1) and what a tile costs around its
+// loop, in stages of 128 bytes of K.  Fitted to the times of 460 int8, fp8 and bf16 and 150 MXFP4 problems on every variant
+// (MI355X; linear layers of 48 to 3000 tokens and 256 .. 8192 rows and columns, K = 128 .. 14592): what they pick takes 1.8 %
+// (MXFP4 1.0 %) more time than the best variant of each problem on average.
+// The variants on the 16x16 MFMA shapes (8, 9) need less energy per multiply-add, which is what bounds a GEMM that keeps the
+// whole chip busy (the board sits at its power cap); on a chip that is partly idle the clock is the bound instead, so they are
+// only chosen for grids that fill the chip; the same tiles at 256x128 and 128x128 measured no better than the 32x32 ones
+// anywhere and are not instantiated.
+struct MfmaTileCost { float efficiency, around; };
+static const MfmaTileCost kMfmaTileCost[kNumMfmaVariants] = {{1.00f, 5.8f}, {0.95f, 6.0f}, {0.82f, 7.6f}, {0.62f, 5.9f}, {0.76f, 9.0f}, {0.43f, 4.4f},
+                                                             {0.41f, 3.4f}, {0.89f, 6.3f}, {1.05f, 5.1f}, {0.89f, 4.6f}, {0.41f, 3.4f}, {1.06f, 5.3f}};
+static const MfmaTileCost kMxTileCost[kNumMfmaVariants] = {{1.00f, 6.0f}, {0.95f, 6.0f}, {0.80f, 9.0f}, {0.70f, 3.3f}, {0.84f, 9.0f}, {0.55f, 3.3f},
+                                                           {0.40f, 2.4f}, {0.92f, 5.3f}, {1.05f, 6.0f}, {0.89f, 6.0f}, {0.40f, 2.4f}, {1.10f, 6.0f}};
+// A last round that fills a part x of the CUs takes this + (1 - this) * x of a full one's time: the clock is higher and memory
+// less busy then.
+constexpr double kPartialRound = 0.65;
 
 static int pick_mfma_variant(const Lowered &l, uint32_t cus) {
   const GemmArgs &g = l.g;
@@ -493,7 +512,7 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus) {
   const bool swapped = g.d_si != 1;
   const uint32_t np = swapped ? g.N : g.M, nq = swapped ? g.M : g.N;
   // cost = rounds of workgroups over the CUs x time of one tile; the tile shapes trade efficiency
-  // per CU against how evenly the problem fills the chip
+  // per CU against how evenly the problem fills the chip and what a tile costs around its K loop
   int best = 0;
   double best_cost = 0;
   for (int v = 0; v < kNumMfmaVariants; v++) {
@@ -501,11 +520,12 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus) {
     const uint64_t tiles = (uint64_t)ceil_div(np, t.bp) * ceil_div(nq, t.bq) * g.batch;
     if (t.stages > 4) continue;  // the deep ring: see below
     if (t.w4) {
-      // The four-wave kernel, for the problems its epilogues serve: level with the best other variant from one round of
-      // tiles on, 4-7 % ahead from four (8192^3: int8 410 us against 429, fp8 360 against 389; 8192 x 4096 x 4096 fp8
-      // 103 against 109; 4096^3 int8 59.4 against 59.5), but not on a short K, where the per-tile work around the loop
-      // shows (16384 x 8192 x 1024 fp8: 167 us against 153 for variant 0)
-      if (w4_epilogue_class(l, true) == W4_CLASS_NONE || g.K < 2048) continue;
+      // The four-wave kernel, for the problems its epilogues serve, but not on a short K, where the per-tile work around the loop
+      // shows: fp8 and int32 outputs from K = 2048 on (16384 x 8192 x 1024 fp8: 167 us against 153 for variant 0), int8 with
+      // float outputs, f16 and bf16 from 1024 on (int8 7904 x 6288 x 1792 131 -> 99 us, bf16 5200 x 5712 x 1024 70 -> 62)
+      const int epi = w4_epilogue_class(l, true);
+      const bool f8 = is_f8(g.a_type);
+      if (epi == W4_CLASS_NONE || g.K < (f8 || epi == W4_CLASS_I32 ? 2048 : 1024)) continue;
       if (tiles < (g.a_type == CUDA_R_8I ? ((uint64_t)cus * 3 + 3) / 4 : (uint64_t)cus)) continue;
     } else if (t.m16) {
       const bool h16 = g.a_type == CUDA_R_16F || g.a_type == CUDA_R_16BF;
@@ -517,8 +537,11 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus) {
       const uint64_t need = (g.a_type == CUDA_R_8I || h16) ? ((uint64_t)cus * 3 + 3) / 4 : (uint64_t)cus * (t.bp == 256 ? 4 : 2);
       if (tiles < need) continue;
     }
-    const uint64_t rounds = (tiles + cus - 1) / cus;
-    const double cost = (double)rounds * t.bp * t.bq / kMfmaVariantEfficiency[v];
+    const uint64_t full = tiles / cus, rem = tiles % cus;
+    const double rounds = (double)full + (rem ? kPartialRound + (1.0 - kPartialRound) * (double)rem / cus : 0.0);
+    const MfmaTileCost &c = (g.a_type == CUDA_R_4F_E2M1 ? kMxTileCost : kMfmaTileCost)[v];
+    const double stages = (double)((int64_t)g.K * type_bits(g.a_type) / 8) / 128;
+    const double cost = rounds * t.bp * t.bq / c.efficiency * (stages + c.around);
     if (v == 0 || cost < best_cost) { best = v; best_cost = cost; }
   }
   return best;

@@ -13,9 +13,9 @@ struct MfmaVariant { int bp, bq, wp, wq, bkb, stages, m16, w4; };  // m16: the 1
 constexpr MfmaVariant kMfmaVariants[] = {
     {256, 256, 2, 4, 128, 2, 0, 0},  // 0: 8 waves, 128x64 per wave
     {256, 256, 2, 2, 128, 2, 0, 0},  // 1: 4 waves, 128x128 per wave
-    {256, 128, 2, 2, 128, 2, 0, 0},  // 2: 4 waves, 128x64 per wave
+    {256, 128, 2, 2, 128, 2, 0, 0},  // 2: 4 waves, 128x64 per wave; or 8 waves, 64x64 per wave, 3 stages (mfma_eight_waves())
     {128, 128, 2, 2, 128, 2, 0, 0},  // 3: 4 waves, 64x64 per wave, two workgroups per CU; many tiles of a short K: mfma_short_k()
-    {128, 128, 2, 2, 64, 4, 0, 0},   // 4: same tile, half-line stages, deeper ring (short K)
+    {128, 128, 2, 2, 128, 3, 0, 0},  // 4: same tile, deeper ring, one workgroup per CU
     {128, 64, 2, 2, 128, 3, 0, 0},   // 5: 4 waves, 64x32 per wave: skinny problems
     {64, 64, 2, 2, 128, 3, 0, 0},    // 6: 4 waves, 32x32 per wave: problems of a few hundred tiles at most
     {192, 256, 2, 4, 128, 2, 0, 0},  // 7: 8 waves, 96x64 per wave: extents that 256 divides badly (3072, 6144, ...)
