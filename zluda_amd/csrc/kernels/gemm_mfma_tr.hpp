@@ -239,8 +239,13 @@ struct TrOperand {
 // gemm_mfma_pipe16.hpp -- the shape that needs less energy per multiply-add, for problems that keep the whole
 // chip busy (see there).  A fragment is then 16 rows x the 64 K bytes of a stage (lane l: row l%16, 16-byte
 // chunk l/16), one MFMA per pair of fragments and stage.
-template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, bool PKC, bool QKC, bool M16 = false>
-__global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams prm) {
+// KG = 2 (16-bit operands; when: tr_two_k_groups()): two groups of four waves share the workgroup's K range, each with LDS stages of its
+// own; their accumulators meet in LDS.  A stage is much waiting for little work (a barrier, an LDS round trip), and where a CU
+// has one workgroup nobody else fills the gaps: bf16 1024 x 512 x 32003 (128 x 128 tiles, eight shares) 76.8 -> 69 us, 80 x 351 x 2459,
+// 21 batches (64 x 64) 23.5 -> 19.1.  Four groups were slower than two on every shape tried.
+template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, bool PKC, bool QKC, bool M16 = false, int KG = 1>
+__global__ __launch_bounds__(WP *WQ * 64 * KG) void gemm_mfma_tr_kernel(MfmaParams prm) {
+  static_assert(KG == 1 || (KG == 2 && !M16 && WP * WQ == 4 && kind_is_h16(KIND)), "groups of four waves");
   static_assert(KIND == KIND_I8 || KIND == KIND_F8 || kind_is_h16(KIND) || KIND == KIND_F32, "8-, 16- or 32-bit operands");
   constexpr int ESZ = kind_esz(KIND);
   constexpr int MPS = KIND == KIND_F32 ? 4 : 1;  // MFMAs per fragment pair and sub-step
@@ -256,11 +261,12 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
   using acc_v = typename std::conditional<KIND == KIND_I8, v16i, v16f>::type;
   using frag_v = typename std::conditional<B16, v4i, v8i>::type;
 
-  __shared__ v4i lds[2 * STAGE_V4];
+  __shared__ v4i lds[KG * 2 * STAGE_V4];
 
   fetch_args(prm);
   const GemmArgs &g = prm.g;
-  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int t = threadIdx.x, lane = t & 63, wave_wg = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int kgrp = KG > 1 ? wave_wg >> 2 : 0, wave = KG > 1 ? wave_wg & 3 : wave_wg;
   const int wp = wave % WP, wq = wave / WP;
   const int lr = lane & 31, gsel = lane >> 5;
 
@@ -280,6 +286,14 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
   if (prm.splits > 1) {
     k0 = item.z * prm.split_stages * (64 / ESZ);
     Kl = max(0, min(g.K - k0, prm.split_stages * (64 / ESZ)));
+  }
+  // (the groups' shares are whole stages; trips counts the barriers of the longest, the first)
+  int trips = 0;
+  if constexpr (KG > 1) {
+    trips = ((Kl * ESZ + 63) / 64 + KG - 1) / KG;
+    const int mine = kgrp * trips * (64 / ESZ);
+    k0 += mine;
+    Kl = max(0, min(Kl - mine, trips * (64 / ESZ)));
   }
   {
     const uint8_t *a = (const uint8_t *)g.A + (g.a_sb * bt + (int64_t)k0 * g.a_sk) * ESZ;
@@ -573,7 +587,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
 
   // two register sets per operand: stage s travels through set s & 1
   int rp0[P.NREG], rp1[P.NREG], rq0[Q.NREG], rq1[Q.NREG];
-  v4i *buf0 = &lds[0], *buf1 = &lds[STAGE_V4];
+  v4i *buf0 = &lds[kgrp * 2 * STAGE_V4], *buf1 = buf0 + STAGE_V4;
   Frags f0;
   load_any(0, rp0, rq0);
   load_any(1, rp1, rq1);
@@ -614,8 +628,44 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_tr_kernel(MfmaParams pr
     }
   }
 
+  if constexpr (KG > 1) {
+    // as many barriers as the longest share has; then the first group adds the others' accumulators, in their order
+    for (int e = KT; e < trips; e++) __syncthreads();
+  }
   // every wave is done with the LDS stages before they become epilogue staging
   __syncthreads();
+  if constexpr (KG > 1) {
+    static_assert(TP * TQ * 4 * 64 * 4 * (KG - 1) <= KG * 2 * STAGE_V4, "the accumulators fit the stages");
+    v4i *part = &lds[(wave * TP * TQ * 4) * 64 + lane];
+    constexpr int GROUP = 4 * TP * TQ * 4 * 64;
+    if (kgrp > 0) {
+#pragma unroll
+      for (int a = 0; a < TQ; a++)
+#pragma unroll
+        for (int b = 0; b < TP; b++)
+#pragma unroll
+          for (int v = 0; v < 4; v++)
+            part[(kgrp - 1) * GROUP + ((a * TP + b) * 4 + v) * 64] =
+                v4i{to_bits(acc[a][b][4 * v]), to_bits(acc[a][b][4 * v + 1]), to_bits(acc[a][b][4 * v + 2]), to_bits(acc[a][b][4 * v + 3])};
+    }
+    __syncthreads();
+    if (kgrp > 0) return;
+#pragma unroll
+    for (int o = 0; o < KG - 1; o++)
+#pragma unroll
+      for (int a = 0; a < TQ; a++)
+#pragma unroll
+        for (int b = 0; b < TP; b++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            const v4i x = part[o * GROUP + ((a * TP + b) * 4 + v) * 64];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              acc[a][b][4 * v + e] += bits2f((uint32_t)x[e]);
+            }
+          }
+    __syncthreads();
+  }
   if constexpr (M16) {
     if (prm.splits > 1) {
       const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;

@@ -25,6 +25,17 @@ inline uint32_t launch_tr_variant(const MfmaParams &prm, const zluda_gemm_plan &
     ZLUDA_TR_MODE(BP, BQ, WP, WQ, false, false) ZLUDA_TR_MODE(BP, BQ, WP, WQ, false, true)                      \
     ZLUDA_TR_MODE(BP, BQ, WP, WQ, true, false) ZLUDA_TR_MODE(BP, BQ, WP, WQ, true, true)                        \
     break;
+#define ZLUDA_TR_KG(V, BP, BQ, PK, QK)                                                                            \
+  if (plan.variant == V && pkc == PK && qkc == QK)                                                               \
+    return launch_kernel(gemm_mfma_tr_kernel<KIND, FQ, FP, BP, BQ, 2, 2, PK, QK, false, 2>, grid, dim3(512), s, prm);
+  if (plan.block == 512 && (plan.variant == 1 || plan.variant == 2)) {  // (tr_two_k_groups())
+    if constexpr (kind_is_h16(KIND)) {
+      ZLUDA_TR_KG(1, 128, 128, false, false) ZLUDA_TR_KG(1, 128, 128, false, true) ZLUDA_TR_KG(1, 128, 128, true, false) ZLUDA_TR_KG(1, 128, 128, true, true)
+      ZLUDA_TR_KG(2, 64, 64, false, false) ZLUDA_TR_KG(2, 64, 64, false, true) ZLUDA_TR_KG(2, 64, 64, true, false) ZLUDA_TR_KG(2, 64, 64, true, true)
+    }
+    return CUBLAS_STATUS_INVALID_VALUE;
+  }
+#undef ZLUDA_TR_KG
   switch (plan.variant) {
     ZLUDA_TR_CASE(0, 256, 256, 2, 4)
     ZLUDA_TR_CASE(1, 128, 128, 2, 2)

@@ -564,6 +564,16 @@ bool tr_lds_reads(const Lowered &l, int variant, uint64_t groups, uint32_t split
   return lds < regs;
 }
 
+// Whether two groups of four waves of a 128 x 128 or 64 x 64 tile share a workgroup's K: at most one workgroup per CU, and enough
+// stages for the gaps to matter (bf16, us: 80 x 351 x 2459, 21 batches 23.5 -> 19.1; 960 x 124 x 31971 45.6 -> 36.5; 1024 x 512 x
+// 32003 76.8 -> 69; 300 x 300 x 1000 11.0 -> 9.7; level at 16 stages).  16-bit operands: f32 gains nothing, its MFMAs alone fill the time,
+// and int8 0.5 us of 7.
+static bool tr_two_k_groups(const Lowered &l, int variant, uint64_t groups, uint32_t splits, uint32_t cus) {
+  const uint32_t t = l.g.a_type;
+  if ((t != CUDA_R_16F && t != CUDA_R_16BF) || (variant != 1 && variant != 2) || groups > cus) return false;
+  return (uint64_t)l.g.K * 2 / std::max(splits, 1u) >= 24 * 64;
+}
+
 static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t workspace_size, zluda_gemm_plan *plan) {
   const GemmArgs &g = l.g;
   const TrVariant &v = kTrVariants[variant];
@@ -587,7 +597,10 @@ static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t w
   const uint64_t slots = (uint64_t)cus * per_cu;
   const bool skinny = std::min(g.M, g.N) <= 64;
   const uint64_t kbytes = (uint64_t)g.K * type_bits(g.a_type) / 8;
-  if (tiles * 2 <= (skinny ? slots : (uint64_t)cus) && kbytes >= 1024 && (uint64_t)ceil_div(np, v.bp) * v.bp <= (1u << 20)) {
+  // (On a shorter K the second kernel costs more than the shorter loop saves, us: int8 512 x 512 x 1024 10.7 split, 6.9 whole; f16
+  // 777 x 333 x 555 9.7 and 7.8; f32 1098 x 419 x 350 12.6 and 10.2; bf16 300 x 300 x 1000 9.7 both.)
+  const uint64_t least = skinny ? 1024 : g.a_type == CUDA_R_32F ? 1536 : type_bits(g.a_type) == 16 ? 2048 : 1088;
+  if (tiles * 2 <= (skinny ? slots : (uint64_t)cus) && kbytes >= least && (uint64_t)ceil_div(np, v.bp) * v.bp <= (1u << 20)) {
     uint32_t s = (uint32_t)std::min<uint64_t>({8, slots / tiles, kbytes / 512});
     const uint64_t per_split = (uint64_t)g.batch * ceil_div(np, v.bp) * v.bp * ceil_div(nq, v.bq) * v.bq * 4;
     while (s > 1 && s * per_split > workspace_size) s--;
@@ -597,6 +610,8 @@ static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t w
       plan->waves = (float)tiles * s / (float)slots;
     }
   }
+  if (!tr_lds_reads(l, variant, tiles * plan->grid_z, plan->grid_z, cus) && tr_two_k_groups(l, variant, tiles * plan->grid_z, plan->grid_z, cus))
+    plan->block = 512;
 }
 
 // Tile choice of the transposing kernel.  A CU runs up to `per_cu` workgroups of a variant side by
