@@ -737,12 +737,14 @@ static int pick_decode_variant(const Lowered &l, uint32_t cus) {
   // (two token blocks on one unit per slab, variant 20, only up to two blocks of rows per CU: 4096 x 32 x 4096
   // 8.9 us against 10.0, but 14336 x 32 x 4096 18.1 against 16.7; with two units, variant 17, it wins
   // throughout: 8192 x 32 x 8192 15.4 against 22.0)
-  // (16-bit weights, which have no other streaming form, also beyond 64 rows per CU when K is long: bf16
-  // 28672 x 16 x 8192 in 1.75 rounds of workgroups 80 us against 99 on 128 x 64 MFMA tiles; at K = 4096 the two are level)
+  // (16-bit weights, which have no other streaming form, also beyond 64 rows per CU, in more than one round of workgroups: with up to
+  // 8 tokens -- bf16, us, against the best MFMA tiles: 37888 x 8 x 3584 49 and 55, 28672 x 8 x 4096 38 and 47, 19000 x 4 x 2048 18.5 and
+  // 20.1 --, with more where K is long: 28672 x 16 x 8192 80 and 99)
   const uint32_t rows = (uint32_t)std::max(l.g.M, l.g.N);
-  const bool h16_long = (l.g.a_type == CUDA_R_16F || l.g.a_type == CUDA_R_16BF) && K * 2 > 8192;
+  const bool h16 = l.g.a_type == CUDA_R_16F || l.g.a_type == CUDA_R_16BF;
+  const bool many_rows = h16 && (K * 2 > 8192 || std::min(l.g.M, l.g.N) <= 8);
   for (int v = 0; v < kNumDecodeVariants; v++)
-    if (kDecodeVariants[v].stream == 2 && decode_variant_ok(l, v) && (rows <= 64 * cus || h16_long) &&
+    if (kDecodeVariants[v].stream == 2 && decode_variant_ok(l, v) && (rows <= 64 * cus || many_rows) &&
         !(kDecodeVariants[v].steps == 8 && rows > 32 * cus))
       return v;
   // the stream instantiation with the least cover that takes K
