@@ -124,19 +124,18 @@ struct WorkItem { int p, q, bt, z; };
 __device__ __forceinline__ uint32_t lesser(uint32_t a, uint32_t b) { return a < b ? a : b; }
 __device__ __forceinline__ WorkItem work_item(const MfmaParams &prm, uint32_t id) {
   const uint32_t tiles = (uint32_t)(prm.tiles_p * prm.tiles_q), batch = (uint32_t)prm.g.batch, n = tiles * batch * (uint32_t)prm.splits;
-  uint32_t w;
+  const uint32_t x = (id & 7) * (n >> 3) + lesser(id & 7, n & 7) + (id >> 3);
+  uint32_t w = x;
   WorkItem it;
   it.bt = it.z = 0;
-  // (kept out of the way of the plain case, whose way to its first loads it would lengthen by instruction cache lines)
-  if (__builtin_expect(n != tiles, 0)) {
+  // (a branch forward over what only batches and shares need: moved behind the kernel's end, it would return over the whole of it)
+  if (n != tiles) {
     const bool by_batch = (tiles & 7) == 0 && tiles >= 256;
-    const uint32_t x = (id & 7) * (n >> 3) + lesser(id & 7, n & 7) + (id >> 3), at = by_batch ? id : x, r = at / tiles;
+    const uint32_t at = by_batch ? id : x, r = at / tiles;
     w = at - r * tiles;
     if (by_batch) w = (w & 7) * (tiles >> 3) + (w >> 3);
     it.z = __builtin_amdgcn_readfirstlane((int)(r / batch));
     it.bt = __builtin_amdgcn_readfirstlane((int)(r % batch));
-  } else {
-    w = (id & 7) * (n >> 3) + lesser(id & 7, n & 7) + (id >> 3);
   }
   const uint32_t group = (uint32_t)(prm.group_p * prm.tiles_q), gid = w / group, first = gid * (uint32_t)prm.group_p;
   const uint32_t in = w - gid * group, rows = lesser((uint32_t)prm.tiles_p - first, (uint32_t)prm.group_p);
