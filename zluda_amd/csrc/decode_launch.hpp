@@ -84,7 +84,8 @@ inline uint32_t launch_decode_slab(const DecodeParams &prm, const zluda_gemm_pla
   dim3 grid(plan.grid_x, plan.grid_y, 1), block(v.nw * 64);
   // 0: element-wise epilogue, 1: packed store, 2: packed store behind a GELU
   const int fast = !decode_packed_output(prm.g, prm.swapped != 0) ? 0 : prm.g.act == ACT_GELU ? 2 : 1;
-  const bool tail = prm.g.K * (kind_is_h16(KIND) ? 2 : 1) < v.nw * v.steps * 64;  // K bytes against the cover
+  const int kbytes = KIND == KIND_MXF4 ? prm.g.K / 2 : kind_is_h16(KIND) ? prm.g.K * 2 : prm.g.K;
+  const bool tail = kbytes < v.nw * v.steps * 64;  // K bytes against the cover
   uint32_t st = CUBLAS_STATUS_NOT_SUPPORTED;
   static_for_host<3>([&](auto fast_c) {
     constexpr int FAST = decltype(fast_c)::value;
@@ -95,11 +96,15 @@ inline uint32_t launch_decode_slab(const DecodeParams &prm, const zluda_gemm_pla
     } else if (v.nw == 8 && nb == 1) {
       static_for_host<3>([&](auto q_c) {
         constexpr int Q = decltype(q_c)::value + 2;
-        if (v.steps == Q * 8) st = launch_kernel(decode_slab_kernel<FAST, KIND, true, 8, 512, Q>, grid, block, s, prm);
+        if constexpr (KIND != KIND_MXF4 || Q < 4) {  // (planner.cpp: decode_variant_ok())
+          if (v.steps == Q * 8) st = launch_kernel(decode_slab_kernel<FAST, KIND, true, 8, 512, Q>, grid, block, s, prm);
+        }
       });
     } else if (v.nw == 8 && nb == 2) {  // two token blocks: one or two units per slab
       if (v.steps == 8) st = launch_kernel(decode_slab_kernel<FAST, KIND, true, 8, 512, 1, 2>, grid, block, s, prm);
-      else if (v.steps == 16) st = launch_kernel(decode_slab_kernel<FAST, KIND, true, 8, 512, 2, 2>, grid, block, s, prm);
+      else if constexpr (KIND != KIND_MXF4) {
+        if (v.steps == 16) st = launch_kernel(decode_slab_kernel<FAST, KIND, true, 8, 512, 2, 2>, grid, block, s, prm);
+      }
     }
   });
   return st;
@@ -107,6 +112,7 @@ inline uint32_t launch_decode_slab(const DecodeParams &prm, const zluda_gemm_pla
 
 uint32_t launch_decode_slab_i8(const DecodeParams &prm, const zluda_gemm_plan &plan, int nb, hipStream_t s);
 uint32_t launch_decode_slab_h16(const DecodeParams &prm, const zluda_gemm_plan &plan, int nb, bool bf16, hipStream_t s);
+uint32_t launch_decode_slab_mx(const DecodeParams &prm, const zluda_gemm_plan &plan, int nb, hipStream_t s);
 uint32_t launch_decode_slab_f8(const DecodeParams &prm, const zluda_gemm_plan &plan, int nb, hipStream_t s);
 uint32_t launch_decode_stream_i8(const DecodeParams &prm, const zluda_gemm_plan &plan, int nb, hipStream_t s);
 uint32_t launch_decode_stream_f8(const DecodeParams &prm, const zluda_gemm_plan &plan, int nb, hipStream_t s);

@@ -5,7 +5,10 @@
 //   out(r, t) = sum_k W[r][k] * X[t][k]     int32 (fp32), then the fused float / integer epilogue
 // The same kernel streams f16 / bf16 weights (KIND_F16 / KIND_BF16: v_mfma_f32_16x16x32_f16 / _bf16 take 16 bytes
 // of K per lane at the byte positions of the int8 instruction, so only the MFMA and the accumulator type
-// differ; every K below is then a count of BYTES, twice the element count).
+// differ; every K below is then a count of BYTES, twice the element count), and MXFP4 weights (KIND_MXF4: K bytes are half the
+// element count; block scales as one more DMA instruction per unit).  MXFP4, 8 tokens, us, on the MFMA tiles before: 8192 x 8192
+// 14.4 -> 8.8, 57344 x 8192 59 -> 45 (250 MB, 5.6 TB/s), 8192 x 23552 29.3 -> 20.2, 4608 x 13824 16.4 -> 10.2; 32 tokens 10240 x 8192
+// 17.1 -> 12.9.
 //
 // What differs from decode_stream_kernel, and what each point bought on a 14336 x 4096 int8 matrix with 16
 // tokens (MI355X, 58.7 MB, a flat read of the same bytes takes 9.95 us; decode_stream_kernel 14.8 us):
@@ -58,8 +61,9 @@ constexpr int kSlabMaxBlocks = 4;   // 16-row blocks a workgroup can run
 constexpr int kSlabFactorLoads = 21;  // vector memory loads of the packed epilogue's factors, per lane
 template <int FAST, int KIND, bool TAIL, int NW = 4, int UB = 1024, int Q = 1, int NB = 1>
 __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) {
-  static_assert(KIND == KIND_I8 || KIND == KIND_F8 || kind_is_h16(KIND), "int8, fp8 (e4m3 x e4m3), f16 or bf16 operands");
-  constexpr int ESZ = kind_is_h16(KIND) ? 2 : 1;           // bytes per element
+  static_assert(KIND == KIND_I8 || KIND == KIND_F8 || KIND == KIND_MXF4 || kind_is_h16(KIND), "int8, fp8 (e4m3 x e4m3), MXFP4, f16 or bf16 operands");
+  constexpr bool MX = KIND == KIND_MXF4;
+  constexpr int EBITS = MX ? 4 : kind_is_h16(KIND) ? 16 : 8;  // per element
   constexpr bool B16 = KIND != KIND_F8;                    // 16 bytes of K per lane and MFMA (fp8: 32)
   static_assert((UB == 1024 || UB == 512) && Q >= 1 && Q * NB <= 4 && (Q * NB == 1 || TAIL), "see above; the shapes beyond the first come with the K checks");
   using acc_t = typename std::conditional<KIND == KIND_I8, v4i, v4f>::type;
@@ -69,9 +73,11 @@ __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) 
   constexpr int CPR = UB / 16;          // 16-byte chunks per row of a unit
   constexpr int NFRAG = UB / 64;        // 16-byte fragments per lane and unit
   constexpr int UNIT_V4 = 16 * CPR;
+  constexpr int SLOT_V4 = UNIT_V4 + (MX ? 64 : 0);  // MXFP4: the unit's scale bytes behind it, one more DMA instruction
+  constexpr int NVM = NDMA + (MX ? 1 : 0);          // vector memory instructions per unit
   static_assert(MAXB * NB <= NW, "one wave per (block, token block) runs the epilogue");
   static_assert(MAXB * NB * 64 <= 2 * UNIT_V4, "a wave's partial tiles fit into its own ring");
-  __shared__ v4i ring[NW][2][UNIT_V4];
+  __shared__ v4i ring[NW][2][SLOT_V4];
 
   const GemmArgs &g = prm.g;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -79,11 +85,11 @@ __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) 
   const int bt = blockIdx.y;
 
   const int R = prm.swapped ? g.N : g.M, T = prm.swapped ? g.M : g.N;
-  const uint8_t *Wg = (const uint8_t *)(prm.swapped ? g.B : g.A) + (prm.swapped ? g.b_sb : g.a_sb) * bt * ESZ;
-  const uint8_t *Xg = (const uint8_t *)(prm.swapped ? g.A : g.B) + (prm.swapped ? g.a_sb : g.b_sb) * bt * ESZ;
-  const int ldw = (int)(prm.swapped ? g.b_sj : g.a_si) * ESZ;  // row pitches and K in bytes
-  const int ldx = (int)(prm.swapped ? g.a_si : g.b_sj) * ESZ;
-  const int K = g.K * ESZ;
+  const uint8_t *Wg = (const uint8_t *)(prm.swapped ? g.B : g.A) + (prm.swapped ? g.b_sb : g.a_sb) * bt * EBITS / 8;
+  const uint8_t *Xg = (const uint8_t *)(prm.swapped ? g.A : g.B) + (prm.swapped ? g.a_sb : g.b_sb) * bt * EBITS / 8;
+  const int ldw = (int)((prm.swapped ? g.b_sj : g.a_si) * EBITS / 8);  // row pitches and K in bytes
+  const int ldx = (int)((prm.swapped ? g.a_si : g.b_sj) * EBITS / 8);
+  const int K = (int)((int64_t)g.K * EBITS / 8);
 
   // Blocks of this workgroup: full_rounds round-robin blocks, then its share [rr0, rr1) (at most 16 rows, a
   // whole number of quads except at the very end of W) of the rows behind the last full round.  The split is
@@ -114,6 +120,23 @@ __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) 
   // issues has all of its lanes out of range, which the counted waits below depend on.
   auto unit_voff = [&](int i, int q, int pitch) { return slab_unit_voff(TAIL, UB, lane, dma_off[i], q, kw, kwave, K, pitch); };
   auto unit_empty = [&](int q) { return slab_unit_empty(TAIL, UB, q, kw, kwave, K); };  // (wave-uniform)
+  // MXFP4: the [row][K/32] scale bytes, one per 16 bytes of a row, through windows of their exact size.  A unit's UB / 16 bytes of
+  // 16 rows are one DMA instruction (UB = 512: its first half), laid out [row][UB / 16].  (An empty unit fetches the row's first ones:
+  // a real load.)
+  const int KB = K / 16;
+  __amdgpu_buffer_rsrc_t rsSW = rsW, rsSX = rsX;
+  constexpr int SPR = UB / 256;  // 16-byte pieces of scales per row of a unit
+  const int srow = lane / SPR, spiece = (lane % SPR) * 16;
+  if constexpr (MX) {
+    rsSW = __builtin_amdgcn_make_buffer_rsrc((void *)((const uint8_t *)(prm.swapped ? g.b_scale : g.a_scale) + (int64_t)bt * R * KB), 0, R * KB, 0x00020000);
+    rsSX = __builtin_amdgcn_make_buffer_rsrc((void *)((const uint8_t *)(prm.swapped ? g.a_scale : g.b_scale) + (int64_t)bt * T * KB), 0, T * KB, 0x00020000);
+  }
+  auto issue_scales = [&](__amdgpu_buffer_rsrc_t rs, int row, int last, int q, v4i *dst) {
+    if constexpr (MX) {
+      const int s0 = unit_empty(q) ? 0 : (kwave + q * UB) / 16;
+      lds_dma16(rs, dst + UNIT_V4, srow < 16 ? min(row + srow, last) * KB + s0 + spiece : (int)0x80000000, 0);
+    }
+  };
   auto issue_w = [&](int b, int q, int slot) {
     const int rb = row_base(b), re = row_end(b);
     v4i *dst = &ring[wave][slot][0];
@@ -124,6 +147,7 @@ __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) 
       const int row = min(rb + RPI * i, re - 1);
       lds_dma16<kWeightStreamAux>(rsW, dst + i * 64, unit_voff(i, q, RPI == 2 && half && row + 1 < re ? ldw : 0), row * ldw);
     }
+    issue_scales(rsSW, rb, re - 1, q, dst);
   };
   // (token 16 * nbk + rho, rho = row of the unit; tokens past T repeat the last one and are never stored)
   auto issue_x = [&](int nbk, int q, int slot) {
@@ -133,17 +157,42 @@ __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) 
       const int tok = min(16 * nbk + RPI * i, T - 1);
       lds_dma16(rsX, dst + i * 64, unit_voff(i, q, RPI == 2 && half && tok + 1 < T ? ldx : 0), tok * ldx);
     }
+    issue_scales(rsSX, 16 * nbk, T - 1, q, dst);
   };
   // fragment f of this lane in a unit: int8, f16, bf16: K step f, 16 bytes at f*64 + g4*16; fp8: half (f & 1) of
-  // the 32 bytes at (f/2)*128 + g4*32 of K step f/2
+  // the 32 bytes at (f/2)*128 + g4*32 of K step f/2; MXFP4: lane group g4 takes a quarter of the unit, piece by piece, so that its
+  // scale bytes lie side by side (the K order of a dot product is free)
   const uint32_t ring_base = lds_addr(&ring[wave][0][l16 * CPR]);
   auto frag_addr = [&](int slot, int f) {
-    const int c = B16 ? 4 * f + g4 : 8 * (f >> 1) + 2 * g4 + (f & 1);
-    return ring_base + slot * (UNIT_V4 * 16) + (((c & ~15) | ((c ^ l16) & 15)) << 4);
+    const int c = MX ? (CPR / 4) * g4 + f : B16 ? 4 * f + g4 : 8 * (f >> 1) + 2 * g4 + (f & 1);
+    return ring_base + slot * (SLOT_V4 * 16) + (((c & ~15) | ((c ^ l16) & 15)) << 4);
   };
   // unit n of this wave = (block n / Q, unit n % Q of the slab), in slot n % 2; the wave runs nblk * Q of them
   auto issue_unit = [&](int n, int slot) { issue_w(n / Q, n % Q, slot); };
 
+  // MXFP4: the lane's scale bytes of unit q in `slot`, one per fragment, fragment f's in byte f % 4 of dword f / 4.  Fragments past the
+  // wave's share or past K are zeros, and the bytes there may be any other row's NaN: they take the bytes of the unit's first
+  // lane group (or of the lane's first half) instead, which are the row's own.
+  const uint32_t scale_base = lds_addr(&ring[wave][0][UNIT_V4]) + l16 * (UB / 16);
+  auto unit_has = [&](int q, int off) { return !TAIL || (q * UB + off < kw && kwave + q * UB + off < K); };  // (whole multiples of 128 bytes)
+  auto scale_group = [&](int q) { return unit_has(q, g4 * (UB / 4)) ? g4 : 0; };
+  auto scales_raw = [&](int slot, int q) {
+    return lds_read16_unordered(scale_base + slot * (SLOT_V4 * 16) + (UB == 1024 ? scale_group(q) : scale_group(q) >> 1) * 16);
+  };
+  struct Scales { int d[NFRAG / 4]; };
+  auto scales_of = [&](const v4i &raw, int q) {
+    Scales s;
+    if constexpr (UB == 1024) {
+      const bool both = unit_has(q, scale_group(q) * 256 + 128);
+      s.d[0] = raw[0]; s.d[1] = raw[1];
+      s.d[NFRAG / 4 - 2] = both ? raw[2] : raw[0]; s.d[NFRAG / 4 - 1] = both ? raw[3] : raw[1];
+    } else {
+      const bool odd = scale_group(q) & 1;
+      s.d[0] = odd ? raw[2] : raw[0]; s.d[1] = odd ? raw[3] : raw[1];
+    }
+    return s;
+  };
+  Scales xs[MX ? NB * Q : 1];
   v4i xf[NB * Q][NFRAG];  // [token block * Q + unit]
   if constexpr (NB * Q == 1) {
     // Activations into slot 1, the first weights behind them, and as soon as the activations are in registers
@@ -151,10 +200,16 @@ __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) 
     // front of the stream.
     issue_x(0, 0, 1);
     issue_unit(0, 0);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");  // all but the youngest unit: the activations
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVM) : "memory");  // all but the youngest unit: the activations
 #pragma unroll
     for (int f = 0; f < NFRAG; f++) xf[0][f] = lds_read16_unordered(frag_addr(1, f));
+    v4i raw[1];
+    if constexpr (MX) raw[0] = scales_raw(1, 0);
     lds_values_ready(xf[0]);
+    if constexpr (MX) {
+      lds_values_ready(raw);
+      xs[0] = scales_of(raw[0], 0);
+    }
   } else {
     // the activations of the whole slab (of every token block), two units at a time through the two slots, then
     // the first weights
@@ -168,6 +223,14 @@ __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) 
       if (c + 1 < NB * Q) {
 #pragma unroll
         for (int f = 0; f < NFRAG; f++) xf[c + 1][f] = lds_read16_unordered(frag_addr(1, f));
+      }
+      if constexpr (MX) {
+        v4i raw[2];
+        raw[0] = scales_raw(0, c % Q);
+        raw[1] = scales_raw(1, (c + 1) % Q);
+        lds_values_ready(raw);
+        xs[c] = scales_of(raw[0], c % Q);
+        if (c + 1 < NB * Q) xs[c + 1] = scales_of(raw[1], (c + 1) % Q);
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
@@ -263,14 +326,17 @@ __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) 
             f_sd = g.d_scale ? f_sd : 1.0f;
           }
         } else if (n == 0 && counted) {
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA + kSlabFactorLoads) : "memory");
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVM + kSlabFactorLoads) : "memory");
         } else {
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVM) : "memory");
         }
         v4i w[NFRAG];
 #pragma unroll
         for (int f = 0; f < NFRAG; f++) w[f] = lds_read16_unordered(frag_addr(n & 1, f));
+        v4i raw[1];
+        if constexpr (MX) raw[0] = scales_raw(n & 1, q);
         lds_values_ready(w);  // in registers before the slot is refilled
+        if constexpr (MX) lds_values_ready(raw);
         if ((n + 2) / Q < nblk) issue_unit(n + 2, n & 1);
         // (a unit that holds no byte of K was fetched for the count only: for 8-bit operands its activation fragments
         // are zero -- see above --, 16-bit ones, whose stray weights may be infinite, skip its MFMAs)
@@ -293,6 +359,14 @@ __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) 
             for (int f = 0; f < NFRAG; f++)
               acc[b][nbk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8b, w[f]), __builtin_bit_cast(v8b, xf[nbk * Q + q][f]),
                                                                     acc[b][nbk], 0, 0, 0);
+          } else if constexpr (MX) {
+            const Scales ws = scales_of(raw[0], q), xq = xs[nbk * Q + q];
+            static_for<NFRAG>([&](auto f_c) {
+              constexpr int f = decltype(f_c)::value;
+              const v4i x = xf[nbk * Q + q][f];
+              const v8i wa = {w[f][0], w[f][1], w[f][2], w[f][3], 0, 0, 0, 0}, xb = {x[0], x[1], x[2], x[3], 0, 0, 0, 0};
+              acc[b][nbk] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wa, xb, acc[b][nbk], 4, 4, f & 3, ws.d[f / 4], f & 3, xq.d[f / 4]);
+            });
           } else {
 #pragma unroll
             for (int f = 0; f < NFRAG; f += 2) {
@@ -319,7 +393,7 @@ __global__ __launch_bounds__(NW * 64) void decode_slab_kernel(DecodeParams prm) 
   v4i part[NW];
   const uint32_t red_base = lds_addr(&ring[0][0][wave * 64 + lane]);
 #pragma unroll
-  for (int w2 = 0; w2 < NW; w2++) part[w2] = lds_read16_unordered(red_base + w2 * (2 * UNIT_V4 * 16));
+  for (int w2 = 0; w2 < NW; w2++) part[w2] = lds_read16_unordered(red_base + w2 * (2 * SLOT_V4 * 16));
   lds_values_ready(part);
   acc_t s = __builtin_bit_cast(acc_t, part[0]);
 #pragma unroll

@@ -253,7 +253,8 @@ static bool decode_variant_ok(const Lowered &l, int variant) {
   const DecodeVariant &v = kDecodeVariants[variant];
   const int T = std::min(g.M, g.N), nb = (T + 15) / 16;
   const bool h16 = g.a_type == CUDA_R_16F || g.a_type == CUDA_R_16BF;
-  if (h16 && v.stream != 2) return false;  // 16-bit weights: the slab form only
+  const bool mx = g.a_type == CUDA_R_4F_E2M1;
+  if ((h16 || mx) && v.stream != 2) return false;  // 16- and 4-bit weights: the slab form only
   // the register-streaming kernel is int8 only; token blocks multiply its fragment registers
   if (!v.stream) return g.a_type == CUDA_R_8I && (nb == 1 || (nb == 2 && v.steps <= 8));
   const bool swapped = g.M < g.N;
@@ -263,10 +264,11 @@ static bool decode_variant_ok(const Lowered &l, int variant) {
     // (the 4-wave shape serves K down to half of its 4096; an 8-wave shape the K above the next smaller cover)
     const int cover = v.nw * v.steps * 64, below = cover == 4096 ? cover / 2 : cover - 4096;
     // one block of tokens; two in the 8-wave shapes of one or two units (the one-unit shape exists for them alone)
-    const bool tokens_ok = v.nw == 4 ? nb == 1 : v.steps == 8 ? nb == 2 : v.steps == 16 ? nb <= 2 : nb == 1;
-    const int64_t esz = h16 ? 2 : 1, kb = (int64_t)g.K * esz;  // covers are bytes of K
-    return tokens_ok && kb <= cover && kb > below && (kb & 15) == 0 && rows * ldw * esz < 0x7fffffffll &&
-           ((int64_t)(T - 1) * ldx + g.K) * esz < 0x7fffffffll;
+    // (MXFP4, whose scales take registers too, has neither two units with two blocks nor four units)
+    const bool tokens_ok = v.nw == 4 ? nb == 1 : v.steps == 8 ? nb == 2 : v.steps == 16 ? nb <= (mx ? 1 : 2) : nb == 1 && !(mx && v.steps == 32);
+    const int64_t bits = type_bits(g.a_type), kb = (int64_t)g.K * bits / 8;  // covers are bytes of K
+    return tokens_ok && kb <= cover && kb > below && (kb & (mx ? 127 : 15)) == 0 && rows * ldw * bits / 8 < 0x7fffffffll &&
+           ((int64_t)(T - 1) * ldx + g.K) * bits / 8 < 0x7fffffffll;
   }
   // a stream instantiation covers nw * steps * 64 bytes of K and takes any K up to that (lanes past the end read
   // zero); more than a quarter of idle lanes is left to the smaller instantiations or to the MFMA tiles
@@ -350,9 +352,10 @@ bool family_supports(uint32_t kernel, const Lowered &l) {
   case ZLUDA_KERNEL_MFMA_TR8: case ZLUDA_KERNEL_MFMA_TR16: case ZLUDA_KERNEL_MFMA_TR32:
     return transposing_family(l, false) == kernel;
   case ZLUDA_KERNEL_DECODE_W8A8:
-    // int8, or e4m3 x e4m3 without block scales (the LDS-streaming variants only), or f16 / bf16 (the slab form only)
+    // int8, or e4m3 x e4m3 without block scales (the LDS-streaming variants only), or f16 / bf16 or MXFP4 (the slab form only)
     return fast_layout && ((g.a_type == CUDA_R_8I && g.b_type == CUDA_R_8I) ||
                            ((g.a_type == CUDA_R_16F || g.a_type == CUDA_R_16BF) && g.b_type == g.a_type) ||
+                           (g.a_type == CUDA_R_4F_E2M1 && family_supports(ZLUDA_KERNEL_MFMA_MXF4, l)) ||
                            (g.a_type == CUDA_R_8F_E4M3 && g.b_type == CUDA_R_8F_E4M3 &&
                             g.a_scale_mode != SCALE_BLOCK32_UE8M0 && g.b_scale_mode != SCALE_BLOCK32_UE8M0)) &&
            std::min(g.M, g.N) <= kDecodeMaxTokens && std::max(g.M, g.N) >= 64 && any_decode_variant_ok(l);
@@ -742,10 +745,14 @@ static int pick_decode_variant(const Lowered &l, uint32_t cus) {
   // 20.1 --, with more where K is long: 28672 x 16 x 8192 80 and 99)
   const uint32_t rows = (uint32_t)std::max(l.g.M, l.g.N);
   const bool h16 = l.g.a_type == CUDA_R_16F || l.g.a_type == CUDA_R_16BF;
-  const bool many_rows = h16 && (K * 2 > 8192 || std::min(l.g.M, l.g.N) <= 8);
+  const bool mx = l.g.a_type == CUDA_R_4F_E2M1;
+  // (MXFP4 beyond 64 rows per CU where the rounds are 70 % full: 57344 x 8 x 8192 in 3.5 rounds 45 us against 59 on MFMA tiles, but
+  // 20480 x 8 x 5120 in 1.25 17.6 against 17.3)
+  const uint64_t round = 64 * (uint64_t)cus;
+  const bool many_rows = (mx && (uint64_t)rows * 10 >= (rows + round - 1) / round * round * 7) || (h16 && (K * 2 > 8192 || std::min(l.g.M, l.g.N) <= 8));
   for (int v = 0; v < kNumDecodeVariants; v++)
     if (kDecodeVariants[v].stream == 2 && decode_variant_ok(l, v) && (rows <= 64 * cus || many_rows) &&
-        !(kDecodeVariants[v].steps == 8 && rows > 32 * cus))
+        !(kDecodeVariants[v].steps == 8 && rows > 32 * cus && !mx))
       return v;
   // the stream instantiation with the least cover that takes K
   int best = -1;
