@@ -493,9 +493,11 @@ static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t
 }
 
 // Relative throughput of one CU inside the K loop on tiles of each variant (variant 0 = 1) and what a tile costs around its
-// loop, in stages of 128 bytes of K.  Fitted to the times of 460 int8, fp8 and bf16 and 150 MXFP4 problems on every variant
-// (MI355X; linear layers of 48 to 3000 tokens and 256 .. 8192 rows and columns, K = 128 .. 14592): what they pick takes 1.8 %
-// (MXFP4 1.0 %) more time than the best variant of each problem on average.
+// loop, in stages of 128 bytes of K.  Fitted to the times of 460 int8, fp8 and bf16 and 270 MXFP4 problems on every variant
+// (MI355X; linear layers of 17 to 4096 tokens and 256 .. 60000 rows, K = 128 .. 24000): what they pick takes 1.8 %
+// (MXFP4 0.3 %; fitted to one half of the problems, 0.6 % on the other) more time than the best variant of each problem on average.
+// MXFP4 counts the rounds of variant 3 over the two workgroups that a CU holds (34304 x 296 x 6400: 70 us, counted one by one
+// variant 5 came out ahead, which takes 94; 8192 x 777 x 8192 41.8, variant 4 48); the other types pick no better for it.
 // The variants on the 16x16 MFMA shapes (8, 9) need less energy per multiply-add, which is what bounds a GEMM that keeps the
 // whole chip busy (the board sits at its power cap); on a chip that is partly idle the clock is the bound instead, so they are
 // only chosen for grids that fill the chip; the same tiles at 256x128 and 128x128 measured no better than the 32x32 ones
@@ -503,8 +505,8 @@ static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t
 struct MfmaTileCost { float efficiency, around; };
 static const MfmaTileCost kMfmaTileCost[kNumMfmaVariants] = {{1.00f, 5.8f}, {0.95f, 6.0f}, {0.82f, 7.6f}, {0.62f, 5.9f}, {0.76f, 9.0f}, {0.43f, 4.4f},
                                                              {0.41f, 3.4f}, {0.89f, 6.3f}, {1.05f, 5.1f}, {0.89f, 4.6f}, {0.41f, 3.4f}, {1.06f, 5.3f}};
-static const MfmaTileCost kMxTileCost[kNumMfmaVariants] = {{1.00f, 6.0f}, {0.95f, 6.0f}, {0.80f, 9.0f}, {0.70f, 3.3f}, {0.84f, 9.0f}, {0.55f, 3.3f},
-                                                           {0.40f, 2.4f}, {0.92f, 5.3f}, {1.05f, 6.0f}, {0.89f, 6.0f}, {0.40f, 2.4f}, {1.10f, 6.0f}};
+static const MfmaTileCost kMxTileCost[kNumMfmaVariants] = {{1.00f, 3.2f}, {0.95f, 3.2f}, {0.82f, 8.5f}, {0.79f, 3.0f}, {0.62f, 5.0f}, {0.46f, 4.4f},
+                                                           {0.26f, 2.9f}, {1.06f, 5.5f}, {1.05f, 3.2f}, {0.89f, 3.2f}, {0.26f, 2.9f}, {1.27f, 5.1f}};
 // A last round that fills a part x of the CUs takes this + (1 - this) * x of a full one's time: the clock is higher and memory
 // less busy then.
 constexpr double kPartialRound = 0.65;
@@ -540,9 +542,10 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus) {
       const uint64_t need = (g.a_type == CUDA_R_8I || h16) ? ((uint64_t)cus * 3 + 3) / 4 : (uint64_t)cus * (t.bp == 256 ? 4 : 2);
       if (tiles < need) continue;
     }
-    const uint64_t full = tiles / cus, rem = tiles % cus;
-    const double rounds = (double)full + (rem ? kPartialRound + (1.0 - kPartialRound) * (double)rem / cus : 0.0);
-    const MfmaTileCost &c = (g.a_type == CUDA_R_4F_E2M1 ? kMxTileCost : kMfmaTileCost)[v];
+    const bool mx = g.a_type == CUDA_R_4F_E2M1;
+    const uint64_t per_cu = mx && v == 3 ? 2 : 1, slots = per_cu * cus, full = tiles / slots, rem = tiles % slots;
+    const double rounds = (double)per_cu * ((double)full + (rem ? kPartialRound + (1.0 - kPartialRound) * (double)rem / slots : 0.0));
+    const MfmaTileCost &c = (mx ? kMxTileCost : kMfmaTileCost)[v];
     const double stages = (double)((int64_t)g.K * type_bits(g.a_type) / 8) / 128;
     const double cost = rounds * t.bp * t.bq / c.efficiency * (stages + c.around);
     if (v == 0 || cost < best_cost) { best = v; best_cost = cost; }
