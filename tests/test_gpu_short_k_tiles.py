@@ -38,3 +38,35 @@ def test_row_major_scales_and_other_roads(gpu_api):
     run(gpu_api, 130, 130, 80, 133, with_c=True, beta=0.5)       # a tile per workgroup
     run(gpu_api, 131, 130, 80, 133, ldd=131)
     run(gpu_api, 130, 130, 80, 133, epilogue=K.CUBLASLT_EPILOGUE_GELU_BIAS)
+
+
+def test_a_plan_for_another_number_of_cus(gpu_api):
+    """64 elements of K in 60 tiles: a plan for 8 CUs has the form (16 workgroups), one for this device would not"""
+    import ctypes as C
+    import torch
+    t = K.CUDA_R_16BF
+    case = Case(dict(a_type=t, b_type=t, d_type=t, c_type=t, compute_type=K.CUBLAS_COMPUTE_32F, scale_type=K.CUDA_R_32F, m=300, n=200, k=64, transa=1, batch=10), 7800)
+    print("case", case.spec, flush=True)
+    keep, ptr, dt = case.upload()
+    p = case.problem(dict(ptr, alpha=case.alpha.ctypes.data, beta=case.beta.ctypes.data))
+    plan = K.zluda_gemm_plan()
+    assert gpu_api.zluda_gemm_plan_problem(C.byref(p), K.ZLUDA_KERNEL_MFMA_H16, 3, 8, C.byref(plan)) == 0
+    assert (plan.variant, plan.grid_x, plan.grid_y, plan.grid_z) == (3, 16, 1, 1)
+    assert gpu_api.zluda_gemm_launch(C.byref(p), C.byref(plan), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    case.compare(case.download(dt), case.run_oracle(), tol=1e-2)
+
+
+@pytest.mark.parametrize("ldd,aux_ld", [(132, 131), (131, 132)])
+def test_a_kept_gelu_input_with_a_pitch_of_its_own(gpu_api, ldd, aux_ld):
+    """the kernel writes the GELU input: the pitch of that matrix decides, not D's"""
+    t = K.CUDA_R_16F   # (D is the GELU of a rounded input u: |u gelu'(u) / gelu(u)| < 16 down to u = -4, times half an ulp of f16: 4e-3)
+    s = dict(a_type=t, b_type=t, d_type=t, c_type=t, compute_type=K.CUBLAS_COMPUTE_32F, scale_type=K.CUDA_R_32F,
+             m=130, n=130, k=72, transa=1, batch=133, ldc=ldd, ldd=ldd, aux_ld=aux_ld, epilogue=K.CUBLASLT_EPILOGUE_GELU_AUX)
+    print("case", s, flush=True)
+    case = Case(s, 7900)
+    ref = case.run_oracle()
+    st, got, kernel, variant = case.run_gpu(gpu_api)
+    assert st == 0 and kernel == K.ZLUDA_KERNEL_MFMA_H16
+    case.compare(got, ref, tol=1e-2)
+    case.compare_aux(case.aux_got, case.aux_ref)

@@ -468,3 +468,24 @@ def test_bias_gradient_epilogues_are_planned_like_the_plain_problem(api):
         assert plan(api, dict(f8, epilogue=epi, aux_ld=512, aux_type=K.CUDA_R_8F_E4M3))[0] == K.CUBLAS_STATUS_NOT_SUPPORTED
     st, _ = plan(api, dict(I8, m=512, n=512, k=512, transa=1, epilogue=K.CUBLASLT_EPILOGUE_GELU_AUX, aux_ld=512))   # int32 scale type
     assert st == K.CUBLAS_STATUS_NOT_SUPPORTED
+
+
+def test_short_k_plans_have_fewer_workgroups_than_tiles_or_one_per_tile(api):
+    """whatever the number of CUs: a plan of the short-K form is told from one of the 128 x 128 tile by its grid alone"""
+    t = K.CUDA_R_16BF
+    forms = set()
+    for cus in (1, 2, 3, 4, 5, 7, 8, 64, 256, 304):
+        for batch in (1, 2, 3, 4, 5, 9, 16, 17, 130):
+            for n in (100, 1000):
+                tiles = 2 * -(-n // 128) * batch
+                st, p = plan(api, dict(a_type=t, b_type=t, d_type=t, compute_type=K.CUBLAS_COMPUTE_32F, scale_type=K.CUDA_R_32F, m=200, n=n, k=64, transa=1, batch=batch),
+                             K.ZLUDA_KERNEL_MFMA_H16, 3, cus)
+                assert st == 0 and p.variant == 3 and p.grid_z == 1 and p.workspace == 0
+                short = p.grid_y == 1 and p.grid_x != tiles // batch
+                if short or (batch > 1 and p.grid_y == 1):
+                    assert p.grid_x % 8 == 0 and 0 < p.grid_x < tiles
+                    forms.add("short")
+                else:
+                    assert (p.grid_x, p.grid_y) == (tiles // batch, batch)
+                    forms.add("tiles")
+    assert forms == {"short", "tiles"}

@@ -86,13 +86,14 @@ uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws,
   prm.tiles_q = (nq + v.bq - 1) / v.bq;
   prm.group_p = 8;
   prm.splits = 1; prm.split_stages = 0; prm.ws = nullptr;
-  if (plan.variant == 3 && plan.kernel == ZLUDA_KERNEL_MFMA_H16 && plan.grid_y == 1 && mfma_short_k(l, true, zluda_gemm_device_cu_count()) &&
-      (plan.grid_x & 7) == 0 && plan.grid_x < (uint64_t)prm.tiles_p * prm.tiles_q * l.g.batch) {
-    // (a beta that is not zero, known only now, runs with one tile per workgroup)
-    if (mfma_short_k(l, false, zluda_gemm_device_cu_count())) {
+  // The short-K form: fewer workgroups than tiles, for which the plan alone counts (it may have been made for another number of CUs).
+  if (plan.variant == 3 && plan.kernel == ZLUDA_KERNEL_MFMA_H16 && plan.grid_y == 1 && plan.grid_z == 1 && plan.grid_x > 0 && (plan.grid_x & 7) == 0 &&
+      plan.grid_x < (uint64_t)prm.tiles_p * prm.tiles_q * l.g.batch && mfma_short_k_operands(l)) {
+    if (mfma_short_k_output(l, false)) {
       prm.split_stages = (int32_t)plan.grid_x;
       return launch_mfma_short(prm, l.g.a_type == CUDA_R_16BF, plan.grid_x, s);
     }
+    // (a beta that is not zero or a D off a dword, known only now, runs with one tile per workgroup)
     plan.grid_x = (uint32_t)(prm.tiles_p * prm.tiles_q); plan.grid_y = l.g.batch; plan.grid_z = 1;
   }
   if ((uint32_t)(prm.tiles_p * prm.tiles_q) != plan.grid_x) return CUBLAS_STATUS_INVALID_VALUE;

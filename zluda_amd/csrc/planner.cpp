@@ -404,19 +404,30 @@ int w4_epilogue_class(const Lowered &l, bool dry) {
   return W4_CLASS_NONE;
 }
 
-// All of K in LDS at once and more tiles than the two workgroups of every CU take in one go: those walk the tiles.  (Columns of
-// D at odd 16-bit addresses are left to the tile kernels, whose narrower stores mind them less: bf16 2459 x 351 x 80, 21
-// batches 23.3 us here, 19.4 there; with a pitch of 2462 or 2464 16 here and 18.5 there.)
-bool mfma_short_k(const Lowered &l, bool dry, uint32_t cus) {
+bool mfma_short_k_operands(const Lowered &l) {
   const GemmArgs &g = l.g;
-  if ((g.a_type != CUDA_R_16F && g.a_type != CUDA_R_16BF) || g.K > 128 || std::min(g.M, g.N) <= 64) return false;
-  if (g.beta_mode != SCALAR_VALUE || (!dry && g.beta_val.f != 0.0f) || (g.d_si != 1 ? g.d_si : g.d_sj) >= kNarrowPitch) return false;
+  if ((g.a_type != CUDA_R_16F && g.a_type != CUDA_R_16BF) || g.K > 128 || std::min(g.M, g.N) <= 64 || g.beta_mode != SCALAR_VALUE) return false;
   if (g.d_type != CUDA_R_16F && g.d_type != CUDA_R_16BF && g.d_type != CUDA_R_32F) return false;
-  const int64_t d_sq = g.d_si != 1 ? g.d_si : g.d_sj;
-  if (g.d_type != CUDA_R_32F && ((d_sq & 1) || (g.batch > 1 && (g.d_sb & 1)) || (!dry && (((uintptr_t)g.D) & 3)))) return false;
   // (its epilogue has one factor for all of D)
-  if (g.act != ACT_NONE || l.has_bias || g.alpha_mode == VECTOR_DEV || g.a_scale_mode == SCALE_OUTER_VEC || g.b_scale_mode == SCALE_OUTER_VEC) return false;
-  return (uint64_t)ceil_div(g.M, 128) * ceil_div(g.N, 128) * g.batch > 2 * (uint64_t)cus;
+  return g.act == ACT_NONE && !l.has_bias && g.alpha_mode != VECTOR_DEV && g.a_scale_mode != SCALE_OUTER_VEC && g.b_scale_mode != SCALE_OUTER_VEC;
+}
+
+// (Columns of D at odd 16-bit addresses are left to the tile kernels, whose narrower stores mind them less: bf16 2459 x 351 x 80, 21
+// batches 23.3 us here, 19.4 there; with a pitch of 2462 or 2464 16 here and 18.5 there.)
+bool mfma_short_k_output(const Lowered &l, bool dry) {
+  const GemmArgs &g = l.g;
+  // (the kernel's output: where the GELU input is kept, that matrix)
+  const bool aux = g.aux_mode == 1, swapped = g.d_si != 1;
+  const int64_t d_sq = aux ? (swapped ? g.aux_si : g.aux_sj) : swapped ? g.d_si : g.d_sj, d_sb = aux ? g.aux_sb : g.d_sb;
+  if (d_sq >= kNarrowPitch || (!dry && g.beta_val.f != 0.0f)) return false;
+  return g.d_type == CUDA_R_32F || !((d_sq & 1) || (g.batch > 1 && (d_sb & 1)) || (!dry && (((uintptr_t)g.D) & 3)));
+}
+
+// All of K in LDS at once and more tiles than the two workgroups of every CU take in one go: those walk the tiles.
+static uint32_t short_k_groups(uint32_t cus) { return std::max(2 * cus / 8 * 8, 8u); }
+static bool mfma_short_k(const Lowered &l, uint32_t cus) {
+  return mfma_short_k_operands(l) && mfma_short_k_output(l, true) &&
+         (uint64_t)ceil_div(l.g.M, 128) * ceil_div(l.g.N, 128) * l.g.batch > std::max(2 * cus, short_k_groups(cus));
 }
 
 // The 256 x 128 tile has a second form on eight waves with three stages, faster on grids of less than two rounds (int8, us:
@@ -452,9 +463,9 @@ static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t
     plan->workspace = 0;
     return;
   }
-  if (variant == 3 && mfma_short_k(l, true, cus)) {
+  if (variant == 3 && mfma_short_k(l, cus)) {
     plan->waves = (float)((double)plan->grid_x * plan->grid_y / (2.0 * cus));
-    plan->grid_x = std::max(2 * cus / 8 * 8, 8u);
+    plan->grid_x = short_k_groups(cus);
     plan->grid_y = 1;
     plan->workspace = 0;
     return;
@@ -513,7 +524,7 @@ constexpr double kPartialRound = 0.65;
 
 static int pick_mfma_variant(const Lowered &l, uint32_t cus) {
   const GemmArgs &g = l.g;
-  if (mfma_short_k(l, true, cus)) return 3;
+  if (mfma_short_k(l, cus)) return 3;
   const bool swapped = g.d_si != 1;
   const uint32_t np = swapped ? g.N : g.M, nq = swapped ? g.M : g.N;
   // cost = rounds of workgroups over the CUs x time of one tile; the tile shapes trade efficiency

@@ -14,7 +14,7 @@ constexpr MfmaVariant kMfmaVariants[] = {
     {256, 256, 2, 4, 128, 2, 0, 0},  // 0: 8 waves, 128x64 per wave
     {256, 256, 2, 2, 128, 2, 0, 0},  // 1: 4 waves, 128x128 per wave
     {256, 128, 2, 2, 128, 2, 0, 0},  // 2: 4 waves, 128x64 per wave; or 8 waves, 64x64 per wave, 3 stages (mfma_eight_waves())
-    {128, 128, 2, 2, 128, 2, 0, 0},  // 3: 4 waves, 64x64 per wave, two workgroups per CU; many tiles of a short K: mfma_short_k()
+    {128, 128, 2, 2, 128, 2, 0, 0},  // 3: 4 waves, 64x64 per wave, two workgroups per CU; many tiles of a short K: short_k_groups()
     {128, 128, 2, 2, 128, 3, 0, 0},  // 4: same tile, deeper ring, one workgroup per CU
     {128, 64, 2, 2, 128, 3, 0, 0},   // 5: 4 waves, 64x32 per wave: skinny problems
     {64, 64, 2, 2, 128, 3, 0, 0},    // 6: 4 waves, 32x32 per wave: problems of a few hundred tiles at most
@@ -108,8 +108,10 @@ uint32_t lower_problem(const zluda_gemm_problem *p, bool dry, Lowered *out);
 // pointers are not known yet and are taken to be zero / aligned)
 int w4_epilogue_class(const Lowered &l, bool dry);
 
-// whether a 16-bit problem runs on the short-K form of variant 3 (kernels/gemm_mfma_short.hpp); `dry` as above
-bool mfma_short_k(const Lowered &l, bool dry, uint32_t cus);
+// Whether the short-K form of variant 3 (kernels/gemm_mfma_short.hpp) takes a 16-bit problem: what the descriptors alone decide, and what
+// also depends on the call (`dry` as above).  A plan of variant 3 has that form where it has fewer workgroups than tiles.
+bool mfma_short_k_operands(const Lowered &l);
+bool mfma_short_k_output(const Lowered &l, bool dry);
 
 // The generic family's fast road: problems that only alignment or a K-contiguous row that ends inside a 16-byte piece keeps
 // from every MFMA family run on the transposing kernel (plan.variant = 1 + its variant, with its grid).  The family whose
