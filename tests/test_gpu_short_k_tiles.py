@@ -70,3 +70,21 @@ def test_a_kept_gelu_input_with_a_pitch_of_its_own(gpu_api, ldd, aux_ld):
     assert st == 0 and kernel == K.ZLUDA_KERNEL_MFMA_H16
     case.compare(got, ref, tol=1e-2)
     case.compare_aux(case.aux_got, case.aux_ref)
+
+
+@pytest.mark.parametrize("d", [K.CUDA_R_16BF, K.CUDA_R_32F])
+def test_zeros_have_the_sign_that_the_tile_kernels_give_them(gpu_api, d):
+    """a row of zeros in A, alpha -1"""
+    t = K.CUDA_R_16BF
+    case = Case(dict(a_type=t, b_type=t, d_type=d, c_type=d, compute_type=K.CUBLAS_COMPUTE_32F, scale_type=K.CUDA_R_32F, m=130, n=130, k=72, transa=1,
+                     batch=133, alpha=-1.0), 7950)
+    case.A.reshape(-1, 72)[::3] = 0
+    print("case", case.spec, flush=True)
+    bits = []
+    for v in (3, 6):
+        st, got, kernel, variant = case.run_gpu(gpu_api, forced_kernel=K.ZLUDA_KERNEL_MFMA_H16, forced_variant=v)
+        assert st == 0 and variant == v
+        bits.append(got.view("u4" if d == K.CUDA_R_32F else "u2").reshape(-1, 130))
+    zero = [(i % 130, b) for b in range(133) for i in range(130) if (b * 130 + i) % 3 == 0]
+    for i, b in zero:
+        assert (bits[0][b * 130:(b + 1) * 130, i] == bits[1][b * 130:(b + 1) * 130, i]).all()

@@ -34,7 +34,7 @@ __device__ __forceinline__ void short_store(__amdgpu_buffer_rsrc_t rs, int d_sq,
 #pragma unroll
       for (int h = 0; h < 2; h++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) x[h][e] = scale * acc[a + h][b][e] * sd;
+        for (int e = 0; e < 4; e++) x[h][e] = (scale * acc[a + h][b][e] + 0.0f) * sd;  // (no -0: the other epilogues add a bias of zero)
       if constexpr (DT == 2) {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
