@@ -489,3 +489,13 @@ def test_short_k_plans_have_fewer_workgroups_than_tiles_or_one_per_tile(api):
                     assert (p.grid_x, p.grid_y) == (tiles // batch, batch)
                     forms.add("tiles")
     assert forms == {"short", "tiles"}
+
+
+@pytest.mark.parametrize("m,n,k,batch,slab", [(428, 25, 4608, 64, False), (2592, 32, 4864, 32, False), (3440, 5, 7936, 4, False), (9000, 15, 8704, 3, False),
+                                              (944, 1, 10240, 18, False), (1608, 2, 10240, 16, False), (252, 2, 10496, 32, True), (552, 16, 23296, 32, True), (192, 5, 7936, 16, True), (380, 5, 24576, 2, True), (2024, 3, 19200, 2, True), (1268, 7, 9728, 4, True)])
+def test_mxfp4_batches_take_the_slab_decode_while_their_workgroups_fit(api, m, n, k, batch, slab):
+    st, p = plan(api, dict(MX, m=m, n=n, k=k, transa=1, batch=batch))
+    assert st == 0 and p.kernel == (K.ZLUDA_KERNEL_DECODE_W8A8 if slab else K.ZLUDA_KERNEL_MFMA_MXF4)
+    if slab:
+        assert p.grid_y == batch and (p.grid_x * batch <= 2 * 256 or k >= 11264)
+    assert plan(api, dict(MX, m=m, n=n, k=k, transa=1, batch=batch), K.ZLUDA_KERNEL_DECODE_W8A8)[0] == 0   # still there to be asked for

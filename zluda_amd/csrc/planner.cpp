@@ -721,6 +721,15 @@ uint32_t transposing_under_generic(const Lowered &l) {
   return family;
 }
 
+// Workgroups of the slab kernel per batch: at most one per CU (its LDS ring fills the CU), more only when the rows would not fit
+// into 4 blocks per workgroup otherwise.
+// (a short block costs its workgroup as many DMA instructions as a full one: the fewest rounds of blocks that
+// fit the CUs, shared out evenly -- 896 blocks on 256 CUs: 224 workgroups x 4)
+static uint32_t slab_groups(uint32_t rows, uint32_t cus) {
+  const uint32_t nrb = ceil_div(rows, 16);
+  return std::max(ceil_div(nrb, ceil_div(nrb, cus)), ceil_div(rows, 64));
+}
+
 static void fill_decode_plan(const Lowered &l, int variant, uint32_t cus, zluda_gemm_plan *plan) {
   const GemmArgs &g = l.g;
   const DecodeVariant &v = kDecodeVariants[variant];
@@ -732,11 +741,7 @@ static void fill_decode_plan(const Lowered &l, int variant, uint32_t cus, zluda_
   // workgroup per CU, two 4-wave ones.
   const uint32_t resident = v.stream == 2 ? cus : v.stream ? cus * (v.nw == 8 ? 1 : 2) : cus * (v.nw == 8 ? 2 : 4);
   uint32_t grid;
-  // slab kernel: at most one workgroup per CU (its LDS ring fills the CU), more only when the rows would not fit
-  // into 4 blocks per workgroup otherwise
-  // (a short block costs its workgroup as many DMA instructions as a full one: the fewest rounds of blocks that
-  // fit the CUs, shared out evenly -- 896 blocks on 256 CUs: 224 workgroups x 4)
-  if (v.stream == 2) grid = std::max(ceil_div(nrb, ceil_div(nrb, cus)), ceil_div(rows, 64));
+  if (v.stream == 2) grid = slab_groups(rows, cus);
   else if (v.stream) grid = std::min(nrb, resident);  // contiguous, balanced row ranges
   else grid = nrb <= resident ? nrb : ceil_div(nrb, ceil_div(nrb, resident));
   plan->variant = variant;
@@ -764,8 +769,13 @@ static int pick_decode_variant(const Lowered &l, uint32_t cus) {
   // 20480 x 8 x 5120 in 1.25 17.6 against 17.3)
   const uint64_t round = 64 * (uint64_t)cus;
   const bool many_rows = (mx && (uint64_t)rows * 10 >= (rows + round - 1) / round * round * 7) || (h16 && (K * 2 > 8192 || std::min(l.g.M, l.g.N) <= 8));
+  // (MXFP4 in batches: a workgroup fetches the activations for as few as 16 rows, and with more than two of them per CU the MFMA tiles
+  // are ahead unless K is long: us on slabs and on tiles, weights from memory, 428 x 25 x 4608, 64 batches, 1728 workgroups 40.4 and 17.0,
+  // 4012 x 16 x 9216, 8, 2008 48 and 30, 9000 x 15 x 8704, 3, 564 31.5 and 26.3; 252 x 2 x 10496, 32, 512 13.1 and 15.7, 828 x 8 x 12288, 8,
+  // 416 13.5 and 17.2, 192 x 5 x 7936, 16, 192 7.4 and 16.2; 15804 x 10 x 11520, 3, 741 51 and 66, 552 x 16 x 23296, 32, 1120 51 and 58)
+  const bool few_groups = !mx || l.g.batch == 1 || K >= 11264 || (uint64_t)slab_groups(rows, cus) * l.g.batch <= 2 * (uint64_t)cus;
   for (int v = 0; v < kNumDecodeVariants; v++)
-    if (kDecodeVariants[v].stream == 2 && decode_variant_ok(l, v) && (rows <= 64 * cus || many_rows) &&
+    if (kDecodeVariants[v].stream == 2 && decode_variant_ok(l, v) && (rows <= 64 * cus || many_rows) && few_groups &&
         !(kDecodeVariants[v].steps == 8 && rows > 32 * cus && !mx))
       return v;
   // the stream instantiation with the least cover that takes K
@@ -890,6 +900,8 @@ extern "C" uint32_t zluda_gemm_plan_problem(const zluda_gemm_problem *p, uint32_
   case ZLUDA_KERNEL_DECODE_W8A8: {
     int v = forced_variant >= 0 ? forced_variant : pick_decode_variant(l, cu_count);
     if (v >= kNumDecodeVariants) return CUBLAS_STATUS_INVALID_VALUE;
+    // (asked for by name: the variant that takes the problem, also where the rules above leave it to another family)
+    for (int n = 0; forced_variant < 0 && n < kNumDecodeVariants && !decode_variant_ok(l, v); n++) v = n;
     if (!decode_variant_ok(l, v)) return CUBLAS_STATUS_NOT_SUPPORTED;
     fill_decode_plan(l, v, cu_count, plan);
     break;
