@@ -339,11 +339,26 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
     so = so_next;
     kt++;
   };
-  while (kt + 2 <= KT) {
-    do_stage(std::integral_constant<int, 0>{});
-    do_stage(std::integral_constant<int, 1>{});
+  // The last stage has its fragments on the way already: it requests nothing and waits for nothing else.  (With the padding stage's
+  // round trip in front of its MFMAs the smallest problems took longer than on one sub-step ahead: fp8 9680 x 48 x 112, one
+  // stage, 4.5 us instead of 4.0.)
+  auto last_stage = [&](auto cur_c) {
+    constexpr int CUR = decltype(cur_c)::value;
+    if constexpr (MX) sc_cur = sc_nxt;
+    static_for<KS>([&](auto s_c) { mfma_all(fr[CUR][decltype(s_c)::value], sc_cur, s_c); });
+  };
+  using E = std::integral_constant<int, 0>;
+  using O = std::integral_constant<int, 1>;
+  while (kt + 2 < KT) {
+    do_stage(E{});
+    do_stage(O{});
   }
-  if (kt < KT) do_stage(std::integral_constant<int, 0>{});
+  if (kt + 1 < KT) {
+    do_stage(E{});
+    last_stage(O{});
+  } else if (kt < KT) {
+    last_stage(E{});
+  }
   } else {
   Frags fa, fb;
   load_frags(0, std::integral_constant<int, 0>{}, fa);
