@@ -499,3 +499,19 @@ def test_mxfp4_batches_take_the_slab_decode_while_their_workgroups_fit(api, m, n
     if slab:
         assert p.grid_y == batch and (p.grid_x * batch <= 2 * 256 or k >= 11264)
     assert plan(api, dict(MX, m=m, n=n, k=k, transa=1, batch=batch), K.ZLUDA_KERNEL_DECODE_W8A8)[0] == 0   # still there to be asked for
+
+
+BF = dict(a_type=K.CUDA_R_16BF, b_type=K.CUDA_R_16BF, d_type=K.CUDA_R_16BF, compute_type=K.CUBLAS_COMPUTE_32F, scale_type=K.CUDA_R_32F)
+
+
+@pytest.mark.parametrize("spec,m,n,k,slab", [
+    (BF, 16384, 8, 1408, True), (BF, 16400, 8, 1408, False), (BF, 49300, 4, 1536, False), (BF, 18000, 8, 2048, True), (BF, 18000, 9, 2048, False), (BF, 18000, 4, 2304, False),
+    (BF, 20480, 4, 4096, True), (BF, 20480, 4, 4088, True), (BF, 16400, 4, 2560, True), (BF, 26000, 4, 2552, False), (BF, 37888, 8, 3584, True), (BF, 28672, 16, 8192, True),
+    (MX, 16384, 4, 4352, True), (MX, 28672, 4, 4352, False), (MX, 28672, 4, 6144, True), (MX, 20480, 4, 8192, False), (MX, 57344, 16, 8192, True), (MX, 57344, 32, 8192, True),
+    (MX, 28672, 24, 6144, False), (MX, 43000, 4, 12288, True), (MX, 43000, 4, 9216, False)])
+def test_slab_decode_beyond_64_rows_per_cu(api, spec, m, n, k, slab):
+    st, p = plan(api, dict(spec, m=m, n=n, k=k, transa=1))
+    assert st == 0 and (p.kernel == K.ZLUDA_KERNEL_DECODE_W8A8) == slab
+    if slab:
+        assert p.grid_x * 64 >= m and p.block in (256, 512)
+    assert plan(api, dict(spec, m=m, n=n, k=k, transa=1), K.ZLUDA_KERNEL_DECODE_W8A8)[0] == 0

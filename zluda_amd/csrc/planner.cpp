@@ -759,23 +759,33 @@ static int pick_decode_variant(const Lowered &l, uint32_t cus) {
   // (two token blocks on one unit per slab, variant 20, only up to two blocks of rows per CU: 4096 x 32 x 4096
   // 8.9 us against 10.0, but 14336 x 32 x 4096 18.1 against 16.7; with two units, variant 17, it wins
   // throughout: 8192 x 32 x 8192 15.4 against 22.0)
-  // (16-bit weights, which have no other streaming form, also beyond 64 rows per CU, in more than one round of workgroups: with up to
-  // 8 tokens -- bf16, us, against the best MFMA tiles: 37888 x 8 x 3584 49 and 55, 28672 x 8 x 4096 38 and 47, 19000 x 4 x 2048 18.5 and
-  // 20.1 --, with more where K is long: 28672 x 16 x 8192 80 and 99)
   const uint32_t rows = (uint32_t)std::max(l.g.M, l.g.N);
   const bool h16 = l.g.a_type == CUDA_R_16F || l.g.a_type == CUDA_R_16BF;
   const bool mx = l.g.a_type == CUDA_R_4F_E2M1;
-  // (MXFP4 beyond 64 rows per CU where the rounds are 70 % full: 57344 x 8 x 8192 in 3.5 rounds 45 us against 59 on MFMA tiles, but
-  // 20480 x 8 x 5120 in 1.25 17.6 against 17.3)
+  // Beyond 64 rows per CU the workgroups take more than one round, each of which costs what a shape's whole cover of K does, however
+  // little of it the problem has.  (us on slabs and on the best MFMA tiles, weights from memory.  A loop over one matrix of less than
+  // 200 MB finds it in the memory-side cache, which the tiles gain more from: 20480 x 4 x 4096 33 and 26, 32768 x 4 x 3072 33 and 30.)
+  //   16-bit weights: with K beyond 4096 always (bf16 28672 x 16 x 8192 80 and 99).  Up to 8 tokens, K that fills the cover (18000 x 4 x 2048
+  //   18.6 and 21.3, 20480 x 4 x 4096 33.7 and 40.2), or five eighths of the 8-wave one (26000 x 4 x 2560 26.2 and 28.4, 18000 x
+  //   4 x 3584 29.9 and 32.5, 37888 x 4 x 3584 48.3 and 59.4; but 18000 x 4 x 2304 23.4 and 21.5, 50000 x 4 x 1408 33.9 and 29.3).
+  //   MXFP4: rounds that are 70 % full (57344 x 4 x 8192 in 3.5 42.7 and 56.5, but 20480 x 8 x 5120 in 1.25 17.6 and 17.3) and K that fills three
+  //   quarters of the cover (28672 x 4 x 6144 19.0 and 21.2, 43000 x 4 x 12288 48.8 and 67.6; but 28672 x 4 x 4352 17.1 and 15.3), all of it with two
+  //   token blocks (43000 x 24 x 8192 40.7 and 54.2; but 28672 x 24 x 5120 19.9 and 18.6).
   const uint64_t round = 64 * (uint64_t)cus;
-  const bool many_rows = (mx && (uint64_t)rows * 10 >= (rows + round - 1) / round * round * 7) || (h16 && (K * 2 > 8192 || std::min(l.g.M, l.g.N) <= 8));
+  auto rounds_ok = [&](int v) {
+    const int cover = kDecodeVariants[v].nw * kDecodeVariants[v].steps * 64, tokens = std::min(l.g.M, l.g.N);
+    const int64_t kb = (int64_t)K * type_bits(l.g.a_type) / 8;
+    if (rows <= round) return true;
+    if (mx) return (uint64_t)rows * 10 >= (rows + round - 1) / round * round * 7 && (tokens > 16 ? kb == cover : kb * 4 >= cover * 3);
+    return h16 && (kb > 8192 || (tokens <= 8 && (kb == cover || kb * 8 >= 8192 * 5)));
+  };
   // (MXFP4 in batches: a workgroup fetches the activations for as few as 16 rows, and with more than two of them per CU the MFMA tiles
   // are ahead unless K is long: us on slabs and on tiles, weights from memory, 428 x 25 x 4608, 64 batches, 1728 workgroups 40.4 and 17.0,
   // 4012 x 16 x 9216, 8, 2008 48 and 30, 9000 x 15 x 8704, 3, 564 31.5 and 26.3; 252 x 2 x 10496, 32, 512 13.1 and 15.7, 828 x 8 x 12288, 8,
   // 416 13.5 and 17.2, 192 x 5 x 7936, 16, 192 7.4 and 16.2; 15804 x 10 x 11520, 3, 741 51 and 66, 552 x 16 x 23296, 32, 1120 51 and 58)
   const bool few_groups = !mx || l.g.batch == 1 || K >= 11264 || (uint64_t)slab_groups(rows, cus) * l.g.batch <= 2 * (uint64_t)cus;
   for (int v = 0; v < kNumDecodeVariants; v++)
-    if (kDecodeVariants[v].stream == 2 && decode_variant_ok(l, v) && (rows <= 64 * cus || many_rows) && few_groups &&
+    if (kDecodeVariants[v].stream == 2 && decode_variant_ok(l, v) && rounds_ok(v) && few_groups &&
         !(kDecodeVariants[v].steps == 8 && rows > 32 * cus && !mx))
       return v;
   // the stream instantiation with the least cover that takes K
