@@ -46,8 +46,7 @@ static int data_after(const std::vector<Ins> &log, int stage) {
 
 // gemm_mfma_pipe_kernel: prologue, then per stage [reads of the next stage's scales] wait, barrier, scale instructions,
 // data of stage kt + nstage
-static void check_pipe(int variant, bool mx, int ks) {
-  const MfmaVariant &v = kMfmaVariants[variant];
+static void check_pipe(const MfmaVariant &v, int variant, bool mx, int ks) {
   const PipeCounts c = pipe_counts(mx, v.bp, v.bq, v.wp, v.wq, v.bkb, v.stages);
   if ((v.stages - 1) * c.nload >= 64) fail("vmcnt range", variant, mx, 0, 0, 0);
   for (int KT = 1; KT <= 3 * c.ch + v.stages + 2; KT++)
@@ -167,15 +166,70 @@ static void check_tr(int esz) {
   }
 }
 
+// gemm_mfma_short_kernel: runs of tiles of every length and start in small grids, whose last tiles along P and Q hang over the ends or
+// not.  Counted by hand here: a wave's 64 x 64 part of a 128 x 128 tile has 16 tiles of 16 x 16 and stores two of them (16-bit D) or one
+// (32 bits) with an instruction; a panel is 128 rows in chunks of 128 bytes, 32 rows per instruction of the four waves.
+static void check_short(int chunks, bool wide) {
+  const ShortCounts c = short_counts(chunks);
+  enum { PANEL, STORE, LOOSE };  // LOOSE: stores that can be dropped, and retire early
+  const int panel_ins = chunks * 128 / 32, store_ins = wide ? 16 : 8;
+  if (short_wait_n(c, 0) >= 64) fail("vmcnt range", -2, 0, 0, 0, 0);
+  long widest = 0;
+  for (int tp = 1; tp <= 3; tp++)
+    for (int tq = 1; tq <= 4; tq++)
+      for (int edges = 0; edges < 4; edges++)
+        for (int first = 0; first < 2 * tp * tq; first++)
+          for (int count = 1; count <= 9; count++) {
+            std::vector<Ins> log;
+            ShortPos use{first / tq % tp, first % tq, first / (tp * tq), count, true}, ask = use;
+            int asked = 0, read = 0, panels = 0, st1 = 0, st2 = 0, tiles = 0, row = -1;  // (row of tiles whose P panel is in registers)
+            auto request = [&]() {
+              if (ask.left == 0) return;
+              for (int i = 0; i < panel_ins; i++) log.push_back(Ins{PANEL, asked});
+              asked++; panels++;
+              short_advance(ask, tp, tq);
+            };
+            request(); request();
+            while (use.left > 0) {
+              const int which = short_wait(c, panels == 2, st1 + st2), n = short_wait_n(c, which);
+              // in order: everything but the loose stores; those may be gone already, so only the others count as outstanding
+              int younger = 0;
+              for (size_t i = log.size(); i-- > 0 && !(log[i].kind == PANEL && log[i].id == read);) younger += log[i].kind != LOOSE;
+              if (n > younger) fail("short K: a panel may still be in flight", -2, 0, chunks, read, count);
+              // the waits are as lax as the kernel has them: between whole tiles of a run nothing younger is waited for
+              if (which == 0) widest++;
+              if (!wide && panels == 2 && st1 + st2 == 2 * store_ins && n != younger) fail("short K: a needless wait", -2, 0, chunks, read, count);
+              checked++;
+              const ShortPos now = use;
+              read++; panels--;
+              request();
+              short_advance(use, tp, tq);
+              st2 = st1;
+              st1 = 0;
+              if (now.p_due) { row = now.bt * tp + now.p; continue; }
+              if (now.bt * tp + now.p != row || row * tq + now.q != first + tiles) fail("short K: another tile's turn", -2, 0, chunks, tiles, count);
+              const bool whole = !((edges & 1) && now.p == tp - 1) && !((edges & 2) && now.q == tq - 1);
+              for (int i = 0; i < store_ins; i++) log.push_back(Ins{whole ? STORE : LOOSE, 0});
+              if (whole) st1 = c.stores;
+              tiles++;
+            }
+            if (tiles != count || asked != read) fail("short K: a run does not hold its tiles", -2, 0, chunks, tiles, count);
+          }
+  if (widest == 0) fail("short K: the widest wait is never reached", -2, 0, chunks, 0, 0);
+}
+
 int main() {
   for (int variant = 0; variant < kNumMfmaVariants; variant++) {
     const MfmaVariant &v = kMfmaVariants[variant];
     if (v.w4) continue;  // every wait of the four-wave kernel is vmcnt(0) (checked on its source)
     if (v.m16) { check_pipe16(variant); continue; }
     // sub-steps per stage: 32 K bytes each, fp8 64; with and without MX scales where the variant serves MXFP4
-    for (int ks : {v.bkb / 32, v.bkb / 64}) check_pipe(variant, false, ks);
-    if (variant < kNumMfmaVariants32) check_pipe(variant, true, v.bkb / 32);
+    for (int ks : {v.bkb / 32, v.bkb / 64}) check_pipe(v, variant, false, ks);
+    if (variant < kNumMfmaVariants32) check_pipe(v, variant, true, v.bkb / 32);
   }
+  for (int ks : {2, 4}) check_pipe(kMfmaEightWaves, 2, false, ks);
+  for (int chunks : {1, 2})
+    for (bool wide : {false, true}) check_short(chunks, wide);
   for (int v : {1, 3}) check_pipe16_mc(kTrVariants[v].bp, kTrVariants[v].bq, kTrVariants[v].wp, kTrVariants[v].wq);
   for (int esz : {1, 2, 4}) check_tr(esz);
   printf("%ld waits checked\n", checked);

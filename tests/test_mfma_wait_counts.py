@@ -40,6 +40,11 @@ MUTATIONS = [
     ("c.wait_prologue = c.nload;", "c.wait_prologue = c.nload - 1;"),
     ("c.wait_stage = 0;", "c.wait_stage = 1;"),
     ("? kl - 2 :", "? kl - 1 :"),
+    ("return ShortCounts{chunks * 4, 8};", "return ShortCounts{chunks * 4 + 1, 8};"),
+    ("return ShortCounts{chunks * 4, 8};", "return ShortCounts{chunks * 4, 9};"),
+    ("return which == 0 ? c.panel + 2 * c.stores :", "return which == 0 ? c.panel + 2 * c.stores + 1 :"),
+    ("const int younger = (panel_behind ? c.panel : 0) + counted_stores;", "const int younger = c.panel + counted_stores;"),
+    ("    c.p_due = true;\n", ""),
     ("c.ls = mx ? (c.sparts + c.nwv * (c.ch - nstage) - 1) / (c.nwv * (c.ch - nstage)) : 0;",
      "c.ls = mx ? (c.sparts + c.nwv * (c.ch - nstage) - 1) / (c.nwv * (c.ch - nstage)) - 1 : 0;"),
 ]
@@ -68,8 +73,11 @@ def test_the_kernels_take_their_waits_from_the_checked_header():
     assert set(waits("gemm_mfma_w4.hpp")) == {"0"}          # the four-wave kernel never counts
     tr = open(os.path.join(KERNELS, "gemm_mfma_tr.hpp")).read()
     assert "tail_from = tr_tail_from(" in tr
+    short = open(os.path.join(KERNELS, "gemm_mfma_short.hpp")).read()
+    assert re.findall(r'"s_waitcnt vmcnt\(%0\)[^"]*" ::"n"\(([^)]*\))\)', short) == ["short_wait_n(SC, %d)" % i for i in range(4)]
+    assert "switch (short_wait(SC, panels == 2, st1 + st2))" in short
     # no other counted wait hides in inline assembly of these kernels
-    for name in ("gemm_mfma_pipe.hpp", "gemm_mfma_pipe16.hpp", "gemm_mfma_w4.hpp", "gemm_mfma_tr.hpp"):
+    for name in ("gemm_mfma_pipe.hpp", "gemm_mfma_pipe16.hpp", "gemm_mfma_w4.hpp", "gemm_mfma_tr.hpp", "gemm_mfma_short.hpp"):
         src = open(os.path.join(KERNELS, name)).read()
         for n in re.findall(r'"s_waitcnt vmcnt\(([^)]*)\)', src):   # (inside assembly strings; comments may say vmcnt(n))
             assert n in ("0", "%0"), (name, n)

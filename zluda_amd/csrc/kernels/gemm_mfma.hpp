@@ -92,14 +92,6 @@ __device__ __forceinline__ void buffer_store_b128_guarded(v4i data, __amdgpu_buf
   asm volatile("s_nop 1" : "+v"(data)::"memory");
 }
 
-// The same guard for a 64-bit store.  The corruption was only ever seen with the 128-bit form, but nothing known about
-// it says the narrower store reads its data registers any earlier, and a wait state per store is not measurable in the
-// epilogues that use it.
-__device__ __forceinline__ void buffer_store_b64_guarded(v2i data, __amdgpu_buffer_rsrc_t rs, int voff, int soff) {
-  __builtin_amdgcn_raw_buffer_store_b64(data, rs, voff, soff, 0);
-  asm volatile("s_nop 1" : "+v"(data)::"memory");
-}
-
 struct MfmaParams {
   GemmArgs g;
   int32_t swapped;           // P = op(B)^T rows, Q = op(A) rows
@@ -108,6 +100,7 @@ struct MfmaParams {
   // split-K (splits > 1): workgroup z of gridDim.z handles stages [z * split_stages, ...) of K and
   // writes its raw partial tile to ws[(z * batch + bt)][tiles_q * BQ][tiles_p * BP] (int32 / fp32)
   int32_t splits, split_stages;
+  int32_t groups;            // workgroups that walk the tiles (gemm_mfma_short.hpp)
   void *ws;
 };
 

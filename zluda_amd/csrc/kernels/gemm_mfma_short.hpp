@@ -80,8 +80,8 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_short_kernel(MfmaParams prm)
   constexpr int KS = 2;                             // MFMAs per fragment pair and chunk
   constexpr int CHUNK_V4 = BP * CPR, SLOT_V4 = NC * CHUNK_V4;
   constexpr int LD = BP / 32;                       // DMA instructions per wave and chunk: 8 rows each, 32 per pass of the workgroup
-  constexpr int kPanel = NC * LD;                   // per wave and panel
-  constexpr int kStores = TP * TQ / 2;              // per wave and whole tile, at least: 16-bit D; D of 32 bits has twice as many
+  constexpr ShortCounts SC = short_counts(NC);      // (mfma_wait_counts.hpp, where a host program replays the waits)
+  static_assert(SC.panel == NC * LD && SC.stores == TP * TQ / 2, "what a wave issues");
   struct Frag { v4i k[KS]; };
 
   __shared__ v4i lds[2 * SLOT_V4];
@@ -101,10 +101,9 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_short_kernel(MfmaParams prm)
   // workgroups are blockIdx.x mod 8), shared out evenly over its workgroups.  Neighbours have neighbouring tiles of P at about the
   // same Q, so the lines that two tiles of D share (a pitch that is no multiple of 128 bytes) meet in the XCD's L2: runs along
   // P took 58 us for bf16 1000 x 1000 x 128, 64 batches, runs along Q take 51.
-  const uint32_t total = (uint32_t)(prm.tiles_p * prm.tiles_q) * (uint32_t)g.batch, groups = (uint32_t)prm.split_stages >> 3;
+  const uint32_t total = (uint32_t)(prm.tiles_p * prm.tiles_q) * (uint32_t)g.batch, groups = (uint32_t)prm.groups >> 3;
   const uint32_t x = blockIdx.x & 7, lo = (uint32_t)((uint64_t)total * x >> 3), cnt = (uint32_t)((uint64_t)total * (x + 1) >> 3) - lo;
-  struct Pos { int p, q, bt, left; bool p_due; };  // the next tile, how many are left, and whether its P panel comes first
-  Pos use;
+  ShortPos use;
   {
     const uint32_t j = blockIdx.x >> 3, at = (uint32_t)((uint64_t)cnt * j / groups), end = (uint32_t)((uint64_t)cnt * (j + 1) / groups);
     const uint32_t id = lo + at, row = id / (uint32_t)prm.tiles_q;
@@ -114,22 +113,11 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_short_kernel(MfmaParams prm)
     use.left = __builtin_amdgcn_readfirstlane((int)(end - at));
     use.p_due = true;
   }
-  // to the panel after this one
-  auto advance = [&](Pos &c) {
-    if (c.p_due) { c.p_due = false; return; }
-    c.left--;
-    if (++c.q == prm.tiles_q) {
-      c.q = 0;
-      c.p_due = true;
-      if (++c.p == prm.tiles_p) { c.p = 0; c.bt++; }
-    }
-  };
-
   const int drow = wave * 8 + lane / CPR;  // (passes advance by 32 rows: same swizzle)
   const int dcg = (lane % CPR) ^ swz(drow);
   // the lanes of the last chunk past the end of K read zeros; every instruction has lanes that are not (K is whole 16-byte pieces)
   const int oob_last = dcg * 16 < Kbytes - (NC - 1) * 128 ? 0 : (int)0x80000000;
-  auto issue_panel = [&](const Pos &c, int slot) {
+  auto issue_panel = [&](const ShortPos &c, int slot) {
     const uint8_t *base = c.p_due ? Pb + p_sb * c.bt : Qb + q_sb * c.bt;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 0x80000000, 0x00020000);
     const int row0 = c.p_due ? c.p * BP : c.q * BQ, last = (c.p_due ? NP : NQ) - 1, ld = c.p_due ? ldp : ldq;
@@ -165,26 +153,27 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_short_kernel(MfmaParams prm)
   // (the host sends only problems with one factor for all of D)
   const EpilogueScalars sc(g);
   const float scale = sc.alpha_s * sc.sa_s * sc.sb_s;
-  Pos ask = use;  // the next panel to request
+  ShortPos ask = use;  // the next panel to request
   int panels = 0;  // of those requested, not read yet
   for (int s = 0; s < 2; s++)
-    if (ask.left > 0) { issue_panel(ask, s); advance(ask); panels++; }
+    if (ask.left > 0) { issue_panel(ask, s); short_advance(ask, prm.tiles_p, prm.tiles_q); panels++; }
   int slot = 0, st1 = 0, st2 = 0;  // stores that count, of the tile before and the one before that
   while (use.left > 0) {
     // wait for the panel; younger: st2, the next panel, st1
-    const int younger = (panels == 2 ? kPanel : 0) + st1 + st2;
-    if (younger == kPanel + 2 * kStores) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kPanel + 2 * kStores) : "memory");
-    else if (younger >= kPanel + kStores) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kPanel + kStores) : "memory");
-    else if (younger >= kPanel) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kPanel) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    const Pos now = use;
+    switch (short_wait(SC, panels == 2, st1 + st2)) {
+    case 0: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(short_wait_n(SC, 0)) : "memory"); break;
+    case 1: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(short_wait_n(SC, 1)) : "memory"); break;
+    case 2: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(short_wait_n(SC, 2)) : "memory"); break;
+    default: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(short_wait_n(SC, 3)) : "memory");
+    }
+    const ShortPos now = use;
     if (now.p_due) load_frags(slot, wp * WTP, pf);
     else load_frags(slot, wq * WTQ, qf);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     panels--;
-    if (ask.left > 0) { issue_panel(ask, slot); advance(ask); panels++; }
+    if (ask.left > 0) { issue_panel(ask, slot); short_advance(ask, prm.tiles_p, prm.tiles_q); panels++; }
     slot ^= 1;
-    advance(use);
+    short_advance(use, prm.tiles_p, prm.tiles_q);
     st2 = st1;
     st1 = 0;
     if (now.p_due) continue;
@@ -222,7 +211,7 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_short_kernel(MfmaParams prm)
     else if (g.d_type == CUDA_R_16F) { ZLUDA_SHORT_STORE(1) }
     else { ZLUDA_SHORT_STORE(2) }
 #undef ZLUDA_SHORT_STORE
-    if (p0 + BP <= NP && q0 + BQ <= NQ) st1 = kStores;
+    if (p0 + BP <= NP && q0 + BQ <= NQ) st1 = SC.stores;
   }
 }
 

@@ -82,4 +82,35 @@ constexpr int tr_tail_from(int kbytes, int esz) {
   return (kbytes & 63) || esz == 2 ? kl - 2 : 0x7fffffff;
 }
 
+// gemm_mfma_short.hpp: panels (128 rows of P or Q, all of K) come through a ring of two LDS slots in the order in which they are
+// used: a run of tiles along Q needs a panel of Q each, behind one of P where the run starts or turns to the next tile of P.
+// In flight at the wait for a panel, younger than it: the panel behind it (if the run has one), and the stores of the tile
+// before and of the one before that, as far as those can be counted -- the stores of a tile that hangs over an end may be
+// dropped and retire early.
+struct ShortPos { int p, q, bt, left; bool p_due; };  // the next tile, how many are left, and whether its P panel comes first
+constexpr void short_advance(ShortPos &c, int tiles_p, int tiles_q) {  // to the panel after this one
+  if (c.p_due) { c.p_due = false; return; }
+  c.left--;
+  if (++c.q == tiles_q) {
+    c.q = 0;
+    c.p_due = true;
+    if (++c.p == tiles_p) { c.p = 0; c.bt++; }
+  }
+}
+
+struct ShortCounts {
+  int panel;   // DMA instructions per wave and panel
+  int stores;  // counted stores per wave and whole tile: those of a 16-bit D; one of 32 bits has twice as many
+};
+constexpr ShortCounts short_counts(int chunks) { return ShortCounts{chunks * 4, 8}; }
+
+// The kernel's waits, N = short_wait_n(c, 0 .. 3); the one for a panel is the first whose N does not exceed what is younger than it
+constexpr int short_wait_n(const ShortCounts &c, int which) {
+  return which == 0 ? c.panel + 2 * c.stores : which == 1 ? c.panel + c.stores : which == 2 ? c.panel : 0;
+}
+constexpr int short_wait(const ShortCounts &c, bool panel_behind, int counted_stores) {
+  const int younger = (panel_behind ? c.panel : 0) + counted_stores;
+  return younger >= short_wait_n(c, 0) ? 0 : younger >= short_wait_n(c, 1) ? 1 : younger >= short_wait_n(c, 2) ? 2 : 3;
+}
+
 } // namespace zluda_amd

@@ -66,7 +66,7 @@ uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws,
       prm.swapped = plan.swapped;
       prm.tiles_p = (np + 255) / 256; prm.tiles_q = (nq + 255) / 256;
       prm.group_p = 8;
-      prm.splits = 1; prm.split_stages = 0; prm.ws = nullptr;
+      prm.splits = 1; prm.split_stages = 0; prm.groups = 0; prm.ws = nullptr;
       return plan.kernel == ZLUDA_KERNEL_MFMA_I8     ? launch_mfma_w4_i8(prm, epi, plan.grid_x, s)
              : plan.kernel == ZLUDA_KERNEL_MFMA_MXF4 ? launch_mfma_w4_mxf4(prm, epi, plan.grid_x, s)
              : plan.kernel == ZLUDA_KERNEL_MFMA_H16  ? (l.g.a_type == CUDA_R_16BF ? launch_mfma_w4_bf16(prm, epi, plan.grid_x, s)
@@ -85,12 +85,12 @@ uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws,
   prm.tiles_p = (np + v.bp - 1) / v.bp;
   prm.tiles_q = (nq + v.bq - 1) / v.bq;
   prm.group_p = 8;
-  prm.splits = 1; prm.split_stages = 0; prm.ws = nullptr;
+  prm.splits = 1; prm.split_stages = 0; prm.groups = 0; prm.ws = nullptr;
   // The short-K form: fewer workgroups than tiles, for which the plan alone counts (it may have been made for another number of CUs).
   if (plan.variant == 3 && plan.kernel == ZLUDA_KERNEL_MFMA_H16 && plan.grid_y == 1 && plan.grid_z == 1 && plan.grid_x > 0 && (plan.grid_x & 7) == 0 &&
       plan.grid_x < (uint64_t)prm.tiles_p * prm.tiles_q * l.g.batch && mfma_short_k_operands(l)) {
     if (mfma_short_k_output(l, false)) {
-      prm.split_stages = (int32_t)plan.grid_x;
+      prm.groups = (int32_t)plan.grid_x;
       return launch_mfma_short(prm, l.g.a_type == CUDA_R_16BF, plan.grid_x, s);
     }
     // (a beta that is not zero or a D off a dword, known only now, runs with one tile per workgroup)
@@ -148,7 +148,7 @@ uint32_t launch_tr(const Lowered &l, const zluda_gemm_plan &plan, void *ws, uint
   prm.tiles_p = (np + v.bp - 1) / v.bp;
   prm.tiles_q = (nq + v.bq - 1) / v.bq;
   prm.group_p = 8;
-  prm.splits = 1; prm.split_stages = 0; prm.ws = nullptr;
+  prm.splits = 1; prm.split_stages = 0; prm.groups = 0; prm.ws = nullptr;
   if ((uint32_t)(prm.tiles_p * prm.tiles_q) != plan.grid_x) return CUBLAS_STATUS_INVALID_VALUE;
   // the same tiles, transposed by the LDS reads: 128 K bytes per stage
   const bool lds_reads = tr_lds_reads(l, (int)plan.variant, (uint64_t)plan.grid_x * plan.grid_y * std::max(plan.grid_z, 1u), plan.grid_z,

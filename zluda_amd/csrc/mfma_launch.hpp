@@ -24,6 +24,8 @@ inline uint32_t launch_mfma_variant(const MfmaParams &prm, const zluda_gemm_plan
   case 2:  // (two forms of one tile, see mfma_eight_waves())
     static_assert(kMfmaVariants[2].bp == 256 && kMfmaVariants[2].bq == 128 && kMfmaVariants[2].wp == 2 && kMfmaVariants[2].wq == 2 &&
                   kMfmaVariants[2].bkb == 128 && kMfmaVariants[2].stages == 2 && !kMfmaVariants[2].m16, "variant table mismatch");
+    static_assert(kMfmaEightWaves.bp == 256 && kMfmaEightWaves.bq == 128 && kMfmaEightWaves.wp == 4 && kMfmaEightWaves.wq == 2 &&
+                  kMfmaEightWaves.bkb == 128 && kMfmaEightWaves.stages == 3, "variant table mismatch");
     if (plan.block != 512) return launch_kernel(gemm_mfma_pipe_kernel<KIND, FQ, FP, 256, 128, 2, 2, 128, 2>, grid, dim3(256), s, prm);
     if constexpr (KIND == KIND_MXF4) return CUBLAS_STATUS_INVALID_VALUE;
     else return launch_kernel(gemm_mfma_pipe_kernel<KIND, FQ, FP, 256, 128, 4, 2, 128, 3>, grid, dim3(512), s, prm);
@@ -60,7 +62,7 @@ uint32_t launch_mfma_f8(const MfmaParams &prm, const zluda_gemm_plan &plan, int 
 uint32_t launch_mfma_mxf4(const MfmaParams &prm, const zluda_gemm_plan &plan, hipStream_t s);
 uint32_t launch_mfma_h16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool bf16, hipStream_t s);
 uint32_t launch_mfma_f32(const MfmaParams &prm, const zluda_gemm_plan &plan, hipStream_t s);
-// variant 3 in the form of kernels/gemm_mfma_short.hpp; `grid` workgroups, prm.split_stages the same number
+// variant 3 in the form of kernels/gemm_mfma_short.hpp; `grid` workgroups, prm.groups the same number
 uint32_t launch_mfma_short(const MfmaParams &prm, bool bf16, uint32_t grid, hipStream_t s);
 // the four-wave persistent kernel (variant 11; kernels/gemm_mfma_w4.hpp), `epi` = W4_CLASS_* of planner.hpp, `grid` workgroups
 uint32_t launch_mfma_w4_i8(const MfmaParams &prm, int epi, uint32_t grid, hipStream_t s);

@@ -471,9 +471,9 @@ static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t
     return;
   }
   const bool eight = variant == 2 && mfma_eight_waves(l, (uint64_t)tp * tq * g.batch, cus);
-  if (eight) plan->block = 512;
+  if (eight) plan->block = kMfmaEightWaves.wp * kMfmaEightWaves.wq * 64;
   // data stages, plus two chunks of 32 scale bytes per tile row for MXFP4
-  const uint32_t lds = (uint32_t)(eight ? 3 : v.stages) * (v.bp + v.bq) * v.bkb + (l.g.a_type == CUDA_R_4F_E2M1 ? 64u * (v.bp + v.bq) : 0u);
+  const uint32_t lds = (uint32_t)(eight ? kMfmaEightWaves : v).stages * (v.bp + v.bq) * v.bkb + (l.g.a_type == CUDA_R_4F_E2M1 ? 64u * (v.bp + v.bq) : 0u);
   const uint32_t per_cu = std::max(1u, std::min(160u * 1024u / lds, 2048u / plan->block));
   plan->waves = (float)plan->grid_x * plan->grid_y / (float)(cus * per_cu);
   plan->workspace = 0;

@@ -30,6 +30,8 @@ constexpr MfmaVariant kMfmaVariants[] = {
     // bf16 operands with the epilogues w4_epilogue_class() admits; no split along K): 5-20 % less time than variant 8 / 0
     {256, 256, 2, 2, 128, 2, 1, 1},  // 11
 };
+// variant 2's second form (plan.block = 512), where mfma_eight_waves() says so
+constexpr MfmaVariant kMfmaEightWaves = {256, 128, 4, 2, 128, 3, 0, 0};
 constexpr int kNumMfmaVariants32 = 8;  // the first ones, on the 32x32 shapes: what MXFP4 has
 constexpr int kNumMfmaVariantsH16 = 12;  // f16 / bf16: all of them
 constexpr int kNumMfmaVariants = sizeof(kMfmaVariants) / sizeof(kMfmaVariants[0]);
