@@ -353,11 +353,11 @@ class Case:
         finally:
             call.close()
 
-    def run_gpu_plan(self, api, forced_kernel, forced_variant=-1, grid_x=None):
+    def run_gpu_plan(self, api, forced_kernel, forced_variant=-1, grid_x=None, edit=None, workspace_bytes=0):
         """The same problem through the inner launch layer (zluda_gemm_plan_problem + zluda_gemm_launch), with the
         plan's grid_x overridden when given: a smaller grid makes every workgroup of the row-streaming decode
-        kernel walk several 16-row blocks without needing a matrix of tens of thousands of rows.
-        Returns (status, D storage, plan)."""
+        kernel walk several 16-row blocks without needing a matrix of tens of thousands of rows.  `edit` gets the
+        plan for any other change.  Returns (status, D storage, plan)."""
         import torch
         keep, ptr, dt = self.upload()
         host = {"alpha": self.alpha.ctypes.data, "beta": self.beta.ctypes.data}
@@ -365,12 +365,17 @@ class Case:
         ptrs["alpha"] = ptr["alpha_dev"] if self.alpha_on_device else host["alpha"]
         ptrs["beta"] = ptr["beta_dev"] if self.beta_on_device else host["beta"]
         p = self.problem(ptrs)
+        if workspace_bytes:
+            ws = torch.empty(workspace_bytes, dtype=torch.uint8, device="cuda:0")
+            p.workspace, p.workspace_size = ws.data_ptr(), workspace_bytes
         plan = abi.zluda_gemm_plan()
         st = api.zluda_gemm_plan_problem(C.byref(p), forced_kernel, forced_variant, api.zluda_gemm_device_cu_count(), C.byref(plan))
         if st:
             return st, None, plan
         if grid_x is not None:
             plan.grid_x = grid_x
+        if edit is not None:
+            edit(plan)
         st = api.zluda_gemm_launch(C.byref(p), C.byref(plan), torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
         return st, self.download(dt), plan

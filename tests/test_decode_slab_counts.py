@@ -21,6 +21,8 @@ def test_every_packed_instantiation_issues_exactly_the_counted_factor_loads(tmp_
     insts = ["%d, %s, %s" % (fast, kind, tail) for fast in (1, 2) for kind in KINDS for tail in ("false", "true")]
     insts += ["%d, %s, true, 8, 512, %d" % (fast, kind, q) for fast in (1, 2) for kind in KINDS for q in (2, 3, 4)]
     insts += ["%d, %s, true, 8, 512, %d, 2" % (fast, kind, q) for fast in (1, 2) for kind in KINDS for q in (1, 2)]
+    # (MXFP4 has neither four units nor two units with two token blocks)
+    insts += ["%d, KIND_MXF4, %s" % (fast, shape) for fast in (1, 2) for shape in ("false", "true", "true, 8, 512, 2", "true, 8, 512, 3", "true, 8, 512, 1, 2")]
     src = tmp_path / "slab_counts.hip"
     src.write_text('#include <hip/hip_runtime.h>\n#include "decode_slab.hpp"\nusing namespace zluda_amd;\n' + "".join(
         "template __global__ void zluda_amd::decode_slab_kernel<%s>(DecodeParams);\n" % i for i in insts))

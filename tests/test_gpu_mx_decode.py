@@ -24,10 +24,8 @@ def run(gpu_api, **spec):
 
 @pytest.mark.parametrize("k,n,variant", [(8192, 16, 16), (4352, 3, 16), (6400, 1, 16), (7936, 9, 16),        # 4 waves, one unit of 1 KiB
                                          (8192, 32, 20), (4352, 17, 20), (6912, 25, 20),                      # 8 waves, one unit, two token blocks
-                                         (16384, 16, 17), (8448, 5, 17), (12544, 1, 17), (16384, 7, 18), (16640, 16, 18), (20736, 11, 18), (24576, 2, 18)])
+                                         (16384, 16, 17), (8448, 5, 17), (12544, 1, 17), (16384, 7, 17), (16640, 16, 18), (20736, 11, 18), (24576, 2, 18)])
 def test_shapes(gpu_api, k, n, variant):
-    if k == 16384 and variant == 18:
-        variant = 17
     assert run(gpu_api, m=300, n=n, k=k) == variant
     assert run(gpu_api, m=16 * 256 + 36, n=n, k=k, epilogue=K.CUBLASLT_EPILOGUE_GELU_BIAS) == variant
 
@@ -55,3 +53,22 @@ def test_a_nan_scale_stays_in_its_row(gpu_api):
         want = plain.view(np.float32).reshape(n, 128)
         got[:, 37] = want[:, 37]
         case.compare(got.reshape(-1).view(plain.dtype), plain)
+
+
+@pytest.mark.parametrize("k,n,variant", [(8192, 16, 16), (4352, 3, 16), (7936, 9, 16), (8192, 32, 20), (4352, 17, 20), (6912, 25, 20), (8448, 5, 17), (16384, 16, 17),
+                                         (16640, 16, 18), (20736, 11, 18)])
+def test_three_and_four_blocks_a_workgroup(gpu_api, k, n, variant):
+    """two workgroups: slots of weights and scales that are filled again and read again, with whole blocks and a short last one"""
+    for m in (96, 116, 128):
+        s = dict(MX, m=m, n=n, k=k)
+        print("case", s, variant, flush=True)
+        case = Case(s, 4600 + k + m)
+        st, got, plan = case.run_gpu_plan(gpu_api, K.ZLUDA_KERNEL_DECODE_W8A8, variant, grid_x=2)
+        assert st == 0 and plan.variant == variant
+        case.compare(got, case.run_oracle())
+
+
+def test_many_rows(gpu_api):
+    """beyond 64 rows per CU: the planner's own grid, four blocks in each workgroup"""
+    assert run(gpu_api, m=28672, n=3, k=6144) == 16
+    assert run(gpu_api, m=28672, n=17, k=8192) == 20
