@@ -515,3 +515,12 @@ def test_slab_decode_beyond_64_rows_per_cu(api, spec, m, n, k, slab):
     if slab:
         assert p.grid_x * 64 >= m and p.block in (256, 512)
     assert plan(api, dict(spec, m=m, n=n, k=k, transa=1), K.ZLUDA_KERNEL_DECODE_W8A8)[0] == 0
+
+
+@pytest.mark.parametrize("spec,m,n,k,more,bad", [
+    (F8, 6608, 2544, 64, {}, (6,)), (F8, 3328, 128, 48, dict(batch=8), (6,)), (F8, 12144, 528, 80, {}, (6,)),      # many tiles of a stage of K
+    (dict(BF, a_type=K.CUDA_R_32F, b_type=K.CUDA_R_32F, d_type=K.CUDA_R_32F), 17280, 1289, 112, {}, (0, 7)),      # f32 multiplies for longer
+    (MX, 3364, 256, 10752, {}, (5,)), (F8, 704, 3248, 176, {}, (3,)), (MX, 5616, 1824, 256, {}, (0,))])
+def test_tiles_that_measured_a_seventh_and_more_slower_are_not_chosen(api, spec, m, n, k, more, bad):
+    st, p = plan(api, dict(spec, m=m, n=n, k=k, transa=1, **more), workspace=4 << 20)
+    assert st == 0 and p.variant not in bad and p.kernel in (K.ZLUDA_KERNEL_MFMA_F8, K.ZLUDA_KERNEL_MFMA_F32, K.ZLUDA_KERNEL_MFMA_MXF4)

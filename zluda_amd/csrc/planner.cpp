@@ -441,6 +441,33 @@ static bool mfma_eight_waves(const Lowered &l, uint64_t tiles, uint32_t cus) {
   return !wide_d || tiles * 4 <= 3 * (uint64_t)cus || (int64_t)l.g.K * type_bits(l.g.a_type) / 8 > 2048;
 }
 
+// Workgroups of a variant that a CU holds: data stages, plus two chunks of 32 scale bytes per tile row for MXFP4
+static uint32_t mfma_per_cu(const Lowered &l, const MfmaVariant &v) {
+  const uint32_t lds = (uint32_t)v.stages * (v.bp + v.bq) * v.bkb + (l.g.a_type == CUDA_R_4F_E2M1 ? 64u * (v.bp + v.bq) : 0u);
+  return std::max(1u, std::min(160u * 1024u / lds, 2048u / (v.wp * v.wq * 64u)));
+}
+
+// Split-K: when even the chosen tiles leave half of the CUs idle and K is long, grid_z workgroups
+// share a tile's K range, write their fp32 / int32 partial tiles to the workspace and a second
+// kernel sums them and applies the epilogue.  Only if the caller's workspace holds the partial
+// tiles (padded to whole tiles).  (MXFP4 shares are whole scale chunks: the launcher rounds.)
+static uint32_t mfma_splits(const Lowered &l, const MfmaVariant &v, uint64_t tiles, uint32_t cus, uint64_t workspace_size) {
+  const GemmArgs &g = l.g;
+  if (tiles * 2 > cus) return 1;
+  // (below ~6 KiB of K per row the second kernel and the workspace traffic cost more than the idle CUs)
+  const uint32_t kbytes = ceil_div((uint32_t)((int64_t)g.K * type_bits(g.a_type) / 8), v.bkb) * v.bkb;
+  // Skinny problems (<= 64 rows or columns) are memory bound: they split from 2 KiB of K per row on
+  // and down to 1 KiB per share, up to two workgroups per CU (fp8 4096x48x4096: 18 -> 13 us; but
+  // 14336x64x4096, 224 tiles, must stay whole: 16.5 us against 23.7 split in three).
+  const bool skinny = std::min(g.M, g.N) <= 64;
+  const bool mx = g.a_type == CUDA_R_4F_E2M1;  // (a byte of FP4 is worth two K steps: 4096x16x4096 loses when split)
+  const uint32_t np = g.d_si != 1 ? g.N : g.M;
+  if (kbytes < (skinny ? (mx ? 4096u : 2048u) : 6144u) || (uint64_t)ceil_div(np, v.bp) * v.bp > (1u << 20)) return 1;
+  uint32_t s = (uint32_t)std::min<uint64_t>({8, (skinny ? 2 * cus : cus) / tiles, kbytes / (skinny ? 1024 : 2048)});
+  while (s > 1 && s * tiles * v.bp * v.bq * 4 > workspace_size) s--;
+  return std::max(s, 1u);
+}
+
 static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t workspace_size,
                            zluda_gemm_plan *plan) {
   const GemmArgs &g = l.g;
@@ -472,63 +499,62 @@ static void fill_mfma_plan(const Lowered &l, int variant, uint32_t cus, uint64_t
   }
   const bool eight = variant == 2 && mfma_eight_waves(l, (uint64_t)tp * tq * g.batch, cus);
   if (eight) plan->block = kMfmaEightWaves.wp * kMfmaEightWaves.wq * 64;
-  // data stages, plus two chunks of 32 scale bytes per tile row for MXFP4
-  const uint32_t lds = (uint32_t)(eight ? kMfmaEightWaves : v).stages * (v.bp + v.bq) * v.bkb + (l.g.a_type == CUDA_R_4F_E2M1 ? 64u * (v.bp + v.bq) : 0u);
-  const uint32_t per_cu = std::max(1u, std::min(160u * 1024u / lds, 2048u / plan->block));
+  const uint32_t per_cu = mfma_per_cu(l, eight ? kMfmaEightWaves : v);
   plan->waves = (float)plan->grid_x * plan->grid_y / (float)(cus * per_cu);
   plan->workspace = 0;
-  // Split-K: when even the chosen tiles leave half of the CUs idle and K is long, grid_z workgroups
-  // share a tile's K range, write their fp32 / int32 partial tiles to the workspace and a second
-  // kernel sums them and applies the epilogue.  Only if the caller's workspace holds the partial
-  // tiles (padded to whole tiles).  (MXFP4 shares are whole scale chunks: the launcher rounds.)
   const uint64_t tiles = (uint64_t)plan->grid_x * plan->grid_y;
-  const uint32_t kt = ceil_div((uint32_t)((int64_t)g.K * type_bits(g.a_type) / 8), v.bkb);
-  // (below ~6 KiB of K per row the second kernel and the workspace traffic cost more than the idle CUs)
-  const uint32_t kbytes = kt * v.bkb;
-  // Skinny problems (<= 64 rows or columns) are memory bound: they split from 2 KiB of K per row on
-  // and down to 1 KiB per share, up to two workgroups per CU (fp8 4096x48x4096: 18 -> 13 us; but
-  // 14336x64x4096, 224 tiles, must stay whole: 16.5 us against 23.7 split in three).
-  const bool skinny = std::min(g.M, g.N) <= 64;
-  const bool mx = g.a_type == CUDA_R_4F_E2M1;  // (a byte of FP4 is worth two K steps: 4096x16x4096 loses when split)
-  if (tiles * 2 <= cus && kbytes >= (skinny ? (mx ? 4096u : 2048u) : 6144u) &&
-      (uint64_t)tp * v.bp <= (1u << 20)) {
-    uint32_t s = (uint32_t)std::min<uint64_t>({8, (skinny ? 2 * cus : cus) / tiles, kbytes / (skinny ? 1024 : 2048)});
-    const uint64_t per_split = (uint64_t)g.batch * tp * v.bp * tq * v.bq * 4;
-    while (s > 1 && s * per_split > workspace_size) s--;
-    if (s > 1) {
-      plan->grid_z = s;
-      plan->workspace = s * per_split;
-      plan->waves = (float)tiles * s / (float)(cus * per_cu);
-    }
+  const uint32_t s = mfma_splits(l, v, tiles, cus, workspace_size);
+  if (s > 1) {
+    plan->grid_z = s;
+    plan->workspace = s * tiles * v.bp * v.bq * 4;
+    plan->waves = (float)tiles * s / (float)(cus * per_cu);
   }
 }
 
-// Relative throughput of one CU inside the K loop on tiles of each variant (variant 0 = 1) and what a tile costs around its
-// loop, in stages of 128 bytes of K.  Fitted to the times of 460 int8, fp8 and bf16 and 270 MXFP4 problems on every variant
-// (MI355X; linear layers of 17 to 4096 tokens and 256 .. 60000 rows, K = 128 .. 24000): what they pick takes 1.8 %
-// (MXFP4 0.3 %; fitted to one half of the problems, 0.6 % on the other) more time than the best variant of each problem on average.
-// MXFP4 counts the rounds of variant 3 over the two workgroups that a CU holds (34304 x 296 x 6400: 70 us, counted one by one
-// variant 5 came out ahead, which takes 94; 8192 x 777 x 8192 41.8, variant 4 48); the other types pick no better for it.
+// What a problem takes on a variant, in the time of one stage (128 bytes of K) of a 256 x 256 tile.  A CU holds one or a few workgroups of a
+// variant at a time (mfma_per_cu()); for each such set it takes `set`, and for each workgroup the tile's area times its stages and what it
+// costs around them that the others of its set do not hide (`around`, in stages) over the relative throughput of one CU inside the K
+// loop (`efficiency`).  With K shared out there is a second kernel, and the partial tiles go through memory.
+// Fitted to the times on every variant, weights from memory and from the caches, of 1900 int8, fp8 and bf16, 620 MXFP4 and 330 f32 problems
+// (MI355X; 64 .. 32768 rows, 17 .. 12000 tokens, K = 32 .. 24000, a quarter of them in batches, workspaces of 0, 4 and 32 MiB).  What they
+// pick takes 0.5 % (MXFP4 0.1 %, f32 0.2 %) more time than the best variant of each problem on average (fitted to one half 0.6, 0.3 and
+// 0.5 % on the other), more than 10 % in 1.5 % of them.  With whole rounds of one workgroup per CU, fractions of a stage, shares not
+// counted and one table for f32 too it was 1.5, 0.6 and 2.4 %, and short or shared K and f32 came out behind by a fifth and more: fp8
+// 6608 x 2544 x 64 20.4 us on 64 x 64 tiles, 15.5 on 192 x 256; MXFP4 3980 x 3 x 8448, 4 batches 25.1 on 128 x 64 in two shares, 16.9 on
+// 64 x 64; f32 17280 x 1289 x 112 80 on 256 x 256, 68 on 256 x 128.
 // The variants on the 16x16 MFMA shapes (8, 9) need less energy per multiply-add, which is what bounds a GEMM that keeps the
 // whole chip busy (the board sits at its power cap); on a chip that is partly idle the clock is the bound instead, so they are
 // only chosen for grids that fill the chip; the same tiles at 256x128 and 128x128 measured no better than the 32x32 ones
 // anywhere and are not instantiated.
-struct MfmaTileCost { float efficiency, around; };
-static const MfmaTileCost kMfmaTileCost[kNumMfmaVariants] = {{1.00f, 5.8f}, {0.95f, 6.0f}, {0.82f, 7.6f}, {0.62f, 5.9f}, {0.76f, 9.0f}, {0.43f, 4.4f},
-                                                             {0.41f, 3.4f}, {0.89f, 6.3f}, {1.05f, 5.1f}, {0.89f, 4.6f}, {0.41f, 3.4f}, {1.06f, 5.3f}};
-static const MfmaTileCost kMxTileCost[kNumMfmaVariants] = {{1.00f, 3.2f}, {0.95f, 3.2f}, {0.82f, 8.5f}, {0.79f, 3.0f}, {0.62f, 5.0f}, {0.46f, 4.4f},
-                                                           {0.26f, 2.9f}, {1.06f, 5.5f}, {1.05f, 3.2f}, {0.89f, 3.2f}, {0.26f, 2.9f}, {1.27f, 5.1f}};
-// A last round that fills a part x of the CUs takes this + (1 - this) * x of a full one's time: the clock is higher and memory
-// less busy then.
-constexpr double kPartialRound = 0.65;
+struct MfmaTileCost { float efficiency, around, set; };
+struct MfmaCost {
+  MfmaTileCost tile[kNumMfmaVariants];
+  // workgroups on a part x of the CUs take partial + (1 - partial) * x of the time of one on each: the clock is higher and memory less busy then
+  float partial;
+  float second_kernel;
+};
+static const MfmaCost kMfmaCost = {{{1.00f, 5.7f}, {0.95f, 8.5f}, {0.84f, 7.0f}, {0.64f, 1.1f, 1.87f}, {0.79f, 8.7f}, {0.46f, 0.8f, 1.44f},
+                                    {0.35f, 0.5f, 1.18f}, {0.88f, 5.4f}, {1.05f, 6.1f}, {0.95f, 6.0f}, {0.37f, 2.9f}, {1.08f, 5.2f}}, 0.84f, 0.38f};
+static const MfmaCost kF32Cost = {{{1.00f, 20.3f}, {0.93f, 10.2f}, {0.81f, 6.7f}, {0.62f, 0.8f, 0.36f}, {0.76f, 10.7f}, {0.64f, 1.1f, 0.90f},
+                                   {0.54f, 0.5f, 0.20f}, {0.85f, 7.4f}}, 0.98f, 0.27f};  // (the others do not exist for f32)
+static const MfmaCost kMxCost = {{{1.00f, 3.3f}, {0.94f, 3.2f}, {0.50f, 8.5f}, {0.61f, 0.5f, 1.26f}, {0.62f, 3.7f}, {0.44f, 1.0f, 1.05f},
+                                  {0.34f, 0.4f, 1.13f}, {0.92f, 4.1f}, {}, {}, {}, {1.24f, 4.9f}}, 0.93f, 0.41f};
+constexpr double kPartialTilesPerMB = 0.2;
 
-static int pick_mfma_variant(const Lowered &l, uint32_t cus) {
+// Skinny problems that end up with at most one 64 x 64 workgroup per CU and are not split along K are bound
+// by what a CU keeps in flight: the 6-stage ring of variant 10 (80 KiB instead of 32) takes 8-17 % less time
+// (bf16 14336x64x4096 29.2 us against 32.0, 4096x64x14336 71 against 87; int8 8192x64x8192 24.4 against 29.0).
+static bool mfma_deep_ring(const Lowered &l, uint64_t tiles, uint32_t splits, uint32_t cus) {
+  const uint32_t t = l.g.a_type;
+  return t != CUDA_R_4F_E2M1 && t != CUDA_R_32F && splits == 1 && tiles <= cus && (int64_t)l.g.K * type_bits(t) / 8 >= 1536;
+}
+
+static int pick_mfma_variant(const Lowered &l, uint32_t cus, uint64_t workspace_size) {
   const GemmArgs &g = l.g;
   if (mfma_short_k(l, cus)) return 3;
   const bool swapped = g.d_si != 1;
   const uint32_t np = swapped ? g.N : g.M, nq = swapped ? g.M : g.N;
-  // cost = rounds of workgroups over the CUs x time of one tile; the tile shapes trade efficiency
-  // per CU against how evenly the problem fills the chip and what a tile costs around its K loop
+  // the tile shapes trade efficiency per CU against how evenly the problem fills the chip and what a tile costs around its K loop
   int best = 0;
   double best_cost = 0;
   for (int v = 0; v < kNumMfmaVariants; v++) {
@@ -553,12 +579,18 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus) {
       const uint64_t need = (g.a_type == CUDA_R_8I || h16) ? ((uint64_t)cus * 3 + 3) / 4 : (uint64_t)cus * (t.bp == 256 ? 4 : 2);
       if (tiles < need) continue;
     }
-    const bool mx = g.a_type == CUDA_R_4F_E2M1;
-    const uint64_t per_cu = mx && v == 3 ? 2 : 1, slots = per_cu * cus, full = tiles / slots, rem = tiles % slots;
-    const double rounds = (double)per_cu * ((double)full + (rem ? kPartialRound + (1.0 - kPartialRound) * (double)rem / slots : 0.0));
-    const MfmaTileCost &c = (mx ? kMxTileCost : kMfmaTileCost)[v];
-    const double stages = (double)((int64_t)g.K * type_bits(g.a_type) / 8) / 128;
-    const double cost = rounds * t.bp * t.bq / c.efficiency * (stages + c.around);
+    const bool mx = g.a_type == CUDA_R_4F_E2M1, f32 = g.a_type == CUDA_R_32F;
+    const MfmaCost &c = f32 ? kF32Cost : mx ? kMxCost : kMfmaCost;
+    const uint32_t s = t.w4 ? 1 : mfma_splits(l, t, tiles, cus, workspace_size);
+    const int as = v == 6 && mfma_deep_ring(l, tiles, s, cus) ? 10 : v;
+    const uint64_t groups = tiles * s, per_cu = mfma_per_cu(l, kMfmaVariants[as]), sets = (groups + per_cu * cus - 1) / (per_cu * cus);
+    const uint64_t each = groups / cus, rem = groups % cus;
+    uint32_t stages = ceil_div(ceil_div((uint32_t)((int64_t)g.K * type_bits(g.a_type) / 8), 128), s);
+    if (mx && s > 1) stages = (stages + 3) / 4 * 4;  // (whole scale chunks)
+    const MfmaTileCost &tc = c.tile[as];
+    const double loops = (double)each + (rem ? c.partial + (1.0 - c.partial) * (double)rem / cus : 0.0);
+    double cost = tc.set * (double)sets + loops * t.bp * t.bq / 65536 / tc.efficiency * (stages + tc.around);
+    if (s > 1) cost += c.second_kernel + kPartialTilesPerMB * 1e-6 * (double)(s * tiles * t.bp * t.bq * 4);
     if (v == 0 || cost < best_cost) { best = v; best_cost = cost; }
   }
   return best;
@@ -855,7 +887,7 @@ extern "C" uint32_t zluda_gemm_plan_problem(const zluda_gemm_problem *p, uint32_
         // against 25; but 2048x16x2560, 32 tiles: 8 against 12)
         zluda_gemm_plan mfma;
         memset(&mfma, 0, sizeof(mfma));
-        fill_mfma_plan(l, pick_mfma_variant(l, cu_count), cu_count, p->workspace_size, &mfma);
+        fill_mfma_plan(l, pick_mfma_variant(l, cu_count, p->workspace_size), cu_count, p->workspace_size, &mfma);
         if ((uint64_t)mfma.grid_x * mfma.grid_y * mfma.grid_z * 2 >= cu_count) continue;
       }
       kernel = k;
@@ -880,7 +912,7 @@ extern "C" uint32_t zluda_gemm_plan_problem(const zluda_gemm_problem *p, uint32_
     break;
   case ZLUDA_KERNEL_MFMA_I8: case ZLUDA_KERNEL_MFMA_F8: case ZLUDA_KERNEL_MFMA_MXF4: case ZLUDA_KERNEL_MFMA_H16:
   case ZLUDA_KERNEL_MFMA_F32: {
-    int v = forced_variant >= 0 ? forced_variant : pick_mfma_variant(l, cu_count);
+    int v = forced_variant >= 0 ? forced_variant : pick_mfma_variant(l, cu_count, p->workspace_size);
     const bool w4 = v < kNumMfmaVariants && kMfmaVariants[v].w4;
     if (v >= kNumMfmaVariants || (v >= kNumMfmaVariants32 && !w4 && kernel != ZLUDA_KERNEL_MFMA_I8 && kernel != ZLUDA_KERNEL_MFMA_F8 &&
                                   kernel != ZLUDA_KERNEL_MFMA_H16) || (v >= kNumMfmaVariantsH16 && kernel == ZLUDA_KERNEL_MFMA_H16) ||
@@ -892,11 +924,7 @@ extern "C" uint32_t zluda_gemm_plan_problem(const zluda_gemm_problem *p, uint32_
                 ((l.g.a_type == CUDA_R_16F || l.g.a_type == CUDA_R_16BF) && l.g.b_type == l.g.a_type)))
       return CUBLAS_STATUS_NOT_SUPPORTED;
     fill_mfma_plan(l, v, cu_count, p->workspace_size, plan);
-    // Skinny problems that end up with at most one 64 x 64 workgroup per CU and are not split along K are bound
-    // by what a CU keeps in flight: the 6-stage ring of variant 10 (80 KiB instead of 32) takes 8-17 % less time
-    // (bf16 14336x64x4096 29.2 us against 32.0, 4096x64x14336 71 against 87; int8 8192x64x8192 24.4 against 29.0).
-    if (forced_variant < 0 && v == 6 && kernel != ZLUDA_KERNEL_MFMA_MXF4 && kernel != ZLUDA_KERNEL_MFMA_F32 && plan->grid_z == 1 &&
-        (uint64_t)plan->grid_x * plan->grid_y <= cu_count && (int64_t)l.g.K * type_bits(l.g.a_type) / 8 >= 1536)
+    if (forced_variant < 0 && v == 6 && mfma_deep_ring(l, (uint64_t)plan->grid_x * plan->grid_y, plan->grid_z, cu_count))
       fill_mfma_plan(l, 10, cu_count, 0, plan);
     break;
   }
