@@ -638,7 +638,7 @@ static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t w
   plan->waves = (float)plan->grid_x * plan->grid_y / (float)(cus * per_cu);
   plan->workspace = 0;
   // Split-K as for the K-contiguous kernels: grid_z workgroups share a tile's K range through the
-  // caller's workspace when K has at least 16 stages and the tiles leave half of the chip idle --
+  // caller's workspace when K is long enough (`least`) and the tiles leave half of the chip idle --
   // half of the CUs, or, for skinny problems (<= 64 rows or columns: memory bound, a workgroup keeps
   // only ~16 KiB in flight), half of the workgroup slots.  N-contiguous weights, 16 tokens, us:
   // 4096x14336 89 -> 25, 4096x4096 31 -> 14, 14336x4096 31 -> 24; 14336x128x4096 would lose (37 -> 42).
@@ -646,8 +646,12 @@ static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t w
   const uint64_t slots = (uint64_t)cus * per_cu;
   const bool skinny = std::min(g.M, g.N) <= 64;
   const uint64_t kbytes = (uint64_t)g.K * type_bits(g.a_type) / 8;
-  // (On a shorter K the second kernel costs more than the shorter loop saves, us: int8 512 x 512 x 1024 10.7 split, 6.9 whole; f16
-  // 777 x 333 x 555 9.7 and 7.8; f32 1098 x 419 x 350 12.6 and 10.2; bf16 300 x 300 x 1000 9.7 both.)
+  // Where the loop that gets shorter outweighs the second kernel and the partial tiles' way through memory depends on both, us whole and in
+  // as many shares as there can be: f32 256 x 256 x 384 9.3 and 8.2, 512 x 512 x 384 9.4 and 10.1, x 1024 19.0 and 14.3; bf16 256 x 256 x 1024
+  // 8.7 and 8.5, 512 x 512 x 1024 8.9 and 10.0, x 2048 12.9 and 12.8; int8 300 x 300 x 1088 8.3 and 9.3, x 1536 10.2 and 9.0, 512 x 512 x 1088
+  // 7.2 and 10.1, x 2048 10.7 and 10.5.  The lines lie at the least K that gains on few tiles; 8-bit operands gain from 1300 to 2500 bytes
+  // on, and are split from 17 stages on as they have been.  (Choosing the number of shares by such a cost gained 2 % over 392 problems whose operands
+  // were in the caches and none where they were not, and lost up to 20 % on some.)
   const uint64_t least = skinny ? 1024 : g.a_type == CUDA_R_32F ? 1536 : type_bits(g.a_type) == 16 ? 2048 : 1088;
   if (tiles * 2 <= (skinny ? slots : (uint64_t)cus) && kbytes >= least && (uint64_t)ceil_div(np, v.bp) * v.bp <= (1u << 20)) {
     uint32_t s = (uint32_t)std::min<uint64_t>({8, slots / tiles, kbytes / 512});
