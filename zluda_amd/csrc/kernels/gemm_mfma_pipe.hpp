@@ -340,8 +340,8 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
     kt++;
   };
   // The last stage has its fragments on the way already: it requests nothing and waits for nothing else.  (With the padding stage's
-  // round trip in front of its MFMAs the smallest problems took longer than on one sub-step ahead: fp8 9680 x 48 x 112, one
-  // stage, 4.5 us instead of 4.0.)
+  // round trip in front of its MFMAs, 90 problems of one to four stages took 1 to 3 % longer on the 128 x 64 and 64 x 64 tiles, the smallest
+  // up to 10 %.)
   auto last_stage = [&](auto cur_c) {
     constexpr int CUR = decltype(cur_c)::value;
     if constexpr (MX) sc_cur = sc_nxt;
