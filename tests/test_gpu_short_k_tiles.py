@@ -88,3 +88,32 @@ def test_zeros_have_the_sign_that_the_tile_kernels_give_them(gpu_api, d):
     zero = [(i % 130, b) for b in range(133) for i in range(130) if (b * 130 + i) % 3 == 0]
     for i, b in zero:
         assert (bits[0][b * 130:(b + 1) * 130, i] == bits[1][b * 130:(b + 1) * 130, i]).all()
+
+
+@pytest.mark.parametrize("k,d,m,n,batch", [(64, K.CUDA_R_16BF, 512, 640, 3), (128, K.CUDA_R_16BF, 512, 640, 3), (128, K.CUDA_R_32F, 384, 1300, 2), (72, K.CUDA_R_16BF, 500, 1300, 2),
+                                           (40, K.CUDA_R_32F, 300, 1100, 3), (128, K.CUDA_R_16F, 130, 4000, 1)])
+def test_runs_of_many_tiles(gpu_api, k, d, m, n, batch):
+    """eight and sixteen workgroups: runs of four to eight tiles, whole ones in a row and turns of P between them, so that every wait is reached"""
+    t = K.CUDA_R_16F if d == K.CUDA_R_16F else K.CUDA_R_16BF
+    s = dict(a_type=t, b_type=t, d_type=d, c_type=d, compute_type=K.CUBLAS_COMPUTE_32F, scale_type=K.CUDA_R_32F, m=m, n=n, k=k, transa=1, batch=batch)
+    case = Case(s, 7960 + k)
+    ref = case.run_oracle()
+    tiles = -(-m // 128) * -(-n // 128)
+    for groups in (8, 16):
+        print("case", s, groups, flush=True)
+
+        def short_form(plan):
+            plan.grid_x, plan.grid_y, plan.grid_z = groups, 1, 1
+        st, got, plan = case.run_gpu_plan(gpu_api, K.ZLUDA_KERNEL_MFMA_H16, 3, edit=short_form)
+        assert st == 0 and plan.variant == 3 and groups < tiles * batch
+        case.compare(got, ref, tol=1e-2)
+
+
+def test_the_planner_gives_the_form(gpu_api):
+    """the problems of test_edges and test_output_types have more tiles than two workgroups per CU take in one go"""
+    for m, n, k, batch in [(130, 130, 8, 130), (128, 256, 64, 260), (300, 70, 72, 175), (66, 65, 128, 520), (256, 384, 120, 90), (1026, 200, 104, 40), (202, 130, 96, 133)]:
+        t = K.CUDA_R_16BF
+        case = Case(dict(a_type=t, b_type=t, d_type=t, c_type=t, compute_type=K.CUBLAS_COMPUTE_32F, scale_type=K.CUDA_R_32F, m=m, n=n, k=k, transa=1, batch=batch), 7970)
+        st, got, plan = case.run_gpu_plan(gpu_api, K.ZLUDA_KERNEL_AUTO)
+        assert st == 0 and (plan.kernel, plan.variant, plan.grid_y, plan.grid_z) == (K.ZLUDA_KERNEL_MFMA_H16, 3, 1, 1)
+        assert plan.grid_x == max(2 * gpu_api.zluda_gemm_device_cu_count() // 8 * 8, 8)
