@@ -1,0 +1,87 @@
+"""GELU with its input kept and GELU's gradient in the epilogues of the 16-bit tile kernels: every accumulator layout, tiles that hang over
+either end of D, pitches and batch strides of aux of their own, and what keeps a problem on the pass behind the matmul."""
+import ctypes as C
+
+import pytest
+
+from oracle.cases import Case
+from zluda_amd import abi as K
+
+pytestmark = pytest.mark.gpu
+AUX, AUX_BIAS, DG, DG_SUMS = (K.CUBLASLT_EPILOGUE_GELU_AUX, K.CUBLASLT_EPILOGUE_GELU_AUX_BIAS, K.CUBLASLT_EPILOGUE_DGELU, K.CUBLASLT_EPILOGUE_DGELU_BGRAD)
+H16, TR16 = K.ZLUDA_KERNEL_MFMA_H16, K.ZLUDA_KERNEL_MFMA_TR16
+BF = dict(a_type=K.CUDA_R_16BF, b_type=K.CUDA_R_16BF, d_type=K.CUDA_R_16BF, compute_type=K.CUBLAS_COMPUTE_32F, scale_type=K.CUDA_R_32F, alpha=0.05)
+# One rounding of D to its type (2^-9 bf16, 2^-12 f16) of sums in another order than the oracle's, and the fast exponential and reciprocal.
+# (The aux matrix is rounded once; the gradient is taken at its stored elements, as the oracle takes it.)
+TOL = {K.CUDA_R_16BF: 1e-2, K.CUDA_R_16F: 2e-3}
+# Behind the matmul GELU sees its input x rounded to bf16: an error of 2^-9 |x gelu'(x)|, at most 0.2 * 2^-9 where x < 0 (it is relative to the
+# result elsewhere).  Compared with a floor of a tenth of D's root mean square (0.2 or more here) that is 10 * 2^-9, and D's own rounding.
+TOL_BEHIND, FLOOR_BEHIND = 12 / 512, 1e-1
+
+
+def run(api, spec, seed, family, variant, ws=4 << 20, block=None, in_epilogue=True):
+    """the case, its plan; `in_epilogue`: the sums of DGELU_BGRAD are counted one per wave along D's columns"""
+    import torch
+    print("case", spec, "family", family, "variant", variant, flush=True)
+    case = Case(spec, seed)
+    ref = case.run_oracle()
+    keep, ptr, dt = case.upload()
+    p = case.problem(dict(ptr, alpha=case.alpha.ctypes.data, beta=case.beta.ctypes.data))
+    scratch = torch.full((max(ws, 16),), 0xFF, dtype=torch.uint8, device="cuda:0")   # (NaN: a sum that is read without being written)
+    p.workspace, p.workspace_size = (scratch.data_ptr() if ws else None), ws
+    plan = K.zluda_gemm_plan()
+    assert api.zluda_gemm_plan_problem(C.byref(p), family, variant, api.zluda_gemm_device_cu_count(), C.byref(plan)) == 0
+    if block:
+        plan.block = block
+    assert api.zluda_gemm_launch(C.byref(p), C.byref(plan), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    case.compare(case.download(dt), ref, tol=TOL[spec["d_type"]] if in_epilogue else TOL_BEHIND,
+                 floor_frac=None if in_epilogue else FLOOR_BEHIND)
+    if case.aux_mode == 1:
+        case.compare_aux(keep[10][:case.aux.nbytes].cpu().numpy().view(case.aux.dtype).copy(), case.aux_ref)
+    if case.bgrad:
+        case.compare_bgrad(keep[3][:case.bias.nbytes].cpu().numpy().view(case.bias.dtype).copy(), case.bgrad_ref, floor_frac=1.0)
+        assert bool((scratch[plan.workspace:] == 0xFF).all())
+    return case, plan
+
+
+# family, variant, block: 32x32 tiles of every wave shape, 16x16 tiles, the four-wave kernel; the layouts of the transposing kernels
+FORMS = [(H16, v, b, 1, 0) for v, b in ((0, 0), (2, 256), (2, 512), (4, 0), (5, 0), (6, 0), (7, 0), (8, 0), (9, 0), (10, 0), (11, 0))] + \
+        [(TR16, v, b, ta, tb) for v, b in ((0, 0), (1, 256), (1, 512), (2, 256), (2, 512), (3, 0)) for ta, tb in ((0, 0), (0, 1), (1, 1))]
+
+
+@pytest.mark.parametrize("epi", [AUX, AUX_BIAS, DG, DG_SUMS])
+@pytest.mark.parametrize("family,variant,block,ta,tb", FORMS)
+def test_every_form(gpu_api, family, variant, block, ta, tb, epi):
+    # (tiles that hang over both ends, at both types of D; K rows of 16-byte pieces)
+    for i, (m, n, k) in enumerate(((264, 131, 128), (520, 300, 200), (8, 1, 72))):
+        spec = dict(BF, m=m, n=n, k=k, transa=ta, transb=tb, epilogue=epi)
+        if i == 1:
+            spec.update(a_type=K.CUDA_R_16F, b_type=K.CUDA_R_16F, d_type=K.CUDA_R_16F, bias_type=K.CUDA_R_32F)
+        if (ta, tb) != (1, 0) and tb:   # (the columns of B lie side by side: a whole number of 16-byte pieces for the LDS reads)
+            spec["ldb"] = (n + 7) // 8 * 8
+        behind = variant == 0 or (family == H16 and block == 256)   # (wave tiles of 128 x 64 on the 32x32 shapes)
+        run(gpu_api, spec, 9700 + 10 * epi + i, family, variant, block=block, in_epilogue=not behind)
+
+
+@pytest.mark.parametrize("family,variant,ta,tb", [(H16, 4, 1, 0), (H16, 8, 1, 0), (H16, 11, 1, 0), (TR16, 1, 0, 0), (TR16, 2, 0, 1)])
+def test_batches_pitches_scales(gpu_api, family, variant, ta, tb):
+    base = dict(BF, m=200, n=136, k=264, batch=3, transa=ta, transb=tb, ldd=208, ldc=208, aux_ld=224, aux_batch_stride=224 * 136 + 40)
+    run(gpu_api, dict(base, epilogue=AUX_BIAS, bias_type=K.CUDA_R_32F, bias_batch_stride=203), 9801, family, variant)
+    run(gpu_api, dict(base, epilogue=AUX_BIAS, bias_batch_stride=203), 9802, family, variant)     # (a bias at odd addresses)
+    run(gpu_api, dict(base, epilogue=DG_SUMS, bias_batch_stride=208), 9803, family, variant)
+
+
+@pytest.mark.parametrize("change", [dict(m=260), dict(ldd=268, ldc=268), dict(aux_ld=268), dict(order_c=1, order_d=1, aux_ld=136), dict(with_c=True),
+                                    dict(d_type=K.CUDA_R_32F), dict(ws=0), dict(k=4096, m=64, n=64)])
+@pytest.mark.parametrize("epi,ta", [(AUX_BIAS, 1), (DG_SUMS, 0)])
+def test_what_keeps_the_pass_behind_the_matmul(gpu_api, epi, ta, change):
+    change = dict(change)
+    ws = change.pop("ws", 4 << 20)
+    spec = dict(BF, m=264, n=136, k=256, transa=ta, epilogue=epi)
+    spec.update(change)
+    if spec["d_type"] == K.CUDA_R_32F:
+        spec["c_type"] = K.CUDA_R_32F
+    if spec.get("with_c") and epi == AUX_BIAS:
+        spec["beta"] = 0.5
+    run(gpu_api, spec, 9850, H16 if ta else TR16, -1, ws=ws, in_epilogue=False)

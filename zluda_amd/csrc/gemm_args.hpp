@@ -13,7 +13,12 @@ namespace zluda_amd {
 
 enum ScalarMode : int32_t { SCALAR_VALUE = 0, SCALAR_DEV = 1, VECTOR_DEV = 2 };
 enum ScaleMode : int32_t { SCALE_NONE = 0, SCALE_SCALAR = 1, SCALE_OUTER_VEC = 2, SCALE_BLOCK32_UE8M0 = 3 };
-enum Activation : int32_t { ACT_NONE = 0, ACT_RELU = 1, ACT_GELU = 2 };
+// (the last two: GELU with its input kept and GELU's gradient where the GEMM kernel does them itself, see aux_mode)
+enum Activation : int32_t { ACT_NONE = 0, ACT_RELU = 1, ACT_GELU = 2, ACT_GELU_KEPT = 3, ACT_DGELU = 4 };
+
+// Wave tiles on the 32x32 MFMA shapes whose kernels carry the last two: larger ones have no registers for them (128 x 128: 14 KiB of spills),
+// and the 16x16 shapes take the grids that fill such tiles
+constexpr bool aux_on_wave_tile32(int wtp, int wtq) { return wtp * wtq <= 96 * 64; }
 
 struct GemmArgs {
   const void *A, *B, *C;
@@ -40,8 +45,9 @@ struct GemmArgs {
   void *bgrad;
   int32_t bgrad_src;
   // GELU with its input kept (aux_mode 1: aux = x, D = gelu(x)) and its gradient (aux_mode 2: D = D * gelu'(aux),
-  // aux_bgrad: the row sums of that D go to `bgrad`).  Run as a second, element-wise pass behind the GEMM
-  // kernel; aux is a matrix of D's type and order, strides in elements.
+  // aux_bgrad: the row sums of that D go to `bgrad`).  aux is a matrix of D's type and
+  // order, strides in elements.  The GEMM kernel does this where
+  // `act` says so; elsewhere a second, element-wise pass behind it.
   void *aux;
   int64_t aux_si, aux_sj, aux_sb;
   int32_t aux_mode, aux_bgrad;

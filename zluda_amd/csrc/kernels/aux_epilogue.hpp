@@ -1,5 +1,5 @@
-// Second, element-wise pass of the epilogues that keep or use the GELU input
-// (cuda_types/src/cublaslt.rs:4601-4660; the aux attributes :4182-4236):
+// Second, element-wise pass of the epilogues that keep or use the GELU input, for the problems whose GEMM kernel does not do it itself
+// (aux_in_epilogue(); cuda_types/src/cublaslt.rs:4601-4660; the aux attributes :4182-4236):
 //   GELU_AUX[_BIAS]  the GEMM kernel has written x = alpha * op(A) op(B) + beta * C (+ bias) into the aux matrix;
 //                    this pass writes D = gelu(x) * d_scale
 //   DGELU[_BGRAD]    the GEMM kernel has written y = alpha * op(A) op(B) + beta * C into D; this pass turns it into
@@ -12,15 +12,6 @@
 #include "bgrad_reduce.hpp"
 
 namespace zluda_amd {
-
-// d/dx of the tanh form of GELU
-__device__ __forceinline__ float dgelu_tanh(float x) {
-  const float k0 = 0.7978845608028654f, k1 = 0.044715f;
-  const float u = k0 * (x + k1 * x * x * x);
-  // tanh(u) = 1 - 2 / (1 + exp(2u)); exp(2u) = inf gives 1, 0 gives -1
-  const float t = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(2.0f * 1.4426950408889634f * u));
-  return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * k0 * (1.0f + 3.0f * k1 * x * x);
-}
 
 template <uint32_t TYPE>
 __device__ __forceinline__ v4u32 piece_of_elems(const float *x) {

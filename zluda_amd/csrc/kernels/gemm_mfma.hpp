@@ -557,6 +557,105 @@ __device__ __forceinline__ void mfma_store_tile_plain(const MfmaParams &prm, Acc
     }
 }
 
+// What the epilogues with an aux matrix read it from, write it to, and put D and the partial sums of its rows
+// (DGELU_BGRAD) into; one column of a wave's tile is `q` elements of that pitch further on.
+// The fused forms take 16-bit floats, a column-major D, beta == 0, one factor for all of D, a multiple of 8 rows and 16-byte aligned
+// columns of D and aux (aux_in_epilogue() of the launch layer); everything else has a pass of its own behind the matmul (aux_epilogue.hpp).
+struct AuxTile {
+  __amdgpu_buffer_rsrc_t rs_d, rs_x;
+  int d_sq, x_sq;
+  float factor;
+  float *sums;  // this wave's partial sums, indexed by P; or NULL
+  __device__ __forceinline__ AuxTile(const MfmaParams &prm, const EpilogueScalars &s, int pc, int qc, int NP, int NQ, int bt, int share, int shares) {
+    const GemmArgs &g = prm.g;
+    d_sq = (int)g.d_sj; x_sq = (int)g.aux_sj;  // < kNarrowPitch
+    const int64_t d_corner = (int64_t)qc * d_sq + pc, x_corner = (int64_t)qc * x_sq + pc;
+    rs_d = __builtin_amdgcn_make_buffer_rsrc((char *)g.D + (g.d_sb * bt + d_corner) * 2, 0, tile_window_bytes(d_sq, NP, NQ, d_corner, 2), 0x00020000);
+    rs_x = __builtin_amdgcn_make_buffer_rsrc((char *)g.aux + (g.aux_sb * bt + x_corner) * 2, 0, tile_window_bytes(x_sq, NP, NQ, x_corner, 2), 0x00020000);
+    factor = s.alpha_s * s.sa_s * s.sb_s;
+    sums = g.aux_bgrad ? (float *)prm.ws + ((int64_t)bt * shares + share) * NP : nullptr;
+  }
+};
+
+// The two 16-bit floats of a dword, and back
+__device__ __forceinline__ float low_half(uint32_t d, bool bf16) { return bf16 ? bits2f(d << 16) : dec_f16((uint16_t)d); }
+__device__ __forceinline__ float high_half(uint32_t d, bool bf16) { return bf16 ? bits2f(d & 0xffff0000u) : dec_f16((uint16_t)(d >> 16)); }
+__device__ __forceinline__ uint32_t pack_halves(float lo, float hi, bool bf16) { return bf16 ? pack_bf16x2(lo, hi) : pack_f16x2(lo, hi); }
+
+// GELU with its input kept (MODE 1: aux = x, D = gelu(x)) and its gradient (MODE 2: D = x * gelu'(aux), and the sums of this
+// wave's part of D's rows): aux goes through the same dwords as D (fast path 2), one 32 x 32 tile at a time.
+template <int WP, int WQ, int WTP, int WTQ, int MODE, class AccV>
+__device__ __forceinline__ void mfma_store_tile_aux(const MfmaParams &prm, AccV (&acc)[WTQ / 32][WTP / 32], int p0, int q0, int NP, int NQ, int bt) {
+  constexpr int TP = WTP / 32, TQ = WTQ / 32;
+  const GemmArgs &g = prm.g;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wp = wave % WP, wq = wave / WP;
+  const int lr = lane & 31, gsel = lane >> 5, odd = lane & 1;
+  const int pc = p0 + wp * WTP, qc = q0 + wq * WTQ;
+  const Epilogue ep(g, bt);
+  const AuxTile at(prm, EpilogueScalars(g), pc, qc, NP, NQ, bt, q0 / WTQ + wq, prm.tiles_q * WQ);
+  const bool bf16 = g.d_type == CUDA_R_16BF;
+  const int vd = ((4 * gsel + odd) * at.d_sq + (lr & ~1)) * 2, vx = ((4 * gsel + odd) * at.x_sq + (lr & ~1)) * 2;
+  float p_bias[TP], sum[TP][2];
+#pragma unroll
+  for (int b = 0; b < TP; b++) {
+    p_bias[b] = MODE == 1 ? ep.bias_at(min(pc + b * 32 + lr, NP - 1)) : 0.0f;
+    sum[b][0] = sum[b][1] = 0.0f;
+  }
+#pragma unroll
+  for (int a = 0; a < TQ; a++) {
+    // (the row's aux dwords in one burst)
+    uint32_t x_in[TP][8];
+    if constexpr (MODE == 2) {
+#pragma unroll
+      for (int b = 0; b < TP; b++)
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+          x_in[b][k] = __builtin_amdgcn_raw_buffer_load_b32(at.rs_x, pc + b * 32 + lr < NP ? vx : kStoreNowhere, (a * 32 + 8 * (k >> 1) + 2 * (k & 1)) * at.x_sq * 2 + b * 64, 0);
+    }
+#pragma unroll
+    for (int b = 0; b < TP; b++) {
+      const bool in = pc + b * 32 + lr < NP;  // (a pair never straddles the end: it is a multiple of 8)
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const float x0 = at.factor * bits2f((uint32_t)to_bits(acc[a][b][2 * k])) + p_bias[b];
+        const float x1 = at.factor * bits2f((uint32_t)to_bits(acc[a][b][2 * k + 1])) + p_bias[b];
+        // even lanes keep row 2k and need the neighbour's row-2k value; odd lanes the other way round
+        const float mine = odd ? x1 : x0, give = odd ? x0 : x1;
+        const float got = bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(give), 0xB1 /* quad_perm [1,0,3,2] */, 0xF, 0xF, true));
+        float lo = odd ? got : mine, hi = odd ? mine : got;
+        const int row = a * 32 + 8 * (k >> 1) + 2 * (k & 1);
+        if constexpr (MODE == 1) {
+          __builtin_amdgcn_raw_buffer_store_b32((int)pack_halves(lo, hi, bf16), at.rs_x, in ? vx : kStoreNowhere, row * at.x_sq * 2 + b * 64, 0);
+          lo = gelu_tanh(lo) * ep.sd;
+          hi = gelu_tanh(hi) * ep.sd;
+        } else {
+          lo *= dgelu_tanh(low_half(x_in[b][k], bf16));
+          hi *= dgelu_tanh(high_half(x_in[b][k], bf16));
+          // (columns past the end hold products of some column)
+          const bool counts = qc + row + 4 * gsel + odd < NQ;
+          sum[b][0] += counts ? lo : 0.0f;
+          sum[b][1] += counts ? hi : 0.0f;
+        }
+        __builtin_amdgcn_raw_buffer_store_b32((int)pack_halves(lo, hi, bf16), at.rs_d, in ? vd : kStoreNowhere, row * at.d_sq * 2 + b * 64, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // one tile at a time: what the scheduler hoists across them spills
+    }
+  }
+  if (MODE == 2 && at.sums) {
+#pragma unroll
+    for (int b = 0; b < TP; b++) {
+#pragma unroll
+      for (int e = 0; e < 2; e++) {  // over the even and the odd lane of a pair of columns, and the lane halves
+        sum[b][e] += __shfl_xor(sum[b][e], 1, 64);
+        sum[b][e] += __shfl_xor(sum[b][e], 32, 64);
+      }
+      const int p = pc + b * 32 + lr;
+      if (gsel == 0 && p < NP) at.sums[p] = sum[b][odd];
+    }
+  }
+}
+
 // Epilogue dispatch: the fast paths for the common configurations, the general path for the rest (C reads, 8-bit outputs,
 // integer outputs of a float epilogue, vectors of alpha in the integer one).  All conditions are workgroup-uniform.  What they
 // and the integer path read is few enough to be kept from the kernel's entry on; the float paths read the arguments again.
@@ -577,6 +676,13 @@ __device__ __forceinline__ void mfma_store_tile(const MfmaParams &prm, AccV (&ac
     }
   }
   const MfmaParams &late = args_again(prm);
+  if constexpr (kind_is_h16(KIND) && aux_on_wave_tile32(WTP, WTQ)) {
+    if (__builtin_expect(g.act > ACT_GELU, 0)) {
+      if (g.act == ACT_GELU_KEPT) mfma_store_tile_aux<WP, WQ, WTP, WTQ, 1>(late, acc, p0, q0, NP, NQ, bt);
+      else mfma_store_tile_aux<WP, WQ, WTP, WTQ, 2>(late, acc, p0, q0, NP, NQ, bt);
+      return;
+    }
+  }
   if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
       (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F)) {
     if (!whole) {

@@ -340,6 +340,109 @@ __device__ __forceinline__ void mfma16_store_general(const MfmaParams &prm, AccV
   }
 }
 
+// GELU with its input kept and GELU's gradient (mfma_store_tile_aux()) in the 16x16 layout: tiles in pairs, the float values trade halves
+// as the 16-bit ones do in mfma16_store_f(), after which a lane has eight consecutive P indices: 16 bytes of D and of aux.
+template <int WP, int WQ, int TP, int TQ, int MODE, class AccV>
+__device__ __forceinline__ void mfma16_store_aux(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt, int wave) {
+  constexpr int WTP = TP * 16, WTQ = TQ * 16;
+  const GemmArgs &g = prm.g;
+  const int lane = lane_here();
+  const int wp = wave % WP, wq = wave / WP;
+  const int pc = p0 + wp * WTP, qc = q0 + wq * WTQ;
+  const EpilogueScalars sc(g);
+  const AuxTile at(prm, sc, pc, qc, NP, NQ, bt, q0 / WTQ + wq, prm.tiles_q * WQ);
+  const bool bf16 = g.d_type == CUDA_R_16BF;
+  const int grp = lane >> 4, first = (grp & 1) ? 4 * grp + 12 : 4 * grp;  // the lane's first P index inside a pair
+  const int vd_in = ((lane & 15) * at.d_sq + first) * 2, vx_in = ((lane & 15) * at.x_sq + first) * 2;
+  const char *bias = MODE == 1 && g.bias ? (const char *)g.bias + g.bias_sb * bt * (g.bias_type == CUDA_R_32F ? 4 : 2) : nullptr;
+#pragma unroll
+  for (int a = 0; a < TP; a += 2) {
+    const int p = pc + a * 16 + first;  // the lane's eight P indices exist or do not (their number is a multiple of 8)
+    const int vd = p < NP ? vd_in : kStoreNowhere, vx = p < NP ? vx_in : kStoreNowhere;
+    float pb[8], sum[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) pb[e] = sum[e] = 0.0f;
+    if (MODE == 1 && bias) {
+      const int at_p = min(p, NP - 8);
+      if (g.bias_type == CUDA_R_32F) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) pb[e] = ((const float *)bias)[at_p + e];
+      } else {
+        uint32_t raw[4];
+        if (((uintptr_t)bias & 15) == 0) {
+          const v4i t = *(const v4i *)(bias + at_p * 2);
+#pragma unroll
+          for (int d = 0; d < 4; d++) raw[d] = (uint32_t)t[d];
+        } else {
+#pragma unroll
+          for (int d = 0; d < 4; d++) raw[d] = ((const uint16_t *)bias)[at_p + 2 * d] | (uint32_t)((const uint16_t *)bias)[at_p + 2 * d + 1] << 16;
+        }
+        const bool bias_bf16 = g.bias_type == CUDA_R_16BF;
+#pragma unroll
+        for (int d = 0; d < 4; d++) { pb[2 * d] = low_half(raw[d], bias_bf16); pb[2 * d + 1] = high_half(raw[d], bias_bf16); }
+      }
+    }
+    // (the pair's aux pieces in one burst)
+    v4i x_in[TQ];
+    if constexpr (MODE == 2) {
+#pragma unroll
+      for (int b = 0; b < TQ; b++) x_in[b] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(at.rs_x, vx, (b * 16 * at.x_sq + a * 16) * 2, 0));
+    }
+#pragma unroll
+    for (int b = 0; b < TQ; b++) {
+      float y[8];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const uint32_t lo = f2bits(at.factor * bits2f((uint32_t)to_bits(acc[a][b][e]))), hi = f2bits(at.factor * bits2f((uint32_t)to_bits(acc[a + 1][b][e])));
+#if defined(__HIP_DEVICE_COMPILE__)
+        const v2u s = __builtin_amdgcn_permlane16_swap(lo, hi, false, false);
+        y[e] = bits2f(s[0]); y[4 + e] = bits2f(s[1]);
+#else
+        y[e] = bits2f(lo); y[4 + e] = bits2f(hi);
+#endif
+      }
+      if constexpr (MODE == 1) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) y[e] += pb[e];
+        v4i keep;
+#pragma unroll
+        for (int d = 0; d < 4; d++) keep[d] = (int)pack_halves(y[2 * d], y[2 * d + 1], bf16);
+        buffer_store_b128_guarded(keep, at.rs_x, vx, (b * 16 * at.x_sq + a * 16) * 2);
+#pragma unroll
+        for (int e = 0; e < 8; e++) y[e] = gelu_tanh(y[e]) * sc.sd;
+      } else {
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+          y[2 * d] *= dgelu_tanh(low_half((uint32_t)x_in[b][d], bf16));
+          y[2 * d + 1] *= dgelu_tanh(high_half((uint32_t)x_in[b][d], bf16));
+        }
+        // (columns past the end hold products of some column)
+        const bool counts = qc + b * 16 + (lane & 15) < NQ;
+#pragma unroll
+        for (int e = 0; e < 8; e++) sum[e] += counts ? y[e] : 0.0f;
+      }
+      v4i pk;
+#pragma unroll
+      for (int d = 0; d < 4; d++) pk[d] = (int)pack_halves(y[2 * d], y[2 * d + 1], bf16);
+      buffer_store_b128_guarded(pk, at.rs_d, vd, (b * 16 * at.d_sq + a * 16) * 2);
+      __builtin_amdgcn_sched_barrier(0);  // one pair at a time: what the scheduler hoists across them spills
+    }
+    if (MODE == 2 && at.sums) {  // over the 16 columns of a lane group
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        sum[e] += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(sum[e]), 0x128 /* row_ror:8 */, 0xF, 0xF, true));
+        sum[e] += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(sum[e]), 0x124, 0xF, 0xF, true));
+        sum[e] += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(sum[e]), 0x122, 0xF, 0xF, true));
+        sum[e] += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(sum[e]), 0x121, 0xF, 0xF, true));
+      }
+      if ((lane & 15) == 0 && p < NP) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) at.sums[p + e] = sum[e];
+      }
+    }
+  }
+}
+
 // The epilogues that store straight from the accumulators; false: this problem needs the general one
 template <int KIND, int WP, int WQ, int TP, int TQ, class AccV>
 __device__ __forceinline__ bool mfma16_store_direct(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt, int wave) {
@@ -362,6 +465,13 @@ __device__ __forceinline__ bool mfma16_store_direct(const MfmaParams &prm, AccV 
     }
   }
   const MfmaParams &late = args_again(prm);
+  if constexpr (kind_is_h16(KIND)) {
+    if (__builtin_expect(g.act > ACT_GELU, 0)) {
+      if (g.act == ACT_GELU_KEPT) mfma16_store_aux<WP, WQ, TP, TQ, 1>(late, acc, p0, q0, NP, NQ, bt, wave);
+      else mfma16_store_aux<WP, WQ, TP, TQ, 2>(late, acc, p0, q0, NP, NQ, bt, wave);
+      return true;
+    }
+  }
   if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
       (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F)) {
 #define ZLUDA_EPI16(DT_, ACT_, EDGE_) mfma16_store_f<KIND, WP, WQ, TP, TQ, DT_, ACT_, EDGE_>(late, acc, p0, q0, NP, NQ, bt, wave)

@@ -48,7 +48,7 @@ __device__ __forceinline__ bool w4_stream_d_i32(const GemmArgs &g) {
 }
 
 // the epilogue an instantiation carries; the planner sends it the problems that one serves (w4_epilogue_class)
-enum { W4_EPI_I32 = 0, W4_EPI_BF16 = 1, W4_EPI_BF16_GELU = 2 };
+enum { W4_EPI_I32 = 0, W4_EPI_BF16 = 1, W4_EPI_BF16_GELU = 2, W4_EPI_GELU_AUX = 3 };  // (the last: GELU with its input kept, 16-bit D)
 
 // one accumulator element, AGPR -> VGPR
 template <class T>
@@ -110,7 +110,8 @@ struct W4Staged {
 // code: one FMA per element, then the activation (ACT fixed at compile time) with D's scale folded into it.
 // QV: the problem has a scale vector along Q (one more multiplication per element, which problems without one are spared).
 // EDGE: the tile hangs over the end of P (its masks cost the whole tiles of fp8 8192^3 2 us: a body of its own).
-template <int KIND, int ACT, bool EDGE, bool QV, int WTP, int WTQ, int TP, int TQ, class AccV>
+// KEPT: the input of the activation (GELU) goes to the aux matrix as well.
+template <int KIND, int ACT, bool KEPT, bool EDGE, bool QV, int WTP, int WTQ, int TP, int TQ, class AccV>
 __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt,
                                              int wp, int wq, const EpilogueScalars &scalars, const W4Staged &st) {
   const GemmArgs &g = prm.g;
@@ -221,6 +222,14 @@ __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[
   const int first = (grp & 1) ? 4 * grp + 12 : 4 * grp;  // the lane's first P index inside a pair of tiles
   const int voff16 = ((lane & 15) * d_sq + first) * 2;
   const int p_left = NP - pc;  // P indices from the wave tile's corner to the end
+  __amdgpu_buffer_rsrc_t rs_x = rs;
+  int x_sq = 0, voff_x = 0;
+  if constexpr (KEPT) {
+    x_sq = (int)g.aux_sj;  // (column-major; < kNarrowPitch)
+    const int64_t x_corner = (int64_t)qc * x_sq + pc;
+    rs_x = __builtin_amdgcn_make_buffer_rsrc((char *)g.aux + (g.aux_sb * bt + x_corner) * 2, 0, tile_window_bytes(x_sq, NP, NQ, x_corner, 2), 0x00020000);
+    voff_x = ((lane & 15) * x_sq + first) * 2;
+  }
 #pragma unroll
   for (int b = 0; b < TQ; b++) {
     // The column's accumulators first, by explicit reads (left to itself the register allocator parks most accumulators
@@ -241,6 +250,46 @@ __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[
         if constexpr (QV) accf *= qs[b];
         x[a][e] = __builtin_fmaf(accf, ps[a][e], pb[a][e]);
       }
+    // bf16 or f16 output: one uniform branch per tile column
+    auto pack_store = [&](auto bf16_c, __amdgpu_buffer_rsrc_t window, int voff16, int pitch) __attribute__((always_inline)) {
+      constexpr bool TO_BF16 = decltype(bf16_c)::value != 0;
+#pragma unroll
+      for (int a = 0; a < TP; a += 2) {
+        uint32_t lo[2], hi[2];  // tile a, tile a + 1
+        if constexpr (TO_BF16) {
+          lo[0] = pack_bf16x2(x[a][0], x[a][1]); lo[1] = pack_bf16x2(x[a][2], x[a][3]);
+          hi[0] = pack_bf16x2(x[a + 1][0], x[a + 1][1]); hi[1] = pack_bf16x2(x[a + 1][2], x[a + 1][3]);
+        } else {
+          lo[0] = pack_f16x2(x[a][0], x[a][1]); lo[1] = pack_f16x2(x[a][2], x[a][3]);
+          hi[0] = pack_f16x2(x[a + 1][0], x[a + 1][1]); hi[1] = pack_f16x2(x[a + 1][2], x[a + 1][3]);
+        }
+        v4i pk;
+#if defined(__HIP_DEVICE_COMPILE__)
+        const v2u s0 = __builtin_amdgcn_permlane16_swap(lo[0], hi[0], false, false);
+        const v2u s1 = __builtin_amdgcn_permlane16_swap(lo[1], hi[1], false, false);
+        pk = v4i{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
+#else
+        pk = v4i{(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
+#endif
+        const int soff = (b * 16 * pitch + a * 16) * 2;
+        if constexpr (!EDGE) {
+          buffer_store_b128_guarded(pk, window, voff16, soff);
+        } else {
+          const int left = w4_vector_here(p_left - a * 16 - first);
+          buffer_store_b128_guarded(pk, window, left >= 8 ? voff16 : kStoreNowhere, soff);
+          if (!KEPT && p_left > a * 16 && p_left < a * 16 + 32 && (p_left & 7)) {  // (uniform)
+#pragma unroll
+            for (int e = 0; e < 7; e++)
+              __builtin_amdgcn_raw_buffer_store_b16((short)(pk[e >> 1] >> (16 * (e & 1))), window, left < 8 && e < left ? voff16 + e * 2 : kStoreNowhere, soff, 0);
+          }
+        }
+      }
+    };
+    // the aux matrix takes the column as it is, D what becomes of it
+    if constexpr (KEPT) {
+      if (to_bf16) pack_store(std::integral_constant<int, 1>{}, rs_x, voff_x, x_sq);
+      else pack_store(std::integral_constant<int, 0>{}, rs_x, voff_x, x_sq);
+    }
     if constexpr (ACT == ACT_GELU) {
       // x * sigmoid(2u) * sd (gelu_tanh of numeric.hpp) with sd folded into the reciprocal: x / ((1 + e) / sd)
       const float c0 = -2.0f * 0.7978845608028654f * 1.4426950408889634f, c1 = 0.044715f * c0;
@@ -282,42 +331,7 @@ __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[
           for (int e = 0; e < 4; e++) x[a][e] = __builtin_amdgcn_fmed3f(x[a][e], clip_lo, clip_hi);
       }
     }
-    // bf16 or f16 output: one uniform branch per tile column
-    auto pack_store = [&](auto bf16_c) __attribute__((always_inline)) {
-      constexpr bool TO_BF16 = decltype(bf16_c)::value != 0;
-#pragma unroll
-      for (int a = 0; a < TP; a += 2) {
-        uint32_t lo[2], hi[2];  // tile a, tile a + 1
-        if constexpr (TO_BF16) {
-          lo[0] = pack_bf16x2(x[a][0], x[a][1]); lo[1] = pack_bf16x2(x[a][2], x[a][3]);
-          hi[0] = pack_bf16x2(x[a + 1][0], x[a + 1][1]); hi[1] = pack_bf16x2(x[a + 1][2], x[a + 1][3]);
-        } else {
-          lo[0] = pack_f16x2(x[a][0], x[a][1]); lo[1] = pack_f16x2(x[a][2], x[a][3]);
-          hi[0] = pack_f16x2(x[a + 1][0], x[a + 1][1]); hi[1] = pack_f16x2(x[a + 1][2], x[a + 1][3]);
-        }
-        v4i pk;
-#if defined(__HIP_DEVICE_COMPILE__)
-        const v2u s0 = __builtin_amdgcn_permlane16_swap(lo[0], hi[0], false, false);
-        const v2u s1 = __builtin_amdgcn_permlane16_swap(lo[1], hi[1], false, false);
-        pk = v4i{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
-#else
-        pk = v4i{(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
-#endif
-        const int soff = (b * 16 * d_sq + a * 16) * 2;
-        if constexpr (!EDGE) {
-          buffer_store_b128_guarded(pk, rs, voff16, soff);
-        } else {
-          const int left = w4_vector_here(p_left - a * 16 - first);
-          buffer_store_b128_guarded(pk, rs, left >= 8 ? voff16 : kStoreNowhere, soff);
-          if (p_left > a * 16 && p_left < a * 16 + 32 && (p_left & 7)) {  // (uniform)
-#pragma unroll
-            for (int e = 0; e < 7; e++)
-              __builtin_amdgcn_raw_buffer_store_b16((short)(pk[e >> 1] >> (16 * (e & 1))), rs, left < 8 && e < left ? voff16 + e * 2 : kStoreNowhere, soff, 0);
-          }
-        }
-      }
-    };
-    if (to_f32) {
+    if (!KEPT && to_f32) {
       const int voff32 = ((lane & 15) * d_sq + 4 * grp) * 4;
 #pragma unroll
       for (int a = 0; a < TP; a++) {
@@ -335,9 +349,9 @@ __device__ __forceinline__ void w4_store_f16(const MfmaParams &prm, AccV (&acc)[
         }
       }
     } else if (to_bf16) {
-      pack_store(std::integral_constant<int, 1>{});
+      pack_store(std::integral_constant<int, 1>{}, rs, voff16, d_sq);
     } else {
-      pack_store(std::integral_constant<int, 0>{});
+      pack_store(std::integral_constant<int, 0>{}, rs, voff16, d_sq);
     }
     __builtin_amdgcn_sched_barrier(0);  // one tile column at a time: what the scheduler hoists across them costs registers
   }
@@ -777,15 +791,16 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
       if (stream_d) w4_store_i32<WTP, WTQ, 2>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, ialpha);
       else w4_store_i32<WTP, WTQ, 0>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, ialpha);
     } else {
-      constexpr int ACT = EPI == W4_EPI_BF16_GELU ? ACT_GELU : ACT_NONE;
+      constexpr int ACT = EPI == W4_EPI_BF16_GELU || EPI == W4_EPI_GELU_AUX ? ACT_GELU : ACT_NONE;
+      constexpr bool KEPT = EPI == W4_EPI_GELU_AUX;
       const bool qv = staged.has[3] || staged.has[4];
       if (p0 + BP <= NP) {
-        if (qv) w4_store_f16<KIND, ACT, false, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
-        else w4_store_f16<KIND, ACT, false, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+        if (qv) w4_store_f16<KIND, ACT, KEPT, false, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+        else w4_store_f16<KIND, ACT, KEPT, false, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
       } else if (qv) {
-        w4_store_f16<KIND, ACT, true, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+        w4_store_f16<KIND, ACT, KEPT, true, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
       } else {
-        w4_store_f16<KIND, ACT, true, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+        w4_store_f16<KIND, ACT, KEPT, true, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
       }
     }
   };

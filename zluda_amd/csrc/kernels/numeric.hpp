@@ -94,6 +94,15 @@ __device__ __forceinline__ float gelu_tanh(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z));
 }
 
+// d/dx of the tanh form of GELU
+__device__ __forceinline__ float dgelu_tanh(float x) {
+  const float k0 = 0.7978845608028654f, k1 = 0.044715f;
+  const float u = k0 * (x + k1 * x * x * x);
+  // tanh(u) = 1 - 2 / (1 + exp(2u)); exp(2u) = inf gives 1, 0 gives -1
+  const float t = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(2.0f * 1.4426950408889634f * u));
+  return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * k0 * (1.0f + 3.0f * k1 * x * x);
+}
+
 // element loads for C / bias / generic operands
 __device__ __forceinline__ float load_elem(const void *base, uint32_t type, int64_t idx) {
   switch (type) {

@@ -67,6 +67,10 @@ uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws,
       prm.tiles_p = (np + 255) / 256; prm.tiles_q = (nq + 255) / 256;
       prm.group_p = 8;
       prm.splits = 1; prm.split_stages = 0; prm.groups = 0; prm.ws = nullptr;
+      if (l.g.act > ACT_GELU) {
+        if (plan.kernel != ZLUDA_KERNEL_MFMA_H16 || l.g.act != ACT_GELU_KEPT || epi != W4_CLASS_BF16) return CUBLAS_STATUS_INTERNAL_ERROR;
+        return l.g.a_type == CUDA_R_16BF ? launch_mfma_w4_bf16(prm, W4_CLASS_GELU_AUX, plan.grid_x, s) : launch_mfma_w4_f16(prm, W4_CLASS_GELU_AUX, plan.grid_x, s);
+      }
       return plan.kernel == ZLUDA_KERNEL_MFMA_I8     ? launch_mfma_w4_i8(prm, epi, plan.grid_x, s)
              : plan.kernel == ZLUDA_KERNEL_MFMA_MXF4 ? launch_mfma_w4_mxf4(prm, epi, plan.grid_x, s)
              : plan.kernel == ZLUDA_KERNEL_MFMA_H16  ? (l.g.a_type == CUDA_R_16BF ? launch_mfma_w4_bf16(prm, epi, plan.grid_x, s)
@@ -85,7 +89,7 @@ uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws,
   prm.tiles_p = (np + v.bp - 1) / v.bp;
   prm.tiles_q = (nq + v.bq - 1) / v.bq;
   prm.group_p = 8;
-  prm.splits = 1; prm.split_stages = 0; prm.groups = 0; prm.ws = nullptr;
+  prm.splits = 1; prm.split_stages = 0; prm.groups = 0; prm.ws = l.g.act == ACT_DGELU ? ws : nullptr;
   // The short-K form: fewer workgroups than tiles, for which the plan alone counts (it may have been made for another number of CUs).
   if (plan.variant == 3 && plan.kernel == ZLUDA_KERNEL_MFMA_H16 && plan.grid_y == 1 && plan.grid_z == 1 && plan.grid_x > 0 && (plan.grid_x & 7) == 0 &&
       plan.grid_x < (uint64_t)prm.tiles_p * prm.tiles_q * l.g.batch && mfma_short_k_operands(l)) {
@@ -149,7 +153,7 @@ uint32_t launch_tr(const Lowered &l, const zluda_gemm_plan &plan, void *ws, uint
   prm.tiles_p = (np + v.bp - 1) / v.bp;
   prm.tiles_q = (nq + v.bq - 1) / v.bq;
   prm.group_p = 8;
-  prm.splits = 1; prm.split_stages = 0; prm.groups = 0; prm.ws = nullptr;
+  prm.splits = 1; prm.split_stages = 0; prm.groups = 0; prm.ws = l.g.act == ACT_DGELU ? ws : nullptr;
   if ((uint32_t)(prm.tiles_p * prm.tiles_q) != plan.grid_x) return CUBLAS_STATUS_INVALID_VALUE;
   // the same tiles, transposed by the LDS reads: 128 K bytes per stage
   const bool lds_reads = tr_lds_reads(l, (int)plan.variant, (uint64_t)plan.grid_x * plan.grid_y * std::max(plan.grid_z, 1u), plan.grid_z,
@@ -379,10 +383,18 @@ uint32_t launch_planned(const zluda_gemm_problem *p, const zluda_gemm_plan *plan
   if (!family_supports(plan->kernel, l)) return CUBLAS_STATUS_INVALID_VALUE;
   if (ws_size < plan->workspace) return CUBLAS_STATUS_INVALID_VALUE;
   if (zluda_gemm_device_cu_count() == 0) return CUBLAS_STATUS_NOT_INITIALIZED;
-  // GELU_AUX: the GEMM kernel writes the GELU input where the caller wants it kept, unscaled; the second pass
-  // below reads it back and writes D.  (DGELU: the kernel writes D as usual and the second pass rewrites it.)
+  // The kernels behind the matmul on its stream take over its scratch: what the plan counted, however much there is, so that
+  // a plan that asks for none writes none and the shares of a sum (its last bits) follow from the plan alone.
+  const uint64_t sums = ws && !(((uintptr_t)ws) & 15) ? std::min<uint64_t>(ws_size, plan->workspace) : 0;
+  // The epilogues with an aux matrix: in the GEMM kernel's own where it has them (and the scratch for the sums).  Elsewhere the kernel sees
+  // a plain problem.  GELU_AUX: it writes the GELU input where the caller wants it kept, unscaled; the second pass below reads
+  // it back and writes D.  (DGELU: the kernel writes D as usual and the second pass rewrites it.)
   const GemmArgs whole = l.g;
-  if (whole.aux_mode == 1) {
+  const uint32_t aux_shares = whole.aux_bgrad && aux_in_epilogue(l, *plan, false) ? aux_sum_shares(l, *plan) : 0;
+  const bool aux_fused = aux_in_epilogue(l, *plan, false) && (uint64_t)aux_shares * whole.M * whole.batch * 4 <= sums;
+  if (aux_fused) {
+    l.g.act = whole.aux_mode == 1 ? ACT_GELU_KEPT : ACT_DGELU;
+  } else if (whole.aux_mode == 1) {
     l.g.D = whole.aux;
     l.g.d_si = whole.aux_si; l.g.d_sj = whole.aux_sj; l.g.d_sb = whole.aux_sb;
     l.g.d_scale = nullptr;
@@ -412,11 +424,10 @@ uint32_t launch_planned(const zluda_gemm_problem *p, const zluda_gemm_plan *plan
   case ZLUDA_KERNEL_MFMA_TR8: case ZLUDA_KERNEL_MFMA_TR16: case ZLUDA_KERNEL_MFMA_TR32: st = launch_tr(l, *plan, ws, ws_size, s); break;
   default: return CUBLAS_STATUS_NOT_SUPPORTED;
   }
-  // The kernels behind the matmul on its stream take over its scratch: what the plan counted, however much there is, so that
-  // a plan that asks for none writes none and the shares of a sum (its last bits) follow from the plan alone.
-  const uint64_t sums = ws && !(((uintptr_t)ws) & 15) ? std::min<uint64_t>(ws_size, plan->workspace) : 0;
   if (st == CUBLAS_STATUS_SUCCESS && l.g.bgrad_src) st = launch_bgrad(l.g, ws, sums, s);
-  if (st == CUBLAS_STATUS_SUCCESS && whole.aux_mode) st = launch_aux(whole, ws, sums, s);
+  if (st == CUBLAS_STATUS_SUCCESS && whole.aux_mode && !aux_fused) st = launch_aux(whole, ws, sums, s);
+  if (st == CUBLAS_STATUS_SUCCESS && aux_fused && whole.aux_bgrad)
+    st = finish_sums(ws, (int)aux_shares, whole.M, whole.batch, false, whole.bgrad, whole.bias_type, whole.bias_sb, s);
   return st;
 }
 

@@ -749,6 +749,39 @@ static uint64_t row_sum_workspace(const GemmArgs &g, uint64_t workspace_size, ui
   return s > 1 ? (uint64_t)s * rows * g.batch * 4 : 0;
 }
 
+// The forms the epilogues with an aux matrix are instantiated for: 16-bit operands on the tile kernels up to a size of the wave tile, unsplit, 16-bit D and aux that the
+// 16-byte stores of eight rows fit.  us with a pass behind the matmul and without: bf16 8192 x 4096 x 2048 GELU_AUX_BIAS 133 -> 122
+// (the product alone 110), A:N B:N DGELU_BGRAD 153 -> 138 (115); 1000 x 700 x 496 8.8 -> 6.6 and 17.3 -> 12.7; 2048 x 1000 x 1024 14.5 -> 11.0
+// and 21.8 -> 16.3.
+bool aux_in_epilogue(const Lowered &l, const zluda_gemm_plan &plan, bool dry) {
+  const GemmArgs &g = l.g;
+  if (!g.aux_mode || (plan.kernel != ZLUDA_KERNEL_MFMA_H16 && plan.kernel != ZLUDA_KERNEL_MFMA_TR16)) return false;
+  if (g.d_type != CUDA_R_16F && g.d_type != CUDA_R_16BF) return false;
+  if (plan.grid_z > 1 || plan.swapped || g.d_si != 1 || g.aux_si != 1) return false;
+  if (g.beta_mode != SCALAR_VALUE || (!dry && g.beta_val.f != 0.0f)) return false;
+  if (g.alpha_mode == VECTOR_DEV || g.a_scale_mode == SCALE_OUTER_VEC || g.b_scale_mode == SCALE_OUTER_VEC) return false;
+  if (g.M & 7) return false;
+  const int64_t pitches = g.d_sj | g.aux_sj | (g.batch > 1 ? g.d_sb | g.aux_sb : 0);
+  if ((pitches & 7) || g.d_sj >= kNarrowPitch || g.aux_sj >= kNarrowPitch) return false;
+  if (!dry && (((uintptr_t)g.D | (uintptr_t)g.aux) & 15)) return false;
+  if (plan.kernel == ZLUDA_KERNEL_MFMA_H16) {
+    if (plan.variant >= (uint32_t)kNumMfmaVariants) return false;
+    const MfmaVariant &v = kMfmaVariants[plan.variant];
+    if (v.w4) return g.aux_mode == 1 && w4_epilogue_class(l, dry) == W4_CLASS_BF16;  // (the gradient: of operands that are not K-contiguous)
+    const MfmaVariant &w = plan.variant == 2 && plan.block == 512 ? kMfmaEightWaves : v;
+    return plan.grid_x == ceil_div(g.M, v.bp) * ceil_div(g.N, v.bq) &&  // (not the short-K form)
+           (v.m16 || aux_on_wave_tile32(w.bp / w.wp, w.bq / w.wq));
+  }
+  if (plan.variant >= (uint32_t)kNumTrVariants) return false;
+  const TrVariant &t = kTrVariants[plan.variant];
+  return t.m16 || aux_on_wave_tile32(t.bp / t.wp, t.bq / t.wq);
+}
+
+uint32_t aux_sum_shares(const Lowered &l, const zluda_gemm_plan &plan) {
+  if (plan.kernel == ZLUDA_KERNEL_MFMA_H16) return ceil_div(l.g.N, kMfmaVariants[plan.variant].bq) * kMfmaVariants[plan.variant].wq;
+  return ceil_div(l.g.N, kTrVariants[plan.variant].bq) * kTrVariants[plan.variant].wq;
+}
+
 uint32_t transposing_under_generic(const Lowered &l) {
   const uint32_t family = transposing_family(l, true);
   if (!family || transposing_family(l, false)) return 0;
@@ -952,5 +985,9 @@ extern "C" uint32_t zluda_gemm_plan_problem(const zluda_gemm_problem *p, uint32_
   }
   // (the sums run behind the matmul and its reduction, in the same scratch)
   plan->workspace = std::max(plan->workspace, row_sum_workspace(l.g, p->workspace_size, cu_count));
+  if (l.g.aux_bgrad && aux_in_epilogue(l, *plan, true)) {
+    const uint64_t sums = (uint64_t)aux_sum_shares(l, *plan) * l.g.M * l.g.batch * 4;
+    if (sums <= p->workspace_size) plan->workspace = std::max(plan->workspace, sums);
+  }
   return CUBLAS_STATUS_SUCCESS;
 }

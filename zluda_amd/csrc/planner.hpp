@@ -92,7 +92,7 @@ constexpr int kDecodeAutoMaxTokensStream = 48;  // ... and when the LDS-streamin
 
 // the fast epilogues the four-wave kernel is instantiated with (gemm_mfma_w4.hpp: W4_EPI_*); what else a problem asks for
 // runs on variant 8
-enum { W4_CLASS_NONE = -1, W4_CLASS_I32 = 0, W4_CLASS_BF16 = 1, W4_CLASS_BF16_GELU = 2 };
+enum { W4_CLASS_NONE = -1, W4_CLASS_I32 = 0, W4_CLASS_BF16 = 1, W4_CLASS_BF16_GELU = 2, W4_CLASS_GELU_AUX = 3 };
 
 struct Lowered {
   GemmArgs g;
@@ -134,6 +134,11 @@ bool tr_lds_reads(const Lowered &l, int variant, uint64_t groups, uint32_t split
 // Row sums along the longer stride (bias gradients): how many workgroups share the `len` terms of each of `rows` sums, given
 // scratch for shares * rows * batch partial sums of 4 bytes; 1: no scratch is used
 uint32_t row_sum_shares(int64_t rows, int64_t len, int64_t batch, uint64_t workspace_size, uint32_t cus);
+
+// Whether the kernel of `plan` carries the aux epilogue of the problem (GELU_AUX, DGELU) itself; `dry`: as above.  And how many partial sums
+// of each row of D it writes for DGELU_BGRAD, one per wave along Q: 4 bytes each, batches, then sums, then rows.
+bool aux_in_epilogue(const Lowered &l, const zluda_gemm_plan &plan, bool dry);
+uint32_t aux_sum_shares(const Lowered &l, const zluda_gemm_plan &plan);
 
 // Lowers `p` with its real pointers and enqueues the kernel `plan` names on `stream` (a hipStream_t).
 // `ws` / `ws_size`: device scratch, at least plan->workspace bytes, of which plan->workspace are used (split-K partial tiles,
