@@ -17,8 +17,11 @@
 //     between neighbouring lane groups): no LDS staging.
 //   * A fragment is 16 rows x 128 K bytes: lane l holds row l%16 and the K bytes of lane group l/16 --
 //     fp8: chunks 2*(l/16) and 2*(l/16)+1 of the 128-byte row (one instruction per stage and tile pair);
-//     int8: chunks l/16 and 4 + l/16 (two instructions, K halves).  Both operands use the same assignment,
-//     which is all a dot product needs.
+//     int8 and 16-bit: the same two chunks, one for each of two instructions.  Both operands use the same assignment,
+//     which is all a dot product needs.  (A ds_read_b128 is served in four parts, the lanes {0-3, 12-15, 20-23, 24-27},
+//     {4-7, 8-11, 16-19, 28-31} and the same of the upper half: two lane groups in each, whose chunks have to be two apart
+//     for the swizzle to keep them on different banks.  With the chunks l/16 and 4 + l/16 every read took twice its time; the loops
+//     wait for other things more: bf16 4096^3 111.6 -> 109.9 us, 8192^3 775 -> 772, int8 8192^3 413 -> 411.)
 //   * A stage is walked in four sub-steps over (P half, Q half) of the wave tile in snake order, so that
 //     consecutive sub-steps share one half and only the other is fetched:
 //         even stages: (P0,Q0) (P0,Q1) | (P1,Q1) (P1,Q0)        odd stages: (P0,Q1) (P0,Q0) | (P1,Q0) (P1,Q1)
@@ -508,6 +511,9 @@ __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&
 // An MC operand's block of LDS (head of this file): the K row of its first lane, and where K row `k` & 36 lies in its block
 __host__ __device__ constexpr int mc_block_k(int blk) { return (blk & 3) + 8 * ((blk >> 2) & 3) + 32 * (blk >> 4); }
 constexpr int kMcPitch = 1056;
+// The chunk swizzle of a K-contiguous operand beside an MC one, whose lane groups hold the K bytes 16 g and 64 + 16 g of a stage: the
+// neighbouring chunks of two lane groups fall on different banks with this one
+__device__ __forceinline__ int swz_mixed(int r) { return r & 6; }
 typedef short v4s_tr __attribute__((ext_vector_type(4)));
 
 // four K elements of one row of an MC operand: 16 lanes, each with the address of 8 bytes (lane 4r + c: K row r, elements
@@ -598,7 +604,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   // slot ^ swizzle(row)
   const int dr = lane / CPR, dslot = lane % CPR;
   const int drow = wave * RPW + dr;  // passes advance by RPP, a multiple of 32: same swizzle
-  const int dcg = dslot ^ swz(drow);
+  const int dcg = dslot ^ (PMC || QMC ? swz_mixed(drow) : swz(drow));
   int voffP[LP], voffQ[LQ];
   // MC: an instruction fills a block; lane l -> K row and 16-byte piece of it.  A piece past the last one of the row index
   // loads that one (rows past the end of D are dropped), which holds at least one element of the operand: with the
@@ -657,7 +663,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
 #pragma unroll
     for (int kk = 0; kk < 2; kk++) {
       const int row = par * 16 + r16;
-      const int ch = (KIND == KIND_F8 ? 2 * g4 + kk : 4 * kk + g4) ^ swz(row);
+      const int ch = PMC || QMC ? (4 * kk + g4) ^ swz_mixed(row) : (2 * g4 + kk) ^ swz(row);
       fragP[par][kk] = (wp * WTP + row) * CPR + ch;
       // (summed in this order: the other one has the compiler hoist two more addresses than the loop has registers for, and
       // their reloads cost 7 % of int8 and bf16 8192 x 4096 x 1024)

@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_short_kernel(MfmaParams prm)
 #pragma unroll
   for (int par = 0; par < 2; par++)
 #pragma unroll
-    for (int kk = 0; kk < 2; kk++) frag_at[par][kk] = (par * 16 + r16) * CPR + ((4 * kk + g4) ^ swz(par * 16 + r16));
+    for (int kk = 0; kk < 2; kk++) frag_at[par][kk] = (par * 16 + r16) * CPR + ((2 * g4 + kk) ^ swz(par * 16 + r16));
   Frag pf[NC][TP], qf[NC][TQ];
   auto load_frags = [&](int slot, int row0, Frag (&f)[NC][4]) {
 #pragma unroll

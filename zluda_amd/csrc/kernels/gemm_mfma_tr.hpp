@@ -22,11 +22,14 @@
 //     dwordx4), 2 v_perm_b32 per 2 x 2 elements, one dword of 2 consecutive K elements per row.
 //     f32: 1 K row x IW row indices per lane; every loaded dword is already one LDS dword (no permute).
 //   * Operand with unit stride along K ("KC"): 16 bytes per lane, ds_write_b128.
-//   * LDS rows have a pitch of 80 bytes and are stored in permuted order, rho(i) = 16 r + ((g + s r) mod 16)
-//     for i = IW g + r, s = 16 / IW.  With that every ds_write_b32 instruction of the transposing path
+//   * LDS rows have a pitch of 80 bytes and are stored in permuted order, rho(i) = 16 r + ((g + 4 r) mod 16)
+//     for i = IW g + r.  With that every ds_write_b32 instruction of the transposing path
 //     hits 64 distinct banks (row pitch 20 dwords: 20 x 16 consecutive rows are 16 distinct multiples
-//     of 4 mod 64) and every ds_read_b128 of 16 consecutive matrix rows hits 16 distinct 16-byte
-//     groups (pitch 5 groups, 5 coprime to 16, rho of 16 consecutive rows distinct mod 16).
+//     of 4 mod 64).  A ds_read_b128 is served in four parts, the lanes {0-3, 12-15, 20-23, 24-27}, {4-7, 8-11, 16-19, 28-31}
+//     and the same of the upper half; over the 32 rows of a fragment either part meets each residue of (g + 4 r) mod 16 once,
+//     i.e. 16 distinct 16-byte groups (pitch 5 groups, 5 coprime to 16).  A fragment of 16 rows has two chunks in each part: those
+//     have to lie two apart.  (With g + 2 r for 128 rows, and neighbouring chunks, half of the LDS cycles of these kernels
+//     were bank conflicts.  us without them: fp8 2048^3 A:N 17.5 -> 17.0, f32 127.8 -> 125.9, int8 4096^3 B:T 73.4 -> 73.2.)
 #pragma once
 #include "gemm_mfma_pipe16.hpp"
 
@@ -35,9 +38,7 @@ namespace zluda_amd {
 // LDS row of matrix row i (0 <= i < ROWS) of a tile operand
 template <int ROWS>
 __device__ __forceinline__ constexpr int tr_rho(int g, int r) {
-  constexpr int IW = ROWS / 16, STEP = 16 / IW;
-  (void)IW;
-  return 16 * r + ((g + STEP * r) & 15);
+  return 16 * r + ((g + 4 * r) & 15);
 }
 template <int ROWS>
 __device__ __forceinline__ int tr_rho_of(int i) {
@@ -238,7 +239,7 @@ struct TrOperand {
 // M16 (int8, f16, bf16): the MFMAs are v_mfma_i32_16x16x64_i8 / v_mfma_f32_16x16x32_f16 / _bf16 with P as operand "A" and the epilogues of
 // gemm_mfma_pipe16.hpp -- the shape that needs less energy per multiply-add, for problems that keep the whole
 // chip busy (see there).  A fragment is then 16 rows x the 64 K bytes of a stage (lane l: row l%16, 16-byte
-// chunk l/16), one MFMA per pair of fragments and stage.
+// chunk l/16 with 1 and 2 exchanged), one MFMA per pair of fragments and stage.
 // KG = 2 (16-bit operands; when: tr_two_k_groups()): two groups of four waves share the workgroup's K range, each with LDS stages of its
 // own; their accumulators meet in LDS.  A stage is much waiting for little work (a barrier, an LDS round trip), and where a CU
 // has one workgroup nobody else fills the gaps: bf16 1024 x 512 x 32003 (128 x 128 tiles, eight shares) 76.8 -> 69 us, 80 x 351 x 2459,
@@ -345,16 +346,17 @@ __global__ __launch_bounds__(WP *WQ * 64 * KG) void gemm_mfma_tr_kernel(MfmaPara
   acc16_v acc16[M16 ? TP16 : 1][M16 ? TQ16 : 1];
   int prow16[M16 ? TP16 : 1], qrow16[M16 ? TQ16 : 1];  // this lane's 16-byte piece of each fragment (v4i units)
   if constexpr (M16) {
-    const int r16 = lane & 15, g4 = lane >> 4;
+    // (the chunks of a pair of lane groups that an LDS access serves together lie two apart, see above)
+    const int r16 = lane & 15, ch = ((lane >> 4) & 1) * 2 + (lane >> 5);
 #pragma unroll
     for (int b = 0; b < TP16; b++) {
       const int i = wp * WTP + b * 16 + r16;
-      prow16[b] = (i / LP * LP + tr_rho_of<LP>(i % LP)) * 5 + g4;
+      prow16[b] = (i / LP * LP + tr_rho_of<LP>(i % LP)) * 5 + ch;
     }
 #pragma unroll
     for (int a = 0; a < TQ16; a++) {
       const int i = wq * WTQ + a * 16 + r16;
-      qrow16[a] = (BP + i / LQ * LQ + tr_rho_of<LQ>(i % LQ)) * 5 + g4;
+      qrow16[a] = (BP + i / LQ * LQ + tr_rho_of<LQ>(i % LQ)) * 5 + ch;
     }
 #pragma unroll
     for (int b = 0; b < TP16; b++)

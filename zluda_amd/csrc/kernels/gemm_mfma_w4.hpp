@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
       const int row = par * 16 + r16;
       // fp8: the lane's 32 bytes of its K group; int8: 16 bytes of each K half; MXFP4: 16 bytes (one scale block of 32
       // elements) of each K step from the lane group's own 32-byte range, so that its two scale bytes are neighbours
-      const int ch = ((KIND == KIND_I8 || H16) ? 4 * kk + g4 : 2 * g4 + kk) ^ swz(row);
+      const int ch = (2 * g4 + kk) ^ swz(row);
       fragP[par][kk] = (wp * WTP + row) * CPR + ch;
       fragQ[par][kk] = (BP + wq * WTQ + row) * CPR + ch;
     }
