@@ -134,6 +134,28 @@ static void check_pipe16_mc(int bp, int bq, int wp, int wq) {
   }
 }
 
+// The same on a ring of more than two stages: a wait of the loop leaves those behind the next one in flight, but nothing where the
+// last stage of K or padding behind it is among them.
+static void check_pipe16_ring(int bp, int bq, int wp, int wq, int nstage) {
+  const Pipe16Counts c = pipe16_counts(bp, bq, wp, wq, nstage);
+  if ((nstage - 1) * c.nload >= 64) fail("vmcnt range", -1, 0, 0, 0, 0);
+  for (int KT = 0; KT <= 3 * nstage + 2; KT++) {
+    std::vector<Ins> log;
+    auto data = [&](int stage) { for (int i = 0; i < c.nload; i++) log.push_back(Ins{DATA, stage}); };
+    for (int s = 0; s < nstage; s++) data(s);
+    if (pipe16_drains_prologue(true, KT, nstage) != (nstage - 1 >= KT - 1)) fail("the prologue's drain", -1, 0, 0, 0, KT);
+    if (!landed(log, log.size(), c.wait_prologue, DATA, 0)) fail("prologue: stage 0 still in flight", -1, 0, 0, 0, KT);
+    if (data_after(log, 0) != c.wait_prologue) fail("prologue: N is not the count of younger data instructions", -1, 0, 0, 0, KT);
+    for (int kt = 0; kt < KT; kt++) {
+      if (pipe16_drains_stage(kt, KT, nstage) != (kt + nstage - 1 >= KT - 1)) fail("a stage's drain", -1, 0, 0, kt, KT);
+      if (!landed(log, log.size(), c.wait_stage, DATA, kt + 1)) fail("next stage still in flight", -1, 0, 0, kt, KT);
+      if (data_after(log, kt + 1) != c.wait_stage) fail("N is not the count of younger data instructions", -1, 0, 0, kt, KT);
+      checked++;
+      data(kt + nstage);
+    }
+  }
+}
+
 // gemm_mfma_tr_kernel: the stages are requested in order, nothing past the last one, kl.  The prologue stores stage 0's registers
 // with stage 1 in flight, trip kt those of stage kt + 1 with stage kt + 2 in flight.
 static void check_tr(int esz) {
@@ -231,6 +253,7 @@ int main() {
   for (int chunks : {1, 2})
     for (bool wide : {false, true}) check_short(chunks, wide);
   for (int v : {1, 3}) check_pipe16_mc(kTrVariants[v].bp, kTrVariants[v].bq, kTrVariants[v].wp, kTrVariants[v].wq);
+  check_pipe16_ring(kTrVariants[1].bp, kTrVariants[1].bq, kTrVariants[1].wp, kTrVariants[1].wq, kTrDeepStages);
   for (int esz : {1, 2, 4}) check_tr(esz);
   printf("%ld waits checked\n", checked);
   return 0;

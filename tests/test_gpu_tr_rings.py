@@ -1,0 +1,33 @@
+"""The two rings of the 128 x 128 tile whose LDS reads transpose, four stages where no CU has more than one workgroup and two elsewhere:
+every position of the ring that K can end at, K tails inside a stage, shares of K of unequal length."""
+import pytest
+
+from oracle.cases import Case
+from zluda_amd import abi as K
+
+pytestmark = pytest.mark.gpu
+BF = dict(a_type=K.CUDA_R_16BF, b_type=K.CUDA_R_16BF, d_type=K.CUDA_R_16BF, compute_type=K.CUBLAS_COMPUTE_32F, scale_type=K.CUDA_R_32F, alpha=0.05)
+# (a stage is 64 elements of K; the form is taken from 11 stages on with one tile to a CU, from 7 on with two)
+SHORT, LONG = [704, 712, 768, 824, 832, 888, 896, 952], [448, 456, 512, 520]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("k,batch", [(k, 1) for k in SHORT] + [(k, 66) for k in LONG])   # 4 and 264 tiles
+def test_every_end_of_the_ring(gpu_api, k, batch, ta, tb):
+    spec = dict(BF, m=200, n=136, k=k, transa=ta, transb=tb, batch=batch)
+    print("case", spec, flush=True)
+    case = Case(spec, 9900 + k)
+    st, got, kernel, variant = case.run_gpu(gpu_api, forced_kernel=K.ZLUDA_KERNEL_MFMA_TR16, forced_variant=1)
+    assert st == 0 and variant == 1
+    case.compare(got, case.run_oracle(), tol=1e-2)   # one rounding to bf16 of sums in another order
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("k", [5632, 5704, 6152])   # eight shares of 11 to 13 stages, the last of 11, 6 and 6
+def test_shares_of_k(gpu_api, k, ta, tb):
+    spec = dict(BF, m=136, n=200, k=k, transa=ta, transb=tb, d_type=K.CUDA_R_32F)
+    print("case", spec, flush=True)
+    case = Case(spec, 9950 + k)
+    st, got, plan = case.run_gpu_plan(gpu_api, K.ZLUDA_KERNEL_MFMA_TR16, 1, workspace_bytes=16 << 20)
+    assert st == 0 and (plan.variant, plan.grid_z) == (1, 8)
+    case.compare(got, case.run_oracle(), tol=1e-3)   # 32-bit sums in another order

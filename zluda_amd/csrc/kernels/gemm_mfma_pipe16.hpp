@@ -35,7 +35,7 @@
 // (16 lanes read 4 K rows x 16 elements; lane i gets the four K elements of row i) transposes on the way into the
 // fragments, so there is no work in registers and no store to LDS.  The kernel of gemm_mfma_tr.hpp, which transposes in
 // registers, spends its stages on that: bf16 8192^3 A:N B:N 1019 us there, 808 here; 4096^3 A:N B:N 110; 128 x 128 tiles,
-// 2048 x 4096 x 8192 A:N B:N 183 and 133 inside a training step.
+// 2048 x 4096 x 8192 A:N B:N 183 and 133 inside a training step.  (The 128 x 128 tile also has a ring of four stages, see mfma_tr_launch.hpp.)
 // LDS layout of such an operand: blocks of 1 KiB, one DMA instruction of a wave each, at a pitch of 1056 bytes.  A block
 // holds the K rows {k, k + 4} (256 elements a row) or {k, k + 4, k + 32, k + 36} (128), and the blocks run over k = 0..3,
 // 8..11, 16..19, ...: a ds_read_b64_tr_b16 takes the rows k..k+3 of four blocks for each of its groups of 16 lanes, 32
@@ -537,7 +537,7 @@ __device__ __forceinline__ void lds_dma16_uncounted(v4i rs, const void *lds_dst,
 #endif
 }
 
-template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, bool PMC = false, bool QMC = false>
+template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, bool PMC = false, bool QMC = false, int NSTAGE = 2>
 __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParams prm) {
   static_assert(!(PMC || QMC) || kind_is_h16(KIND), "the transposing LDS reads are those of 16-bit elements");
   static_assert((!PMC || BP == 256 || BP == 128) && (!QMC || BQ == 256 || BQ == 128), "rows of 1 KiB / 2 or / 4");
@@ -545,7 +545,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   constexpr int ESZ = kind_esz(KIND);          // f16 / bf16: the byte geometry of int8 (v_mfma_f32_16x16x32_*: 16 bytes of K per lane)
   constexpr int NT = WP * WQ * 64, NWV = NT / 64;
   constexpr int BKB = 128, CPR = 8, RPW = 8;
-  constexpr Pipe16Counts PC = pipe16_counts(BP, BQ, WP, WQ);  // (shared with the host program that checks the waits)
+  constexpr Pipe16Counts PC = pipe16_counts(BP, BQ, WP, WQ, NSTAGE);  // (shared with the host program that checks the waits)
   constexpr int RPP = PC.rpp;                  // rows filled per DMA pass of the workgroup
   constexpr int LP = PC.lp, LQ = PC.lq;        // DMA instructions per thread, stage and operand
   constexpr int NLOAD = PC.nload;
@@ -553,7 +553,6 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   constexpr int WTP = BP / WP, WTQ = BQ / WQ, TP = WTP / 16, TQ = WTQ / 16;
   constexpr int HP = TP / 2, HQ = TQ / 2;      // fragments per half of the wave tile
   constexpr int KS = KIND == KIND_F8 ? 1 : 2;  // MFMAs per fragment pair (K halves of the 128-byte stage)
-  constexpr int NSTAGE = 2;
   // one slot in 16-byte words: P rows, then Q rows
   constexpr int P_V4 = PMC ? BP / 8 * (kMcPitch / 16) : BP * CPR, Q_V4 = QMC ? BQ / 8 * (kMcPitch / 16) : BQ * CPR;
   constexpr int STAGE_V4 = P_V4 + Q_V4;
@@ -768,11 +767,10 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   };
 
   // ---- prologue: stages 0 and 1 in flight, stage 0 landed, its first fragments in registers -----------------
-  issue_stage(0, 0);
-  issue_stage(1, STAGE_V4);
+  static_for<NSTAGE>([&](auto s_c) { issue_stage(decltype(s_c)::value, decltype(s_c)::value * STAGE_V4); });
   // (MC: an instruction of the last stage's K tail may hold no K row that exists and retires early, so nothing is counted
   // where one is in flight)
-  if (pipe16_drains_prologue(MC, KT)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (pipe16_drains_prologue(MC, KT, NSTAGE)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   wait_vmcnt_barrier<PC.wait_prologue>();
   load_p_half(0, std::integral_constant<int, 0>{});
   load_q_half(0, std::integral_constant<int, 0>{});
@@ -807,8 +805,11 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     pattern(std::integral_constant<int, DSP - PD * EARLY>{}, std::integral_constant<int, 0>{});
     // every fragment of the stage has been requested: wait for them and for this wave's share of stage
     // kt+1, meet the other waves; then the slot is free and the other one readable
+    if constexpr (NSTAGE > 2) {
+      if (pipe16_drains_stage(kt, KT, NSTAGE)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
     wait_vmcnt_barrier<PC.wait_stage>();
-    // (P1, QB): refill this slot with stage kt+2, P half 0 of stage kt+1 arrives
+    // (P1, QB): refill this slot with stage kt+NSTAGE, P half 0 of stage kt+1 arrives
     load_p_part(so_next, P0{}, I0{}, IL{});
     if constexpr (MC) {
       // (the scheduler does not know the asm for a memory instruction: its place among the MFMAs is written out)
@@ -832,11 +833,23 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   };
 
   int kt = 0;
-  for (; kt + 2 <= KT; kt += 2) {
-    do_stage(kt, 0, STAGE_V4, std::integral_constant<int, 0>{});
-    do_stage(kt + 1, STAGE_V4, 0, std::integral_constant<int, 1>{});
+  if constexpr (NSTAGE == 2) {
+    for (; kt + 2 <= KT; kt += 2) {
+      do_stage(kt, 0, STAGE_V4, std::integral_constant<int, 0>{});
+      do_stage(kt + 1, STAGE_V4, 0, std::integral_constant<int, 1>{});
+    }
+    if (kt < KT) do_stage(kt, 0, STAGE_V4, std::integral_constant<int, 0>{});
+  } else {
+    auto behind = [](int so) { return so == (NSTAGE - 1) * STAGE_V4 ? 0 : so + STAGE_V4; };
+    int so = 0;
+    for (; kt + 2 <= KT; kt += 2) {
+      const int so1 = behind(so), so2 = behind(so1);
+      do_stage(kt, so, so1, std::integral_constant<int, 0>{});
+      do_stage(kt + 1, so1, so2, std::integral_constant<int, 1>{});
+      so = so2;
+    }
+    if (kt < KT) do_stage(kt, so, behind(so), std::integral_constant<int, 0>{});
   }
-  if (kt < KT) do_stage(kt, 0, STAGE_V4, std::integral_constant<int, 0>{});
 
   __builtin_amdgcn_s_waitcnt(0);  // every DMA of the padding stages has landed before the LDS is reused or the wave ends
   if (prm.splits > 1) {

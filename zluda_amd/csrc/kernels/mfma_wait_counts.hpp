@@ -49,14 +49,15 @@ constexpr PipeCounts pipe_counts(bool mx, int bp, int bq, int wp, int wq, int bk
   return c;
 }
 
-// gemm_mfma_pipe16.hpp: two stages of 128 K bytes, eight rows per DMA instruction, no scale instructions
+// gemm_mfma_pipe16.hpp: two stages of 128 K bytes (four in a form for operands along their row index), eight rows per DMA
+// instruction, no scale instructions
 struct Pipe16Counts {
   int rpp, lp, lq, nload;
-  int wait_prologue;  // stages 0 and 1 issued: stage 0 has landed
-  int wait_stage;     // in stage kt, before its slot is refilled: stage kt + 1 has landed (nothing younger is in flight)
+  int wait_prologue;  // stages 0 .. nstage - 1 issued: stage 0 has landed
+  int wait_stage;     // in stage kt, before its slot is refilled: stage kt + 1 has landed (of two stages, nothing younger is in flight)
 };
 
-constexpr Pipe16Counts pipe16_counts(int bp, int bq, int wp, int wq) {
+constexpr Pipe16Counts pipe16_counts(int bp, int bq, int wp, int wq, int nstage = 2) {
   Pipe16Counts c{};
   c.rpp = wp * wq * 8;
   c.lp = bp / c.rpp;
@@ -64,12 +65,16 @@ constexpr Pipe16Counts pipe16_counts(int bp, int bq, int wp, int wq) {
   c.nload = c.lp + c.lq;
   c.wait_prologue = c.nload;
   c.wait_stage = 0;
+  c.wait_prologue += (nstage - 2) * c.nload;
+  c.wait_stage += (nstage - 2) * c.nload;
   return c;
 }
 
 // The form of gemm_mfma_pipe16.hpp whose operands lie along their row index ("MC"): an instruction of the last stage may hold
-// no K row that exists.  The prologue, the one place that counts, waits for everything where stage 0 or 1 is that stage.
-constexpr bool pipe16_drains_prologue(bool mc, int kt) { return mc && kt <= 2; }
+// no K row that exists.  Where that stage or one behind it is in flight the prologue waits for everything, and so does a stage of a ring of
+// more than two slots.
+constexpr bool pipe16_drains_prologue(bool mc, int kt, int nstage = 2) { return mc && kt <= nstage; }
+constexpr bool pipe16_drains_stage(int stage, int kt, int nstage) { return stage + nstage >= kt; }
 
 // gemm_mfma_tr.hpp leaves its waits to the compiler, which counts: before the LDS stores of trip kt (stage kt + 1's
 // registers) it waits until only stage kt + 2's loads are outstanding.  Stages hold 64 K bytes; nothing past the last one that

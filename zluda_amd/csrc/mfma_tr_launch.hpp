@@ -72,6 +72,17 @@ uint32_t launch_tr_f32(const MfmaParams &prm, const zluda_gemm_plan &plan, bool 
 template <int KIND>
 inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s) {
   const dim3 grid(plan.grid_x, plan.grid_y, plan.grid_z > 1 ? plan.grid_z : 1);
+  // One workgroup to a CU: four stages of 33 KiB instead of two, all but the one that is multiplied on their way (a stage's time is far
+  // below a round trip to memory; with two workgroups the other one fills the gaps, and two rings of four do not fit).  bf16, us:
+  // 2048^3 A:N B:N 33.4 -> 25.7, A:N B:T 32.7 -> 25.2, 1024 x 4096 x 4096 60.6 -> 44.3, 1000^3 (64 tiles) 17.0 -> 15.4, level at 11
+  // stages; on 512 tiles 2048 x 4096 x 8192 132 -> 165, 4096 x 2048 x 512 15 -> 20.
+  if (plan.variant == 1 && (uint64_t)grid.x * grid.y * grid.z <= zluda_gemm_device_cu_count()) {
+#define ZLUDA_TRL_DEEP(PK, QK)                                                                                        \
+  if (pkc == PK && qkc == QK)                                                                                        \
+    return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, 128, 128, 2, 2, !PK, !QK, kTrDeepStages>, grid, dim3(256), s, prm);
+    ZLUDA_TRL_DEEP(false, false) ZLUDA_TRL_DEEP(false, true) ZLUDA_TRL_DEEP(true, false)
+#undef ZLUDA_TRL_DEEP
+  }
 #define ZLUDA_TRL_MODE(BP, BQ, WP, WQ, PK, QK)                                                                       \
   if (pkc == PK && qkc == QK)                                                                                        \
     return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, BP, BQ, WP, WQ, !PK, !QK>, grid, dim3(WP * WQ * 64), s, prm);

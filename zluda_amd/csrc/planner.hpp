@@ -45,6 +45,8 @@ constexpr TrVariant kTrVariants[] = {
     {64, 64, 2, 2, 0},    // 2: 4 waves, 32x32 per wave, four or more per CU: small and skinny problems
     {256, 256, 2, 4, 1},  // 3: variant 0 on the 16x16 MFMA shape, int8 / f16 / bf16: grids that fill the chip
 };
+// stages of variant 1 by the LDS reads where no CU has more than one workgroup (mfma_tr_launch.hpp)
+constexpr int kTrDeepStages = 4;
 constexpr int kNumTrVariants = sizeof(kTrVariants) / sizeof(kTrVariants[0]);
 
 // decode configurations (index = plan.variant for ZLUDA_KERNEL_DECODE_W8A8).
