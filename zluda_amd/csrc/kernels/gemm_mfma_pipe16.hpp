@@ -468,14 +468,7 @@ __device__ __forceinline__ bool mfma16_store_direct(const MfmaParams &prm, AccV 
     }
   }
   const MfmaParams &late = args_again(prm);
-  if constexpr (kind_is_h16(KIND)) {
-    if (__builtin_expect(g.act > ACT_GELU, 0)) {
-      if (g.act == ACT_GELU_KEPT) mfma16_store_aux<WP, WQ, TP, TQ, 1>(late, acc, p0, q0, NP, NQ, bt, wave);
-      else mfma16_store_aux<WP, WQ, TP, TQ, 2>(late, acc, p0, q0, NP, NQ, bt, wave);
-      return true;
-    }
-  }
-  if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
+  if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f && g.act <= ACT_GELU &&
       (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F)) {
 #define ZLUDA_EPI16(DT_, ACT_, EDGE_) mfma16_store_f<KIND, WP, WQ, TP, TQ, DT_, ACT_, EDGE_>(late, acc, p0, q0, NP, NQ, bt, wave)
 #define ZLUDA_EPI16_ACT(DT_)                                 \
@@ -495,6 +488,13 @@ __device__ __forceinline__ bool mfma16_store_direct(const MfmaParams &prm, AccV 
 #undef ZLUDA_EPI16_ACT
 #undef ZLUDA_EPI16
     return true;
+  }
+  if constexpr (kind_is_h16(KIND)) {
+    if (g.act > ACT_GELU) {
+      if (g.act == ACT_GELU_KEPT) mfma16_store_aux<WP, WQ, TP, TQ, 1>(late, acc, p0, q0, NP, NQ, bt, wave);
+      else mfma16_store_aux<WP, WQ, TP, TQ, 2>(late, acc, p0, q0, NP, NQ, bt, wave);
+      return true;
+    }
   }
   return false;
 }
