@@ -254,6 +254,10 @@ int main() {
     for (bool wide : {false, true}) check_short(chunks, wide);
   for (int v : {1, 3}) check_pipe16_mc(kTrVariants[v].bp, kTrVariants[v].bq, kTrVariants[v].wp, kTrVariants[v].wq);
   check_pipe16_ring(kTrVariants[1].bp, kTrVariants[1].bq, kTrVariants[1].wp, kTrVariants[1].wq, kTrDeepStages);
+  for (int nstage : kTr64Stages) {
+    if (nstage > 2) check_pipe16_ring(kTrVariants[2].bp, kTrVariants[2].bq, kTrVariants[2].wp, kTrVariants[2].wq, nstage);
+    else check_pipe16_mc(kTrVariants[2].bp, kTrVariants[2].bq, kTrVariants[2].wp, kTrVariants[2].wq);
+  }
   for (int esz : {1, 2, 4}) check_tr(esz);
   printf("%ld waits checked\n", checked);
   return 0;

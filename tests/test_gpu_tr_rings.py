@@ -1,5 +1,5 @@
-"""The two rings of the 128 x 128 tile whose LDS reads transpose, four stages where no CU has more than one workgroup and two elsewhere:
-every position of the ring that K can end at, K tails inside a stage, shares of K of unequal length."""
+"""The rings of the 128 x 128 and 64 x 64 tiles whose LDS reads transpose, deeper ones where fewer workgroups share a CU: every position of
+the ring that K can end at, K tails inside a stage, shares of K of unequal length."""
 import pytest
 
 from oracle.cases import Case
@@ -31,3 +31,15 @@ def test_shares_of_k(gpu_api, k, ta, tb):
     st, got, plan = case.run_gpu_plan(gpu_api, K.ZLUDA_KERNEL_MFMA_TR16, 1, workspace_bytes=16 << 20)
     assert st == 0 and (plan.variant, plan.grid_z) == (1, 8)
     case.compare(got, case.run_oracle(), tol=1e-3)   # 32-bit sums in another order
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("batch", [1, 44, 130])   # 6, 264 and 780 tiles of 64 x 64: rings of six, three and two stages
+def test_small_tiles(gpu_api, batch, ta, tb):
+    for k in (8, 64, 72, 128, 192, 200, 256, 320, 384, 392, 448, 512) if batch < 130 else (8, 64, 72, 128, 192, 200):
+        spec = dict(BF, m=136, n=72, k=k, transa=ta, transb=tb, batch=batch)
+        print("case", spec, flush=True)
+        case = Case(spec, 9970 + k)
+        st, got, kernel, variant = case.run_gpu(gpu_api, forced_kernel=K.ZLUDA_KERNEL_MFMA_TR16, forced_variant=2)
+        assert st == 0 and variant == 2
+        case.compare(got, case.run_oracle(), tol=1e-2)

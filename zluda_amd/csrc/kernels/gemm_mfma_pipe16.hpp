@@ -37,8 +37,8 @@
 // registers, spends its stages on that: bf16 8192^3 A:N B:N 1019 us there, 808 here; 4096^3 A:N B:N 110; 128 x 128 tiles,
 // 2048 x 4096 x 8192 A:N B:N 183 and 133 inside a training step.  (The 128 x 128 tile also has a ring of four stages, see mfma_tr_launch.hpp.)
 // LDS layout of such an operand: blocks of 1 KiB, one DMA instruction of a wave each, at a pitch of 1056 bytes.  A block
-// holds the K rows {k, k + 4} (256 elements a row) or {k, k + 4, k + 32, k + 36} (128), and the blocks run over k = 0..3,
-// 8..11, 16..19, ...: a ds_read_b64_tr_b16 takes the rows k..k+3 of four blocks for each of its groups of 16 lanes, 32
+// holds the K rows {k, k + 4} (256 elements a row), {k, k + 4, k + 32, k + 36} (128) or {k, k + 4, k + 16, k + 20} and those 32
+// further on (64), and the blocks run over k = 0..3, 8..11, 16..19, ... (64: to 11): a ds_read_b64_tr_b16 takes the rows k..k+3 of four blocks for each of its groups of 16 lanes, 32
 // bytes of each; the pitch puts eight blocks in a row on different banks, and every fragment of a stage is one register
 // plus an immediate away.
 #pragma once
@@ -511,6 +511,14 @@ __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&
 // An MC operand's block of LDS (head of this file): the K row of its first lane, and where K row `k` & 36 lies in its block
 __host__ __device__ constexpr int mc_block_k(int blk) { return (blk & 3) + 8 * ((blk >> 2) & 3) + 32 * (blk >> 4); }
 constexpr int kMcPitch = 1056;
+// the K row of a lane's 16 bytes in a block of operands of `rows` rows, less its first lane's
+__host__ __device__ constexpr int mc_lane_k(int rows, int lane) {
+  return rows == 256 ? 4 * (lane >> 5) : rows == 128 ? 4 * ((lane >> 4) & 1) + 32 * (lane >> 5) : 4 * ((lane >> 3) & 1) + 16 * ((lane >> 4) & 1) + 32 * (lane >> 5);
+}
+// where the lane group g4 finds the K rows 8 g4 .. 8 g4 + 3 of a stage: row r of them in bytes
+__host__ __device__ constexpr int mc_frag_at(int rows, int g4, int r) {
+  return rows == 64 ? (r + 4 * (g4 & 1)) * kMcPitch + (g4 >> 1) * 256 : (r + 4 * g4) * kMcPitch;
+}
 // The chunk swizzle of a K-contiguous operand beside an MC one, whose lane groups hold the K bytes 16 g and 64 + 16 g of a stage: the
 // neighbouring chunks of two lane groups fall on different banks with this one
 __device__ __forceinline__ int swz_mixed(int r) { return r & 6; }
@@ -540,7 +548,7 @@ __device__ __forceinline__ void lds_dma16_uncounted(v4i rs, const void *lds_dst,
 template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, bool PMC = false, bool QMC = false, int NSTAGE = 2>
 __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParams prm) {
   static_assert(!(PMC || QMC) || kind_is_h16(KIND), "the transposing LDS reads are those of 16-bit elements");
-  static_assert((!PMC || BP == 256 || BP == 128) && (!QMC || BQ == 256 || BQ == 128), "rows of 1 KiB / 2 or / 4");
+  static_assert((!PMC || BP == 256 || BP == 128 || BP == 64) && (!QMC || BQ == 256 || BQ == 128 || BQ == 64), "rows of 1 KiB / 2, / 4 or / 8");
   static_assert(KIND == KIND_I8 || KIND == KIND_F8 || kind_is_h16(KIND), "int8, fp8, f16 and bf16 operands");
   constexpr int ESZ = kind_esz(KIND);          // f16 / bf16: the byte geometry of int8 (v_mfma_f32_16x16x32_*: 16 bytes of K per lane)
   constexpr int NT = WP * WQ * 64, NWV = NT / 64;
@@ -608,8 +616,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   // MC: an instruction fills a block; lane l -> K row and 16-byte piece of it.  A piece past the last one of the row index
   // loads that one (rows past the end of D are dropped), which holds at least one element of the operand: with the
   // 16-byte aligned pitch the planner asks for it lies in the operand's own 16-byte granules.
-  const int mkP = mc_block_k(wave) + (BP == 256 ? 4 * (lane >> 5) : 4 * ((lane >> 4) & 1) + 32 * (lane >> 5));
-  const int mkQ = mc_block_k(wave) + (BQ == 256 ? 4 * (lane >> 5) : 4 * ((lane >> 4) & 1) + 32 * (lane >> 5));
+  const int mkP = mc_block_k(wave) + mc_lane_k(BP, lane), mkQ = mc_block_k(wave) + mc_lane_k(BQ, lane);
 #pragma unroll
   for (int i = 0; i < LP; i++)
     if constexpr (PMC) voffP[i] = i ? 0 : mkP * ldp + min(p0 + 8 * (lane & (BP / 8 - 1)), (NP - 1) & ~7) * ESZ;
@@ -669,8 +676,8 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
       fragQ[par][kk] = PMC ? P_V4 + (wq * WTQ + row) * CPR + ch : (BP + wq * WTQ + row) * CPR + ch;
     }
   // MC: K row 8 * (l / 16) + (l % 16) / 4, elements 4 * (l % 4) .. +3 of the wave tile, in bytes inside a slot
-  const int mfrag = ((r16 >> 2) + 4 * g4) * kMcPitch + 8 * (r16 & 3);
-  const int mfragP = mfrag + wp * WTP * 2, mfragQ = P_V4 * 16 + mfrag + wq * WTQ * 2;
+  const int mfragP = mc_frag_at(BP, g4, r16 >> 2) + 8 * (r16 & 3) + wp * WTP * 2;
+  const int mfragQ = P_V4 * 16 + mc_frag_at(BQ, g4, r16 >> 2) + 8 * (r16 & 3) + wq * WTQ * 2;
   // 16-row tile `tile` of the wave tile, from the stage in the slot at `so`
   auto load_frag = [&](int so, const int (&fr)[2][2], auto tile_c, Frag &f) {
     constexpr int tile = decltype(tile_c)::value;
@@ -686,7 +693,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
 
   auto load_frag_mc = [&](int so, int fr, auto rows_c, auto tile_c, Frag &f) {
     constexpr int B = decltype(rows_c)::value, tile = decltype(tile_c)::value;
-    constexpr int UP4 = B == 256 ? 512 : 256, UP32 = B == 256 ? 16 * kMcPitch : 512;  // bytes to the K row 4 / 32 further on
+    constexpr int UP4 = B * 2, UP32 = B == 256 ? 16 * kMcPitch : 512;  // bytes to the K row 4 / 32 further on
     const char *base = (const char *)&lds[so] + fr + tile * 32;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {

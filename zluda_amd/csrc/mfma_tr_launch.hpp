@@ -58,7 +58,7 @@ inline uint32_t launch_tr_variant(const MfmaParams &prm, const zluda_gemm_plan &
   return CUBLAS_STATUS_INVALID_VALUE;
 }
 
-// the variants 1 and 3 where tr_lds_reads() says so: their grids, with the transposition in the LDS reads
+// the variants 1, 2 and 3 where tr_lds_reads() says so: their grids, with the transposition in the LDS reads
 uint32_t launch_trl_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_trl_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_i8(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
@@ -72,6 +72,21 @@ uint32_t launch_tr_f32(const MfmaParams &prm, const zluda_gemm_plan &plan, bool 
 template <int KIND>
 inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s) {
   const dim3 grid(plan.grid_x, plan.grid_y, plan.grid_z > 1 ? plan.grid_z : 1);
+  if (plan.variant == 2) {
+    // 17 KiB a stage: as many of them as the workgroups that share a CU have room for.  (64 x 64 tiles, bf16, us, transposed in registers before:
+    // 704 x 1000 x 2104, 176 workgroups 14.8 -> 13.6; 2104 x 704 x 1000, 363, 14.5 -> 12.4; 1536 x 1536 x 1024, 576, 17.8 -> 13.5.)
+    const uint64_t groups = (uint64_t)grid.x * grid.y * grid.z, cus = zluda_gemm_device_cu_count();
+#define ZLUDA_TRL_64(PK, QK, NS)                                                                                      \
+  if (pkc == PK && qkc == QK)                                                                                        \
+    return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, 64, 64, 2, 2, !PK, !QK, NS>, grid, dim3(256), s, prm);
+#define ZLUDA_TRL_64_RING(NS) { ZLUDA_TRL_64(false, false, NS) ZLUDA_TRL_64(false, true, NS) ZLUDA_TRL_64(true, false, NS) }
+    if (groups <= cus) ZLUDA_TRL_64_RING(kTr64Stages[0])
+    else if (groups <= 3 * cus) ZLUDA_TRL_64_RING(kTr64Stages[1])
+    else ZLUDA_TRL_64_RING(kTr64Stages[2])
+#undef ZLUDA_TRL_64_RING
+#undef ZLUDA_TRL_64
+    return CUBLAS_STATUS_INVALID_VALUE;
+  }
   // One workgroup to a CU: four stages of 33 KiB instead of two, all but the one that is multiplied on their way (a stage's time is far
   // below a round trip to memory; with two workgroups the other one fills the gaps, and two rings of four do not fit).  bf16, us:
   // 2048^3 A:N B:N 33.4 -> 25.7, A:N B:T 32.7 -> 25.2, 1024 x 4096 x 4096 60.6 -> 44.3, 1000^3 (64 tiles) 17.0 -> 15.4, level at 11

@@ -602,10 +602,11 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus, uint64_t workspace_
 //   transposed in registers  4.6 + 1.2 n + (7.5 + 15.3 n) u
 //   by the LDS reads         6.2 + 1.45 n + 2.4 per round behind the first + 27.8 u per round of two on a CU, 17.4 u for one
 // -- level at K = 700 for n = 1, 430 for two, 1200 for three.  (2048 x 2048 x 128: 7.5 us in registers, 9.7 by the LDS reads;
-// 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 tile is faster by the LDS reads at every K.
+// 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 and the 64 x 64 tile are faster by the LDS reads at every K (the latter bf16, us: 512 x 512 x 128
+// 5.4 and 5.3, 512^3 7.9 and 6.7, 1024^3 A:N B:T 9.8 and 8.7, 2104 x 704 x 1000 14.5 and 12.4, 1536 x 1536 x 1024 17.8 and 13.5).
 bool tr_lds_reads(const Lowered &l, int variant, uint64_t groups, uint32_t splits, uint32_t cus) {
-  if ((variant != 1 && variant != 3) || !lds_transposable(l)) return false;
-  if (variant == 3) return true;
+  if (variant == 0 || !lds_transposable(l)) return false;
+  if (variant != 1) return true;
   const uint64_t n = (groups + cus - 1) / std::max(cus, 1u), rounds = (n + 1) / 2;
   const double u = (double)l.g.K * 2 / 4096 / std::max(splits, 1u);
   const double regs = 4.6 + 1.2 * (double)n + (7.5 + 15.3 * (double)n) * u;
@@ -678,7 +679,9 @@ static const TrCost kTrCost[kNumTrVariants] = {{1, 0.0f, 71.0f}, {2, 26.0f, 11.0
 // (tr_lds_reads()) the variants 1 and 3 have times of their own.  us for 4096 bytes of K:
 // 128x128 25 + 3.3 n, 256x256 53 on a full chip (8192 x 4096 x 2048 121 us against 174 on 128x128; 2048 x 4096 x 8192, 128
 // tiles, 164 against 130); the others as above.  Around the loop 4 us, and for a split the second kernel and the partial
-// tiles' way through memory at 3 TB/s (1024 x 512 x 1024 on 128x128 would take 20 us split, 64x64 take 10).
+// tiles' way through memory at 3 TB/s.  (The small tiles and their deeper rings take less than that by now, all alike: over 440 problems of 128 to 4096
+// rows and columns and K = 128 to 8192 what these pick takes 0.3 % more time than the best variant on average, times fitted anew 2 %.)
+// (1024 x 512 x 1024 on 128x128 would take 20 us split, 64x64 take 10).
 static const TrCost kTrCostLds[kNumTrVariants] = {{1, 0.0f, 71.0f}, {2, 25.0f, 3.3f}, {4, 16.0f, 6.0f}, {1, 0.0f, 53.0f}};
 
 static int pick_tr_variant_h16(const Lowered &l, uint32_t cus, uint64_t workspace_size) {

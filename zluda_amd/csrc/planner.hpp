@@ -47,6 +47,7 @@ constexpr TrVariant kTrVariants[] = {
 };
 // stages of variant 1 by the LDS reads where no CU has more than one workgroup (mfma_tr_launch.hpp)
 constexpr int kTrDeepStages = 4;
+constexpr int kTr64Stages[] = {6, 3, 2};  // and of variant 2: up to one workgroup per CU, up to three, more
 constexpr int kNumTrVariants = sizeof(kTrVariants) / sizeof(kTrVariants[0]);
 
 // decode configurations (index = plan.variant for ZLUDA_KERNEL_DECODE_W8A8).
@@ -130,7 +131,7 @@ bool family_supports(uint32_t kernel, const Lowered &l);
 bool lds_transposable(const Lowered &l);
 
 // whether `groups` workgroups (all shares and batches) of a variant of the transposing family do so, each share holding
-// K / splits: the tiles 1 and 3 of operands that allow it, the former from the K on where that is the faster form
+// K / splits: the tiles 1, 2 and 3 of operands that allow it, the first from the K on where that is the faster form
 bool tr_lds_reads(const Lowered &l, int variant, uint64_t groups, uint32_t splits, uint32_t cus);
 
 // Row sums along the longer stride (bias gradients): how many workgroups share the `len` terms of each of `rows` sums, given
