@@ -29,7 +29,8 @@
 //     and the same of the upper half; over the 32 rows of a fragment either part meets each residue of (g + 4 r) mod 16 once,
 //     i.e. 16 distinct 16-byte groups (pitch 5 groups, 5 coprime to 16).  A fragment of 16 rows has two chunks in each part: those
 //     have to lie two apart.  (With g + 2 r for 128 rows, and neighbouring chunks, half of the LDS cycles of these kernels
-//     were bank conflicts.  us without them: fp8 2048^3 A:N 17.5 -> 17.0, f32 127.8 -> 125.9, int8 4096^3 B:T 73.4 -> 73.2.)
+//     were bank conflicts, now a fifth to three tenths.  us before and now: fp8 2048^3 A:N 17.5 and 17.0, f32 127.8 and 125.9, int8 4096^3 B:T 73.4
+//     and 73.2.)
 #pragma once
 #include "gemm_mfma_pipe16.hpp"
 
