@@ -1,0 +1,57 @@
+"""Which plans carry an epilogue with an aux matrix in their own kernel: only grids that cover every tile of every batch, one workgroup each."""
+import ctypes as C
+
+import pytest
+
+import planner_probe
+from zluda_amd import abi as K
+
+AUX, AUX_BIAS, DG, DG_SUMS = (K.CUBLASLT_EPILOGUE_GELU_AUX, K.CUBLASLT_EPILOGUE_GELU_AUX_BIAS, K.CUBLASLT_EPILOGUE_DGELU, K.CUBLASLT_EPILOGUE_DGELU_BGRAD)
+H16, TR16 = K.ZLUDA_KERNEL_MFMA_H16, K.ZLUDA_KERNEL_MFMA_TR16
+BASE = 1 << 40   # (an aligned address; nothing is read from it)
+
+
+def planned(api, m, n, k, batch, epi, ta=1, tb=0, workspace=32 << 20, family=0, variant=-1, cus=256):
+    p, plan, one, zero = K.zluda_gemm_problem(), K.zluda_gemm_plan(), C.c_float(1), C.c_float(0)
+    for dst, rows, cols in ((p.a, k if ta else m, m if ta else k), (p.b, n if tb else k, k if tb else n), (p.c, m, n), (p.d, m, n)):
+        dst.type, dst.order, dst.rows, dst.cols, dst.ld, dst.batch_count, dst.batch_stride = K.CUDA_R_16BF, K.CUBLASLT_ORDER_COL, rows, cols, rows, batch, rows * cols
+    o = p.op
+    o.compute_type, o.scale_type, o.transa, o.transb = K.CUBLAS_COMPUTE_32F, K.CUDA_R_32F, ta, tb
+    o.epilogue, o.bias_type, o.epilogue_aux_type = epi, -1, -1
+    o.epilogue_aux, o.epilogue_aux_ld, o.epilogue_aux_batch_stride, o.bias, o.bias_batch_stride = BASE, m, m * n, BASE, m
+    p.A = p.B = p.C = p.D = BASE
+    p.workspace, p.workspace_size = BASE, workspace
+    status = api.zluda_gemm_plan_problem(C.byref(p), family, variant, cus, C.byref(plan))
+    p.alpha, p.beta = C.addressof(one), C.addressof(zero)
+    return status, p, plan, (one, zero)
+
+
+@pytest.mark.parametrize("epi", [AUX, DG, DG_SUMS])
+@pytest.mark.parametrize("m,n,k,batch", [(2048, 4096, 128, 2), (4096, 2000, 64, 3), (512, 16384, 120, 9)])   # 512 tiles of 128 x 128 a batch
+def test_walked_tiles_with_a_grid_of_one_batch(api, m, n, k, batch, epi):
+    status, p, plan, keep = planned(api, m, n, k, batch, epi)
+    assert status == 0 and (plan.kernel, plan.variant, plan.grid_x, plan.grid_y) == (H16, 3, 512, 1)
+    assert planner_probe.aux_in_epilogue(p, plan) == 0
+
+
+@pytest.mark.parametrize("epi", [AUX, AUX_BIAS, DG, DG_SUMS])
+@pytest.mark.parametrize("cus", [64, 256])
+def test_every_plan_that_carries_it_covers_the_batches(api, cus, epi):
+    carried = 0
+    for ta, tb in ((1, 0), (0, 0), (0, 1), (1, 1)):
+        for m in (8, 64, 264, 1024, 2048):
+            for n in (1, 65, 512, 2048):
+                for k in (64, 128, 136, 2048):
+                    for batch in (1, 2, 5, 8):
+                        for family, variants in ((0, (-1,)), (H16, range(12)), (TR16, range(4))):
+                            for v in variants:
+                                status, p, plan, keep = planned(api, m, n, k, batch, epi, ta, tb, family=family, variant=v, cus=cus)
+                                if status or planner_probe.aux_in_epilogue(p, plan) != 1:
+                                    continue
+                                carried += 1
+                                if plan.kernel == H16 and plan.variant == 11:
+                                    continue   # (the persistent kernel walks the batches itself)
+                                assert plan.grid_y == batch and plan.grid_z == 1
+                                if epi == DG_SUMS:
+                                    assert plan.workspace >= planner_probe.aux_sum_bytes(p, plan)
+    assert carried > 1000

@@ -85,3 +85,25 @@ def test_what_keeps_the_pass_behind_the_matmul(gpu_api, epi, ta, change):
     if spec.get("with_c") and epi == AUX_BIAS:
         spec["beta"] = 0.5
     run(gpu_api, spec, 9850, H16 if ta else TR16, -1, ws=ws, in_epilogue=False)
+
+
+@pytest.mark.parametrize("epi", [AUX, DG, DG_SUMS])
+def test_walked_tiles_with_a_grid_of_one_batch(gpu_api, epi):
+    # (512 tiles of 128 x 128 in each of two batches: as many workgroups walk them all on 256 CUs)
+    case, plan = run(gpu_api, dict(BF, m=1928, n=3969, k=16, transa=1, batch=2, epilogue=epi, bias_batch_stride=1928 if epi == DG_SUMS else 0),
+                     9870, H16, -1, ws=32 << 20, in_epilogue=False)
+    assert (plan.variant, plan.grid_x, plan.grid_y) == (3, 512, 1)
+
+
+@pytest.mark.parametrize("family,ta", [(H16, 1), (TR16, 0)])
+def test_a_plan_for_fewer_batches_is_refused(gpu_api, family, ta):
+    import torch
+    case = Case(dict(BF, m=200, n=136, k=264, transa=ta, batch=3), 9880)
+    keep, ptr, dt = case.upload()
+    p = case.problem(dict(ptr, alpha=case.alpha.ctypes.data, beta=case.beta.ctypes.data))
+    plan = K.zluda_gemm_plan()
+    assert gpu_api.zluda_gemm_plan_problem(C.byref(p), family, -1, 256, C.byref(plan)) == 0 and plan.grid_y == 3
+    plan.grid_y = 1
+    assert gpu_api.zluda_gemm_launch(C.byref(p), C.byref(plan), torch.cuda.current_stream().cuda_stream) == K.CUBLAS_STATUS_INVALID_VALUE
+    torch.cuda.synchronize()
+    assert bool((case.download(dt) == case.new_d()).all())

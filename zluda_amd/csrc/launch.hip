@@ -101,7 +101,7 @@ uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws,
     // beta 1 298 us, on the 256 x 256 tiles that the cost would pick 502)
     plan.grid_x = (uint32_t)(prm.tiles_p * prm.tiles_q); plan.grid_y = l.g.batch; plan.grid_z = 1;
   }
-  if ((uint32_t)(prm.tiles_p * prm.tiles_q) != plan.grid_x) return CUBLAS_STATUS_INVALID_VALUE;
+  if ((uint32_t)(prm.tiles_p * prm.tiles_q) != plan.grid_x || (uint32_t)l.g.batch != plan.grid_y) return CUBLAS_STATUS_INVALID_VALUE;
   if (plan.grid_z > 1) {
     // split-K: partial tiles go through the caller's workspace
     const uint64_t need = (uint64_t)plan.grid_z * l.g.batch * prm.tiles_p * v.bp * prm.tiles_q * v.bq * 4;
@@ -154,7 +154,7 @@ uint32_t launch_tr(const Lowered &l, const zluda_gemm_plan &plan, void *ws, uint
   prm.tiles_q = (nq + v.bq - 1) / v.bq;
   prm.group_p = 8;
   prm.splits = 1; prm.split_stages = 0; prm.groups = 0; prm.ws = l.g.act == ACT_DGELU ? ws : nullptr;
-  if ((uint32_t)(prm.tiles_p * prm.tiles_q) != plan.grid_x) return CUBLAS_STATUS_INVALID_VALUE;
+  if ((uint32_t)(prm.tiles_p * prm.tiles_q) != plan.grid_x || (uint32_t)l.g.batch != plan.grid_y) return CUBLAS_STATUS_INVALID_VALUE;
   // the same tiles, transposed by the LDS reads: 128 K bytes per stage
   const bool lds_reads = tr_lds_reads(l, (int)plan.variant, (uint64_t)plan.grid_x * plan.grid_y * std::max(plan.grid_z, 1u), plan.grid_z,
                                       zluda_gemm_device_cu_count());

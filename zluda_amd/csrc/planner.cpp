@@ -772,7 +772,8 @@ bool aux_in_epilogue(const Lowered &l, const zluda_gemm_plan &plan, bool dry) {
     const MfmaVariant &v = kMfmaVariants[plan.variant];
     if (v.w4) return g.aux_mode == 1 && w4_epilogue_class(l, dry) == W4_CLASS_BF16;  // (the gradient: of operands that are not K-contiguous)
     const MfmaVariant &w = plan.variant == 2 && plan.block == 512 ? kMfmaEightWaves : v;
-    return plan.grid_x == ceil_div(g.M, v.bp) * ceil_div(g.N, v.bq) &&  // (not the short-K form)
+    // (not the short-K form, whose workgroups walk the tiles of all batches: as many of them as one batch has tiles, with 512 of those)
+    return plan.grid_x == ceil_div(g.M, v.bp) * ceil_div(g.N, v.bq) && plan.grid_y == (uint32_t)g.batch &&
            (v.m16 || aux_on_wave_tile32(w.bp / w.wp, w.bq / w.wq));
   }
   if (plan.variant >= (uint32_t)kNumTrVariants) return false;
