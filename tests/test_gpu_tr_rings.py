@@ -43,3 +43,19 @@ def test_small_tiles(gpu_api, batch, ta, tb):
         st, got, kernel, variant = case.run_gpu(gpu_api, forced_kernel=K.ZLUDA_KERNEL_MFMA_TR16, forced_variant=2)
         assert st == 0 and variant == 2
         case.compare(got, case.run_oracle(), tol=1e-2)
+
+
+# whole turns of the ring and what is left of K behind them, at every number of stages that can be left
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("variant,batch,least,turn", [(2, 1, 13, 6), (2, 44, 10, 6), (1, 1, 9, 4)])
+def test_turns(gpu_api, variant, batch, least, turn, ta, tb):
+    for stages in range(least - 1, least + 2 * turn + 1):
+        for k in (64 * stages, 64 * stages - 56):
+            if variant == 1 and k < 704:
+                continue   # (transposed in registers)
+            spec = dict(BF, m=136, n=72, k=k, transa=ta, transb=tb, batch=batch)
+            print("case", spec, flush=True)
+            case = Case(spec, 10000 + k)
+            st, got, kernel, chosen = case.run_gpu(gpu_api, forced_kernel=K.ZLUDA_KERNEL_MFMA_TR16, forced_variant=variant)
+            assert st == 0 and chosen == variant
+            case.compare(got, case.run_oracle(), tol=1e-2)

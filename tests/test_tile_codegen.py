@@ -15,14 +15,14 @@ HIPCC = "/opt/rocm/bin/hipcc"
 pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
 
 
-def kernels(instances):
+def kernels(instances, *flags):
     """the instruction lines of the kernels instantiated in `instances`, in their order"""
     with tempfile.TemporaryDirectory() as tmp:
         src, out = os.path.join(tmp, "k.hip"), os.path.join(tmp, "k.s")
         with open(src, "w") as f:
             f.write('#include "mfma_launch.hpp"\nnamespace zluda_amd {\n%s\n}\n' % "\n".join("template __global__ void %s(MfmaParams);" % i for i in instances))
         cmd = [HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Xclang", "-target-feature", "-Xclang",
-               "-packed-fp32-ops", "--cuda-device-only", "-S", "-I" + CSRC, src, "-o", out]
+               "-packed-fp32-ops", *flags, "--cuda-device-only", "-S", "-I" + CSRC, src, "-o", out]
         res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
         assert res.returncode == 0, res.stdout[-2000:]
         text = open(out).read()
@@ -49,3 +49,21 @@ def test_no_reload_in_the_loop_of_a_256x256_tile():
         body = k_loop(lines)
         assert sum(x.startswith("v_mfma") for x in body) == 128, kind
         assert not [x for x in body if x.startswith("scratch_")], kind
+
+
+# (bf16, A:N B:T and one operand K-contiguous; the flag is that of the units which hold these kernels)
+@pytest.mark.parametrize("tile,stages,turn", [(64, 6, 6), (64, 3, 6), (128, 4, 4)])
+def test_turns_of_a_deep_ring_address_nothing_at_run_time(tile, stages, turn):
+    names = ["gemm_mfma_pipe16_kernel<KIND_BF16, 0, 0, %d, %d, 2, 2, %s, %d>" % (tile, tile, mc, stages) for mc in ("true, true", "true, false")]
+    for lines in kernels(names, "-mllvm", "-amdgpu-mfma-vgpr-form=1"):
+        body = k_loop(lines)
+        mfmas = (tile // 32) ** 2 * 2
+        assert sum(x.startswith("v_mfma") for x in body) == turn * mfmas
+        assert sum(x.startswith("s_barrier") for x in body) == turn
+        assert not [x for x in body if x.startswith("scratch_")]
+        # beside the MFMAs: with a slot in a register and the masks of the last stages 13 to 29 vector instructions a stage
+        assert len([x for x in body if x.startswith("v_") and not x.startswith("v_mfma")]) <= turn
+        # the scalar ones: offsets, M0 and its wait states of each DMA instruction, the barrier (38 to 65 a stage before)
+        loads = sum(x.startswith("buffer_load") for x in body)
+        scalar = [x for x in body if x.startswith("s_") and not x.startswith(("s_waitcnt", "s_barrier"))]
+        assert len(scalar) <= 3.5 * loads + 4 * turn

@@ -659,6 +659,20 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     }
   };
   auto issue_stage = [&](int kt, int so) { static_for<NLOAD>([&](auto n_c) { issue_one(kt, so, n_c); }); };
+  // the same for a stage that neither ends K nor lies behind its end (operands along their row index)
+  auto issue_inside = [&](int kt, int so, auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    constexpr bool is_p = n < LP, mc = is_p ? PMC : QMC;
+    constexpr int i = is_p ? n : n - LP;
+    const int *voff = is_p ? voffP : voffQ;
+    v4i *base = &lds[so] + (is_p ? 0 : P_V4);
+    if constexpr (mc) {
+      const int ld = is_p ? ldp : ldq;
+      lds_dma16_uncounted(is_p ? rawP : rawQ, base + (wave + NWV * i) * (kMcPitch / 16), voff[0], (k0 + kt * BKB) / ESZ * ld + mc_block_k(i * NWV) * ld);
+    } else {
+      lds_dma16_uncounted(is_p ? rawP : rawQ, base + (wave * RPW + RPP * i) * CPR, voff[i], k0 + kt * BKB);
+    }
+  };
 
   // ---- fragment addressing --------------------------------------------------------------------------------
   // Tiles start on multiples of 16 rows; the swizzle depends on the row mod 32, so even and odd tiles
@@ -788,7 +802,8 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   // ---- one stage ----------------------------------------------------------------------------------------------
   // ODD = 0: on entry P half 0 and Q half 0 of the stage are in registers; the next stage will find P half 0
   // and Q half 1 of its own.  ODD = 1: the same with the Q halves exchanged.
-  auto do_stage = [&](int kt, int so, int so_next, auto odd_c) {
+  auto do_stage = [&](int kt, int so, int so_next, auto odd_c, auto inside_c) {
+    constexpr bool INSIDE = decltype(inside_c)::value != 0;  // nothing of this stage's turn of the ring ends K or lies behind it
     constexpr int QA = decltype(odd_c)::value, QB_ = 1 - QA;  // the Q half that is resident / that is fetched
     using P0 = std::integral_constant<int, 0>;
     using P1 = std::integral_constant<int, 1>;
@@ -815,7 +830,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     pattern(std::integral_constant<int, DSP - PD * EARLY>{}, std::integral_constant<int, 0>{});
     // every fragment of the stage has been requested: wait for them and for this wave's share of stage
     // kt+1, meet the other waves; then the slot is free and the other one readable
-    if constexpr (NSTAGE > 2) {
+    if constexpr (NSTAGE > 2 && !INSIDE) {
       if (pipe16_drains_stage(kt, KT, NSTAGE)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     wait_vmcnt_barrier<PC.wait_stage>();
@@ -827,7 +842,8 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
       static_for<NLOAD>([&](auto n_c) {
         constexpr int n = decltype(n_c)::value;
         mfma_part(P1{}, QBc{}, std::integral_constant<int, NM * n / NLOAD>{}, std::integral_constant<int, NM * (n + 1) / NLOAD>{});
-        issue_one(kt + NSTAGE, so, n_c);
+        if constexpr (INSIDE) issue_inside(kt + NSTAGE, so, n_c);
+        else issue_one(kt + NSTAGE, so, n_c);
         __builtin_amdgcn_sched_barrier(0);
       });
     } else {
@@ -843,22 +859,29 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   };
 
   int kt = 0;
+  using E = std::integral_constant<int, 0>;  // an even stage; not inside
+  using O = std::integral_constant<int, 1>;  // an odd one; inside
   if constexpr (NSTAGE == 2) {
     for (; kt + 2 <= KT; kt += 2) {
-      do_stage(kt, 0, STAGE_V4, std::integral_constant<int, 0>{});
-      do_stage(kt + 1, STAGE_V4, 0, std::integral_constant<int, 1>{});
+      do_stage(kt, 0, STAGE_V4, E{}, E{});
+      do_stage(kt + 1, STAGE_V4, 0, O{}, E{});
     }
-    if (kt < KT) do_stage(kt, 0, STAGE_V4, std::integral_constant<int, 0>{});
+    if (kt < KT) do_stage(kt, 0, STAGE_V4, E{}, E{});
   } else {
-    auto behind = [](int so) { return so == (NSTAGE - 1) * STAGE_V4 ? 0 : so + STAGE_V4; };
-    int so = 0;
-    for (; kt + 2 <= KT; kt += 2) {
-      const int so1 = behind(so), so2 = behind(so1);
-      do_stage(kt, so, so1, std::integral_constant<int, 0>{});
-      do_stage(kt + 1, so1, so2, std::integral_constant<int, 1>{});
-      so = so2;
-    }
-    if (kt < KT) do_stage(kt, so, behind(so), std::integral_constant<int, 0>{});
+    static_assert(MC, "issue_inside()");
+    // Whole turns of the ring with its slots fixed at compile time and without the masks of the last stages: with the slot in a register
+    // and the masks a stage of a 64 x 64 tile has 42 scalar and 15 vector instructions beside its 8 MFMAs, a lone workgroup's time
+    constexpr int TURN = pipe16_turn(NSTAGE);
+    for (; pipe16_inside(kt, KT, NSTAGE); kt += TURN)
+      static_for<TURN>([&](auto u_c) {
+        constexpr int u = decltype(u_c)::value;
+        do_stage(kt + u, u % NSTAGE * STAGE_V4, (u + 1) % NSTAGE * STAGE_V4, std::integral_constant<int, u & 1>{}, O{});
+      });
+    for (; kt < KT; kt += TURN)
+      static_for<TURN>([&](auto u_c) {
+        constexpr int u = decltype(u_c)::value;
+        if (kt + u < KT) do_stage(kt + u, u % NSTAGE * STAGE_V4, (u + 1) % NSTAGE * STAGE_V4, std::integral_constant<int, u & 1>{}, E{});
+      });
   }
 
   __builtin_amdgcn_s_waitcnt(0);  // every DMA of the padding stages has landed before the LDS is reused or the wave ends

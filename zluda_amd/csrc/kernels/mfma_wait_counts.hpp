@@ -76,6 +76,10 @@ constexpr Pipe16Counts pipe16_counts(int bp, int bq, int wp, int wq, int nstage 
 constexpr bool pipe16_drains_prologue(bool mc, int kt) { return mc && kt <= 2; }
 constexpr bool pipe16_drains_prologue(bool mc, int kt, int nstage) { return pipe16_drains_prologue(mc, kt - (nstage - 2)); }
 constexpr bool pipe16_drains_stage(int stage, int kt, int nstage) { return stage + nstage >= kt; }
+// Rings of more than two slots are walked in turns of pipe16_turn() stages (whole turns of the ring, an even number of stages) from `stage`
+// on while none of them requests the last stage or one behind it; those waits drain nothing.
+constexpr int pipe16_turn(int nstage) { return nstage % 2 ? 2 * nstage : nstage; }
+constexpr bool pipe16_inside(int stage, int kt, int nstage) { return stage + pipe16_turn(nstage) + nstage < kt; }
 
 // gemm_mfma_tr.hpp leaves its waits to the compiler, which counts: before the LDS stores of trip kt (stage kt + 1's
 // registers) it waits until only stage kt + 2's loads are outstanding.  Stages hold 64 K bytes; nothing past the last one that
