@@ -1,29 +1,12 @@
 """Which plans carry an epilogue with an aux matrix in their own kernel: only grids that cover every tile of every batch, one workgroup each."""
-import ctypes as C
-
 import pytest
 
 import planner_probe
+from planner_probe import planned
 from zluda_amd import abi as K
 
 AUX, AUX_BIAS, DG, DG_SUMS = (K.CUBLASLT_EPILOGUE_GELU_AUX, K.CUBLASLT_EPILOGUE_GELU_AUX_BIAS, K.CUBLASLT_EPILOGUE_DGELU, K.CUBLASLT_EPILOGUE_DGELU_BGRAD)
 H16, TR16 = K.ZLUDA_KERNEL_MFMA_H16, K.ZLUDA_KERNEL_MFMA_TR16
-BASE = 1 << 40   # (an aligned address; nothing is read from it)
-
-
-def planned(api, m, n, k, batch, epi, ta=1, tb=0, workspace=32 << 20, family=0, variant=-1, cus=256):
-    p, plan, one, zero = K.zluda_gemm_problem(), K.zluda_gemm_plan(), C.c_float(1), C.c_float(0)
-    for dst, rows, cols in ((p.a, k if ta else m, m if ta else k), (p.b, n if tb else k, k if tb else n), (p.c, m, n), (p.d, m, n)):
-        dst.type, dst.order, dst.rows, dst.cols, dst.ld, dst.batch_count, dst.batch_stride = K.CUDA_R_16BF, K.CUBLASLT_ORDER_COL, rows, cols, rows, batch, rows * cols
-    o = p.op
-    o.compute_type, o.scale_type, o.transa, o.transb = K.CUBLAS_COMPUTE_32F, K.CUDA_R_32F, ta, tb
-    o.epilogue, o.bias_type, o.epilogue_aux_type = epi, -1, -1
-    o.epilogue_aux, o.epilogue_aux_ld, o.epilogue_aux_batch_stride, o.bias, o.bias_batch_stride = BASE, m, m * n, BASE, m
-    p.A = p.B = p.C = p.D = BASE
-    p.workspace, p.workspace_size = BASE, workspace
-    status = api.zluda_gemm_plan_problem(C.byref(p), family, variant, cus, C.byref(plan))
-    p.alpha, p.beta = C.addressof(one), C.addressof(zero)
-    return status, p, plan, (one, zero)
 
 
 @pytest.mark.parametrize("epi", [AUX, DG, DG_SUMS])

@@ -59,3 +59,14 @@ def test_turns(gpu_api, variant, batch, least, turn, ta, tb):
             st, got, kernel, chosen = case.run_gpu(gpu_api, forced_kernel=K.ZLUDA_KERNEL_MFMA_TR16, forced_variant=variant)
             assert st == 0 and chosen == variant
             case.compare(got, case.run_oracle(), tol=1e-2)
+
+
+@pytest.mark.parametrize("m,n,ta,tb", [(50000, 16, 0, 0), (49160, 1, 0, 0), (16, 50000, 1, 1)])
+def test_a_long_operand_along_its_row_index(gpu_api, m, n, ta, tb):
+    for k in (120, 128, 136, 264):   # by the LDS reads, then in registers
+        spec = dict(BF, m=m, n=n, k=k, transa=ta, transb=tb)
+        print("case", spec, flush=True)
+        case = Case(spec, 10300 + k)
+        st, got, kernel, variant = case.run_gpu(gpu_api, forced_kernel=K.ZLUDA_KERNEL_MFMA_TR16, forced_variant=2)
+        assert st == 0 and variant == 2
+        case.compare(got, case.run_oracle(), tol=1e-2)

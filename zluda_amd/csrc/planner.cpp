@@ -602,11 +602,19 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus, uint64_t workspace_
 //   transposed in registers  4.6 + 1.2 n + (7.5 + 15.3 n) u
 //   by the LDS reads         6.2 + 1.45 n + 2.4 per round behind the first + 27.8 u per round of two on a CU, 17.4 u for one
 // -- level at K = 700 for n = 1, 430 for two, 1200 for three.  (2048 x 2048 x 128: 7.5 us in registers, 9.7 by the LDS reads;
-// 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 and the 64 x 64 tile are faster by the LDS reads at every K (the latter bf16, us: 512 x 512 x 128
-// 5.4 and 5.3, 512^3 7.9 and 6.7, 1024^3 A:N B:T 9.8 and 8.7, 2104 x 704 x 1000 14.5 and 12.4, 1536 x 1536 x 1024 17.8 and 13.5).
+// 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 tile is faster by the LDS reads at every K, the 64 x 64 tile too (bf16, us: 512 x 512 x 128
+// 5.4 and 5.3, 512^3 7.9 and 6.7, 1024^3 A:N B:T 9.8 and 8.7, 2104 x 704 x 1000 14.5 and 12.4, 1536 x 1536 x 1024 17.8 and 13.5), but for
+// a long operand along its row index beside up to 16 K-contiguous tokens on four to six workgroups per CU: memory bound, and the two-stage ring
+// has less on its way than the registers (us from memory, in registers and by the LDS reads: 65536 x 16 x 512 17.2 and 18.7, x 2048 57 and 61, 14336 x 1 x
+// 4096 in four shares 32.2 and 33.8, x 16 level; x 33 39.3 and 37.5; level at K = 64 and on eight workgroups per CU; up to three of them run
+// on deeper rings: 3584 x 4 x 18944 in eight shares 38.4 and 35.3).
 bool tr_lds_reads(const Lowered &l, int variant, uint64_t groups, uint32_t splits, uint32_t cus) {
   if (variant == 0 || !lds_transposable(l)) return false;
-  if (variant != 1) return true;
+  if (variant == 2) {
+    const bool a_long = l.g.M >= l.g.N, one_long = (a_long ? l.b_kcontig : l.a_kcontig) && std::min(l.g.M, l.g.N) <= 16;
+    return !(one_long && groups > 3 * (uint64_t)cus && groups <= 6 * (uint64_t)cus && (uint64_t)l.g.K >= 128 * (uint64_t)std::max(splits, 1u));
+  }
+  if (variant == 3) return true;
   const uint64_t n = (groups + cus - 1) / std::max(cus, 1u), rounds = (n + 1) / 2;
   const double u = (double)l.g.K * 2 / 4096 / std::max(splits, 1u);
   const double regs = 4.6 + 1.2 * (double)n + (7.5 + 15.3 * (double)n) * u;
