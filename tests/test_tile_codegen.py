@@ -67,3 +67,13 @@ def test_turns_of_a_deep_ring_address_nothing_at_run_time(tile, stages, turn):
         loads = sum(x.startswith("buffer_load") for x in body)
         scalar = [x for x in body if x.startswith("s_") and not x.startswith(("s_waitcnt", "s_barrier"))]
         assert len(scalar) <= 3.5 * loads + 4 * turn
+
+
+def test_epilogues_with_an_aux_matrix_have_kernels_of_their_own():
+    plain, aux = kernels(["gemm_mfma_pipe16_kernel<KIND_BF16, 0, 0, 128, 128, 2, 2, true, true, 2%s>" % more for more in ("", ", true")],
+                         "-mllvm", "-amdgpu-mfma-vgpr-form=1")
+    # the gradient's aux matrix: dwordx4 loads that do not go to LDS, one for each pair of the 4 x 4 tiles of a wave
+    to_registers = lambda lines: sum(x.startswith("buffer_load_dwordx4") and " lds" not in x for x in lines)
+    assert to_registers(aux) == 8 and to_registers(plain) == 0
+    # and one exponential per element and epilogue: GELU, its gradient
+    assert sum(x.startswith("v_exp_f32") for x in aux) == 2 * 4 * 4 * 4

@@ -36,7 +36,7 @@ __device__ __forceinline__ void wait_vmcnt_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, int BKB_, int NSTAGE>
+template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, int BKB_, int NSTAGE, bool AUX = false>
 __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams prm) {
   constexpr int NT = WP * WQ * 64;
   // The DMA side's instruction counts and the counted waits come from mfma_wait_counts.hpp, where the rule they rest on
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
   int k0 = 0;
   int sk0 = 0;  // MX: first scale byte of this workgroup's K range in a row of scales (the host keeps
                 // split_stages a multiple of the CH stages of a scale chunk)
-  if (prm.splits > 1) {
+  if (!AUX && prm.splits > 1) {
     k0 = item.z * prm.split_stages * BKB_;
     Kbytes_local = max(0, min(Kbytes - k0, prm.split_stages * BKB_));
     sk0 = k0 / 16;
@@ -433,13 +433,13 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe_kernel(MfmaParams 
   // every wave is done with the LDS tiles (and every DMA has landed) before they become staging
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if (prm.splits > 1) {
+  if (!AUX && prm.splits > 1) {
     const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
     int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)item.z * g.batch + bt) * ws_np * ws_nq + (int64_t)q0 * ws_np + p0;
     mfma_store_tile_raw<WP, WQ, WTP, WTQ>(ws_tile, ws_np, acc);
     return;
   }
-  mfma_store_tile<KIND, WP, WQ, WTP, WTQ>(prm, acc, (int *)&lds[0], sizeof(lds), p0, q0, NP, NQ, bt);
+  mfma_store_tile<KIND, WP, WQ, WTP, WTQ, AUX>(prm, acc, (int *)&lds[0], sizeof(lds), p0, q0, NP, NQ, bt);
 }
 
 } // namespace zluda_amd

@@ -468,7 +468,7 @@ __device__ __forceinline__ bool mfma16_store_direct(const MfmaParams &prm, AccV 
     }
   }
   const MfmaParams &late = args_again(prm);
-  if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f && g.act <= ACT_GELU &&
+  if (!g.int_scale && narrow && g.beta_mode == SCALAR_VALUE && g.beta_val.f == 0.0f &&
       (g.d_type == CUDA_R_16BF || g.d_type == CUDA_R_16F || g.d_type == CUDA_R_32F)) {
 #define ZLUDA_EPI16(DT_, ACT_, EDGE_) mfma16_store_f<KIND, WP, WQ, TP, TQ, DT_, ACT_, EDGE_>(late, acc, p0, q0, NP, NQ, bt, wave)
 #define ZLUDA_EPI16_ACT(DT_)                                 \
@@ -489,19 +489,20 @@ __device__ __forceinline__ bool mfma16_store_direct(const MfmaParams &prm, AccV 
 #undef ZLUDA_EPI16
     return true;
   }
-  if constexpr (kind_is_h16(KIND)) {
-    if (g.act > ACT_GELU) {
-      if (g.act == ACT_GELU_KEPT) mfma16_store_aux<WP, WQ, TP, TQ, 1>(late, acc, p0, q0, NP, NQ, bt, wave);
-      else mfma16_store_aux<WP, WQ, TP, TQ, 2>(late, acc, p0, q0, NP, NQ, bt, wave);
-      return true;
-    }
-  }
   return false;
 }
 
-template <int KIND, int WP, int WQ, int TP, int TQ, int LDS_BYTES, class AccV>
+// AUX: as in mfma_store_tile()
+template <int KIND, int WP, int WQ, int TP, int TQ, int LDS_BYTES, bool AUX, class AccV>
 __device__ __forceinline__ void mfma16_store_tile(const MfmaParams &prm, AccV (&acc)[TP][TQ], int *lds_words, int p0, int q0, int NP,
                                                   int NQ, int bt, int wave) {
+  if constexpr (AUX) {
+    static_assert(kind_is_h16(KIND), "aux_in_epilogue()");
+    const MfmaParams &late = args_again(prm);
+    if (prm.g.act == ACT_GELU_KEPT) mfma16_store_aux<WP, WQ, TP, TQ, 1>(late, acc, p0, q0, NP, NQ, bt, wave);
+    else mfma16_store_aux<WP, WQ, TP, TQ, 2>(late, acc, p0, q0, NP, NQ, bt, wave);
+    return;
+  }
   if (mfma16_store_direct<KIND, WP, WQ, TP, TQ>(prm, acc, p0, q0, NP, NQ, bt, wave)) return;
   __syncthreads();  // (workgroup-uniform branch) the LDS tiles become staging
   mfma16_store_general<KIND, WP, WQ, TP, TQ, LDS_BYTES>(args_again(prm), acc, lds_words, p0, q0, NP, NQ, bt, wave);
@@ -545,7 +546,7 @@ __device__ __forceinline__ void lds_dma16_uncounted(v4i rs, const void *lds_dst,
 #endif
 }
 
-template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, bool PMC = false, bool QMC = false, int NSTAGE = 2>
+template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, bool PMC = false, bool QMC = false, int NSTAGE = 2, bool AUX = false>
 __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParams prm) {
   static_assert(!(PMC || QMC) || kind_is_h16(KIND), "the transposing LDS reads are those of 16-bit elements");
   static_assert((!PMC || BP == 256 || BP == 128 || BP == 64) && (!QMC || BQ == 256 || BQ == 128 || BQ == 64), "rows of 1 KiB / 2, / 4 or / 8");
@@ -596,7 +597,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   }
   // split-K: this workgroup's share of the stages starts k0 bytes into every row
   int Kbytes_local = Kbytes, k0 = 0;
-  if (prm.splits > 1) {
+  if (!AUX && prm.splits > 1) {
     k0 = item.z * prm.split_stages * BKB;
     Kbytes_local = max(0, min(Kbytes - k0, prm.split_stages * BKB));
   }
@@ -885,14 +886,14 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   }
 
   __builtin_amdgcn_s_waitcnt(0);  // every DMA of the padding stages has landed before the LDS is reused or the wave ends
-  if (prm.splits > 1) {
+  if (!AUX && prm.splits > 1) {
     const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
     int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)item.z * g.batch + bt) * ws_np * ws_nq + (int64_t)(q0 + wq * WTQ) * ws_np + p0 + wp * WTP;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)ws_tile, 0, 0xFFFFFFFF, 0x00020000);
     mfma16_store_raw<false>(rs, ws_np, acc, 1, 0);
     return;
   }
-  mfma16_store_tile<KIND, WP, WQ, TP, TQ, (int)sizeof(lds)>(prm, acc, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
+  mfma16_store_tile<KIND, WP, WQ, TP, TQ, (int)sizeof(lds), AUX>(prm, acc, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
 }
 
 } // namespace zluda_amd

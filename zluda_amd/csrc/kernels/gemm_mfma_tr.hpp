@@ -245,7 +245,7 @@ struct TrOperand {
 // own; their accumulators meet in LDS.  A stage is much waiting for little work (a barrier, an LDS round trip), and where a CU
 // has one workgroup nobody else fills the gaps: bf16 1024 x 512 x 32003 (128 x 128 tiles, eight shares) 76.8 -> 69 us, 80 x 351 x 2459,
 // 21 batches (64 x 64) 23.5 -> 19.1.  Four groups were slower than two on every shape tried.
-template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, bool PKC, bool QKC, bool M16 = false, int KG = 1>
+template <int KIND, int FQ, int FP, int BP, int BQ, int WP, int WQ, bool PKC, bool QKC, bool M16 = false, int KG = 1, bool AUX = false>
 __global__ __launch_bounds__(WP *WQ * 64 * KG) void gemm_mfma_tr_kernel(MfmaParams prm) {
   static_assert(KG == 1 || (KG == 2 && !M16 && WP * WQ == 4 && kind_is_h16(KIND)), "groups of four waves");
   static_assert(KIND == KIND_I8 || KIND == KIND_F8 || kind_is_h16(KIND) || KIND == KIND_F32, "8-, 16- or 32-bit operands");
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(WP *WQ * 64 * KG) void gemm_mfma_tr_kernel(MfmaPara
   // of K; the operands start k0 further along K and the rest of the kernel sees a shorter K
   // (k0, Kl in elements; a stage is 64 bytes of K)
   int k0 = 0, Kl = g.K;
-  if (prm.splits > 1) {
+  if (!AUX && prm.splits > 1) {
     k0 = item.z * prm.split_stages * (64 / ESZ);
     Kl = max(0, min(g.K - k0, prm.split_stages * (64 / ESZ)));
   }
@@ -670,22 +670,22 @@ __global__ __launch_bounds__(WP *WQ * 64 * KG) void gemm_mfma_tr_kernel(MfmaPara
     __syncthreads();
   }
   if constexpr (M16) {
-    if (prm.splits > 1) {
+    if (!AUX && prm.splits > 1) {
       const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
       int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)item.z * g.batch + bt) * ws_np * ws_nq + (int64_t)(q0 + wq * WTQ) * ws_np + p0 + wp * WTP;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)ws_tile, 0, 0xFFFFFFFF, 0x00020000);
       mfma16_store_raw<false>(rs, ws_np, acc16, 1, 0);
       return;
     }
-    mfma16_store_tile<KIND, WP, WQ, TP16, TQ16, (int)sizeof(lds)>(prm, acc16, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
+    mfma16_store_tile<KIND, WP, WQ, TP16, TQ16, (int)sizeof(lds), AUX>(prm, acc16, (int *)&lds[0], p0, q0, NP, NQ, bt, wave);
   } else {
-  if (prm.splits > 1) {
+  if (!AUX && prm.splits > 1) {
     const int ws_np = prm.tiles_p * BP, ws_nq = prm.tiles_q * BQ;
     int32_t *ws_tile = (int32_t *)prm.ws + ((int64_t)item.z * g.batch + bt) * ws_np * ws_nq + (int64_t)q0 * ws_np + p0;
     mfma_store_tile_raw<WP, WQ, WTP, WTQ>(ws_tile, ws_np, acc);
     return;
   }
-  mfma_store_tile<KIND, WP, WQ, WTP, WTQ>(prm, acc, (int *)&lds[0], sizeof(lds), p0, q0, NP, NQ, bt);
+  mfma_store_tile<KIND, WP, WQ, WTP, WTQ, AUX>(prm, acc, (int *)&lds[0], sizeof(lds), p0, q0, NP, NQ, bt);
   }
 }
 

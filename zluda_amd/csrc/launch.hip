@@ -121,7 +121,10 @@ uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws,
   switch (plan.kernel) {
   case ZLUDA_KERNEL_MFMA_I8: st = launch_mfma_i8(prm, plan, s); break;
   case ZLUDA_KERNEL_MFMA_MXF4: st = launch_mfma_mxf4(prm, plan, s); break;
-  case ZLUDA_KERNEL_MFMA_H16: st = launch_mfma_h16(prm, plan, l.g.a_type == CUDA_R_16BF, s); break;
+  case ZLUDA_KERNEL_MFMA_H16:
+    if (l.g.act > ACT_GELU) st = l.g.a_type == CUDA_R_16BF ? launch_mfma_aux_bf16(prm, plan, s) : launch_mfma_aux_f16(prm, plan, s);
+    else st = launch_mfma_h16(prm, plan, l.g.a_type == CUDA_R_16BF, s);
+    break;
   case ZLUDA_KERNEL_MFMA_F32: st = launch_mfma_f32(prm, plan, s); break;
   case ZLUDA_KERNEL_MFMA_F8: {
     // MFMA operand "A" is Q, operand "B" is P (see gemm_mfma.hpp)
@@ -170,7 +173,10 @@ uint32_t launch_tr(const Lowered &l, const zluda_gemm_plan &plan, void *ws, uint
   // P is op(A) for a column-major D, op(B)^T otherwise
   const bool pkc = plan.swapped ? l.b_kcontig : l.a_kcontig, qkc = plan.swapped ? l.a_kcontig : l.b_kcontig;
   uint32_t st;
-  if (lds_reads) {
+  if (l.g.act > ACT_GELU) {
+    st = l.g.a_type == CUDA_R_16BF ? (lds_reads ? launch_trl_aux_bf16 : launch_tr_aux_bf16)(prm, plan, pkc, qkc, s)
+                                   : (lds_reads ? launch_trl_aux_f16 : launch_tr_aux_f16)(prm, plan, pkc, qkc, s);
+  } else if (lds_reads) {
     st = l.g.a_type == CUDA_R_16BF ? launch_trl_bf16(prm, plan, pkc, qkc, s) : launch_trl_f16(prm, plan, pkc, qkc, s);
   } else if (l.g.a_type == CUDA_R_8I) {
     st = launch_tr_i8(prm, plan, pkc, qkc, s);

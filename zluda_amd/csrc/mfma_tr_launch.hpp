@@ -10,24 +10,27 @@
 
 namespace zluda_amd {
 
-// plan.variant indexes kTrVariants (planner.hpp); pkc / qkc: operand P / Q has unit stride along K
-template <int KIND, int FQ, int FP>
+// plan.variant indexes kTrVariants (planner.hpp); pkc / qkc: operand P / Q has unit stride along K.  AUX: the epilogues with an aux
+// matrix, on the variants that have them (aux_in_epilogue()).
+template <int KIND, int FQ, int FP, bool AUX = false>
 inline uint32_t launch_tr_variant(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s) {
   const dim3 grid(plan.grid_x, plan.grid_y, plan.grid_z > 1 ? plan.grid_z : 1);  // z: split-K shares
 #define ZLUDA_TR_MODE(BP, BQ, WP, WQ, PK, QK)                                                                   \
   if (pkc == PK && qkc == QK) {                                                                                 \
-    return launch_kernel(gemm_mfma_tr_kernel<KIND, FQ, FP, BP, BQ, WP, WQ, PK, QK>, grid, dim3(WP * WQ * 64), s, prm); \
+    return launch_kernel(gemm_mfma_tr_kernel<KIND, FQ, FP, BP, BQ, WP, WQ, PK, QK, false, 1, AUX>, grid, dim3(WP * WQ * 64), s, prm); \
   }
 #define ZLUDA_TR_CASE(V, BP, BQ, WP, WQ)                                                                        \
   case V:                                                                                                       \
     static_assert(kTrVariants[V].bp == BP && kTrVariants[V].bq == BQ && kTrVariants[V].wp == WP &&              \
                   kTrVariants[V].wq == WQ && !kTrVariants[V].m16, "variant table mismatch");                                           \
-    ZLUDA_TR_MODE(BP, BQ, WP, WQ, false, false) ZLUDA_TR_MODE(BP, BQ, WP, WQ, false, true)                      \
-    ZLUDA_TR_MODE(BP, BQ, WP, WQ, true, false) ZLUDA_TR_MODE(BP, BQ, WP, WQ, true, true)                        \
+    if constexpr (!AUX || aux_on_wave_tile32(BP / WP, BQ / WQ)) {                                               \
+      ZLUDA_TR_MODE(BP, BQ, WP, WQ, false, false) ZLUDA_TR_MODE(BP, BQ, WP, WQ, false, true)                    \
+      ZLUDA_TR_MODE(BP, BQ, WP, WQ, true, false) ZLUDA_TR_MODE(BP, BQ, WP, WQ, true, true)                      \
+    }                                                                                                           \
     break;
 #define ZLUDA_TR_KG(V, BP, BQ, PK, QK)                                                                            \
   if (plan.variant == V && pkc == PK && qkc == QK)                                                               \
-    return launch_kernel(gemm_mfma_tr_kernel<KIND, FQ, FP, BP, BQ, 2, 2, PK, QK, false, 2>, grid, dim3(512), s, prm);
+    return launch_kernel(gemm_mfma_tr_kernel<KIND, FQ, FP, BP, BQ, 2, 2, PK, QK, false, 2, AUX>, grid, dim3(512), s, prm);
   if (plan.block == 512 && (plan.variant == 1 || plan.variant == 2)) {  // (tr_two_k_groups())
     if constexpr (kind_is_h16(KIND)) {
       ZLUDA_TR_KG(1, 128, 128, false, false) ZLUDA_TR_KG(1, 128, 128, false, true) ZLUDA_TR_KG(1, 128, 128, true, false) ZLUDA_TR_KG(1, 128, 128, true, true)
@@ -46,7 +49,7 @@ inline uint32_t launch_tr_variant(const MfmaParams &prm, const zluda_gemm_plan &
     if constexpr (KIND == KIND_I8 || kind_is_h16(KIND)) {
 #define ZLUDA_TR16_MODE(PK, QK)                                                                                  \
   if (pkc == PK && qkc == QK)                                                                                    \
-    return launch_kernel(gemm_mfma_tr_kernel<KIND, FQ, FP, 256, 256, 2, 4, PK, QK, true>, grid, dim3(512), s, prm);
+    return launch_kernel(gemm_mfma_tr_kernel<KIND, FQ, FP, 256, 256, 2, 4, PK, QK, true, 1, AUX>, grid, dim3(512), s, prm);
       ZLUDA_TR16_MODE(false, false) ZLUDA_TR16_MODE(false, true) ZLUDA_TR16_MODE(true, false) ZLUDA_TR16_MODE(true, true)
 #undef ZLUDA_TR16_MODE
     }
@@ -61,6 +64,11 @@ inline uint32_t launch_tr_variant(const MfmaParams &prm, const zluda_gemm_plan &
 // the variants 1, 2 and 3 where tr_lds_reads() says so: their grids, with the transposition in the LDS reads
 uint32_t launch_trl_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_trl_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
+// (a problem whose `act` is an epilogue with an aux matrix)
+uint32_t launch_trl_aux_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
+uint32_t launch_trl_aux_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
+uint32_t launch_tr_aux_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
+uint32_t launch_tr_aux_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_i8(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_f8(const MfmaParams &prm, const zluda_gemm_plan &plan, int fq, int fp, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_f8_e5m2q(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
@@ -69,7 +77,7 @@ uint32_t launch_tr_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool 
 uint32_t launch_tr_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_f32(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 
-template <int KIND>
+template <int KIND, bool AUX = false>
 inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s) {
   const dim3 grid(plan.grid_x, plan.grid_y, plan.grid_z > 1 ? plan.grid_z : 1);
   if (plan.variant == 2) {
@@ -78,7 +86,7 @@ inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, b
     const uint64_t groups = (uint64_t)grid.x * grid.y * grid.z, cus = zluda_gemm_device_cu_count();
 #define ZLUDA_TRL_64(PK, QK, NS)                                                                                      \
   if (pkc == PK && qkc == QK)                                                                                        \
-    return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, 64, 64, 2, 2, !PK, !QK, NS>, grid, dim3(256), s, prm);
+    return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, 64, 64, 2, 2, !PK, !QK, NS, AUX>, grid, dim3(256), s, prm);
 #define ZLUDA_TRL_64_RING(NS) { ZLUDA_TRL_64(false, false, NS) ZLUDA_TRL_64(false, true, NS) ZLUDA_TRL_64(true, false, NS) }
     if (groups <= cus) ZLUDA_TRL_64_RING(kTr64Stages[0])
     else if (groups <= 3 * cus) ZLUDA_TRL_64_RING(kTr64Stages[1])
@@ -94,13 +102,13 @@ inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, b
   if (plan.variant == 1 && (uint64_t)grid.x * grid.y * grid.z <= zluda_gemm_device_cu_count()) {
 #define ZLUDA_TRL_DEEP(PK, QK)                                                                                        \
   if (pkc == PK && qkc == QK)                                                                                        \
-    return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, 128, 128, 2, 2, !PK, !QK, kTrDeepStages>, grid, dim3(256), s, prm);
+    return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, 128, 128, 2, 2, !PK, !QK, kTrDeepStages, AUX>, grid, dim3(256), s, prm);
     ZLUDA_TRL_DEEP(false, false) ZLUDA_TRL_DEEP(false, true) ZLUDA_TRL_DEEP(true, false)
 #undef ZLUDA_TRL_DEEP
   }
 #define ZLUDA_TRL_MODE(BP, BQ, WP, WQ, PK, QK)                                                                       \
   if (pkc == PK && qkc == QK)                                                                                        \
-    return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, BP, BQ, WP, WQ, !PK, !QK>, grid, dim3(WP * WQ * 64), s, prm);
+    return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, BP, BQ, WP, WQ, !PK, !QK, 2, AUX>, grid, dim3(WP * WQ * 64), s, prm);
 #define ZLUDA_TRL_CASE(V, BP, BQ, WP, WQ)                                                                            \
   case V:                                                                                                            \
     static_assert(kTrVariants[V].bp == BP && kTrVariants[V].bq == BQ && kTrVariants[V].wp == WP &&                   \
