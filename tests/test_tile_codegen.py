@@ -77,3 +77,16 @@ def test_epilogues_with_an_aux_matrix_have_kernels_of_their_own():
     assert to_registers(aux) == 8 and to_registers(plain) == 0
     # and one exponential per element and epilogue: GELU, its gradient
     assert sum(x.startswith("v_exp_f32") for x in aux) == 2 * 4 * 4 * 4
+
+
+def test_aux_epilogues_store_whole_lines():
+    # 256 x 256 tiles: D's and aux's stores run along a column's rows, 64 bytes further on with each (the gradient's first, then GELU's)
+    lines = kernels(["gemm_mfma_pipe16_kernel<KIND_BF16, 0, 0, 256, 256, 2, 4, false, false, 2, true>"])[0]
+    assert not [x for x in k_loop(lines) if x.startswith("scratch_")]
+    offsets = {}   # window -> the scalar offsets of its stores
+    for x in lines:
+        m = re.match(r"buffer_store_dwordx4 v\[\d+:\d+\], v\d+, (s\[\d+:\d+\]), (\S+) offen", x)
+        if m:
+            offsets.setdefault(m.group(1), []).append(m.group(2))
+    assert sorted(len(v) for v in offsets.values()) == [16, 16, 16]
+    assert all(v[:2] == ["0", "64"] for v in offsets.values())

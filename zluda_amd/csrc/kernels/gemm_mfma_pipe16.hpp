@@ -347,7 +347,7 @@ __device__ __forceinline__ void mfma16_store_general(const MfmaParams &prm, AccV
 // as the 16-bit ones do in mfma16_store_f(), after which a lane has eight consecutive P indices: 16 bytes of D and of aux.
 template <int WP, int WQ, int TP, int TQ, int MODE, class AccV>
 __device__ __forceinline__ void mfma16_store_aux(const MfmaParams &prm, AccV (&acc)[TP][TQ], int p0, int q0, int NP, int NQ, int bt, int wave) {
-  constexpr int WTP = TP * 16, WTQ = TQ * 16;
+  constexpr int WTP = TP * 16, WTQ = TQ * 16, PAIRS = TP / 2;
   const GemmArgs &g = prm.g;
   const int lane = lane_here();
   const int wp = wave % WP, wq = wave / WP;
@@ -358,18 +358,17 @@ __device__ __forceinline__ void mfma16_store_aux(const MfmaParams &prm, AccV (&a
   const int grp = lane >> 4, first = (grp & 1) ? 4 * grp + 12 : 4 * grp;  // the lane's first P index inside a pair
   const int vd_in = ((lane & 15) * at.d_sq + first) * 2, vx_in = ((lane & 15) * at.x_sq + first) * 2;
   const char *bias = MODE == 1 && g.bias ? (const char *)g.bias + g.bias_sb * bt * (g.bias_type == CUDA_R_32F ? 4 : 2) : nullptr;
+  // the bias of a pair's eight rows (1), or their sums (2)
+  float row[PAIRS][8];
 #pragma unroll
-  for (int a = 0; a < TP; a += 2) {
-    const int p = pc + a * 16 + first;  // the lane's eight P indices exist or do not (their number is a multiple of 8)
-    const int vd = p < NP ? vd_in : kStoreNowhere, vx = p < NP ? vx_in : kStoreNowhere;
-    float pb[8], sum[8];
+  for (int a = 0; a < PAIRS; a++) {
+    const int at_p = min(pc + a * 32 + first, NP - 8);  // the lane's eight P indices exist or do not (their number is a multiple of 8)
 #pragma unroll
-    for (int e = 0; e < 8; e++) pb[e] = sum[e] = 0.0f;
+    for (int e = 0; e < 8; e++) row[a][e] = 0.0f;
     if (MODE == 1 && bias) {
-      const int at_p = min(p, NP - 8);
       if (g.bias_type == CUDA_R_32F) {
 #pragma unroll
-        for (int e = 0; e < 8; e++) pb[e] = ((const float *)bias)[at_p + e];
+        for (int e = 0; e < 8; e++) row[a][e] = ((const float *)bias)[at_p + e];
       } else {
         uint32_t raw[4];
         if (((uintptr_t)bias & 15) == 0) {
@@ -382,21 +381,29 @@ __device__ __forceinline__ void mfma16_store_aux(const MfmaParams &prm, AccV (&a
         }
         const bool bias_bf16 = g.bias_type == CUDA_R_16BF;
 #pragma unroll
-        for (int d = 0; d < 4; d++) { pb[2 * d] = low_half(raw[d], bias_bf16); pb[2 * d + 1] = high_half(raw[d], bias_bf16); }
+        for (int d = 0; d < 4; d++) { row[a][2 * d] = low_half(raw[d], bias_bf16); row[a][2 * d + 1] = high_half(raw[d], bias_bf16); }
       }
     }
-    // (the pair's aux pieces in one burst)
-    v4i x_in[TQ];
+  }
+  // Along P first: a pair of tiles stores 64 bytes of a column, half a line, and with another column's halves in between both matrices' lines left the
+  // L2 of an XCD (whose 32 tiles of 256 x 256 are 8 MiB of them) half written: bf16 1480 x 29920 x 176, two batches, GELU_AUX_BIAS 209 us.
+#pragma unroll
+  for (int b = 0; b < TQ; b++) {
+    // (the column's aux pieces in one burst)
+    v4i x_in[PAIRS];
     if constexpr (MODE == 2) {
 #pragma unroll
-      for (int b = 0; b < TQ; b++) x_in[b] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(at.rs_x, vx, (b * 16 * at.x_sq + a * 16) * 2, 0));
+      for (int a = 0; a < PAIRS; a++)
+        x_in[a] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(at.rs_x, pc + a * 32 + first < NP ? vx_in : kStoreNowhere, (b * 16 * at.x_sq + a * 32) * 2, 0));
     }
 #pragma unroll
-    for (int b = 0; b < TQ; b++) {
+    for (int a = 0; a < PAIRS; a++) {
+      const bool in = pc + a * 32 + first < NP;
+      const int vd = in ? vd_in : kStoreNowhere, vx = in ? vx_in : kStoreNowhere;
       float y[8];
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const uint32_t lo = f2bits(at.factor * bits2f((uint32_t)to_bits(acc[a][b][e]))), hi = f2bits(at.factor * bits2f((uint32_t)to_bits(acc[a + 1][b][e])));
+        const uint32_t lo = f2bits(at.factor * bits2f((uint32_t)to_bits(acc[2 * a][b][e]))), hi = f2bits(at.factor * bits2f((uint32_t)to_bits(acc[2 * a + 1][b][e])));
 #if defined(__HIP_DEVICE_COMPILE__)
         const v2u s = __builtin_amdgcn_permlane16_swap(lo, hi, false, false);
         y[e] = bits2f(s[0]); y[4 + e] = bits2f(s[1]);
@@ -406,41 +413,46 @@ __device__ __forceinline__ void mfma16_store_aux(const MfmaParams &prm, AccV (&a
       }
       if constexpr (MODE == 1) {
 #pragma unroll
-        for (int e = 0; e < 8; e++) y[e] += pb[e];
+        for (int e = 0; e < 8; e++) y[e] += row[a][e];
         v4i keep;
 #pragma unroll
         for (int d = 0; d < 4; d++) keep[d] = (int)pack_halves(y[2 * d], y[2 * d + 1], bf16);
-        buffer_store_b128_guarded(keep, at.rs_x, vx, (b * 16 * at.x_sq + a * 16) * 2);
+        buffer_store_b128_guarded(keep, at.rs_x, vx, (b * 16 * at.x_sq + a * 32) * 2);
 #pragma unroll
         for (int e = 0; e < 8; e++) y[e] = gelu_tanh(y[e]) * sc.sd;
       } else {
 #pragma unroll
         for (int d = 0; d < 4; d++) {
-          y[2 * d] *= dgelu_tanh(low_half((uint32_t)x_in[b][d], bf16));
-          y[2 * d + 1] *= dgelu_tanh(high_half((uint32_t)x_in[b][d], bf16));
+          y[2 * d] *= dgelu_tanh(low_half((uint32_t)x_in[a][d], bf16));
+          y[2 * d + 1] *= dgelu_tanh(high_half((uint32_t)x_in[a][d], bf16));
         }
         // (columns past the end hold products of some column)
         const bool counts = qc + b * 16 + (lane & 15) < NQ;
 #pragma unroll
-        for (int e = 0; e < 8; e++) sum[e] += counts ? y[e] : 0.0f;
+        for (int e = 0; e < 8; e++) row[a][e] += counts ? y[e] : 0.0f;
       }
       v4i pk;
 #pragma unroll
       for (int d = 0; d < 4; d++) pk[d] = (int)pack_halves(y[2 * d], y[2 * d + 1], bf16);
-      buffer_store_b128_guarded(pk, at.rs_d, vd, (b * 16 * at.d_sq + a * 16) * 2);
+      buffer_store_b128_guarded(pk, at.rs_d, vd, (b * 16 * at.d_sq + a * 32) * 2);
       __builtin_amdgcn_sched_barrier(0);  // one pair at a time: what the scheduler hoists across them spills
     }
-    if (MODE == 2 && at.sums) {  // over the 16 columns of a lane group
+  }
+  if (MODE == 2 && at.sums) {  // over the 16 columns of a lane group
+#pragma unroll
+    for (int a = 0; a < PAIRS; a++) {
+      const int p = pc + a * 32 + first;
 #pragma unroll
       for (int e = 0; e < 8; e++) {
-        sum[e] += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(sum[e]), 0x128 /* row_ror:8 */, 0xF, 0xF, true));
-        sum[e] += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(sum[e]), 0x124, 0xF, 0xF, true));
-        sum[e] += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(sum[e]), 0x122, 0xF, 0xF, true));
-        sum[e] += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(sum[e]), 0x121, 0xF, 0xF, true));
+        float &t = row[a][e];
+        t += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(t), 0x128 /* row_ror:8 */, 0xF, 0xF, true));
+        t += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(t), 0x124, 0xF, 0xF, true));
+        t += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(t), 0x122, 0xF, 0xF, true));
+        t += bits2f((uint32_t)__builtin_amdgcn_mov_dpp((int)f2bits(t), 0x121, 0xF, 0xF, true));
       }
       if ((lane & 15) == 0 && p < NP) {
 #pragma unroll
-        for (int e = 0; e < 8; e++) at.sums[p + e] = sum[e];
+        for (int e = 0; e < 8; e++) at.sums[p + e] = row[a][e];
       }
     }
   }
