@@ -107,3 +107,11 @@ def test_a_plan_for_fewer_batches_is_refused(gpu_api, family, ta):
     assert gpu_api.zluda_gemm_launch(C.byref(p), C.byref(plan), torch.cuda.current_stream().cuda_stream) == K.CUBLAS_STATUS_INVALID_VALUE
     torch.cuda.synchronize()
     assert bool((case.download(dt) == case.new_d()).all())
+
+
+@pytest.mark.parametrize("m,n,batch", [(72, 2048, 1), (72, 2049, 1), (8, 9000, 2), (200, 9000, 1)])
+@pytest.mark.parametrize("bias_type", [-1, K.CUDA_R_32F])
+def test_sums_of_many_waves(gpu_api, m, n, batch, bias_type):
+    # (64 x 64 tiles, two waves along D's columns: 64 partial sums of a row by four threads, 66 and 282 by 64)
+    run(gpu_api, dict(BF, m=m, n=n, k=72, transa=1, batch=batch, epilogue=DG_SUMS, bias_type=bias_type, bias_batch_stride=m if batch > 1 else 0),
+        9890, H16, 6, ws=1 << 20)

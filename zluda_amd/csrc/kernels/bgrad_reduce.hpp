@@ -149,7 +149,7 @@ __global__ __launch_bounds__(512) void bgrad_cols_kernel(BgradParams prm) {
   });
 }
 
-// The sums of the `shares` workgroups of a row, added in their order; grid (ceil(rows / 64), 1, batch)
+// The sums of the `shares` workgroups (or waves) of a row, added in their order; grid (ceil(rows / ROWS), 1, batch), PHASES threads a row.
 struct BgradFinishParams {
   const void *part;  // [batch][shares][rows]
   int32_t shares, rows, ints;
@@ -157,15 +157,16 @@ struct BgradFinishParams {
   uint32_t out_type;
   int64_t out_sb;
 };
-__global__ __launch_bounds__(256) void bgrad_finish_kernel(BgradFinishParams prm) {
-  __shared__ float pf[256];
-  __shared__ int32_t pi[256];
-  const int r = blockIdx.x * 64 + (threadIdx.x & 63), phase = threadIdx.x >> 6, bt = blockIdx.z;
+template <int ROWS, int PHASES>
+__global__ __launch_bounds__(ROWS *PHASES) void bgrad_finish_kernel(BgradFinishParams prm) {
+  __shared__ float pf[ROWS * PHASES];
+  __shared__ int32_t pi[ROWS * PHASES];
+  const int t = threadIdx.x % ROWS, r = blockIdx.x * ROWS + t, phase = threadIdx.x / ROWS, bt = blockIdx.z;
   float s = 0.0f;
   int32_t si = 0;
   if (r < prm.rows) {
     const int64_t base = (int64_t)bt * prm.shares * prm.rows + r;
-    const int per = (prm.shares + 3) / 4, y1 = min(prm.shares, (phase + 1) * per);
+    const int per = (prm.shares + PHASES - 1) / PHASES, y1 = min(prm.shares, (phase + 1) * per);
 #pragma unroll 8
     for (int y = phase * per; y < y1; y++) {
       const uint32_t raw = ((const uint32_t *)prm.part)[base + (int64_t)y * prm.rows];
@@ -177,8 +178,19 @@ __global__ __launch_bounds__(256) void bgrad_finish_kernel(BgradFinishParams prm
   pi[threadIdx.x] = si;
   __syncthreads();
   if (phase == 0 && r < prm.rows) {
-    const int t = threadIdx.x;
-    const float total = prm.ints ? (float)(pi[t] + pi[t + 64] + pi[t + 128] + pi[t + 192]) : (pf[t] + pf[t + 64]) + (pf[t + 128] + pf[t + 192]);
+    float qf[4];
+    int32_t qi[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {  // a quarter of the phases each
+      qf[q] = pf[q * (PHASES / 4) * ROWS + t];
+      qi[q] = pi[q * (PHASES / 4) * ROWS + t];
+#pragma unroll
+      for (int ph = 1; ph < PHASES / 4; ph++) {
+        qf[q] += pf[(q * (PHASES / 4) + ph) * ROWS + t];
+        qi[q] += pi[(q * (PHASES / 4) + ph) * ROWS + t];
+      }
+    }
+    const float total = prm.ints ? (float)(qi[0] + qi[1] + qi[2] + qi[3]) : (qf[0] + qf[1]) + (qf[2] + qf[3]);
     store_elem(prm.out, prm.out_type, (int64_t)bt * prm.out_sb + r, total);
   }
 }

@@ -386,7 +386,7 @@ __device__ __forceinline__ void mfma16_store_aux(const MfmaParams &prm, AccV (&a
     }
   }
   // Along P first: a pair of tiles stores 64 bytes of a column, half a line, and with another column's halves in between both matrices' lines left the
-  // L2 of an XCD (whose 32 tiles of 256 x 256 are 8 MiB of them) half written: bf16 1480 x 29920 x 176, two batches, GELU_AUX_BIAS 209 us.
+  // L2 of an XCD (whose 32 tiles of 256 x 256 are 8 MiB of them) half written: bf16 1480 x 29920 x 176, two batches, GELU_AUX_BIAS 209 us, now 137.
 #pragma unroll
   for (int b = 0; b < TQ; b++) {
     // (the column's aux pieces in one burst)

@@ -293,9 +293,13 @@ namespace zluda_amd {
 
 namespace {
 
+// Up to 64 sums of a row four threads each take a quarter of them; more are 64 threads' (us of the whole call, bf16 DGELU_BGRAD, K = 64: 64 x 512
+// 7.8 and 8.0, 64 x 8192 (256 sums) 9.7 and 9.0, 64 x 131072 58.8 and 22.2, 512 x 32768 30.5 and 25.8; level from 2048 rows on)
+constexpr int kFinishWide = 64;
 uint32_t finish_sums(const void *part, int shares, int rows, int batch, bool ints, void *out, uint32_t out_type, int64_t out_sb, hipStream_t s) {
   BgradFinishParams f{part, shares, rows, ints ? 1 : 0, out, out_type, out_sb};
-  return launch_kernel(bgrad_finish_kernel, dim3((rows + 63) / 64, 1, batch), dim3(256), s, f);
+  if (shares > kFinishWide) return launch_kernel(bgrad_finish_kernel<16, 64>, dim3((rows + 15) / 16, 1, batch), dim3(1024), s, f);
+  return launch_kernel(bgrad_finish_kernel<64, 4>, dim3((rows + 63) / 64, 1, batch), dim3(256), s, f);
 }
 
 // LANES of the row-sum kernels: 16-byte pieces side by side.  Four (whole 64-byte pieces of memory) give the most
