@@ -38,3 +38,11 @@ def test_every_plan_that_carries_it_covers_the_batches(api, cus, epi):
                                 if epi == DG_SUMS:
                                     assert plan.workspace >= planner_probe.aux_sum_bytes(p, plan)
     assert carried > 1000
+
+
+def test_a_scale_of_d_keeps_the_pass_behind_the_persistent_kernel(api):
+    status, p, plan, keep = planned(api, 4096, 4096, 2048, epi=AUX_BIAS)
+    assert status == 0 and (plan.kernel, plan.variant) == (H16, 11)
+    assert planner_probe.aux_in_epilogue(p, plan) == 1
+    p.op.d_scale = planner_probe.BASE
+    assert planner_probe.aux_in_epilogue(p, plan) == 0

@@ -115,3 +115,21 @@ def test_sums_of_many_waves(gpu_api, m, n, batch, bias_type):
     # (64 x 64 tiles, two waves along D's columns: 64 partial sums of a row by four threads, 66 and 282 by 64)
     run(gpu_api, dict(BF, m=m, n=n, k=72, transa=1, batch=batch, epilogue=DG_SUMS, bias_type=bias_type, bias_batch_stride=m if batch > 1 else 0),
         9890, H16, 6, ws=1 << 20)
+
+
+@pytest.mark.parametrize("family,variant,ta", [(H16, 11, 1), (H16, 8, 1), (H16, 6, 1), (TR16, 3, 0), (TR16, 2, 0)])
+def test_a_scale_of_zero(gpu_api, family, variant, ta):
+    # (inputs of GELU well beyond where its exponential is zero)
+    import torch
+    case = Case(dict(BF, m=264, n=136, k=512, transa=ta, epilogue=AUX, alpha=1, with_cd_scales=True), 9895)
+    case.d_scale[:] = 0
+    case.run_oracle()
+    keep, ptr, dt = case.upload()
+    p = case.problem(dict(ptr, alpha=case.alpha.ctypes.data, beta=case.beta.ctypes.data))
+    plan = K.zluda_gemm_plan()
+    print("variant", family, variant, flush=True)
+    assert gpu_api.zluda_gemm_plan_problem(C.byref(p), family, variant, gpu_api.zluda_gemm_device_cu_count(), C.byref(plan)) == 0
+    assert gpu_api.zluda_gemm_launch(C.byref(p), C.byref(plan), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert bool(((case.download(dt) & 0x7FFF) == 0).all())
+    case.compare_aux(keep[10][:case.aux.nbytes].cpu().numpy().view(case.aux.dtype).copy(), case.aux_ref)

@@ -778,7 +778,9 @@ bool aux_in_epilogue(const Lowered &l, const zluda_gemm_plan &plan, bool dry) {
   if (plan.kernel == ZLUDA_KERNEL_MFMA_H16) {
     if (plan.variant >= (uint32_t)kNumMfmaVariants) return false;
     const MfmaVariant &v = kMfmaVariants[plan.variant];
-    if (v.w4) return g.aux_mode == 1 && w4_epilogue_class(l, dry) == W4_CLASS_BF16;  // (the gradient: of operands that are not K-contiguous)
+    // (the gradient: of operands that are not K-contiguous; D's scale is folded into GELU's reciprocal there, which makes NaN of large inputs
+    // where the scale is zero)
+    if (v.w4) return g.aux_mode == 1 && !g.d_scale && w4_epilogue_class(l, dry) == W4_CLASS_BF16;
     const MfmaVariant &w = plan.variant == 2 && plan.block == 512 ? kMfmaEightWaves : v;
     // (not the short-K form, whose workgroups walk the tiles of all batches: as many of them as one batch has tiles, with 512 of those)
     return plan.grid_x == ceil_div(g.M, v.bp) * ceil_div(g.N, v.bq) && plan.grid_y == (uint32_t)g.batch &&
