@@ -28,3 +28,13 @@ def test_shares_of_k_count(api):
     assert planner_probe.lds_reads(p, plan, 256) == 0
     status, p, plan, keep = planned(api, 14336, 16, 4096, ta=0, workspace=0, family=TR16, variant=2)
     assert planner_probe.lds_reads(p, plan, 256) == 1
+
+
+# LDS of a CU: 132 KiB of a ring of four stages of 128 x 128 tiles, 66 of two; 99, 50 and 33 of 64 x 64 tiles on six, three and two; in registers four
+# workgroups
+@pytest.mark.parametrize("m,n,k,ta,tb,variant,per_cu", [
+    (2048, 2048, 2048, 0, 0, 1, 1), (2048, 2176, 2048, 0, 0, 1, 2), (1024, 1024, 1024, 0, 1, 2, 1), (1024, 1088, 1024, 0, 1, 2, 3),
+    (4096, 1024, 1024, 0, 1, 2, 4), (65536, 16, 512, 0, 0, 2, 4), (2048, 2048, 128, 0, 0, 1, 4), (2044, 2048, 512, 0, 0, 1, 4), (4096, 4096, 512, 0, 0, 3, 1)])
+def test_waves_are_those_of_the_form_that_runs(api, m, n, k, ta, tb, variant, per_cu):
+    status, p, plan, keep = planned(api, m, n, k, ta=ta, tb=tb, workspace=0, family=TR16, variant=variant)
+    assert status == 0 and plan.waves == pytest.approx(plan.grid_x / (256 * per_cu))

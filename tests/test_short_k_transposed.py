@@ -1,6 +1,7 @@
 """16-bit operands with unit stride along their row index on 128 x 128 tiles: a short K is transposed in registers, a long one by
 the LDS reads, which cost more in front of and behind the loop and less in it.  The plan's waves tell the forms apart (four and
-two workgroups fit a CU); on the GPU both sides of the change-over run with ends of K and of the rows inside pieces."""
+two workgroups fit a CU, one with the deep ring of a grid that has no more); on the GPU both sides of the change-over run with ends of K and of the
+rows inside pieces."""
 import ctypes as C
 
 import pytest
@@ -24,8 +25,8 @@ def waves(api, m, n, k, ta=0, tb=1, variant=1, cus=256):
 
 
 def test_the_form_follows_k_and_the_number_of_tiles(api):
-    registers, lds = 0.25, 0.5
-    for k, want in ((32, registers), (128, registers), (512, registers), (768, lds), (4096, lds)):
+    registers, lds, alone = 0.25, 0.5, 1.0
+    for k, want in ((32, registers), (128, registers), (512, registers), (768, alone), (4096, alone)):
         assert waves(api, 2048, 2048, k) == want, k      # one tile on a CU
     for k, want in ((256, registers), (512, lds), (2048, lds)):
         assert waves(api, 8192, 1024, k) == want, k      # two

@@ -80,16 +80,16 @@ uint32_t launch_tr_f32(const MfmaParams &prm, const zluda_gemm_plan &plan, bool 
 template <int KIND, bool AUX = false>
 inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s) {
   const dim3 grid(plan.grid_x, plan.grid_y, plan.grid_z > 1 ? plan.grid_z : 1);
+  const int stages = tr_ring_stages((int)plan.variant, (uint64_t)grid.x * grid.y * grid.z, zluda_gemm_device_cu_count());
   if (plan.variant == 2) {
     // 17 KiB a stage: as many of them as the workgroups that share a CU have room for.  (64 x 64 tiles, bf16, us, transposed in registers before:
     // 704 x 1000 x 2104, 176 workgroups 14.8 -> 13.6; 2104 x 704 x 1000, 363, 14.5 -> 12.4; 1536 x 1536 x 1024, 576, 17.8 -> 13.5.)
-    const uint64_t groups = (uint64_t)grid.x * grid.y * grid.z, cus = zluda_gemm_device_cu_count();
 #define ZLUDA_TRL_64(PK, QK, NS)                                                                                      \
   if (pkc == PK && qkc == QK)                                                                                        \
     return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, 64, 64, 2, 2, !PK, !QK, NS, AUX>, grid, dim3(256), s, prm);
 #define ZLUDA_TRL_64_RING(NS) { ZLUDA_TRL_64(false, false, NS) ZLUDA_TRL_64(false, true, NS) ZLUDA_TRL_64(true, false, NS) }
-    if (groups <= cus) ZLUDA_TRL_64_RING(kTr64Stages[0])
-    else if (groups <= 3 * cus) ZLUDA_TRL_64_RING(kTr64Stages[1])
+    if (stages == kTr64Stages[0]) ZLUDA_TRL_64_RING(kTr64Stages[0])
+    else if (stages == kTr64Stages[1]) ZLUDA_TRL_64_RING(kTr64Stages[1])
     else ZLUDA_TRL_64_RING(kTr64Stages[2])
 #undef ZLUDA_TRL_64_RING
 #undef ZLUDA_TRL_64
@@ -99,7 +99,7 @@ inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, b
   // below a round trip to memory; with two workgroups the other one fills the gaps, and two rings of four do not fit).  bf16, us:
   // 2048^3 A:N B:N 33.4 -> 25.7, A:N B:T 32.7 -> 25.2, 1024 x 4096 x 4096 60.6 -> 44.3, 1000^3 (64 tiles) 17.0 -> 15.4, level at 11
   // stages; on 512 tiles 2048 x 4096 x 8192 132 -> 165, 4096 x 2048 x 512 15 -> 20.
-  if (plan.variant == 1 && (uint64_t)grid.x * grid.y * grid.z <= zluda_gemm_device_cu_count()) {
+  if (plan.variant == 1 && stages == kTrDeepStages) {
 #define ZLUDA_TRL_DEEP(PK, QK)                                                                                        \
   if (pkc == PK && qkc == QK)                                                                                        \
     return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, 128, 128, 2, 2, !PK, !QK, kTrDeepStages, AUX>, grid, dim3(256), s, prm);

@@ -641,10 +641,10 @@ static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t w
   plan->swapped = swapped;
   plan->grid_x = ceil_div(np, v.bp) * ceil_div(nq, v.bq); plan->grid_y = g.batch; plan->grid_z = 1;
   plan->block = v.wp * v.wq * 64;
-  // workgroups that share a CU: two stages of 80-byte rows each, or two of 128 K bytes at a pitch of 1056 bytes per KiB
-  const bool lds_reads = tr_lds_reads(l, variant, (uint64_t)plan->grid_x * plan->grid_y, 1, cus);
-  const uint32_t per_cu = std::min(160u * 1024u / (lds_reads ? 2u * (v.bp + v.bq) * 132u : 2u * (v.bp + v.bq) * 80u), 4u);
-  plan->waves = (float)plan->grid_x * plan->grid_y / (float)(cus * per_cu);
+  // workgroups that share a CU: stages of 80-byte rows, or of 128 K bytes at a pitch of 1056 bytes per KiB
+  auto per_cu_of = [&](bool by_lds, uint64_t stages) { return (uint32_t)std::min<uint64_t>(160u * 1024u / (stages * (v.bp + v.bq) * (by_lds ? 132u : 80u)), 4u); };
+  // (two stages each: what the rule below was measured with, and the least that any form has)
+  const uint32_t per_cu = per_cu_of(tr_lds_reads(l, variant, (uint64_t)plan->grid_x * plan->grid_y, 1, cus), 2);
   plan->workspace = 0;
   // Split-K as for the K-contiguous kernels: grid_z workgroups share a tile's K range through the
   // caller's workspace when K is long enough (`least`) and the tiles leave half of the chip idle --
@@ -669,11 +669,12 @@ static void fill_tr_plan(const Lowered &l, int variant, uint32_t cus, uint64_t w
     if (s > 1) {
       plan->grid_z = s;
       plan->workspace = s * per_split;
-      plan->waves = (float)tiles * s / (float)slots;
     }
   }
-  if (!tr_lds_reads(l, variant, tiles * plan->grid_z, plan->grid_z, cus) && tr_two_k_groups(l, variant, tiles * plan->grid_z, plan->grid_z, cus))
-    plan->block = 512;
+  const uint64_t groups = tiles * plan->grid_z;
+  const bool lds_reads = tr_lds_reads(l, variant, groups, plan->grid_z, cus);
+  if (!lds_reads && tr_two_k_groups(l, variant, groups, plan->grid_z, cus)) plan->block = 512;
+  plan->waves = (float)groups / (float)(cus * per_cu_of(lds_reads, lds_reads ? tr_ring_stages(variant, groups, cus) : 2));
 }
 
 // Tile choice of the transposing kernel.  A CU runs up to `per_cu` workgroups of a variant side by
@@ -684,11 +685,13 @@ struct TrCost { uint32_t per_cu; float base, slope; };
 static const TrCost kTrCost[kNumTrVariants] = {{1, 0.0f, 71.0f}, {2, 26.0f, 11.0f}, {4, 16.0f, 6.0f}, {1, 0.0f, 67.0f}};
 
 // f16 and bf16: the split along K that the variant would get counts as well, and where the LDS reads transpose
-// (tr_lds_reads()) the variants 1 and 3 have times of their own.  us for 4096 bytes of K:
+// (tr_lds_reads()) the variants 1 and 3 have times of their own (kTrCostLds).  us for 4096 bytes of K:
 // 128x128 25 + 3.3 n, 256x256 53 on a full chip (8192 x 4096 x 2048 121 us against 174 on 128x128; 2048 x 4096 x 8192, 128
 // tiles, 164 against 130); the others as above.  Around the loop 4 us, and for a split the second kernel and the partial
-// tiles' way through memory at 3 TB/s.  (The small tiles and their deeper rings take less than that by now, all alike: over 440 problems of 128 to 4096
-// rows and columns and K = 128 to 8192 what these pick takes 0.3 % more time than the best variant on average, times fitted anew 2 %.)
+// tiles' way through memory at 3 TB/s.  (The variants 1 and 2 by the LDS reads take less than that by now, both alike, and variant 2 is left
+// with its time in registers: over 300 problems of 128 to 4096 rows and columns and K = 128 to 8192 what these pick takes 0.3 % more time than the best
+// variant on average with operands from memory, 1.2 % from the caches; more than 10 % in 2 and 12 of them: 1376 x 448 x 3000 A:N B:T from the caches 22.7 us
+// on 128 x 128 tiles, 14.3 on 64 x 64.)
 // (1024 x 512 x 1024 on 128x128 would take 20 us split, 64x64 take 10).
 static const TrCost kTrCostLds[kNumTrVariants] = {{1, 0.0f, 71.0f}, {2, 25.0f, 3.3f}, {4, 16.0f, 6.0f}, {1, 0.0f, 53.0f}};
 

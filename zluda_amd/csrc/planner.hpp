@@ -48,6 +48,9 @@ constexpr TrVariant kTrVariants[] = {
 // stages of variant 1 by the LDS reads where no CU has more than one workgroup (mfma_tr_launch.hpp)
 constexpr int kTrDeepStages = 4;
 constexpr int kTr64Stages[] = {6, 3, 2};  // and of variant 2: up to one workgroup per CU, up to three, more
+constexpr int tr_ring_stages(int variant, uint64_t groups, uint64_t cus) {
+  return variant == 1 ? (groups <= cus ? kTrDeepStages : 2) : variant == 2 ? kTr64Stages[groups <= cus ? 0 : groups <= 3 * cus ? 1 : 2] : 2;
+}
 constexpr int kNumTrVariants = sizeof(kTrVariants) / sizeof(kTrVariants[0]);
 
 // decode configurations (index = plan.variant for ZLUDA_KERNEL_DECODE_W8A8).
