@@ -39,4 +39,4 @@ def test_the_kernels_take_the_rules_from_the_checked_header():
     kernels = os.path.join(ROOT, "zluda_amd", "csrc", "kernels")
     tr = open(os.path.join(kernels, "gemm_mfma_tr.hpp")).read()
     assert tr.count("tail_from = ") == 1 and "tail_from = tr_tail_from(Kl * ESZ, ESZ)" in tr
-    assert "if (pipe16_drains_prologue(MC, KT)) asm volatile(\"s_waitcnt vmcnt(0)\"" in open(os.path.join(kernels, "gemm_mfma_pipe16.hpp")).read()
+    assert "if (pipe16_drains_prologue(MC, KT, NSTAGE)) asm volatile(\"s_waitcnt vmcnt(0)\"" in open(os.path.join(kernels, "gemm_mfma_pipe16.hpp")).read()

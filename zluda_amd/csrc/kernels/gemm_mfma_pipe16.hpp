@@ -800,14 +800,11 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // ---- prologue: stages 0 and 1 in flight, stage 0 landed, its first fragments in registers -----------------
+  // ---- prologue: the first NSTAGE stages in flight, stage 0 landed, its first fragments in registers ---------
   static_for<NSTAGE>([&](auto s_c) { issue_stage(decltype(s_c)::value, decltype(s_c)::value * STAGE_V4); });
   // (MC: an instruction of the last stage's K tail may hold no K row that exists and retires early, so nothing is counted
   // where one is in flight)
-  if (pipe16_drains_prologue(MC, KT)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if constexpr (NSTAGE > 2) {
-    if (pipe16_drains_prologue(MC, KT, NSTAGE)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  }
+  if (pipe16_drains_prologue(MC, KT, NSTAGE)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   wait_vmcnt_barrier<PC.wait_prologue>();
   load_p_half(0, std::integral_constant<int, 0>{});
   load_q_half(0, std::integral_constant<int, 0>{});

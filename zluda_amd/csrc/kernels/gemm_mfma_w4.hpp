@@ -542,8 +542,8 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
 #pragma unroll
     for (int kk = 0; kk < 2; kk++) {
       const int row = par * 16 + r16;
-      // fp8: the lane's 32 bytes of its K group; int8: 16 bytes of each K half; MXFP4: 16 bytes (one scale block of 32
-      // elements) of each K step from the lane group's own 32-byte range, so that its two scale bytes are neighbours
+      // the lane group's 32 neighbouring bytes: fp8 in one MFMA; int8 and 16-bit 16 bytes in each of two; MXFP4 16 bytes (one scale
+      // block of 32 elements) in each K step, so that its two scale bytes are neighbours
       const int ch = (2 * g4 + kk) ^ swz(row);
       fragP[par][kk] = (wp * WTP + row) * CPR + ch;
       fragQ[par][kk] = (BP + wq * WTQ + row) * CPR + ch;
@@ -794,13 +794,16 @@ __global__ __launch_bounds__(256) void gemm_mfma_w4_kernel(MfmaParams prm) {
       constexpr int ACT = EPI == W4_EPI_BF16_GELU || EPI == W4_EPI_GELU_AUX ? ACT_GELU : ACT_NONE;
       constexpr bool KEPT = EPI == W4_EPI_GELU_AUX;
       const bool qv = staged.has[3] || staged.has[4];
-      if (p0 + BP <= NP) {
-        if (qv) w4_store_f16<KIND, ACT, KEPT, false, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
-        else w4_store_f16<KIND, ACT, KEPT, false, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+      if constexpr (KEPT) {  // (no vector along Q: aux_in_epilogue())
+        if (p0 + BP <= NP) w4_store_f16<KIND, ACT, true, false, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+        else w4_store_f16<KIND, ACT, true, true, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+      } else if (p0 + BP <= NP) {
+        if (qv) w4_store_f16<KIND, ACT, false, false, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+        else w4_store_f16<KIND, ACT, false, false, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
       } else if (qv) {
-        w4_store_f16<KIND, ACT, KEPT, true, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+        w4_store_f16<KIND, ACT, false, true, true, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
       } else {
-        w4_store_f16<KIND, ACT, KEPT, true, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
+        w4_store_f16<KIND, ACT, false, true, false, WTP, WTQ>(prm, acc, p0, q0, NP, NQ, bt, wp, wq, scalars, staged);
       }
     }
   };

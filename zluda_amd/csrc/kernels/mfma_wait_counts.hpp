@@ -49,8 +49,8 @@ constexpr PipeCounts pipe_counts(bool mx, int bp, int bq, int wp, int wq, int bk
   return c;
 }
 
-// gemm_mfma_pipe16.hpp: two stages of 128 K bytes (four in a form for operands along their row index), eight rows per DMA
-// instruction, no scale instructions
+// gemm_mfma_pipe16.hpp: `nstage` stages of 128 K bytes (two; up to six in the forms for operands along their row index), eight
+// rows per DMA instruction, no scale instructions
 struct Pipe16Counts {
   int rpp, lp, lq, nload;
   int wait_prologue;  // stages 0 .. nstage - 1 issued: stage 0 has landed

@@ -53,7 +53,7 @@ uint32_t launch_mfma(const Lowered &l, const zluda_gemm_plan &plan_in, void *ws,
   if (plan_in.variant >= (uint32_t)kNumMfmaVariants) return CUBLAS_STATUS_INVALID_VALUE;
   zluda_gemm_plan plan = plan_in;
   if (kMfmaVariants[plan.variant].w4) {
-    // The four-wave kernel carries three epilogues.  What the call turns out to ask for beyond them (a beta that is not
+    // The four-wave kernel carries four epilogues.  What the call turns out to ask for beyond them (a beta that is not
     // zero, a D that is not 16-byte aligned: known only now) runs on the eight-wave kernel with the same tile, which
     // needs no workspace either.
     const uint32_t cus = zluda_gemm_device_cu_count();

@@ -177,8 +177,8 @@ uint32_t lower_problem(const zluda_gemm_problem *p, bool dry, Lowered *out) {
   // the bias buffer is an output here: sums over K of op(A)'s rows / op(B)'s columns, D as with DEFAULT
   case CUBLASLT_EPILOGUE_BGRADA: g.act = ACT_NONE; g.bgrad_src = 1; break;
   case CUBLASLT_EPILOGUE_BGRADB: g.act = ACT_NONE; g.bgrad_src = 2; break;
-  // GELU with its input kept, and GELU's gradient: the GEMM kernel runs without the activation, a second
-  // element-wise pass (kernels/aux_epilogue.hpp) finishes D
+  // GELU with its input kept, and GELU's gradient: in the GEMM kernel's epilogue where aux_in_epilogue() says so; elsewhere it runs
+  // without the activation, and a second element-wise pass (kernels/aux_epilogue.hpp) finishes D
   case CUBLASLT_EPILOGUE_GELU_AUX: g.act = ACT_NONE; g.aux_mode = 1; break;
   case CUBLASLT_EPILOGUE_GELU_AUX_BIAS: g.act = ACT_NONE; g.aux_mode = 1; has_bias = true; break;
   case CUBLASLT_EPILOGUE_DGELU: g.act = ACT_NONE; g.aux_mode = 2; break;
@@ -367,8 +367,8 @@ static uint32_t ceil_div(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
 int w4_epilogue_class(const Lowered &l, bool dry) {
   const GemmArgs &g = l.g;
-  // (the epilogues with an aux matrix are plain problems to the GEMM kernel: launch_planned points D at the aux matrix or
-  // runs the gradient pass behind it)
+  // (GELU with its input kept has an epilogue of its own where a plain problem has W4_CLASS_BF16 and aux_in_epilogue() holds; the other
+  // epilogues with an aux matrix are plain problems here: launch_planned points D at the aux matrix or runs the gradient pass behind it)
   if (g.beta_mode != SCALAR_VALUE) return W4_CLASS_NONE;
   const bool swapped = g.d_si != 1;
   const int64_t d_sq = swapped ? g.d_si : g.d_sj;
