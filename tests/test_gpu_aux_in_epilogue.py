@@ -1,9 +1,11 @@
 """GELU with its input kept and GELU's gradient in the epilogues of the 16-bit tile kernels: every accumulator layout, tiles that hang over
-either end of D, pitches and batch strides of aux of their own, and what keeps a problem on the pass behind the matmul."""
+either end of D, pitches and batch strides of aux of their own, and what keeps a problem on the pass behind the matmul.  Which of the two ways
+a problem goes is asked of the planner's own rule and read off the scratch that the sums of a gradient leave."""
 import ctypes as C
 
 import pytest
 
+import planner_probe
 from oracle.cases import Case
 from zluda_amd import abi as K
 
@@ -19,8 +21,8 @@ TOL = {K.CUDA_R_16BF: 1e-2, K.CUDA_R_16F: 2e-3}
 TOL_BEHIND, FLOOR_BEHIND = 12 / 512, 1e-1
 
 
-def run(api, spec, seed, family, variant, ws=4 << 20, block=None, in_epilogue=True):
-    """the case, its plan; `in_epilogue`: the sums of DGELU_BGRAD are counted one per wave along D's columns"""
+def run(api, spec, seed, family, variant, ws=4 << 20, block=None, in_epilogue=True, lds=None):
+    """the case, its plan; `in_epilogue`: the kernel does it all, else there is a pass behind it; `lds`: transposed by the LDS reads"""
     import torch
     print("case", spec, "family", family, "variant", variant, flush=True)
     case = Case(spec, seed)
@@ -33,6 +35,10 @@ def run(api, spec, seed, family, variant, ws=4 << 20, block=None, in_epilogue=Tr
     assert api.zluda_gemm_plan_problem(C.byref(p), family, variant, api.zluda_gemm_device_cu_count(), C.byref(plan)) == 0
     if block:
         plan.block = block
+    sums = planner_probe.aux_sum_bytes(p, plan) if case.bgrad else 0
+    assert (planner_probe.aux_in_epilogue(p, plan) == 1 and sums <= plan.workspace) == in_epilogue
+    if lds is not None:
+        assert planner_probe.lds_reads(p, plan, api.zluda_gemm_device_cu_count()) == lds
     assert api.zluda_gemm_launch(C.byref(p), C.byref(plan), torch.cuda.current_stream().cuda_stream) == 0
     torch.cuda.synchronize()
     case.compare(case.download(dt), ref, tol=TOL[spec["d_type"]] if in_epilogue else TOL_BEHIND,
@@ -42,12 +48,16 @@ def run(api, spec, seed, family, variant, ws=4 << 20, block=None, in_epilogue=Tr
     if case.bgrad:
         case.compare_bgrad(keep[3][:case.bias.nbytes].cpu().numpy().view(case.bias.dtype).copy(), case.bgrad_ref, floor_frac=1.0)
         assert bool((scratch[plan.workspace:] == 0xFF).all())
+        if in_epilogue:   # one sum per wave and row, each of them written, and nothing else
+            import torch
+            assert bool((scratch[:sums].view(torch.int32) != -1).all()) and bool((scratch[sums:] == 0xFF).all())
     return case, plan
 
 
-# family, variant, block: 32x32 tiles of every wave shape, 16x16 tiles, the four-wave kernel; the layouts of the transposing kernels
+# family, variant, block: 32x32 tiles of every wave shape, 16x16 tiles, the four-wave kernel; the layouts of the transposing kernels (the 64 x 64 tile
+# by the LDS reads, the 128 x 128 tile in registers: K is short)
 FORMS = [(H16, v, b, 1, 0) for v, b in ((0, 0), (2, 256), (2, 512), (4, 0), (5, 0), (6, 0), (7, 0), (8, 0), (9, 0), (10, 0), (11, 0))] + \
-        [(TR16, v, b, ta, tb) for v, b in ((0, 0), (1, 256), (1, 512), (2, 256), (2, 512), (3, 0)) for ta, tb in ((0, 0), (0, 1), (1, 1))]
+        [(TR16, v, b, ta, tb) for v, b in ((0, 0), (1, 256), (1, 512), (2, 0), (3, 0)) for ta, tb in ((0, 0), (0, 1), (1, 1))]
 
 
 @pytest.mark.parametrize("epi", [AUX, AUX_BIAS, DG, DG_SUMS])
@@ -61,7 +71,35 @@ def test_every_form(gpu_api, family, variant, block, ta, tb, epi):
         if (ta, tb) != (1, 0) and tb:   # (the columns of B lie side by side: a whole number of 16-byte pieces for the LDS reads)
             spec["ldb"] = (n + 7) // 8 * 8
         behind = variant == 0 or (family == H16 and block == 256)   # (wave tiles of 128 x 64 on the 32x32 shapes)
-        run(gpu_api, spec, 9700 + 10 * epi + i, family, variant, block=block, in_epilogue=not behind)
+        if family == H16 and variant == 11 and epi in (DG, DG_SUMS):
+            behind = True   # (the four-wave kernel keeps GELU's input, and has no gradient)
+        run(gpu_api, spec, 9700 + 10 * epi + i, family, variant, block=block, in_epilogue=not behind,
+            lds=None if family == H16 else int(variant in (2, 3)))
+
+
+# Operands off 16 bytes (pitches of whole dwords) are transposed in registers: 64 x 64 tiles with one group of waves and with two that share K,
+# the 256 x 256 tile of the 16x16 shapes
+@pytest.mark.parametrize("epi", [AUX_BIAS, DG, DG_SUMS])
+@pytest.mark.parametrize("variant,block", [(2, 256), (2, 512), (3, 512)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 1), (1, 0)])
+def test_forms_in_registers(gpu_api, ta, tb, variant, block, epi):
+    for i, (m, n, k) in enumerate(((264, 131, 264), (72, 65, 800), (8, 1, 72))):
+        off = lambda x: x + (2 if x % 4 == 0 else 3 if x % 2 else 4)   # (a multiple of 2, of 4 at the most)
+        spec = dict(BF, m=m, n=n, k=k, transa=ta, transb=tb, epilogue=epi, lda=off(k if ta else m), ldb=off(n if tb else k))
+        run(gpu_api, spec, 9820 + i, TR16, variant, block=block, lds=0)
+
+
+# ... and by the LDS reads: the 128 x 128 tile on its ring of four stages (6 tiles) and of two (264), the 64 x 64 tile on three (660) and two (990)
+@pytest.mark.parametrize("epi", [AUX_BIAS, DG, DG_SUMS])
+@pytest.mark.parametrize("variant,k,batch", [(1, 712, 1), (1, 1016, 1), (1, 456, 44), (2, 832, 1), (2, 136, 44), (2, 136, 66)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 1)])
+def test_forms_by_the_lds_reads(gpu_api, ta, tb, variant, k, batch, epi):
+    spec = dict(BF, m=264, n=131, k=k, transa=ta, transb=tb, batch=batch, epilogue=epi)
+    if tb:
+        spec["ldb"] = 136
+    if batch > 1:
+        spec["bias_batch_stride"] = 264
+    run(gpu_api, spec, 9840, TR16, variant, ws=16 << 20, lds=1)
 
 
 @pytest.mark.parametrize("family,variant,ta,tb", [(H16, 4, 1, 0), (H16, 8, 1, 0), (H16, 11, 1, 0), (TR16, 1, 0, 0), (TR16, 2, 0, 1)])
@@ -69,7 +107,7 @@ def test_batches_pitches_scales(gpu_api, family, variant, ta, tb):
     base = dict(BF, m=200, n=136, k=264, batch=3, transa=ta, transb=tb, ldd=208, ldc=208, aux_ld=224, aux_batch_stride=224 * 136 + 40)
     run(gpu_api, dict(base, epilogue=AUX_BIAS, bias_type=K.CUDA_R_32F, bias_batch_stride=203), 9801, family, variant)
     run(gpu_api, dict(base, epilogue=AUX_BIAS, bias_batch_stride=203), 9802, family, variant)     # (a bias at odd addresses)
-    run(gpu_api, dict(base, epilogue=DG_SUMS, bias_batch_stride=208), 9803, family, variant)
+    run(gpu_api, dict(base, epilogue=DG_SUMS, bias_batch_stride=208), 9803, family, variant, in_epilogue=variant != 11)
 
 
 @pytest.mark.parametrize("change", [dict(m=260), dict(ldd=268, ldc=268), dict(aux_ld=268), dict(order_c=1, order_d=1, aux_ld=136), dict(with_c=True),
@@ -84,7 +122,8 @@ def test_what_keeps_the_pass_behind_the_matmul(gpu_api, epi, ta, change):
         spec["c_type"] = K.CUDA_R_32F
     if spec.get("with_c") and epi == AUX_BIAS:
         spec["beta"] = 0.5
-    run(gpu_api, spec, 9850, H16 if ta else TR16, -1, ws=ws, in_epilogue=False)
+    # (without scratch only the sums of a gradient want the pass)
+    run(gpu_api, spec, 9850, H16 if ta else TR16, -1, ws=ws, in_epilogue=ws == 0 and epi == AUX_BIAS)
 
 
 @pytest.mark.parametrize("epi", [AUX, DG, DG_SUMS])

@@ -24,7 +24,7 @@ def check(gpu_api, s, seed, ws=0):
     print("case", s, flush=True)
     case = Case(s, seed)
     ref = case.run_oracle()
-    for v in (1, 3):
+    for v in (1, 2, 3):
         st, got, kernel, variant = case.run_gpu(gpu_api, forced_kernel=K.ZLUDA_KERNEL_MFMA_TR16, forced_variant=v, workspace_bytes=ws)
         assert st == 0 and (kernel, variant) == (K.ZLUDA_KERNEL_MFMA_TR16, v)
         case.compare(got, ref, tol=1e-2)   # one rounding to 16 bits of sums in another order
