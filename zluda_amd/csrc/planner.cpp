@@ -602,8 +602,9 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus, uint64_t workspace_
 //   transposed in registers  4.6 + 1.2 n + (7.5 + 15.3 n) u
 //   by the LDS reads         6.2 + 1.45 n + 2.4 per round behind the first + 27.8 u per round of two on a CU, 17.4 u for one
 // -- level at K = 700 for n = 1, 430 for two, 1200 for three.  (2048 x 2048 x 128: 7.5 us in registers, 9.7 by the LDS reads;
-// 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 tile is faster by the LDS reads at every K, the 64 x 64 tile too (bf16, us: 512 x 512 x 128
-// 5.4 and 5.3, 512^3 7.9 and 6.7, 1024^3 A:N B:T 9.8 and 8.7, 2104 x 704 x 1000 14.5 and 12.4, 1536 x 1536 x 1024 17.8 and 13.5), but for
+// 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 tile is faster by the LDS reads at every K, the 64 x 64 tile too (bf16, us from memory: 512 x 512 x 128
+// 5.2 and 4.8, 512^3 7.8 and 6.5, 1024^3 A:N B:T 11.3 and 9.2, 2104 x 704 x 1000 16.7 and 13.7, 64 x 64 x 16384 69 and 47.5; from the caches 4.6 and 4.5,
+// 6.4 and 6.0, 9.1 and 7.6, 11.8 and 10.6, 60 and 47), but for
 // a long operand along its row index beside up to 16 K-contiguous tokens on four to six workgroups per CU: memory bound, and the two-stage ring
 // has less on its way than the registers (us from memory, in registers and by the LDS reads: 65536 x 16 x 512 17.2 and 18.7, x 2048 57 and 61, 14336 x 1 x
 // 4096 in four shares 32.2 and 33.8, x 16 level; x 33 39.3 and 37.5; level at K = 64 and on eight workgroups per CU; up to three of them run
@@ -763,10 +764,10 @@ static uint64_t row_sum_workspace(const GemmArgs &g, uint64_t workspace_size, ui
   return s > 1 ? (uint64_t)s * rows * g.batch * 4 : 0;
 }
 
-// The forms the epilogues with an aux matrix are instantiated for: 16-bit operands on the tile kernels up to a size of the wave tile, unsplit, 16-bit D and aux that the
-// 16-byte stores of eight rows fit.  us with a pass behind the matmul and without: bf16 8192 x 4096 x 2048 GELU_AUX_BIAS 133 -> 122
-// (the product alone 110), A:N B:N DGELU_BGRAD 153 -> 138 (115); 1000 x 700 x 496 8.8 -> 6.6 and 17.3 -> 12.7; 2048 x 1000 x 1024 14.5 -> 11.0
-// and 21.8 -> 16.3.
+// The forms the epilogues with an aux matrix are instantiated for: 16-bit operands on the tile kernels up to a size of the wave tile, unsplit,
+// 16-bit D and aux that the 16-byte stores of eight rows fit.  us with a pass behind the matmul and without (bf16, operands in the caches):
+// 8192 x 4096 x 2048 GELU_AUX_BIAS 122 -> 110, A:N B:N DGELU_BGRAD 152 -> 138; 2048 x 1000 x 1024 13.2 -> 10.1 and 21.1 -> 13.4; 1000 x 700 x 496
+// 9.0 -> 7.1 and 16.5 -> 12.2.
 bool aux_in_epilogue(const Lowered &l, const zluda_gemm_plan &plan, bool dry) {
   const GemmArgs &g = l.g;
   if (!g.aux_mode || (plan.kernel != ZLUDA_KERNEL_MFMA_H16 && plan.kernel != ZLUDA_KERNEL_MFMA_TR16)) return false;
