@@ -135,17 +135,18 @@ static void check_pipe16_mc(int bp, int bq, int wp, int wq) {
 }
 
 // The same on a ring of more than two stages: a wait of the loop leaves those behind the next one in flight, but nothing where the
-// last stage of K or padding behind it is among them.
+// last stage of K is among them; nothing behind that one is requested.
 static void check_pipe16_ring(int bp, int bq, int wp, int wq, int nstage) {
   const Pipe16Counts c = pipe16_counts(bp, bq, wp, wq, nstage);
   if ((nstage - 1) * c.nload >= 64) fail("vmcnt range", -1, 0, 0, 0, 0);
   for (int KT = 0; KT <= 5 * nstage + 2; KT++) {
     std::vector<Ins> log;
     auto data = [&](int stage) { for (int i = 0; i < c.nload; i++) log.push_back(Ins{DATA, stage}); };
-    for (int s = 0; s < nstage; s++) data(s);
-    if (pipe16_drains_prologue(true, KT, nstage) != (nstage - 1 >= KT - 1)) fail("the prologue's drain", -1, 0, 0, 0, KT);
-    if (!landed(log, log.size(), c.wait_prologue, DATA, 0)) fail("prologue: stage 0 still in flight", -1, 0, 0, 0, KT);
-    if (data_after(log, 0) != c.wait_prologue) fail("prologue: N is not the count of younger data instructions", -1, 0, 0, 0, KT);
+    for (int s = 0; s < nstage && s < KT; s++) data(s);
+    const bool drained = pipe16_drains_prologue(true, KT, nstage);
+    if (drained != (nstage - 1 >= KT - 1)) fail("the prologue's drain", -1, 0, 0, 0, KT);
+    if (!drained && !landed(log, log.size(), c.wait_prologue, DATA, 0)) fail("prologue: stage 0 still in flight", -1, 0, 0, 0, KT);
+    if (!drained && data_after(log, 0) != c.wait_prologue) fail("prologue: N is not the count of younger data instructions", -1, 0, 0, 0, KT);
     // the turns at compile time: none of their stages drains, or requests what is not a whole stage
     int inside = 0;
     for (; pipe16_inside(inside, KT, nstage); inside += pipe16_turn(nstage))
@@ -154,10 +155,13 @@ static void check_pipe16_ring(int bp, int bq, int wp, int wq, int nstage) {
     if (inside % nstage || inside % 2) fail("a turn leaves the ring inside it", -1, 0, 0, inside, KT);
     if (inside + pipe16_turn(nstage) + nstage + 1 <= KT) fail("a turn is left out", -1, 0, 0, inside, KT);
     for (int kt = 0; kt < KT; kt++) {
-      if (pipe16_drains_stage(kt, KT, nstage) != (kt + nstage - 1 >= KT - 1)) fail("a stage's drain", -1, 0, 0, kt, KT);
+      const bool drains = pipe16_drains_stage(kt, KT, nstage);
+      if (drains != (kt + nstage - 1 >= KT - 1)) fail("a stage's drain", -1, 0, 0, kt, KT);
+      checked++;
+      if (drains) continue;  // (and requests nothing)
+      if (kt + nstage >= KT) fail("a stage behind the last one is requested", -1, 0, 0, kt, KT);
       if (!landed(log, log.size(), c.wait_stage, DATA, kt + 1)) fail("next stage still in flight", -1, 0, 0, kt, KT);
       if (data_after(log, kt + 1) != c.wait_stage) fail("N is not the count of younger data instructions", -1, 0, 0, kt, KT);
-      checked++;
       data(kt + nstage);
     }
   }

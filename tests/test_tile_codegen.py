@@ -32,14 +32,16 @@ def kernels(instances, *flags):
     return found
 
 
-def k_loop(lines):
-    """the loop with the most MFMAs"""
+def k_loop(lines, first=False):
+    """the loop with the most MFMAs, or the first one that has any"""
     labels = {m.group(1): i for i, l in enumerate(lines) for m in [re.match(r"(\.LBB\d+_\d+):", l)] if m}
     loops = []
     for i, l in enumerate(lines):
         m = re.match(r"s_c?branch\S*\s+(\.LBB\d+_\d+)", l)
         if m and labels.get(m.group(1), i) < i:
             loops.append(lines[labels[m.group(1)]:i])
+    if first:
+        return next(b for b in loops if any(x.startswith("v_mfma") for x in b))
     return max(loops, key=lambda b: sum(x.startswith("v_mfma") for x in b))
 
 
@@ -56,7 +58,7 @@ def test_no_reload_in_the_loop_of_a_256x256_tile():
 def test_turns_of_a_deep_ring_address_nothing_at_run_time(tile, stages, turn):
     names = ["gemm_mfma_pipe16_kernel<KIND_BF16, 0, 0, %d, %d, 2, 2, %s, %d>" % (tile, tile, mc, stages) for mc in ("true, true", "true, false")]
     for lines in kernels(names, "-mllvm", "-amdgpu-mfma-vgpr-form=1"):
-        body = k_loop(lines)
+        body = k_loop(lines, first=True)
         mfmas = (tile // 32) ** 2 * 2
         assert sum(x.startswith("v_mfma") for x in body) == turn * mfmas
         assert sum(x.startswith("s_barrier") for x in body) == turn

@@ -648,12 +648,12 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   // stage kt -> LDS slot at 16-byte offset `so`, DMA instruction `n` of LP + LQ.  Stages kt >= KT are never multiplied; they
   // are issued only so that every stage has the same vector memory operations in flight, as real loads of one cache
   // line (an instruction whose lanes are all out of range completes without a memory round trip and can
-  // retire ahead of older loads).
+  // retire ahead of older loads).  Rings of more than two slots drain where such a stage would be in flight, and request none.
   auto issue_one = [&](int kt, int so, auto n_c) {
     constexpr int n = decltype(n_c)::value;
     constexpr bool is_p = n < LP, mc = is_p ? PMC : QMC;
     constexpr int i = is_p ? n : n - LP;
-    const int live = kt < KT ? -1 : 0;  // uniform
+    const int live = NSTAGE > 2 || kt < KT ? -1 : 0;  // uniform
     const int *voff = is_p ? voffP : voffQ;
     v4i *base = &lds[so] + (is_p ? 0 : P_V4);
     if constexpr (mc) {
@@ -801,7 +801,9 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   };
 
   // ---- prologue: the first NSTAGE stages in flight, stage 0 landed, its first fragments in registers ---------
-  static_for<NSTAGE>([&](auto s_c) { issue_stage(decltype(s_c)::value, decltype(s_c)::value * STAGE_V4); });
+  static_for<NSTAGE>([&](auto s_c) {
+    if (NSTAGE == 2 || decltype(s_c)::value < KT) issue_stage(decltype(s_c)::value, decltype(s_c)::value * STAGE_V4);
+  });
   // (MC: an instruction of the last stage's K tail may hold no K row that exists and retires early, so nothing is counted
   // where one is in flight)
   if (pipe16_drains_prologue(MC, KT, NSTAGE)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -812,8 +814,9 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   // ---- one stage ----------------------------------------------------------------------------------------------
   // ODD = 0: on entry P half 0 and Q half 0 of the stage are in registers; the next stage will find P half 0
   // and Q half 1 of its own.  ODD = 1: the same with the Q halves exchanged.
-  auto do_stage = [&](int kt, int so, int so_next, auto odd_c, auto inside_c) {
-    constexpr bool INSIDE = decltype(inside_c)::value != 0;  // nothing of this stage's turn of the ring ends K or lies behind it
+  // `requests`: stage kt + NSTAGE, masked (0), as one inside K (1), or nothing (2: none is left, and what is in flight has to land)
+  auto do_stage = [&](int kt, int so, int so_next, auto odd_c, auto requests_c) {
+    constexpr int REQ = decltype(requests_c)::value;
     constexpr int QA = decltype(odd_c)::value, QB_ = 1 - QA;  // the Q half that is resident / that is fetched
     using P0 = std::integral_constant<int, 0>;
     using P1 = std::integral_constant<int, 1>;
@@ -840,9 +843,7 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     pattern(std::integral_constant<int, DSP - PD * EARLY>{}, std::integral_constant<int, 0>{});
     // every fragment of the stage has been requested: wait for them and for this wave's share of stage
     // kt+1, meet the other waves; then the slot is free and the other one readable
-    if constexpr (NSTAGE > 2 && !INSIDE) {
-      if (pipe16_drains_stage(kt, KT, NSTAGE)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+    if constexpr (REQ == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     wait_vmcnt_barrier<PC.wait_stage>();
     // (P1, QB): refill this slot with stage kt+NSTAGE, P half 0 of stage kt+1 arrives
     load_p_part(so_next, P0{}, I0{}, IL{});
@@ -852,8 +853,8 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
       static_for<NLOAD>([&](auto n_c) {
         constexpr int n = decltype(n_c)::value;
         mfma_part(P1{}, QBc{}, std::integral_constant<int, NM * n / NLOAD>{}, std::integral_constant<int, NM * (n + 1) / NLOAD>{});
-        if constexpr (INSIDE) issue_inside(kt + NSTAGE, so, n_c);
-        else issue_one(kt + NSTAGE, so, n_c);
+        if constexpr (REQ == 1) issue_inside(kt + NSTAGE, so, n_c);
+        else if constexpr (REQ == 0) issue_one(kt + NSTAGE, so, n_c);
         __builtin_amdgcn_sched_barrier(0);
       });
     } else {
@@ -869,8 +870,8 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
   };
 
   int kt = 0;
-  using E = std::integral_constant<int, 0>;  // an even stage; not inside
-  using O = std::integral_constant<int, 1>;  // an odd one; inside
+  using E = std::integral_constant<int, 0>;  // an even stage; masked requests
+  using O = std::integral_constant<int, 1>;  // an odd one
   if constexpr (NSTAGE == 2) {
     for (; kt + 2 <= KT; kt += 2) {
       do_stage(kt, 0, STAGE_V4, E{}, E{});
@@ -882,15 +883,18 @@ __global__ __launch_bounds__(WP *WQ * 64) void gemm_mfma_pipe16_kernel(MfmaParam
     // Whole turns of the ring with its slots fixed at compile time and without the masks of the last stages: with the slot in a register
     // and the masks a stage of a 64 x 64 tile has 42 scalar and 15 vector instructions beside its 8 MFMAs, a lone workgroup's time
     constexpr int TURN = pipe16_turn(NSTAGE);
-    for (; pipe16_inside(kt, KT, NSTAGE); kt += TURN)
+    auto turn = [&](auto stage) {
       static_for<TURN>([&](auto u_c) {
         constexpr int u = decltype(u_c)::value;
-        do_stage(kt + u, u % NSTAGE * STAGE_V4, (u + 1) % NSTAGE * STAGE_V4, std::integral_constant<int, u & 1>{}, O{});
+        stage(kt + u, u % NSTAGE * STAGE_V4, (u + 1) % NSTAGE * STAGE_V4, std::integral_constant<int, u & 1>{});
       });
+    };
+    for (; pipe16_inside(kt, KT, NSTAGE); kt += TURN)
+      turn([&](int k, int so, int so_next, auto odd_c) { do_stage(k, so, so_next, odd_c, std::integral_constant<int, 1>{}); });
     for (; kt < KT; kt += TURN)
-      static_for<TURN>([&](auto u_c) {
-        constexpr int u = decltype(u_c)::value;
-        if (kt + u < KT) do_stage(kt + u, u % NSTAGE * STAGE_V4, (u + 1) % NSTAGE * STAGE_V4, std::integral_constant<int, u & 1>{}, E{});
+      turn([&](int k, int so, int so_next, auto odd_c) {
+        if (!pipe16_drains_stage(k, KT, NSTAGE)) do_stage(k, so, so_next, odd_c, std::integral_constant<int, 0>{});
+        else if (k < KT) do_stage(k, so, so_next, odd_c, std::integral_constant<int, 2>{});
       });
   }
 

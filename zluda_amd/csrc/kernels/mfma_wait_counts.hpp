@@ -71,8 +71,8 @@ constexpr Pipe16Counts pipe16_counts(int bp, int bq, int wp, int wq, int nstage 
 }
 
 // The form of gemm_mfma_pipe16.hpp whose operands lie along their row index ("MC"): an instruction of the last stage may hold
-// no K row that exists.  Where that stage or one behind it is in flight the prologue waits for everything, and so does a stage of a ring of
-// more than two slots.
+// no K row that exists.  Where that stage is in flight the prologue waits for everything, and so does a stage of a ring of more than two
+// slots, which then requests no further one: what lies behind the last stage is never asked for there.
 constexpr bool pipe16_drains_prologue(bool mc, int kt) { return mc && kt <= 2; }
 constexpr bool pipe16_drains_prologue(bool mc, int kt, int nstage) { return pipe16_drains_prologue(mc, kt - (nstage - 2)); }
 constexpr bool pipe16_drains_stage(int stage, int kt, int nstage) { return stage + nstage >= kt; }
