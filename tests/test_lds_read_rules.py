@@ -1,5 +1,5 @@
 """Which form of the transposing family's 64 x 64 tile runs 16-byte aligned 16-bit operands: transposed by the LDS reads, but in registers for
-a long operand along its row index beside a few K-contiguous tokens on four to six workgroups per CU."""
+a K of one stage there and for a long operand along its row index beside a few K-contiguous tokens on four to six workgroups per CU."""
 import pytest
 
 import planner_probe
@@ -12,10 +12,10 @@ TR16 = K.ZLUDA_KERNEL_MFMA_TR16
 @pytest.mark.parametrize("m,n,k,ta,tb,lds", [
     (65536, 16, 512, 0, 0, 0), (16, 65536, 512, 1, 1, 0),      # 1024 workgroups, either operand the long one
     (65536, 16, 512, 0, 1, 1), (65536, 16, 512, 1, 1, 1),      # both along their row index; the long one K-contiguous
-    (65536, 16, 64, 0, 0, 1), (65536, 17, 512, 0, 0, 1),
+    (65536, 16, 72, 0, 0, 1), (65536, 17, 512, 0, 0, 1),
     (49152, 16, 512, 0, 0, 1), (49160, 16, 512, 0, 0, 0),      # three workgroups per CU, and more
     (98304, 16, 512, 0, 0, 0), (98312, 16, 512, 0, 0, 1),      # six, and more
-    (1024, 1024, 512, 0, 0, 1)])
+    (1024, 1024, 512, 0, 0, 1), (1024, 1024, 32, 0, 1, 0), (1024, 1024, 40, 0, 1, 1), (1024, 1024, 64, 0, 0, 0), (1024, 1024, 72, 1, 1, 1)])
 def test_sixty_four_square(api, m, n, k, ta, tb, lds):
     status, p, plan, keep = planned(api, m, n, k, ta=ta, tb=tb, workspace=0, family=TR16, variant=2)
     assert status == 0 and plan.grid_z == 1

@@ -602,9 +602,10 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus, uint64_t workspace_
 //   transposed in registers  4.6 + 1.2 n + (7.5 + 15.3 n) u
 //   by the LDS reads         6.2 + 1.45 n + 2.4 per round behind the first + 27.8 u per round of two on a CU, 17.4 u for one
 // -- level at K = 700 for n = 1, 430 for two, 1200 for three.  (2048 x 2048 x 128: 7.5 us in registers, 9.7 by the LDS reads;
-// 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 tile is faster by the LDS reads at every K, the 64 x 64 tile too (bf16, us from memory: 512 x 512 x 128
-// 5.2 and 4.8, 512^3 7.8 and 6.5, 1024^3 A:N B:T 11.3 and 9.2, 2104 x 704 x 1000 16.7 and 13.7, 64 x 64 x 16384 69 and 47.5; from the caches 4.6 and 4.5,
-// 6.4 and 6.0, 9.1 and 7.6, 11.8 and 10.6, 60 and 47), but for
+// 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 tile is faster by the LDS reads at every K, the 64 x 64 tile beyond one stage in registers
+// (K = 16 and 32: 3 to 9 % slower by the LDS reads, from the caches and from memory; 64 with one operand K-contiguous 4 and 0 %, with none 2 and 5 % faster).
+// (bf16, us from memory: 512 x 512 x 128 5.2 and 4.8, 512^3 7.8 and 6.5, 1024^3 A:N B:T 11.3 and 9.2, 2104 x 704 x 1000 16.7 and 13.7, 64 x 64 x 16384 69 and 47.5; from the caches 4.6 and 4.5,
+// 6.4 and 6.0, 9.1 and 7.6, 11.8 and 10.6, 60 and 47.)  Another exception is
 // a long operand along its row index beside up to 16 K-contiguous tokens on four to six workgroups per CU: memory bound, and the two-stage ring
 // has less on its way than the registers (us from memory, in registers and by the LDS reads: 65536 x 16 x 512 17.2 and 18.7, x 2048 57 and 61, 14336 x 1 x
 // 4096 in four shares 32.2 and 33.8, x 16 level; x 33 39.3 and 37.5; level at K = 64 and on eight workgroups per CU; up to three of them run
@@ -612,6 +613,7 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus, uint64_t workspace_
 bool tr_lds_reads(const Lowered &l, int variant, uint64_t groups, uint32_t splits, uint32_t cus) {
   if (variant == 0 || !lds_transposable(l)) return false;
   if (variant == 2) {
+    if ((uint64_t)l.g.K <= (l.a_kcontig || l.b_kcontig ? 64 : 32) * (uint64_t)std::max(splits, 1u)) return false;
     const bool a_long = l.g.M >= l.g.N, one_long = (a_long ? l.b_kcontig : l.a_kcontig) && std::min(l.g.M, l.g.N) <= 16;
     return !(one_long && groups > 3 * (uint64_t)cus && groups <= 6 * (uint64_t)cus && (uint64_t)l.g.K >= 128 * (uint64_t)std::max(splits, 1u));
   }
