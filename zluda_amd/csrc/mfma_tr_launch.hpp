@@ -63,6 +63,8 @@ inline uint32_t launch_tr_variant(const MfmaParams &prm, const zluda_gemm_plan &
 
 // the variants 1, 2 and 3 where tr_lds_reads() says so: their grids, with the transposition in the LDS reads
 uint32_t launch_trl_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
+uint32_t launch_trl_rings_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
+uint32_t launch_trl_rings_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_trl_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 // (a problem whose `act` is an epilogue with an aux matrix)
 uint32_t launch_trl_aux_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
@@ -77,8 +79,14 @@ uint32_t launch_tr_f16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool 
 uint32_t launch_tr_bf16(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 uint32_t launch_tr_f32(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s);
 
+// Which of the two below: the variant 2, and the variant 1 on its deep ring.  Their kernels have a translation unit, i.e. a code object, of their
+// own (mfma_trl_rings_*.hip): in one with them the 256 x 256 tiles took 1 to 2 % longer (bf16 4096 x 4096 x 256 A:N B:N, same code).
+inline bool trl_on_rings(const zluda_gemm_plan &plan) {
+  return plan.variant == 2 || tr_ring_stages((int)plan.variant, (uint64_t)plan.grid_x * plan.grid_y * (plan.grid_z > 1 ? plan.grid_z : 1), zluda_gemm_device_cu_count()) > 2;
+}
+
 template <int KIND, bool AUX = false>
-inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s) {
+inline uint32_t launch_trl_rings(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s) {
   const dim3 grid(plan.grid_x, plan.grid_y, plan.grid_z > 1 ? plan.grid_z : 1);
   const int stages = tr_ring_stages((int)plan.variant, (uint64_t)grid.x * grid.y * grid.z, zluda_gemm_device_cu_count());
   if (plan.variant == 2) {
@@ -106,6 +114,12 @@ inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, b
     ZLUDA_TRL_DEEP(false, false) ZLUDA_TRL_DEEP(false, true) ZLUDA_TRL_DEEP(true, false)
 #undef ZLUDA_TRL_DEEP
   }
+  return CUBLAS_STATUS_INVALID_VALUE;
+}
+
+template <int KIND, bool AUX = false>
+inline uint32_t launch_trl(const MfmaParams &prm, const zluda_gemm_plan &plan, bool pkc, bool qkc, hipStream_t s) {
+  const dim3 grid(plan.grid_x, plan.grid_y, plan.grid_z > 1 ? plan.grid_z : 1);
 #define ZLUDA_TRL_MODE(BP, BQ, WP, WQ, PK, QK)                                                                       \
   if (pkc == PK && qkc == QK)                                                                                        \
     return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, BP, BQ, WP, WQ, !PK, !QK, 2, AUX>, grid, dim3(WP * WQ * 64), s, prm);
