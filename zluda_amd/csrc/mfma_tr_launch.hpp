@@ -91,7 +91,7 @@ inline uint32_t launch_trl_rings(const MfmaParams &prm, const zluda_gemm_plan &p
   const int stages = tr_ring_stages((int)plan.variant, (uint64_t)grid.x * grid.y * grid.z, zluda_gemm_device_cu_count());
   if (plan.variant == 2) {
     // 17 KiB a stage: as many of them as the workgroups that share a CU have room for.  (64 x 64 tiles, bf16, us from memory and from the caches,
-    // transposed in registers before: 704 x 1000 x 2104, 176 workgroups 18.1 -> 14.3 and 13.5 -> 10.5; 2104 x 704 x 1000, 363, 16.7 -> 13.7 and 11.8 -> 10.6.)
+    // transposed in registers before: 704 x 1000 x 2104, 176 workgroups 17.9 -> 14.2 and 13.5 -> 10.6; 2104 x 704 x 1000, 363, 16.9 -> 13.8 and 11.9 -> 10.7.)
 #define ZLUDA_TRL_64(PK, QK, NS)                                                                                      \
   if (pkc == PK && qkc == QK)                                                                                        \
     return launch_kernel(gemm_mfma_pipe16_kernel<KIND, 0, 0, 64, 64, 2, 2, !PK, !QK, NS, AUX>, grid, dim3(256), s, prm);
@@ -105,8 +105,8 @@ inline uint32_t launch_trl_rings(const MfmaParams &prm, const zluda_gemm_plan &p
   }
   // One workgroup to a CU: four stages of 33 KiB instead of two, all but the one that is multiplied on their way (a stage's time is far
   // below a round trip to memory; with two workgroups the other one fills the gaps, and two rings of four do not fit).  bf16, us from
-  // memory and from the caches: 2048^3 A:N B:N 33.8 -> 25.9 and 28.3 -> 22.3, A:N B:T 33.5 -> 25.6 and 29.2 -> 21.6, 1024 x 4096 x 4096 59.8 -> 41.8 and
-  // 46.4 -> 34.8; at 11 stages 2048 x 2048 x 704 13.7 -> 13.0 and 11.5 -> 11.8; on 512 tiles 2048 x 4096 x 8192 132 -> 165, 4096 x 2048 x 512 15 -> 20.
+  // memory and from the caches: 2048^3 A:N B:N 34.2 -> 25.0 and 28.4 -> 21.3, A:N B:T 33.0 -> 25.0 and 29.3 -> 21.3, 1024 x 4096 x 4096 61.1 -> 41.7 and
+  // 46.9 -> 34.4; at 11 stages 2048 x 2048 x 704 14.0 -> 12.6 and level; on 512 tiles 2048 x 4096 x 8192 132 -> 165, 4096 x 2048 x 512 15 -> 20.
   if (plan.variant == 1 && stages == kTrDeepStages) {
 #define ZLUDA_TRL_DEEP(PK, QK)                                                                                        \
   if (pkc == PK && qkc == QK)                                                                                        \

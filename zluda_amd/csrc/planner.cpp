@@ -601,11 +601,12 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus, uint64_t workspace_
 // of the better one there):
 //   transposed in registers  4.6 + 1.2 n + (7.5 + 15.3 n) u
 //   by the LDS reads         6.2 + 1.45 n + 2.4 per round behind the first + 27.8 u per round of two on a CU, 17.4 u for one
-// -- level at K = 700 for n = 1, 430 for two, 1200 for three.  (2048 x 2048 x 128: 7.5 us in registers, 9.7 by the LDS reads;
+// -- level at K = 700 for n = 1, 430 for two, 1200 for three.  (Two stages each; the deeper ring that n = 1 has takes less: level at
+// K = 704 from the caches, 10 % ahead there from memory.)  (2048 x 2048 x 128: 7.5 us in registers, 9.7 by the LDS reads;
 // 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 tile is faster by the LDS reads at every K, the 64 x 64 tile beyond one stage in registers
 // (K = 16 and 32: 3 to 9 % slower by the LDS reads, from the caches and from memory; 64 with one operand K-contiguous 4 and 0 %, with none 2 and 5 % faster).
-// (bf16, us from memory: 512 x 512 x 128 5.2 and 4.8, 512^3 7.8 and 6.5, 1024^3 A:N B:T 11.3 and 9.2, 2104 x 704 x 1000 16.7 and 13.7, 64 x 64 x 16384 69 and 47.5; from the caches 4.6 and 4.5,
-// 6.4 and 6.0, 9.1 and 7.6, 11.8 and 10.6, 60 and 47.)  Another exception is
+// (bf16, us from memory: 512 x 512 x 128 5.6 and 5.2, 512^3 7.9 and 6.8, 1024^3 A:N B:T 11.3 and 9.2, 2104 x 704 x 1000 16.9 and 13.8, 64 x 64 x 16384
+// 70 and 48; from the caches 5.0 and 5.1, 6.7 and 6.4, 9.2 and 7.5, 11.9 and 10.7, 61 and 48.)  Another exception is
 // a long operand along its row index beside up to 16 K-contiguous tokens on four to six workgroups per CU: memory bound, and the two-stage ring
 // has less on its way than the registers (us from memory, in registers and by the LDS reads: 65536 x 16 x 512 17.2 and 18.7, x 2048 57 and 61, 14336 x 1 x
 // 4096 in four shares 32.2 and 33.8, x 16 level; x 33 39.3 and 37.5; level at K = 64 and on eight workgroups per CU; up to three of them run
@@ -693,8 +694,8 @@ static const TrCost kTrCost[kNumTrVariants] = {{1, 0.0f, 71.0f}, {2, 26.0f, 11.0
 // tiles, 164 against 130); the others as above.  Around the loop 4 us, and for a split the second kernel and the partial
 // tiles' way through memory at 3 TB/s.  (The variants 1 and 2 by the LDS reads take less than that by now, both alike, and variant 2 is left
 // with its time in registers: over 300 problems of 128 to 4096 rows and columns and K = 128 to 8192 what these pick takes 0.3 % more time than the best
-// variant on average with operands from memory, 1.2 % from the caches; more than 10 % in 2 and 12 of them: 1376 x 448 x 3000 A:N B:T from the caches 22.7 us
-// on 128 x 128 tiles, 14.3 on 64 x 64.)
+// variant on average with operands from memory, 1.3 % from the caches; more than 10 % in 2 and 11 of them: 1376 x 448 x 3000 A:N B:T from the caches 22.5 us
+// on 128 x 128 tiles, 13.7 on 64 x 64.)
 // (1024 x 512 x 1024 on 128x128 would take 20 us split, 64x64 take 10).
 static const TrCost kTrCostLds[kNumTrVariants] = {{1, 0.0f, 71.0f}, {2, 25.0f, 3.3f}, {4, 16.0f, 6.0f}, {1, 0.0f, 53.0f}};
 
