@@ -21,10 +21,12 @@ TOL = {K.CUDA_R_16BF: 1e-2, K.CUDA_R_16F: 2e-3}
 TOL_BEHIND, FLOOR_BEHIND = 12 / 512, 1e-1
 
 
-def run(api, spec, seed, family, variant, ws=4 << 20, block=None, in_epilogue=True, lds=None):
-    """the case, its plan; `in_epilogue`: the kernel does it all, else there is a pass behind it; `lds`: transposed by the LDS reads"""
+def run(api, spec, seed, family, variant, ws=4 << 20, block=None, in_epilogue=True, lds=None, one_rounding=None):
+    """the case, its plan; `in_epilogue`: the kernel does it all, else there is a pass behind it; `lds`: transposed by the LDS reads;
+    `one_rounding`: held to the bounds of a single rounding, which these inputs meet behind some plans as well"""
     import torch
     print("case", spec, "family", family, "variant", variant, flush=True)
+    one_rounding = in_epilogue if one_rounding is None else one_rounding
     case = Case(spec, seed)
     ref = case.run_oracle()
     keep, ptr, dt = case.upload()
@@ -41,8 +43,8 @@ def run(api, spec, seed, family, variant, ws=4 << 20, block=None, in_epilogue=Tr
         assert planner_probe.lds_reads(p, plan, api.zluda_gemm_device_cu_count()) == lds
     assert api.zluda_gemm_launch(C.byref(p), C.byref(plan), torch.cuda.current_stream().cuda_stream) == 0
     torch.cuda.synchronize()
-    case.compare(case.download(dt), ref, tol=TOL[spec["d_type"]] if in_epilogue else TOL_BEHIND,
-                 floor_frac=None if in_epilogue else FLOOR_BEHIND)
+    case.compare(case.download(dt), ref, tol=TOL[spec["d_type"]] if one_rounding else TOL_BEHIND,
+                 floor_frac=None if one_rounding else FLOOR_BEHIND)
     if case.aux_mode == 1:
         case.compare_aux(keep[10][:case.aux.nbytes].cpu().numpy().view(case.aux.dtype).copy(), case.aux_ref)
     if case.bgrad:
@@ -55,9 +57,9 @@ def run(api, spec, seed, family, variant, ws=4 << 20, block=None, in_epilogue=Tr
 
 
 # family, variant, block: 32x32 tiles of every wave shape, 16x16 tiles, the four-wave kernel; the layouts of the transposing kernels (the 64 x 64 tile
-# by the LDS reads, the 128 x 128 tile in registers: K is short)
+# by the LDS reads whatever the block, the 128 x 128 tile in registers: K is short)
 FORMS = [(H16, v, b, 1, 0) for v, b in ((0, 0), (2, 256), (2, 512), (4, 0), (5, 0), (6, 0), (7, 0), (8, 0), (9, 0), (10, 0), (11, 0))] + \
-        [(TR16, v, b, ta, tb) for v, b in ((0, 0), (1, 256), (1, 512), (2, 0), (3, 0)) for ta, tb in ((0, 0), (0, 1), (1, 1))]
+        [(TR16, v, b, ta, tb) for v, b in ((0, 0), (1, 256), (1, 512), (2, 256), (2, 512), (3, 0)) for ta, tb in ((0, 0), (0, 1), (1, 1))]
 
 
 @pytest.mark.parametrize("epi", [AUX, AUX_BIAS, DG, DG_SUMS])
@@ -71,10 +73,9 @@ def test_every_form(gpu_api, family, variant, block, ta, tb, epi):
         if (ta, tb) != (1, 0) and tb:   # (the columns of B lie side by side: a whole number of 16-byte pieces for the LDS reads)
             spec["ldb"] = (n + 7) // 8 * 8
         behind = variant == 0 or (family == H16 and block == 256)   # (wave tiles of 128 x 64 on the 32x32 shapes)
-        if family == H16 and variant == 11 and epi in (DG, DG_SUMS):
-            behind = True   # (the four-wave kernel keeps GELU's input, and has no gradient)
-        run(gpu_api, spec, 9700 + 10 * epi + i, family, variant, block=block, in_epilogue=not behind,
-            lds=None if family == H16 else int(variant in (2, 3)))
+        no_gradient = family == H16 and variant == 11 and epi in (DG, DG_SUMS)   # (the four-wave kernel keeps GELU's input)
+        run(gpu_api, spec, 9700 + 10 * epi + i, family, variant, block=block, in_epilogue=not behind and not no_gradient,
+            lds=None if family == H16 else int(variant in (2, 3)), one_rounding=not behind)
 
 
 # Operands off 16 bytes (pitches of whole dwords) are transposed in registers: 64 x 64 tiles with one group of waves and with two that share K,
@@ -107,7 +108,7 @@ def test_batches_pitches_scales(gpu_api, family, variant, ta, tb):
     base = dict(BF, m=200, n=136, k=264, batch=3, transa=ta, transb=tb, ldd=208, ldc=208, aux_ld=224, aux_batch_stride=224 * 136 + 40)
     run(gpu_api, dict(base, epilogue=AUX_BIAS, bias_type=K.CUDA_R_32F, bias_batch_stride=203), 9801, family, variant)
     run(gpu_api, dict(base, epilogue=AUX_BIAS, bias_batch_stride=203), 9802, family, variant)     # (a bias at odd addresses)
-    run(gpu_api, dict(base, epilogue=DG_SUMS, bias_batch_stride=208), 9803, family, variant, in_epilogue=variant != 11)
+    run(gpu_api, dict(base, epilogue=DG_SUMS, bias_batch_stride=208), 9803, family, variant, in_epilogue=variant != 11, one_rounding=True)
 
 
 @pytest.mark.parametrize("change", [dict(m=260), dict(ldd=268, ldc=268), dict(aux_ld=268), dict(order_c=1, order_d=1, aux_ld=136), dict(with_c=True),
