@@ -604,7 +604,8 @@ static int pick_mfma_variant(const Lowered &l, uint32_t cus, uint64_t workspace_
 // -- level at K = 700 for n = 1, 430 for two, 1200 for three.  (Two stages each; the deeper ring that n = 1 has takes less: level at
 // K = 704 from the caches, 10 % ahead there from memory.)  (2048 x 2048 x 128: 7.5 us in registers, 9.7 by the LDS reads;
 // 3072 x 2048 x 1024: 24.3 and 20.9.)  The 256 x 256 tile is faster by the LDS reads at every K, the 64 x 64 tile beyond one stage in registers
-// (K = 16 and 32: 3 to 9 % slower by the LDS reads, from the caches and from memory; 64 with one operand K-contiguous 4 and 0 %, with none 2 and 5 % faster).
+// (K = 16 and 32: 3 to 9 % slower by the LDS reads, from the caches and from memory; 64 with one operand K-contiguous 4 and 0 %, with none 2 and 5 % faster;
+// 72 to 96 with one 2 to 3 % slower from the caches and 2 to 5 % faster from memory: 2048 x 1024 x 96 A:N B:N 5.20 and 5.34, 6.28 and 5.98).
 // (bf16, us from memory: 512 x 512 x 128 5.6 and 5.2, 512^3 7.9 and 6.8, 1024^3 A:N B:T 11.3 and 9.2, 2104 x 704 x 1000 16.9 and 13.8, 64 x 64 x 16384
 // 70 and 48; from the caches 5.0 and 5.1, 6.7 and 6.4, 9.2 and 7.5, 11.9 and 10.7, 61 and 48.)  Another exception is
 // a long operand along its row index beside up to 16 K-contiguous tokens on four to six workgroups per CU: memory bound, and the two-stage ring
